@@ -20,7 +20,10 @@ LIB = os.path.join(HERE, "libfastnn_hip.so")
 HIP_SOURCES = ["api.hip", "qgemv.hip", "qgemm_generic.hip", "qgemm_tiled.hip", "qgemm_i8.hip", "qgemm_digits.hip", "qgemv_mfma.hip", "qgemv_i8dot.hip", "qgemv_rows16.hip", "i8act.hip", "qconv.hip", "qconv_float.hip", "qconv_implicit.hip", "eltwise.hip",
                "qgemm_stream.hip", "qgemm_stream_i8.hip", "qgemm_stream_i4.hip", "qgemm_stream_u4.hip", "qgemm_stream_u8.hip",
                "qgemm_stream_f8.hip", "qgemm_stream_f8r.hip", "qgemm_stream_f4.hip", "qgemm_stream_i4cb.hip"]
-HOST_SOURCES = ["quantize_host.cpp", "hip_backend.cpp"]
+HOST_SOURCES = ["quantize_host.cpp", "quantize_simd_avx512.cpp", "quantize_simd_avx2.cpp", "quantize_simd_base.cpp", "host_pool.cpp", "hip_backend.cpp"]
+# the weight packers are compiled once per instruction set and chosen at run time
+SOURCE_FLAGS = {"quantize_simd_avx512.cpp": ["-O3", "-mavx512f", "-mavx512bw", "-mavx512dq", "-mavx512vl", "-mprefer-vector-width=512"],
+                "quantize_simd_avx2.cpp": ["-O3", "-mavx2", "-Wno-psabi"], "quantize_simd_base.cpp": ["-O3", "-Wno-psabi"]}
 
 # -ffp-contract=off: the integer/quantisation formulas must evaluate exactly as written;
 # hot loops ask for fused multiply-adds explicitly.  Packed-FP32 instructions are disabled.
@@ -73,7 +76,7 @@ def build(force: bool = False, verbose: bool = False) -> str:
         o = os.path.join(OBJ, src + ".o")
         objs.append(o)
         if force or _stale(o, [s] + headers):
-            jobs.append(["g++"] + HOST_FLAGS + ["-I/opt/rocm/include", "-D__HIP_PLATFORM_AMD__", "-c", s, "-o", o])
+            jobs.append(["g++"] + HOST_FLAGS + SOURCE_FLAGS.get(src, []) + ["-I/opt/rocm/include", "-D__HIP_PLATFORM_AMD__", "-c", s, "-o", o])
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs)))) as ex:
         for out in ex.map(_run, jobs):
             if verbose and out.strip():

@@ -4,17 +4,22 @@
 // fastnn's: strict binary32 arithmetic in the reference's evaluation order (this file is
 // compiled with FMA contraction off); only order-independent work is spread over threads.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
-#include <thread>
+#include <memory>
+#include <new>
 #include <vector>
 
 #include "../../include/fastnn_hip.h"
+#include "host_pool.h"
+#include "quantize_simd.h"
 
 namespace {
 
 constexpr size_t kMargin = 16;  // SIMD_MARGIN words after the last row (src/packed_tensor.rs:980-982)
+constexpr int64_t kPanel = 32;  // channels a packing task takes at a time
 
 inline int lanes_of(int dt)
 {
@@ -25,226 +30,160 @@ inline int lanes_of(int dt)
     }
 }
 
-inline float clamp_keep_nan(float x, float lo, float hi) { return x < lo ? lo : (x > hi ? hi : x); }
-
-// `as iN` after clamp+round: value already in range, NaN becomes 0
-inline int32_t to_int(float f) { return std::isnan(f) ? 0 : (int32_t)f; }
-
-// ---- single-lane encoders (pack_from_f32 of each PackedWord) -----------------------
-
-struct EncI8 {  // src/dtypes/i8x4.rs:34-43
-    static constexpr int kBits = 8;
-    static uint32_t enc(float v) { return (uint32_t)(uint8_t)(int8_t)to_int(std::round(clamp_keep_nan(v, -128.f, 127.f))); }
-};
-struct EncI4 {  // src/dtypes/i4x8.rs:34-42
-    static constexpr int kBits = 4;
-    static uint32_t enc(float v) { return (uint32_t)(uint8_t)(int8_t)to_int(std::round(clamp_keep_nan(v, -8.f, 7.f))) & 0xFu; }
-};
-struct EncU8 {  // src/dtypes/u8x4.rs:33-40
-    static constexpr int kBits = 8;
-    static uint32_t enc(float v) { return (uint32_t)to_int(std::round(clamp_keep_nan(v, 0.f, 255.f))) & 0xFFu; }
-};
-struct EncU4 {  // src/dtypes/u4x8.rs:34-41
-    static constexpr int kBits = 4;
-    static uint32_t enc(float v) { return (uint32_t)to_int(std::round(clamp_keep_nan(v, 0.f, 15.f))) & 0xFu; }
-};
-
-// Minifloat encoder shared by E4M3 (src/dtypes/f8x4.rs:41-77) and E5M2
-// (src/dtypes/f8x4r.rs:48-88): mantissa rounded half away from zero, carry into the
-// exponent, saturation at `max_code`, subnormals scaled by `sub_mul`.
-template <int MBITS, int BIAS, int EMAX>
-uint32_t enc_minifloat(float v, float max_val, float sub_limit, float sub_mul, uint32_t max_code, bool has_inf)
+const FnnQuantKernels &kernels()
 {
-    if (std::isnan(v)) return 0x7F;
-    const uint32_t sign = (v < 0.0f) ? 0x80u : 0u;
-    float a = std::fabs(v);
-    if (a == 0.0f) return std::signbit(v) ? 0x80u : 0u;
-    if (has_inf && std::isinf(v)) return v > 0.0f ? 0x7Cu : 0xFCu;
-    a = std::min(a, max_val);
-    constexpr int MONE = 1 << MBITS;
-    if (a < sub_limit) {
-        float r = std::round(a * sub_mul);
-        int m = r >= 255.0f ? 255 : (int)r;
-        if (m >= MONE) return sign | (uint32_t)MONE;
-        return sign | (uint32_t)m;
-    }
-    int ex;
-    (void)std::frexp(a, &ex);
-    const int e = ex - 1;  // floor(log2 a); see the oracle's note on why this equals log2().floor() here
-    const int biased = e + BIAS;
-    const float normalized = a / std::ldexp(1.0f, e);
-    float r = std::round((normalized - 1.0f) * (float)MONE);
-    int mant = std::isnan(r) ? 0 : (r <= 0.0f ? 0 : (r >= 255.0f ? 255 : (int)r));
-    if (mant >= MONE) {
-        const int nb = biased + 1;
-        if (nb >= EMAX) return sign | max_code;
-        return sign | (uint32_t)(nb << MBITS);
-    }
-    if (biased >= EMAX) return sign | max_code;
-    return sign | (uint32_t)(biased << MBITS) | (uint32_t)mant;
+    static const FnnQuantKernels &k = __builtin_cpu_supports("avx512f") && __builtin_cpu_supports("avx512bw") && __builtin_cpu_supports("avx512dq") && __builtin_cpu_supports("avx512vl")
+                                          ? fnn_quant_avx512
+                                          : (__builtin_cpu_supports("avx2") ? fnn_quant_avx2 : fnn_quant_base);
+    return k;
 }
 
-struct EncF8 {
-    static constexpr int kBits = 8;
-    static uint32_t enc(float v) { return enc_minifloat<3, 7, 15>(v, 240.0f, 0.015625f, 512.0f, 0x7Bu, false); }
-};
-struct EncF8R {
-    static constexpr int kBits = 8;
-    static uint32_t enc(float v) { return enc_minifloat<2, 15, 31>(v, 57344.0f, 1.0f / 16384.0f, 16384.0f, 0x7Cu, true); }
-};
-struct EncF4 {  // src/dtypes/f4x8.rs:49-70
-    static constexpr int kBits = 4;
-    static uint32_t enc(float v)
+int threads_for(int64_t elements) { return elements < (1 << 16) ? 1 : fnn_host_threads(); }
+
+// A task's working copy of a panel (inner x 32 floats), kept by its thread up to 4 MB so that no call pays for fresh pages.
+struct PanelBuffer {
+    std::unique_ptr<float[]> own;
+    size_t cap = 0;
+    float *get(size_t n)
     {
-        static const float mag[8] = {0.0f, 0.5f, 1.0f, 1.5f, 2.0f, 3.0f, 4.0f, 6.0f};
-        if (std::isnan(v)) return 0;
-        const float a = std::fabs(v);
-        uint32_t best = 0;
-        float best_d = a;
-        for (uint32_t i = 0; i < 8; i++) {
-            const float d = std::fabs(a - mag[i]);
-            if (d < best_d) { best_d = d; best = i; }
-        }
-        return (std::signbit(v) && best != 0) ? (best | 0x8u) : best;
+        if (n > cap) { own.reset(); own.reset(new float[n]); cap = n; }
+        return own.get();
     }
+    void done() { if (cap > (1u << 20)) { own.reset(); cap = 0; } }
 };
+thread_local PanelBuffer t_panel;
 
-// Pack one row: lane value f(x); lanes past the row end are the value 0.0
-// (src/packed_tensor.rs:993-1003).
-template <class Enc, class F>
-void pack_row(const float *row, int64_t inner, uint32_t *dst, F f)
+// Per-channel packing of an [inner, rows] matrix (kn: channels along the fast axis, as a graph holds a MatMul weight: a
+// panel is read where it lies) or of its transpose (each panel is turned first).  src/packed_tensor.rs:661-742, 852-1049.
+// A [4096, 11008] matrix to 4-bit words on 16 EPYC threads: 251 ms as a serial transpose followed by scalar packing,
+// 1.2 ms in this form (169 GB/s of floats read, the host memory's rate).
+bool quant_per_channel(int dtype, const float *w, int64_t rows, int64_t inner, bool kn, uint32_t *words, float *scales, float *zeros)
 {
-    constexpr int items = 32 / Enc::kBits;
+    const FnnQuantKernels &kern = kernels();
+    const int items = lanes_of(dtype);
     const int64_t kp = (inner + items - 1) / items;
-    for (int64_t wd = 0; wd < kp; wd++) {
-        uint32_t w = 0;
-        for (int i = 0; i < items; i++) {
-            const int64_t e = wd * items + i;
-            const float lane = (e < inner) ? f(row[e]) : 0.0f;
-            w |= Enc::enc(lane) << (Enc::kBits * i);
-        }
-        dst[wd] = w;
-    }
-}
-
-template <class Fn>
-void parallel_rows(int64_t rows, int64_t work_per_row, Fn fn)
-{
-    unsigned hw = std::thread::hardware_concurrency();
-    int64_t nt = hw ? (int64_t)hw : 4;
-    if (nt > 16) nt = 16;
-    if (rows * work_per_row < (1 << 18)) nt = 1;
-    if (nt > rows) nt = rows > 0 ? rows : 1;
-    if (nt <= 1) { fn(0, rows); return; }
-    std::vector<std::thread> th;
-    const int64_t per = (rows + nt - 1) / nt;
-    for (int64_t t = 0; t < nt; t++) {
-        const int64_t r0 = t * per, r1 = std::min(rows, r0 + per);
-        if (r0 >= r1) break;
-        th.emplace_back([=] { fn(r0, r1); });
-    }
-    for (auto &t : th) t.join();
-}
-
-// from_f32_per_channel_asymmetric, group_size 0 (src/packed_tensor.rs:852-1049)
-template <class Enc, bool FP4>
-void quant_asym(const float *w, int64_t rows, int64_t inner, uint32_t *words, float *scales, float *zeros)
-{
-    constexpr int items = 32 / Enc::kBits;
-    const int64_t kp = (inner + items - 1) / items;
-    const float umax = (float)((1u << Enc::kBits) - 1u);
-    const float sbias = (float)(1u << (Enc::kBits - 1));
-    parallel_rows(rows, inner, [=](int64_t r0, int64_t r1) {
-        for (int64_t r = r0; r < r1; r++) {
-            const float *row = w + r * inner;
-            float mn = 3.40282347e+38f, mx = -3.40282347e+38f;
-            for (int64_t i = 0; i < inner; i++) { mn = std::fmin(mn, row[i]); mx = std::fmax(mx, row[i]); }
-            const float range = mx - mn;
-            float scale, zero;
-            if (range == 0.0f) {
-                scale = 1.0f; zero = 0.0f;
-            } else if (FP4) {
-                float sum = 0.0f;
-                for (int64_t i = 0; i < inner; i++) sum += row[i];
-                const float mean = sum / (float)inner;
-                const float dev = std::fmax(std::fabs(mean - mn), std::fabs(mx - mean));
-                scale = (dev == 0.0f ? 1e-10f : dev) / 4.0f;
-                zero = mean;
+    std::atomic<bool> ok{true};
+    fnn_parallel((rows + kPanel - 1) / kPanel, threads_for(rows * inner), [&](int64_t p) {
+        const int64_t r0 = p * kPanel;
+        const int have = (int)std::min(kPanel, rows - r0);
+        const float *src = w + r0;
+        int64_t ld = rows;
+        if (!kn || have < kPanel) {
+            float *buf;
+            try { buf = t_panel.get((size_t)inner * kPanel); } catch (const std::bad_alloc &) { ok = false; return; }
+            if (kn) {
+                for (int64_t k = 0; k < inner; k++) {
+                    std::memcpy(buf + k * kPanel, w + k * rows + r0, (size_t)have * 4);
+                    std::memset(buf + k * kPanel + have, 0, (size_t)(kPanel - have) * 4);
+                }
             } else {
-                const float init = range / umax;
-                const float lo = mn - init, hi = mx + init;
-                scale = (hi - lo) / umax;
-                zero = lo + sbias * scale;
+                kern.panel_from_rows(w + r0 * inner, inner, have, buf);
             }
-            scales[r] = scale;
-            zeros[r] = zero;
-            const float inv = (scale != 0.0f) ? 1.0f / scale : 0.0f;
-            pack_row<Enc>(row, inner, words + r * kp, [=](float x) { return (x - zero) * inv; });
+            src = buf;
+            ld = kPanel;
         }
+        kern.quant_panel(dtype, src, ld, inner, have, words + r0 * kp, kp, scales + r0, zeros + r0);
+        t_panel.done();
     });
+    return ok;
 }
 
-// from_f32_per_channel (src/packed_tensor.rs:661-742)
-template <class Enc>
-void quant_sym(const float *w, int64_t rows, int64_t inner, float max_val, uint32_t *words, float *scales, float *zeros)
-{
-    constexpr int items = 32 / Enc::kBits;
-    const int64_t kp = (inner + items - 1) / items;
-    parallel_rows(rows, inner, [=](int64_t r0, int64_t r1) {
-        for (int64_t r = r0; r < r1; r++) {
-            const float *row = w + r * inner;
-            float max_abs = 0.0f;
-            for (int64_t i = 0; i < inner; i++) max_abs = std::fmax(max_abs, std::fabs(row[i]));
-            const float scale = (max_abs == 0.0f) ? 1.0f : max_abs / max_val;
-            scales[r] = scale;
-            zeros[r] = 0.0f;
-            const float inv = (scale != 1.0f) ? 1.0f / scale : 1.0f;
-            pack_row<Enc>(row, inner, words + r * kp, [=](float x) { return x * inv; });
-        }
-    });
-}
+// ---- codebook
 
-inline uint32_t nearest16(float v, const float *cb)
+constexpr int64_t kChunk = 1 << 14;   // values of one task of the flat passes
+
+// The values at 16 positions of the stable ascending order of `vals` (-0.0 and +0.0 are equal there and keep the order
+// they came in).  Histogram of the upper 16 bits of the order-preserving integer image, then a selection inside the
+// buckets that hold the positions: what a full sort gives at these positions (1 M values: 75 ms sorted, 2 ms here).
+void order_statistics(const std::vector<float> &vals, const size_t *at, float *out)
 {
-    float best_d = std::fabs(v - cb[0]);
-    uint32_t best = 0;
-    for (uint32_t i = 1; i < 16; i++) {
-        const float d = std::fabs(v - cb[i]);
-        if (d < best_d) { best_d = d; best = i; }
+    const int64_t n = (int64_t)vals.size();
+    auto key = [](float f) -> uint32_t {
+        uint32_t u;
+        std::memcpy(&u, &f, 4);
+        if ((u << 1) == 0) u = 0;
+        return u & 0x80000000u ? ~u : u | 0x80000000u;
+    };
+    const int threads = threads_for(n);
+    std::vector<std::vector<uint32_t>> part((size_t)threads, std::vector<uint32_t>(1 << 16, 0));
+    const int64_t per = (n + threads - 1) / threads;
+    fnn_parallel(threads, threads, [&](int64_t t) {
+        for (int64_t i = t * per; i < std::min(n, (t + 1) * per); i++) part[(size_t)t][key(vals[(size_t)i]) >> 16]++;
+    });
+    std::vector<uint64_t> before((1 << 16) + 1, 0);
+    for (size_t b = 0; b < 1 << 16; b++) {
+        uint64_t c = 0;
+        for (auto &p : part) c += p[b];
+        before[b + 1] = before[b] + c;
     }
-    return best;
+    uint32_t bucket[16];
+    for (int j = 0; j < 16; j++)
+        bucket[j] = (uint32_t)(std::upper_bound(before.begin(), before.end(), (uint64_t)at[j]) - before.begin() - 1);
+    std::vector<std::vector<uint32_t>> found(16);
+    std::vector<uint8_t> slot(1 << 16, 255);
+    for (int j = 0; j < 16; j++) if (slot[bucket[j]] == 255) slot[bucket[j]] = (uint8_t)j;
+    for (int j = 0; j < 16; j++) if (slot[bucket[j]] == j) found[(size_t)j].reserve(before[bucket[j] + 1] - before[bucket[j]]);
+    for (float v : vals) {
+        const uint32_t k = key(v);
+        if (const uint8_t s = slot[k >> 16]; s != 255) found[s].push_back(k);
+    }
+    for (int j = 0; j < 16; j++) {
+        std::vector<uint32_t> &f = found[slot[bucket[j]]];
+        const size_t pos = at[j] - before[bucket[j]];
+        std::nth_element(f.begin(), f.begin() + (ptrdiff_t)pos, f.end());
+        const uint32_t k = f[pos], u = k & 0x80000000u ? k & 0x7fffffffu : ~k;
+        std::memcpy(&out[j], &u, 4);
+        if (out[j] == 0.0f) {   // which of the zeros, in the order they came
+            size_t below = 0, nth = 0;
+            for (float v : vals) below += v < 0.0f;
+            for (float v : vals)
+                if (v == 0.0f && nth++ == at[j] - below) { out[j] = v; break; }
+        }
+    }
 }
 
-// kmeans_16 (src/packed_tensor.rs:18-75).  The assignment step is independent per value
-// and runs on threads; the f32 cluster sums must follow data order and stay sequential.
+// kmeans_16 (src/packed_tensor.rs:18-75).  The assignment is independent per value; the f32 sum of a cluster must follow
+// data order: the chunks are grouped by cluster side by side, then one task per cluster adds its runs chunk after chunk
+// (bound by the latency of n / 16 dependent additions).
 bool kmeans16(const std::vector<float> &vals, int iters, float *c)
 {
+    const FnnQuantKernels &kern = kernels();
     const size_t n = vals.size();
     std::fill(c, c + 16, 0.0f);
     if (n == 0) return true;
     if (n == 1) { std::fill(c, c + 16, vals[0]); return true; }
     for (float v : vals) if (std::isnan(v)) return false;  // the reference panics on NaN
     {
-        std::vector<float> sorted(vals);
-        // stable, with -0.0 == +0.0, like sort_by(partial_cmp)
-        std::stable_sort(sorted.begin(), sorted.end(), [](float a, float b) { return a < b; });
+        size_t at[16];
         for (int i = 0; i < 16; i++) {
             const float pct = ((float)i + 0.5f) / 16.0f;
-            size_t idx = (size_t)(pct * (float)n);
-            c[i] = sorted[std::min(idx, n - 1)];
+            at[i] = std::min((size_t)(pct * (float)n), n - 1);
         }
+        order_statistics(vals, at, c);
     }
+    const int threads = threads_for((int64_t)n);
+    const int64_t chunks = ((int64_t)n + kChunk - 1) / kChunk;
     std::vector<uint8_t> assign(n);
+    std::vector<float> grouped(n);
+    std::vector<int32_t> start((size_t)chunks * 17);
     for (int it = 0; it < iters; it++) {
         float cc[16];
         std::memcpy(cc, c, sizeof(cc));
-        parallel_rows((int64_t)n, 16, [&](int64_t i0, int64_t i1) {
-            for (int64_t i = i0; i < i1; i++) assign[(size_t)i] = (uint8_t)nearest16(vals[(size_t)i], cc);
+        fnn_parallel(chunks, threads, [&](int64_t t) {
+            const int64_t i0 = t * kChunk;
+            kern.group16(vals.data() + i0, std::min(kChunk, (int64_t)n - i0), cc, assign.data() + i0, grouped.data() + i0, &start[(size_t)t * 17]);
         });
-        size_t counts[16] = {0};
-        float sums[16] = {0};
-        for (size_t i = 0; i < n; i++) { counts[assign[i]]++; sums[assign[i]] += vals[i]; }
-        for (int k = 0; k < 16; k++) if (counts[k] > 0) c[k] = sums[k] / (float)counts[k];
+        fnn_parallel(16, threads, [&](int64_t k) {
+            float sum = 0.0f;
+            size_t count = 0;
+            for (int64_t t = 0; t < chunks; t++) {
+                const int32_t s0 = start[(size_t)(t * 17 + k)], s1 = start[(size_t)(t * 17 + k + 1)];
+                const float *g = grouped.data() + t * kChunk;
+                for (int32_t i = s0; i < s1; i++) sum += g[i];
+                count += (size_t)(s1 - s0);
+            }
+            if (count > 0) c[k] = sum / (float)count;
+        });
     }
     std::stable_sort(c, c + 16, [](float a, float b) { return a < b; });
     return true;
@@ -253,42 +192,70 @@ bool kmeans16(const std::vector<float> &vals, int iters, float *c)
 // from_f32_per_block_codebook (src/packed_tensor.rs:1209-1313)
 int quant_codebook(const float *w, int64_t rows, int64_t inner, int64_t qb, uint32_t *words, float *bscales, float *cb)
 {
+    const FnnQuantKernels &kern = kernels();
     const int64_t bpr = (inner + qb - 1) / qb, kp = (inner + 7) / 8;
+    const int threads = threads_for(rows * inner);
     std::vector<float> norm((size_t)(rows * inner));
-    parallel_rows(rows, inner, [&](int64_t r0, int64_t r1) {
-        for (int64_t r = r0; r < r1; r++)
-            for (int64_t b = 0; b < bpr; b++) {
-                const int64_t base = r * inner + b * qb, end = std::min(base + qb, (r + 1) * inner);
-                float mx = 0.0f;
-                for (int64_t i = base; i < end; i++) mx = std::fmax(mx, std::fabs(w[i]));
-                bscales[r * bpr + b] = mx;
-                if (mx > 0.0f) {
-                    const float inv = 1.0f / mx;
-                    for (int64_t i = base; i < end; i++) norm[(size_t)i] = w[i] * inv;
-                } else {
-                    for (int64_t i = base; i < end; i++) norm[(size_t)i] = 0.0f;
-                }
+    fnn_parallel(rows, threads, [&](int64_t r) {
+        for (int64_t b = 0; b < bpr; b++) {
+            const int64_t base = r * inner + b * qb, end = std::min(base + qb, (r + 1) * inner);
+            float mx = 0.0f;
+            for (int64_t i = base; i < end; i++) mx = std::fmax(mx, std::fabs(w[i]));
+            bscales[r * bpr + b] = mx;
+            if (mx > 0.0f) {
+                const float inv = 1.0f / mx;
+                for (int64_t i = base; i < end; i++) norm[(size_t)i] = w[i] * inv;
+            } else {
+                for (int64_t i = base; i < end; i++) norm[(size_t)i] = 0.0f;
             }
+        }
     });
     // block order of the reference's normalised list == element order (blocks tile each row)
     if (!kmeans16(norm, 30, cb)) return FNN_ERR_COMPILATION;
-    parallel_rows(rows, inner, [&](int64_t r0, int64_t r1) {
-        for (int64_t r = r0; r < r1; r++)
-            for (int64_t b = 0; b < bpr; b++) {
-                const float s = bscales[r * bpr + b];
-                const float inv = s > 0.0f ? 1.0f / s : 0.0f;
-                const int64_t base = r * inner + b * qb, end = std::min(base + qb, (r + 1) * inner);
-                for (int64_t eb = 0; eb < end - base; eb += 8) {
-                    uint32_t word = 0;
-                    for (int i = 0; i < 8; i++) {
-                        const int64_t e = base + eb + i;
-                        if (e < end) word |= nearest16(w[e] * inv, cb) << (4 * i);
-                    }
-                    words[r * kp + (b * qb + eb) / 8] = word;  // a straddling word keeps the later block's value
+    std::vector<uint8_t> index((size_t)(rows * inner));
+    fnn_parallel(rows, threads, [&](int64_t r) {
+        for (int64_t b = 0; b < bpr; b++) {
+            const float s = bscales[r * bpr + b];
+            const float inv = s > 0.0f ? 1.0f / s : 0.0f;
+            const int64_t base = r * inner + b * qb, end = std::min(base + qb, (r + 1) * inner);
+            for (int64_t i = base; i < end; i++) norm[(size_t)i] = w[i] * inv;
+        }
+        kern.nearest16(norm.data() + r * inner, inner, cb, index.data() + r * inner);
+        for (int64_t b = 0; b < bpr; b++) {
+            const int64_t base = r * inner + b * qb, end = std::min(base + qb, (r + 1) * inner);
+            for (int64_t eb = 0; eb < end - base; eb += 8) {
+                uint32_t word = 0;
+                for (int i = 0; i < 8; i++) {
+                    const int64_t e = base + eb + i;
+                    if (e < end) word |= (uint32_t)index[(size_t)e] << (4 * i);
                 }
+                words[r * kp + (b * qb + eb) / 8] = word;  // a straddling word keeps the later block's value
             }
+        }
     });
     return FNN_OK;
+}
+
+int quantize(int dtype, const float *w, int64_t rows, int64_t inner, bool kn, int qblock, uint32_t *words, float *scales,
+             float *zeros, float *codebook16)
+{
+    const int items = lanes_of(dtype);
+    if (!items || !w || !words || !scales || rows <= 0 || inner <= 0) return FNN_ERR_COMPILATION;
+    if (dtype != FNN_DT_I4CB) {
+        if (!zeros) return FNN_ERR_COMPILATION;
+        std::memset(words + rows * ((inner + items - 1) / items), 0, kMargin * sizeof(uint32_t));
+        return quant_per_channel(dtype, w, rows, inner, kn, words, scales, zeros) ? FNN_OK : FNN_ERR_MEMORY;
+    }
+    if (qblock <= 0 || !codebook16) return FNN_ERR_COMPILATION;
+    try {
+        std::memset(words, 0, fnn_packed_words(dtype, rows, inner) * sizeof(uint32_t));   // (short blocks leave words out)
+        if (!kn) return quant_codebook(w, rows, inner, qblock, words, scales, codebook16);
+        std::unique_ptr<float[]> t(new float[(size_t)(rows * inner)]);
+        fnn_transpose_kn_to_nk(w, inner, rows, t.get());
+        return quant_codebook(t.get(), rows, inner, qblock, words, scales, codebook16);
+    } catch (const std::bad_alloc &) {
+        return FNN_ERR_MEMORY;
+    }
 }
 
 }  // namespace
@@ -305,32 +272,24 @@ size_t fnn_packed_words(int dtype, int64_t rows, int64_t inner)
 void fnn_transpose_kn_to_nk(const float *w_kn, int64_t k, int64_t n, float *w_nk)
 {
     constexpr int64_t T = 32;
-    for (int64_t k0 = 0; k0 < k; k0 += T)
-        for (int64_t n0 = 0; n0 < n; n0 += T)
-            for (int64_t kk = k0; kk < std::min(k, k0 + T); kk++)
-                for (int64_t nn = n0; nn < std::min(n, n0 + T); nn++) w_nk[nn * k + kk] = w_kn[kk * n + nn];
+    fnn_parallel((n + T - 1) / T, threads_for(k * n), [&](int64_t t) {
+        const int64_t n0 = t * T, n1 = std::min(n, n0 + T);
+        for (int64_t k0 = 0; k0 < k; k0 += T)
+            for (int64_t nn = n0; nn < n1; nn++)
+                for (int64_t kk = k0; kk < std::min(k, k0 + T); kk++) w_nk[nn * k + kk] = w_kn[kk * n + nn];
+    });
 }
 
 int fnn_quantize_weights(int dtype, const float *w, int64_t rows, int64_t inner, int qblock,
                          uint32_t *words, float *scales, float *zeros, float *codebook16)
 {
-    const int items = lanes_of(dtype);
-    if (!items || !w || !words || !scales || rows <= 0 || inner <= 0) return FNN_ERR_COMPILATION;
-    if (dtype != FNN_DT_I4CB && !zeros) return FNN_ERR_COMPILATION;
-    std::memset(words, 0, fnn_packed_words(dtype, rows, inner) * sizeof(uint32_t));
-    switch (dtype) {
-    case FNN_DT_I8: quant_asym<EncI8, false>(w, rows, inner, words, scales, zeros); return FNN_OK;
-    case FNN_DT_I4: quant_asym<EncI4, false>(w, rows, inner, words, scales, zeros); return FNN_OK;
-    case FNN_DT_U8: quant_asym<EncU8, false>(w, rows, inner, words, scales, zeros); return FNN_OK;
-    case FNN_DT_U4: quant_asym<EncU4, false>(w, rows, inner, words, scales, zeros); return FNN_OK;
-    case FNN_DT_F4: quant_asym<EncF4, true>(w, rows, inner, words, scales, zeros); return FNN_OK;
-    case FNN_DT_F8: quant_sym<EncF8>(w, rows, inner, 240.0f, words, scales, zeros); return FNN_OK;
-    case FNN_DT_F8R: quant_sym<EncF8R>(w, rows, inner, 57344.0f, words, scales, zeros); return FNN_OK;
-    case FNN_DT_I4CB:
-        if (qblock <= 0 || !codebook16) return FNN_ERR_COMPILATION;
-        return quant_codebook(w, rows, inner, qblock, words, scales, codebook16);
-    default: return FNN_ERR_COMPILATION;
-    }
+    return quantize(dtype, w, rows, inner, false, qblock, words, scales, zeros, codebook16);
+}
+
+int fnn_quantize_weights_kn(int dtype, const float *w_kn, int64_t k, int64_t n, int qblock,
+                            uint32_t *words, float *scales, float *zeros, float *codebook16)
+{
+    return quantize(dtype, w_kn, n, k, true, qblock, words, scales, zeros, codebook16);
 }
 
 }  // extern "C"

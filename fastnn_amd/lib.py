@@ -58,7 +58,7 @@ EXPORTED_SYMBOLS = [
     "fnn_hip_timer_start", "fnn_hip_timer_stop",
     "fnn_hip_graph_begin", "fnn_hip_graph_end", "fnn_hip_graph_launch", "fnn_hip_graph_destroy",
     "fnn_hip_workspace_epoch",
-    "fnn_packed_words", "fnn_quantize_weights", "fnn_transpose_kn_to_nk", "fnn_hip_version",
+    "fnn_packed_words", "fnn_quantize_weights", "fnn_quantize_weights_kn", "fnn_transpose_kn_to_nk", "fnn_hip_version",
 ]
 # every symbol include/fastnn_hip_backend.h declares
 BACKEND_SYMBOLS = [
@@ -170,6 +170,7 @@ def _prototype(l):
     l.fnn_packed_words.argtypes = [C.c_int, _i64, _i64]
     l.fnn_packed_words.restype = _sz
     l.fnn_quantize_weights.argtypes = [C.c_int, _vp, _i64, _i64, C.c_int, _vp, _vp, _vp, _vp]
+    l.fnn_quantize_weights_kn.argtypes = [C.c_int, _vp, _i64, _i64, C.c_int, _vp, _vp, _vp, _vp]
     l.fnn_transpose_kn_to_nk.argtypes = [_vp, _i64, _i64, _vp]
     l.fnn_transpose_kn_to_nk.restype = None
     l.fnn_hip_version.restype = C.c_char_p
@@ -260,39 +261,37 @@ class PackedWeight:
         return self.rows * (-(-self.inner // items)) * 4
 
 
-def quantize_weights(dtype: int, w_nk: np.ndarray, qblock: int = 32) -> PackedWeight:
-    """Quantise a transposed [N,K] f32 matrix with fastnn's packer for `dtype` (host, no GPU)."""
-    l = load_library()
-    w = np.ascontiguousarray(w_nk, dtype=np.float32)
-    if w.ndim != 2:
-        raise FnnError(4, "quantize_weights expects a 2-D [N,K] matrix")
-    rows, inner = w.shape
-    words = np.zeros(l.fnn_packed_words(dtype, rows, inner), np.uint32)
+def _quantize(dtype: int, w: np.ndarray, rows: int, inner: int, qblock: int, entry) -> PackedWeight:
+    words = np.empty(load_library().fnn_packed_words(dtype, rows, inner), np.uint32)
     if dtype == DT_I4CB:
-        bpr = -(-inner // qblock)
-        scales = np.zeros(rows * bpr, np.float32)
+        scales = np.zeros(rows * (-(-inner // qblock)), np.float32)
         zeros = np.zeros(0, np.float32)
         cb = np.zeros(16, np.float32)
     else:
-        scales = np.zeros(rows, np.float32)
-        zeros = np.zeros(rows, np.float32)
+        scales = np.empty(rows, np.float32)
+        zeros = np.empty(rows, np.float32)
         cb = None
-    rc = l.fnn_quantize_weights(dtype, _np_ptr(w), rows, inner, qblock if dtype == DT_I4CB else 0,
-                                _np_ptr(words), _np_ptr(scales), _np_ptr(zeros) if zeros.size else None,
-                                _np_ptr(cb))
+    qb = qblock if dtype == DT_I4CB else 0
+    rc = entry(dtype, _np_ptr(w), w.shape[0], w.shape[1], qb, _np_ptr(words), _np_ptr(scales), _np_ptr(zeros) if zeros.size else None,
+               _np_ptr(cb))
     if rc:
         raise FnnError(rc, f"fnn_quantize_weights failed for dtype {dtype} (NaN in a codebook weight?)")
-    return PackedWeight(dtype, rows, inner, words, scales, zeros, qblock if dtype == DT_I4CB else 0, cb)
+    return PackedWeight(dtype, rows, inner, words, scales, zeros, qb, cb)
+
+
+def quantize_weights(dtype: int, w_nk: np.ndarray, qblock: int = 32) -> PackedWeight:
+    """Quantise a transposed [N,K] f32 matrix with fastnn's packer for `dtype` (host, no GPU)."""
+    w = np.ascontiguousarray(w_nk, dtype=np.float32)
+    if w.ndim != 2:
+        raise FnnError(4, "quantize_weights expects a 2-D [N,K] matrix")
+    return _quantize(dtype, w, w.shape[0], w.shape[1], qblock, load_library().fnn_quantize_weights)
 
 
 def quantize_weights_kn(dtype: int, w_kn: np.ndarray, qblock: int = 32) -> PackedWeight:
-    """Logical [K,N] weight (as a graph holds it) -> transposed -> packed [N,K]."""
-    l = load_library()
+    """Logical [K,N] weight (as a graph holds it) -> packed [N,K]."""
     w = np.ascontiguousarray(w_kn, dtype=np.float32)
     k, n = w.shape
-    t = np.empty((n, k), np.float32)
-    l.fnn_transpose_kn_to_nk(_np_ptr(w), k, n, _np_ptr(t))
-    return quantize_weights(dtype, t, qblock)
+    return _quantize(dtype, w, n, k, qblock, load_library().fnn_quantize_weights_kn)
 
 
 class DeviceBuffer:

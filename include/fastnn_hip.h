@@ -312,6 +312,10 @@ size_t fnn_packed_words(int dtype, int64_t rows, int64_t inner);
 int fnn_quantize_weights(int dtype, const float *w_nk, int64_t rows, int64_t inner,
                          int quant_block_size, uint32_t *words, float *scales, float *zeros,
                          float *codebook16);
+/* The same for a [K,N] matrix as a graph holds it: transpose and packing in one pass over the matrix. */
+int fnn_quantize_weights_kn(int dtype, const float *w_kn, int64_t k, int64_t n,
+                            int quant_block_size, uint32_t *words, float *scales, float *zeros,
+                            float *codebook16);
 /* [K,N] -> [N,K] (quantization.rs:144-156) */
 void fnn_transpose_kn_to_nk(const float *w_kn, int64_t k, int64_t n, float *w_nk);
 
