@@ -532,6 +532,7 @@ class AotExecutor:
 
     def forward(self, inputs: Dict[str, np.ndarray]) -> Dict[str, np.ndarray]:
         self._ensure_plan()
+        ins = []
         for name in self.input_names:
             if name not in inputs:
                 raise FnnError(1, f"forward: missing input '{name}'")
@@ -539,12 +540,11 @@ class AotExecutor:
             x = np.ascontiguousarray(inputs[name], dtype=np.float32)
             if x.shape != v.shape:
                 raise FnnError(1, f"forward: input '{name}' has shape {x.shape}, compiled for {v.shape}")
-            self._backend.write_arena(v.slot[0], x)
-        self._backend.dispatch(self._plan)
+            ins.append((v.slot[0], x))
         out = {}
         for name in self.output_names:
-            v = self._values[name]
-            out[name] = self._backend.read_arena(*v.slot, np.float32).reshape(v.shape).copy()
+            out[name] = _l.result_array(self._values[name].shape)
+        self._backend.forward(self._plan, ins, [(self._values[name].slot[0], y) for name, y in out.items()])
         return out
 
     def set_option(self, option: int, value: int):
@@ -577,7 +577,7 @@ class AotExecutor:
         if name in self._dropped:
             raise FnnError(4, f"AotExecutor: '{name}' is not computed: nothing reads it; name it in output_names to keep it")
         v = self._values[name]
-        return self._backend.read_arena(*v.slot, np.float32).reshape(v.shape).copy()
+        return self._backend.read_arena(*v.slot, np.float32).reshape(v.shape)
 
     @property
     def replayed(self) -> bool:

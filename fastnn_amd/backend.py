@@ -199,7 +199,7 @@ class HipBackend:
         self._check(self.lib.fnn_backend_write_arena(self.handle, offset, buf.ctypes.data_as(C.c_void_p), buf.nbytes))
 
     def read_arena(self, offset: int, size: int, dtype=np.uint8) -> np.ndarray:
-        out = np.empty(size, np.uint8)
+        out = _l.result_array(size, np.uint8)
         self._check(self.lib.fnn_backend_read_arena(self.handle, offset, out.ctypes.data_as(C.c_void_p), size))
         return out.view(dtype)
 
@@ -223,6 +223,13 @@ class HipBackend:
         names = (C.c_char_p * len(shape_env))(*[k.encode() for k in shape_env])
         values = (C.c_uint64 * len(shape_env))(*[int(v) for v in shape_env.values()])
         self._check(self.lib.fnn_backend_dispatch_env(self.handle, plan.handle, names, values, len(shape_env)))
+
+    def forward(self, plan: ExecutablePlan, inputs, outputs):
+        """write_arena, dispatch and read_arena in one call that waits once: inputs and outputs are (offset, array) pairs,
+        the arrays C-contiguous."""
+        ins = (_l.HostSlice * max(len(inputs), 1))(*[(off, a.nbytes, a.ctypes.data) for off, a in inputs])
+        outs = (_l.HostSlice * max(len(outputs), 1))(*[(off, a.nbytes, a.ctypes.data) for off, a in outputs])
+        self._check(self.lib.fnn_backend_forward(self.handle, plan.handle, ins, len(inputs), outs, len(outputs)))
 
     def dispatch_from(self, plan: ExecutablePlan, first: int = 0, shape_env: Optional[dict] = None):
         """One segment of a dispatch (fnn_backend_dispatch_from): returns None when the end of the plan was reached,

@@ -14,6 +14,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "host_io.h"
 #include "i8act.h"
 #include "range_io.h"
 #include "mfma.h"
@@ -40,6 +41,8 @@ struct fnn_hip_graph {
     hipGraphExec_t exec = nullptr;
 };
 
+constexpr size_t kResultSlot = 64u << 10;
+
 struct Staging {
     void *ptr = nullptr;
     size_t cap = 0;
@@ -63,6 +66,7 @@ struct fnn_hip_ctx {
     FnnResidualIo residual;               // a residual addition handed to the next MatMul call (range_io.h)
     FnnPrepIo prep;                       // a prepared operand handed from one MatMul call to the next (range_io.h)
     FnnPreparedOperand prepared;
+    FnnHostIo io;                         // transfers of the calls that take host pointers
 };
 
 // Workspace of fnn_hip_qmatmul_static, part of the library's device image: every GPU the library runs on holds one
@@ -107,7 +111,7 @@ int fail(fnn_hip_ctx *ctx, int code, const char *fmt, ...) noexcept
 // Every extern "C" body runs inside this: a C++ exception (std::bad_alloc from a container, std::length_error, ...)
 // becomes a status code and a message instead of unwinding into the caller's language.
 template <class F>
-int guarded(fnn_hip_ctx *ctx, const char *fn, F &&body) noexcept
+int guarded_body(fnn_hip_ctx *ctx, const char *fn, F &&body) noexcept
 {
     try {
         return body();
@@ -118,6 +122,14 @@ int guarded(fnn_hip_ctx *ctx, const char *fn, F &&body) noexcept
     } catch (...) {
         return fail(ctx, FNN_ERR_DISPATCH, "%s: unknown C++ exception", fn);
     }
+}
+
+template <class F>
+int guarded(fnn_hip_ctx *ctx, const char *fn, F &&body) noexcept
+{
+    const int rc = guarded_body(ctx, fn, body);
+    if (rc && ctx) ctx->io.pending.clear();   // results of a call that failed half way go nowhere
+    return rc;
 }
 
 // option defaults, and the range fnn_hip_set_option accepts
@@ -171,6 +183,27 @@ int ensure(fnn_hip_ctx *ctx, Staging &s, size_t bytes)
     HIP_TRY(ctx, FNN_ERR_MEMORY, hipMalloc(&s.ptr, cap));
     s.cap = cap;
     ctx->ws_epoch++;
+    return FNN_OK;
+}
+
+// A call on host pointers: its inputs and outputs go through pinned memory (host_io.h); finish() ends it.
+int stage_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t bytes)
+{
+    if (ctx->capturing) return fail(ctx, FNN_ERR_DISPATCH, "transfer from host memory during graph capture");
+    HIP_TRY(ctx, FNN_ERR_MEMORY, ctx->io.in(ctx->stream, dst_dev, src, bytes));
+    return FNN_OK;
+}
+
+int stage_out(fnn_hip_ctx *ctx, void *dst, const void *src_dev, size_t bytes)
+{
+    if (ctx->capturing) return fail(ctx, FNN_ERR_DISPATCH, "transfer to host memory during graph capture");
+    HIP_TRY(ctx, FNN_ERR_MEMORY, ctx->io.out(ctx->stream, dst, src_dev, bytes));
+    return FNN_OK;
+}
+
+int finish(fnn_hip_ctx *ctx)
+{
+    HIP_TRY(ctx, FNN_ERR_DISPATCH, ctx->io.wait(ctx->stream));
     return FNN_OK;
 }
 
@@ -241,6 +274,7 @@ int fnn_hip_create(int device, fnn_hip_ctx **out)
         fnn_hip_ctx *ctx = new (std::nothrow) fnn_hip_ctx();
         if (!ctx) return fail(nullptr, FNN_ERR_MEMORY, "fnn_hip_create: out of host memory");
         ctx->device = device;
+        ctx->io.device = device;
         for (int i = 0; i < FNN_OPT_COUNT; i++) ctx->options[i] = kOptions[i].dflt;
         if ((e = hipSetDevice(device)) != hipSuccess ||
             (e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking)) != hipSuccess ||
@@ -266,6 +300,7 @@ void fnn_hip_destroy(fnn_hip_ctx *ctx)
     for (auto &kv : ctx->weights) free_weight(kv.second);
     for (Staging *s : {&ctx->st_a, &ctx->st_out, &ctx->st_bias, &ctx->st_acc, &ctx->st_tmp, &ctx->st_tmp2, &ctx->st_tmp3, &ctx->st_tmp4, &ctx->st_col, &ctx->st_rows})
         if (s->ptr) (void)hipFree(s->ptr);
+    ctx->io.destroy();
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     if (ctx->stream_counters) (void)hipFree(ctx->stream_counters);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
@@ -310,6 +345,18 @@ int fnn_hip_get_option(fnn_hip_ctx *ctx, int option, int64_t *value)
     });
 }
 
+void *fnn_hip_host_alloc(size_t bytes)
+{
+    void *p = nullptr;
+    (void)guarded(nullptr, "fnn_hip_host_alloc", [&]() -> int { p = fnn_pinned_alloc(bytes); return FNN_OK; });
+    return p;
+}
+
+void fnn_hip_host_free(void *p)
+{
+    (void)guarded(nullptr, "fnn_hip_host_free", [&]() -> int { fnn_pinned_free(p); return FNN_OK; });
+}
+
 void *fnn_hip_stream(fnn_hip_ctx *ctx) { return ctx ? (void *)ctx->stream : nullptr; }
 
 int fnn_hip_malloc(fnn_hip_ctx *ctx, size_t bytes, void **dptr)
@@ -339,9 +386,8 @@ int fnn_hip_upload(fnn_hip_ctx *ctx, void *dst, const void *src, size_t bytes)
     return guarded(ctx, "fnn_hip_upload", [&]() -> int {
         if (!ctx || (bytes && (!dst || !src))) return fail(ctx, FNN_ERR_MEMORY, "fnn_hip_upload: NULL argument");
         if (!bytes) return FNN_OK;
-        HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
-        HIP_TRY(ctx, FNN_ERR_MEMORY, hipStreamSynchronize(ctx->stream));
-        return FNN_OK;
+        const int rc = stage_in(ctx, dst, src, bytes);
+        return rc ? rc : finish(ctx);
     });
 }
 
@@ -350,9 +396,8 @@ int fnn_hip_download(fnn_hip_ctx *ctx, void *dst, const void *src, size_t bytes)
     return guarded(ctx, "fnn_hip_download", [&]() -> int {
         if (!ctx || (bytes && (!dst || !src))) return fail(ctx, FNN_ERR_MEMORY, "fnn_hip_download: NULL argument");
         if (!bytes) return FNN_OK;
-        HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-        HIP_TRY(ctx, FNN_ERR_MEMORY, hipStreamSynchronize(ctx->stream));
-        return FNN_OK;
+        const int rc = stage_out(ctx, dst, src, bytes);
+        return rc ? rc : finish(ctx);
     });
 }
 
@@ -518,8 +563,8 @@ int fnn_hip_dequant(fnn_hip_ctx *ctx, const fnn_hip_weight *w, float *out, int f
         }
         HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_dequant(w, dout, ctx->stream));
         if (!(flags & FNN_FLAG_DEVICE_PTRS)) {
-            HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(out, dout, bytes, hipMemcpyDeviceToHost, ctx->stream));
-            HIP_TRY(ctx, FNN_ERR_DISPATCH, hipStreamSynchronize(ctx->stream));
+            const int rc = stage_out(ctx, out, dout, bytes);
+            return rc ? rc : finish(ctx);
         }
         return FNN_OK;
     });
@@ -541,20 +586,23 @@ int fnn_hip_qmatmul(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *a, i
         const int64_t n = w->rows, k = w->inner;
         const bool dev = (flags & FNN_FLAG_DEVICE_PTRS) != 0;
         const float *da = a, *dbias = bias;
-        float *dout = out;
+        float *dout = out, *slot = nullptr;
         if (!dev) {
             int rc;
-            if ((rc = ensure(ctx, ctx->st_a, (size_t)(m * k) * 4))) return rc;
-            if ((rc = ensure(ctx, ctx->st_out, (size_t)(m * n) * 4))) return rc;
-            HIP_TRY(ctx, FNN_ERR_MEMORY,
-                    hipMemcpyAsync(ctx->st_a.ptr, a, (size_t)(m * k) * 4, hipMemcpyHostToDevice, ctx->stream));
+            // one staging buffer for the activations and the bias; a small result is stored by the kernel itself into
+            // pinned memory (every element once; 64 KB cross the link in 2 us)
+            const size_t abytes = (size_t)(m * k) * 4, obytes = (size_t)(m * n) * 4, boff = (abytes + 255) / 256 * 256;
+            if ((rc = ensure(ctx, ctx->st_a, boff + (bias ? (size_t)n * 4 : 0)))) return rc;
+            if ((rc = stage_in(ctx, ctx->st_a.ptr, a, abytes))) return rc;
             da = (const float *)ctx->st_a.ptr;
-            dout = (float *)ctx->st_out.ptr;
             if (bias) {
-                if ((rc = ensure(ctx, ctx->st_bias, (size_t)n * 4))) return rc;
-                HIP_TRY(ctx, FNN_ERR_MEMORY,
-                        hipMemcpyAsync(ctx->st_bias.ptr, bias, (size_t)n * 4, hipMemcpyHostToDevice, ctx->stream));
-                dbias = (const float *)ctx->st_bias.ptr;
+                dbias = (const float *)((const char *)ctx->st_a.ptr + boff);
+                if ((rc = stage_in(ctx, (void *)dbias, bias, (size_t)n * 4))) return rc;
+            }
+            if (obytes <= kResultSlot) dout = slot = (float *)ctx->io.result_slot(out, obytes);
+            if (!slot) {
+                if ((rc = ensure(ctx, ctx->st_out, obytes))) return rc;
+                dout = (float *)ctx->st_out.ptr;
             }
         }
         QMatmulArgs p;
@@ -591,8 +639,8 @@ int fnn_hip_qmatmul(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *a, i
                 if (!done) HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_qgemm_i8act_generic(w->dtype, q8, ctx->stream));
             }
             if (!dev) {
-                HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(out, dout, (size_t)(m * n) * 4, hipMemcpyDeviceToHost, ctx->stream));
-                HIP_TRY(ctx, FNN_ERR_DISPATCH, hipStreamSynchronize(ctx->stream));
+                if (!slot) if (int rc_ = stage_out(ctx, out, dout, (size_t)(m * n) * 4)) return rc_;
+                if (int rc_ = finish(ctx)) return rc_;
             }
             return FNN_OK;
         }
@@ -632,9 +680,8 @@ int fnn_hip_qmatmul(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *a, i
         }
         if (!handled) HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_qgemm_generic(w->dtype, p, ctx->stream));
         if (!dev) {
-            HIP_TRY(ctx, FNN_ERR_MEMORY,
-                    hipMemcpyAsync(out, dout, (size_t)(m * n) * 4, hipMemcpyDeviceToHost, ctx->stream));
-            HIP_TRY(ctx, FNN_ERR_DISPATCH, hipStreamSynchronize(ctx->stream));
+            if (!slot) if (int rc_ = stage_out(ctx, out, dout, (size_t)(m * n) * 4)) return rc_;
+            if (int rc_ = finish(ctx)) return rc_;
         }
         return FNN_OK;
     });
@@ -672,14 +719,14 @@ int fnn_hip_quantize_activations(fnn_hip_ctx *ctx, const float *x, int64_t numel
             int rc;
             if ((rc = ensure(ctx, ctx->st_a, (size_t)numel * 4 + 16))) return rc;
             if ((rc = ensure(ctx, ctx->st_out, (size_t)numel + 16))) return rc;
-            HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(ctx->st_a.ptr, x, (size_t)numel * 4, hipMemcpyHostToDevice, ctx->stream));
+            if ((rc = stage_in(ctx, ctx->st_a.ptr, x, (size_t)numel * 4))) return rc;
             dx = (const float *)ctx->st_a.ptr;
             dp = (uint8_t *)ctx->st_out.ptr;
         }
         HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_quantize_activations(dx, numel, scale, zp, dp, ctx->scratch, ctx->stream));
         if (!dev) {
-            HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(payload, dp, (size_t)numel + 8, hipMemcpyDeviceToHost, ctx->stream));
-            HIP_TRY(ctx, FNN_ERR_DISPATCH, hipStreamSynchronize(ctx->stream));
+            if (int rc_ = stage_out(ctx, payload, dp, (size_t)numel + 8)) return rc_;
+            if (int rc_ = finish(ctx)) return rc_;
         }
         return FNN_OK;
     });
@@ -748,7 +795,7 @@ int fnn_hip_qmatmul_i8act(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const uint8
             int rc;
             if ((rc = ensure(ctx, ctx->st_a, (size_t)(m * k) + 8 + 16))) return rc;
             if ((rc = ensure(ctx, ctx->st_out, (size_t)(m * n) * 4))) return rc;
-            HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(ctx->st_a.ptr, payload, (size_t)(m * k) + 8, hipMemcpyHostToDevice, ctx->stream));
+            if ((rc = stage_in(ctx, ctx->st_a.ptr, payload, (size_t)(m * k) + 8))) return rc;
             dp = (const uint8_t *)ctx->st_a.ptr;
             dout = (float *)ctx->st_out.ptr;
             if (acc_out) {
@@ -766,10 +813,10 @@ int fnn_hip_qmatmul_i8act(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const uint8
         }
         if (!handled) HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_qgemm_i8act_generic(w->dtype, p, ctx->stream));
         if (!dev) {
-            HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(out, dout, (size_t)(m * n) * 4, hipMemcpyDeviceToHost, ctx->stream));
+            if (int rc_ = stage_out(ctx, out, dout, (size_t)(m * n) * 4)) return rc_;
             if (acc_out)
-                HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(acc_out, dacc, (size_t)(m * n) * 4, hipMemcpyDeviceToHost, ctx->stream));
-            HIP_TRY(ctx, FNN_ERR_DISPATCH, hipStreamSynchronize(ctx->stream));
+                if (int rc_ = stage_out(ctx, acc_out, dacc, (size_t)(m * n) * 4)) return rc_;
+            if (int rc_ = finish(ctx)) return rc_;
         }
         return FNN_OK;
     });
@@ -819,12 +866,12 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
         if (!dev) {
             if ((rc = ensure(ctx, ctx->st_a, xin))) return rc;
             if ((rc = ensure(ctx, ctx->st_out, yout))) return rc;
-            HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(ctx->st_a.ptr, x, xin, hipMemcpyHostToDevice, ctx->stream));
+            if ((rc = stage_in(ctx, ctx->st_a.ptr, x, xin))) return rc;
             dx = (const float *)ctx->st_a.ptr;
             dy = (float *)ctx->st_out.ptr;
             if (bias) {
                 if ((rc = ensure(ctx, ctx->st_bias, (size_t)oc * 4))) return rc;
-                HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(ctx->st_bias.ptr, bias, (size_t)oc * 4, hipMemcpyHostToDevice, ctx->stream));
+                if ((rc = stage_in(ctx, ctx->st_bias.ptr, bias, (size_t)oc * 4))) return rc;
                 dbias = (const float *)ctx->st_bias.ptr;
             }
             if (acc_out) {
@@ -859,8 +906,8 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
                 HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_rows_to_nchw(rows_out, dy, b, np, oc, (int64_t)g * ocg, ocg, ctx->stream));
             }
             if (!dev) {
-                HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(y, dy, yout, hipMemcpyDeviceToHost, ctx->stream));
-                HIP_TRY(ctx, FNN_ERR_DISPATCH, hipStreamSynchronize(ctx->stream));
+                if (int rc_ = stage_out(ctx, y, dy, yout)) return rc_;
+                if (int rc_ = finish(ctx)) return rc_;
             }
             return FNN_OK;
         }
@@ -936,9 +983,9 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
             rio.out_parts += range_base;
         }
         if (!dev) {
-            HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(y, dy, yout, hipMemcpyDeviceToHost, ctx->stream));
-            if (acc_out) HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(acc_out, dacc, yout, hipMemcpyDeviceToHost, ctx->stream));
-            HIP_TRY(ctx, FNN_ERR_DISPATCH, hipStreamSynchronize(ctx->stream));
+            if (int rc_ = stage_out(ctx, y, dy, yout)) return rc_;
+            if (acc_out) if (int rc_ = stage_out(ctx, acc_out, dacc, yout)) return rc_;
+            if (int rc_ = finish(ctx)) return rc_;
         }
         return FNN_OK;
     });
@@ -989,12 +1036,12 @@ int fnn_hip_qconv2d_i8act(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const uint8
         if (!dev) {
             if ((rc = ensure(ctx, ctx->st_a, xin))) return rc;
             if ((rc = ensure(ctx, ctx->st_out, yout))) return rc;
-            HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(ctx->st_a.ptr, payload, xin, hipMemcpyHostToDevice, ctx->stream));
+            if ((rc = stage_in(ctx, ctx->st_a.ptr, payload, xin))) return rc;
             dp = (const uint8_t *)ctx->st_a.ptr;
             dy = (float *)ctx->st_out.ptr;
             if (bias) {
                 if ((rc = ensure(ctx, ctx->st_bias, (size_t)oc * 4))) return rc;
-                HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(ctx->st_bias.ptr, bias, (size_t)oc * 4, hipMemcpyHostToDevice, ctx->stream));
+                if ((rc = stage_in(ctx, ctx->st_bias.ptr, bias, (size_t)oc * 4))) return rc;
                 dbias = (const float *)ctx->st_bias.ptr;
             }
         }
@@ -1015,8 +1062,8 @@ int fnn_hip_qconv2d_i8act(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const uint8
         if ((rc = fnn_i8_tiled_conv(ctx, ctx->stream, w, p, &handled))) return rc;
         if (!handled) return fail(ctx, FNN_ERR_UNSUPPORTED_OP, "conv2d_i8_i8: shape outside the integer GEMM's limits");
         if (!dev) {
-            HIP_TRY(ctx, FNN_ERR_MEMORY, hipMemcpyAsync(y, dy, yout, hipMemcpyDeviceToHost, ctx->stream));
-            HIP_TRY(ctx, FNN_ERR_DISPATCH, hipStreamSynchronize(ctx->stream));
+            if (int rc_ = stage_out(ctx, y, dy, yout)) return rc_;
+            if (int rc_ = finish(ctx)) return rc_;
         }
         return FNN_OK;
     });
@@ -1238,6 +1285,10 @@ bool fnn_ctx_no_alloc(fnn_hip_ctx *ctx) { return ctx->capturing || ctx->static_m
 int fnn_ctx_fail(fnn_hip_ctx *ctx, int code, const char *msg) { return fail(ctx, code, "%s", msg); }
 
 int64_t fnn_ctx_option(const fnn_hip_ctx *ctx, int option) { return ctx->options[option]; }
+int fnn_ctx_copy_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t bytes) { return guarded(ctx, "copy in", [&] { return stage_in(ctx, dst_dev, src, bytes); }); }
+int fnn_ctx_copy_out(fnn_hip_ctx *ctx, void *dst, const void *src_dev, size_t bytes) { return guarded(ctx, "copy out", [&] { return stage_out(ctx, dst, src_dev, bytes); }); }
+int fnn_ctx_wait(fnn_hip_ctx *ctx) { return guarded(ctx, "wait", [&] { return finish(ctx); }); }
+void fnn_ctx_drop(fnn_hip_ctx *ctx) { ctx->io.pending.clear(); }
 uint32_t *fnn_ctx_stream_counters(fnn_hip_ctx *ctx) { return ctx->stream_counters; }
 FnnRangeIo *fnn_ctx_range_io(fnn_hip_ctx *ctx) { return &ctx->range; }
 FnnResidualIo *fnn_ctx_residual_io(fnn_hip_ctx *ctx) { return &ctx->residual; }

@@ -1113,7 +1113,7 @@ int run_instr(fnn_backend *b, fnn_plan *p, size_t idx, bool consts_resident)
 // first / stopped_at: a caller that runs unsupported kernels elsewhere dispatches in segments.  With stopped_at given,
 // an instruction that returns FNN_ERR_UNSUPPORTED_OP ends the segment (index in *stopped_at, nothing of it has run)
 // and the caller resumes at the next index; a plan that ever stopped this way is not replayed as a graph.
-int dispatch_impl(fnn_backend *b, fnn_plan *p, uint64_t *elapsed_ns, uint64_t n_elapsed, uint64_t first = 0, uint64_t *stopped_at = nullptr)
+int dispatch_impl(fnn_backend *b, fnn_plan *p, uint64_t *elapsed_ns, uint64_t n_elapsed, uint64_t first = 0, uint64_t *stopped_at = nullptr, bool wait = true)
 {
     if (!b || !p) return fail(b, FNN_ERR_DISPATCH, "dispatch: NULL argument");
     if (first > p->instrs.size()) return fail(b, FNN_ERR_DISPATCH, "dispatch: first instruction %llu of %zu", (unsigned long long)first, p->instrs.size());
@@ -1177,7 +1177,7 @@ int dispatch_impl(fnn_backend *b, fnn_plan *p, uint64_t *elapsed_ns, uint64_t n_
     p->last_replayed = false;
     if (p->graph) {
         int st = lift(b, fnn_hip_graph_launch(b->ctx, p->graph));
-        if (st == FNN_OK) st = lift(b, fnn_hip_sync(b->ctx));
+        if (st == FNN_OK && wait) st = lift(b, fnn_ctx_wait(b->ctx));
         p->last_replayed = st == FNN_OK;
         if (st == FNN_OK) note_dispatched(b, p);
         return st;
@@ -1215,9 +1215,31 @@ int dispatch_impl(fnn_backend *b, fnn_plan *p, uint64_t *elapsed_ns, uint64_t n_
         }
         if (elapsed_ns) elapsed_ns[i] = (uint64_t)std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now() - t0).count();
     }
-    int st = lift(b, fnn_hip_sync(b->ctx));
+    int st = wait ? lift(b, fnn_ctx_wait(b->ctx)) : FNN_OK;
     if (st == FNN_OK) note_dispatched(b, p);
     return st;
+}
+
+// write_arena without the wait: the copy is ordered by the stream
+int write_slice(fnn_backend *b, uint64_t offset, const void *data, uint64_t size)
+{
+    fnn_slice s{offset, size};
+    if (!b->arena || !in_arena(b, s)) return fail(b, FNN_ERR_MEMORY, "write_arena: %llu bytes at %llu outside the arena of %llu bytes", (unsigned long long)size, (unsigned long long)offset, (unsigned long long)b->arena_bytes);
+    if (size == 0) return FNN_OK;
+    if (!data) return fail(b, FNN_ERR_DISPATCH, "write_arena: NULL data");
+    drop_weights_overlapping(b, s);
+    b->write_seq++;
+    log_write(b, s);
+    return lift(b, fnn_ctx_copy_in(b->ctx, b->arena + offset, data, size));
+}
+
+int read_slice(fnn_backend *b, uint64_t offset, void *out, uint64_t size)
+{
+    fnn_slice s{offset, size};
+    if (!b->arena || !in_arena(b, s)) return fail(b, FNN_ERR_MEMORY, "read_arena: %llu bytes at %llu outside the arena of %llu bytes", (unsigned long long)size, (unsigned long long)offset, (unsigned long long)b->arena_bytes);
+    if (size == 0) return FNN_OK;
+    if (!out) return fail(b, FNN_ERR_DISPATCH, "read_arena: NULL destination");
+    return lift(b, fnn_ctx_copy_out(b->ctx, out, b->arena + offset, size));
 }
 
 }  // namespace
@@ -1318,14 +1340,7 @@ int fnn_backend_write_arena(fnn_backend *b, uint64_t offset, const void *data, u
 {
     return guarded(b, "fnn_backend_write_arena", [&]() -> int {
         if (!b) return fail(nullptr, FNN_ERR_DISPATCH, "fnn_backend_write_arena: NULL backend");
-        fnn_slice s{offset, size};
-        if (!b->arena || !in_arena(b, s)) return fail(b, FNN_ERR_MEMORY, "write_arena: %llu bytes at %llu outside the arena of %llu bytes", (unsigned long long)size, (unsigned long long)offset, (unsigned long long)b->arena_bytes);
-        if (size == 0) return FNN_OK;
-        if (!data) return fail(b, FNN_ERR_DISPATCH, "write_arena: NULL data");
-        drop_weights_overlapping(b, s);
-        b->write_seq++;
-        log_write(b, s);
-        return lift(b, fnn_hip_upload(b->ctx, b->arena + offset, data, size));
+        return write_slice(b, offset, data, size);
     });
 }
 
@@ -1333,11 +1348,8 @@ int fnn_backend_read_arena(fnn_backend *b, uint64_t offset, void *out, uint64_t 
 {
     return guarded(b, "fnn_backend_read_arena", [&]() -> int {
         if (!b) return fail(nullptr, FNN_ERR_DISPATCH, "fnn_backend_read_arena: NULL backend");
-        fnn_slice s{offset, size};
-        if (!b->arena || !in_arena(b, s)) return fail(b, FNN_ERR_MEMORY, "read_arena: %llu bytes at %llu outside the arena of %llu bytes", (unsigned long long)size, (unsigned long long)offset, (unsigned long long)b->arena_bytes);
-        if (size == 0) return FNN_OK;
-        if (!out) return fail(b, FNN_ERR_DISPATCH, "read_arena: NULL destination");
-        return lift(b, fnn_hip_download(b->ctx, out, b->arena + offset, size));
+        const int st = read_slice(b, offset, out, size);
+        return st || size == 0 ? st : lift(b, fnn_ctx_wait(b->ctx));
     });
 }
 
@@ -1510,6 +1522,23 @@ int fnn_backend_dispatch(fnn_backend *b, fnn_plan *p)
     return guarded(b, "fnn_backend_dispatch", [&]() -> int {
         if (b) { b->shape_env.clear(); b->shape_env_sig.clear(); }
         return dispatch_impl(b, p, nullptr, 0);
+    });
+}
+
+int fnn_backend_forward(fnn_backend *b, fnn_plan *p, const fnn_host_slice *inputs, uint64_t n_inputs, const fnn_host_slice *outputs, uint64_t n_outputs)
+{
+    return guarded(b, "fnn_backend_forward", [&]() -> int {
+        if (!b || !p || (n_inputs && !inputs) || (n_outputs && !outputs)) return fail(b, FNN_ERR_DISPATCH, "forward: NULL argument");
+        b->shape_env.clear();
+        b->shape_env_sig.clear();
+        int st = FNN_OK;
+        for (uint64_t i = 0; i < n_inputs && !st; i++) st = write_slice(b, inputs[i].offset, inputs[i].data, inputs[i].size);
+        if (!st) st = dispatch_impl(b, p, nullptr, 0, 0, nullptr, false);
+        for (uint64_t i = 0; i < n_outputs && !st; i++) st = read_slice(b, outputs[i].offset, outputs[i].data, outputs[i].size);
+        if (!st) return lift(b, fnn_ctx_wait(b->ctx));
+        fnn_hip_sync(b->ctx);
+        fnn_ctx_drop(b->ctx);
+        return st;
     });
 }
 

@@ -11,36 +11,23 @@
 
 namespace {
 
-struct Job {
-    void (*fn)(void *, int64_t);
-    void *arg;
-    int64_t tasks;
-    std::atomic<int64_t> next{0};
-    int helpers = 0;       // workers inside run(), under Pool::mu
-    int helpers_max = 0;
-    void run()
-    {
-        for (int64_t i; (i = next.fetch_add(1, std::memory_order_relaxed)) < tasks;) fn(arg, i);
-    }
-};
-
 struct Pool {
     std::mutex mu;
     std::condition_variable work, left;
-    std::list<Job *> jobs;
+    std::list<FnnJob *> jobs;
     int workers = 0;
 
     void serve()
     {
         std::unique_lock<std::mutex> lock(mu);
         for (;;) {
-            Job *job = nullptr;
-            for (Job *j : jobs)
+            FnnJob *job = nullptr;
+            for (FnnJob *j : jobs)
                 if (j->helpers < j->helpers_max && j->next.load(std::memory_order_relaxed) < j->tasks) { job = j; break; }
             if (!job) { work.wait(lock); continue; }
             job->helpers++;
             lock.unlock();
-            job->run();
+            while (job->run_one()) {}
             lock.lock();
             if (--job->helpers == 0) left.notify_all();
         }
@@ -65,32 +52,34 @@ int fnn_host_threads()
     return n;
 }
 
-void fnn_parallel_raw(int64_t tasks, int threads, void (*fn)(void *, int64_t), void *arg)
+void FnnJob::begin(int threads)
 {
     Pool &p = *g_pool;
-    Job job;
-    job.fn = fn; job.arg = arg; job.tasks = tasks;
-    const int64_t want = tasks - 1;
-    int helpers = threads - 1 < want ? threads - 1 : (int)want;
-    if (helpers <= 0) { job.run(); return; }
-    job.helpers_max = helpers;
-    std::list<Job *>::iterator at;
+    helpers_max = (int)(threads - 1 < tasks - 1 ? threads - 1 : tasks - 1);
+    if (helpers_max <= 0) return;
     {
         std::lock_guard<std::mutex> lock(p.mu);
         const int most = fnn_host_threads() - 1;
         try {
-            while (p.workers < helpers && p.workers < most) {
+            while (p.workers < helpers_max && p.workers < most) {
                 std::thread([&p] { p.serve(); }).detach();
                 p.workers++;
             }
         } catch (...) {   // (no more threads to be had: those that run, and the caller, do the work)
         }
-        at = p.jobs.insert(p.jobs.end(), &job);
+        p.jobs.push_back(this);
+        queued = true;
     }
-    if (helpers >= 4) p.work.notify_all();
-    else for (int i = 0; i < helpers; i++) p.work.notify_one();
-    job.run();
+    if (helpers_max >= 4) p.work.notify_all();
+    else for (int i = 0; i < helpers_max; i++) p.work.notify_one();
+}
+
+void FnnJob::end()
+{
+    while (run_one()) {}
+    if (!queued) return;
+    Pool &p = *g_pool;
     std::unique_lock<std::mutex> lock(p.mu);
-    p.jobs.erase(at);
-    p.left.wait(lock, [&] { return job.helpers == 0; });
+    p.jobs.remove(this);
+    p.left.wait(lock, [&] { return helpers == 0; });
 }

@@ -74,3 +74,11 @@ struct FnnPreparedOperand {
     int precise = 0, interleaved = 0;
 };
 FnnPreparedOperand *fnn_ctx_prepared(fnn_hip_ctx *ctx);
+
+// Transfers between host memory and the context's stream (host_io.h) without the wait that ends a host-pointer call:
+// copy_in returns when the source may be reused, copy_out's destination holds the result after fnn_ctx_wait, and
+// fnn_ctx_drop forgets results that nobody waits for any more.
+int fnn_ctx_copy_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t bytes);
+int fnn_ctx_copy_out(fnn_hip_ctx *ctx, void *dst, const void *src_dev, size_t bytes);
+int fnn_ctx_wait(fnn_hip_ctx *ctx);
+void fnn_ctx_drop(fnn_hip_ctx *ctx);

@@ -6,6 +6,7 @@ point fails, an exception is raised.
 from __future__ import annotations
 
 import ctypes as C
+import math
 import os
 from dataclasses import dataclass
 from typing import Optional
@@ -52,7 +53,7 @@ STATUS_NAMES = {0: "Ok", 1: "Dispatch", 2: "Memory", 3: "UnsupportedOp", 4: "Com
 # every symbol include/fastnn_hip.h declares
 EXPORTED_SYMBOLS = [
     "fnn_hip_device_count", "fnn_hip_create", "fnn_hip_destroy", "fnn_hip_last_error", "fnn_hip_sync", "fnn_hip_set_option", "fnn_hip_get_option", "fnn_hip_stream",
-    "fnn_hip_malloc", "fnn_hip_free", "fnn_hip_upload", "fnn_hip_download",
+    "fnn_hip_malloc", "fnn_hip_free", "fnn_hip_host_alloc", "fnn_hip_host_free", "fnn_hip_upload", "fnn_hip_download",
     "fnn_hip_weight_register", "fnn_hip_weight_lookup", "fnn_hip_weight_release", "fnn_hip_dequant",
     "fnn_hip_qmatmul", "fnn_hip_qmatmul_static", "fnn_hip_quantize_activations", "fnn_hip_dequantize_activations", "fnn_hip_quantize_activations_per_channel", "fnn_hip_dequantize_activations_per_channel", "fnn_hip_qmatmul_i8act", "fnn_hip_qconv2d", "fnn_hip_qconv2d_i8act",
     "fnn_hip_timer_start", "fnn_hip_timer_stop",
@@ -68,7 +69,7 @@ BACKEND_SYMBOLS = [
     "fnn_plan_create", "fnn_plan_destroy", "fnn_plan_add_write_const", "fnn_plan_add_fill",
     "fnn_plan_add_memcopy", "fnn_plan_add_call_kernel", "fnn_plan_len", "fnn_plan_replayed", "fnn_plan_ranges_used", "fnn_plan_residuals_fused", "fnn_plan_operands_handed", "fnn_plan_arena_size",
     "fnn_plan_set_param_dims", "fnn_plan_from_bincode", "fnn_plan_to_bincode", "fnn_plan_describe",
-    "fnn_backend_dispatch", "fnn_backend_dispatch_env", "fnn_backend_dispatch_from", "fnn_backend_dispatch_profile",
+    "fnn_backend_dispatch", "fnn_backend_forward", "fnn_backend_dispatch_env", "fnn_backend_dispatch_from", "fnn_backend_dispatch_profile",
     "fnn_backend_dispatch_profile_env",
     "fnn_hip_elementwise", "fnn_hip_fill_f32", "fnn_hip_copy",
     "fnn_hip_copy2d_f32", "fnn_hip_concat_f32", "fnn_hip_maxpool2d_f32", "fnn_hip_avgpool2d_f32", "fnn_hip_upsample_nearest2d_f32",
@@ -116,6 +117,11 @@ class Slice(C.Structure):
     _fields_ = [("offset", C.c_uint64), ("size", C.c_uint64)]
 
 
+class HostSlice(C.Structure):
+    """fnn_host_slice: an arena range and the host memory it is copied from or to."""
+    _fields_ = [("offset", C.c_uint64), ("size", C.c_uint64), ("data", _vp)]
+
+
 class DimExpr(C.Structure):
     """fnn_dim_expr: kind 0 Known(value), 1 Symbol(symbol), 2 Bounded{sym: symbol, max: value}."""
     _fields_ = [("kind", C.c_uint32), ("value", C.c_uint64), ("symbol", C.c_char_p)]
@@ -142,6 +148,10 @@ def _prototype(l):
     l.fnn_hip_stream.restype = _vp
     l.fnn_hip_malloc.argtypes = [_vp, _sz, C.POINTER(_vp)]
     l.fnn_hip_free.argtypes = [_vp, _vp]
+    l.fnn_hip_host_alloc.argtypes = [_sz]
+    l.fnn_hip_host_alloc.restype = _vp
+    l.fnn_hip_host_free.argtypes = [_vp]
+    l.fnn_hip_host_free.restype = None
     l.fnn_hip_upload.argtypes = [_vp, _vp, _vp, _sz]
     l.fnn_hip_download.argtypes = [_vp, _vp, _vp, _sz]
     l.fnn_hip_weight_register.argtypes = [_vp, C.c_uint64, C.c_int, _vp, _sz, _i64, _i64, _vp, _sz, _vp, _sz,
@@ -206,6 +216,7 @@ def _prototype(l):
     l.fnn_plan_operands_handed.argtypes = [_vp]
     l.fnn_plan_operands_handed.restype = C.c_uint64
     l.fnn_backend_dispatch.argtypes = [_vp, _vp]
+    l.fnn_backend_forward.argtypes = [_vp, _vp, C.POINTER(HostSlice), _u64, C.POINTER(HostSlice), _u64]
     l.fnn_backend_dispatch_env.argtypes = [_vp, _vp, C.POINTER(C.c_char_p), C.POINTER(_u64), _u64]
     l.fnn_backend_dispatch_from.argtypes = [_vp, _vp, C.POINTER(C.c_char_p), C.POINTER(_u64), _u64, _u64, C.POINTER(_u64)]
     l.fnn_plan_arena_size.argtypes = [_vp]
@@ -228,6 +239,33 @@ def _prototype(l):
 
 def _np_ptr(a: Optional[np.ndarray]):
     return None if a is None else a.ctypes.data_as(_vp)
+
+
+class _PinnedBlock:
+    """Pinned memory that a result array keeps alive through its base."""
+    __slots__ = ("ptr", "__array_interface__")
+
+    def __init__(self, ptr: int, nbytes: int):
+        self.ptr = ptr
+        self.__array_interface__ = {"data": (ptr, False), "shape": (nbytes,), "typestr": "|u1", "version": 3}
+
+    def __del__(self):
+        _lib.fnn_hip_host_free(self.ptr)
+
+
+_PINNED_MIN = 1 << 15   # (smaller results are cheaper to copy out of the staging memory)
+
+
+def result_array(shape, dtype=np.float32) -> np.ndarray:
+    """An uninitialised array for a call's result: pinned memory where it is large, so that the device writes it in place."""
+    dtype = np.dtype(dtype)
+    shape = (shape,) if isinstance(shape, (int, np.integer)) else tuple(shape)
+    nbytes = math.prod(shape) * dtype.itemsize
+    if nbytes >= _PINNED_MIN:
+        p = load_library().fnn_hip_host_alloc(nbytes)
+        if p:
+            return np.asarray(_PinnedBlock(p, nbytes)).view(dtype).reshape(shape)
+    return np.empty(shape, dtype)
 
 
 def _as_ptr(x):
@@ -311,7 +349,7 @@ class DeviceBuffer:
         return self
 
     def download(self, dtype, count: int, offset: int = 0) -> np.ndarray:
-        out = np.empty(count, dtype=dtype)
+        out = result_array(count, dtype)
         assert offset + out.nbytes <= self.nbytes
         self.ctx._check(self.ctx.lib.fnn_hip_download(self.ctx.handle, _np_ptr(out), _vp(self.ptr + offset), out.nbytes))
         return out
@@ -385,7 +423,7 @@ class HipContext:
         self._check(self.lib.fnn_hip_weight_release(self.handle, wh))
 
     def dequant(self, wh, rows: int, inner: int) -> np.ndarray:
-        out = np.empty((rows, inner), np.float32)
+        out = result_array((rows, inner))
         self._check(self.lib.fnn_hip_dequant(self.handle, wh, _np_ptr(out), 0))
         return out
 
@@ -395,7 +433,7 @@ class HipContext:
         """Host-pointer call: copies in, runs, copies out, synchronises."""
         a = np.ascontiguousarray(a, dtype=np.float32)
         m = a.shape[0]
-        out = np.empty((m, n), np.float32)
+        out = result_array((m, n))
         b = None if bias is None else np.ascontiguousarray(bias, dtype=np.float32)
         self._check(self.lib.fnn_hip_qmatmul(self.handle, wh, _np_ptr(a), m, _np_ptr(b), act, _np_ptr(out), flags))
         return out
@@ -453,7 +491,7 @@ class HipContext:
 
     def qmatmul_i8act(self, wh, payload: np.ndarray, m: int, n: int, want_acc: bool = False, flags: int = 0):
         payload = np.ascontiguousarray(payload, dtype=np.uint8)
-        out = np.empty((m, n), np.float32)
+        out = result_array((m, n))
         acc = np.zeros((m, n), np.int32) if want_acc else None
         self._check(self.lib.fnn_hip_qmatmul_i8act(self.handle, wh, _np_ptr(payload), m, _np_ptr(out), _np_ptr(acc),
                                                    flags))
@@ -468,7 +506,7 @@ class HipContext:
             dk = (k - 1) * dil + 1
             return (i + 2 * pad - dk) // stride + 1 if i + 2 * pad >= dk else 0
         ho, wo = osz(h, kh), osz(w, kw)
-        y = np.zeros((b, oc, ho, wo), np.float32)
+        y = result_array((b, oc, ho, wo))
         acc = np.zeros((b, oc, ho, wo), np.int32) if want_acc else None
         bb = None if bias is None else np.ascontiguousarray(bias, dtype=np.float32)
         self._check(self.lib.fnn_hip_qconv2d(self.handle, wh, _np_ptr(x), b, c, h, w, kh, kw, stride, pad, dil, groups,
@@ -486,7 +524,7 @@ class HipContext:
         def osz(i, k):
             dk = (k - 1) * dil + 1
             return (i + 2 * pad - dk) // stride + 1 if i + 2 * pad >= dk else 0
-        y = np.zeros((b, oc, osz(h, kh), osz(w, kw)), np.float32)
+        y = result_array((b, oc, osz(h, kh), osz(w, kw)))
         bb = None if bias is None else np.ascontiguousarray(bias, dtype=np.float32)
         self._check(self.lib.fnn_hip_qconv2d_i8act(self.handle, wh, _np_ptr(payload), b, c, h, w, kh, kw, stride, pad,
                                                    dil, groups, _np_ptr(bb), act, _np_ptr(y), flags))

@@ -172,6 +172,12 @@ int fnn_hip_get_option(fnn_hip_ctx *ctx, int option, int64_t *value);
  * library's (no counterpart in fastnn). */
 void *fnn_hip_stream(fnn_hip_ctx *ctx);
 
+/* Pinned host memory for arrays that host-pointer calls read or write: results land in it without a copy by the host.
+ * Blocks come from a pool of the process (at most 1 GiB in existence, 256 MiB of it kept unused); NULL: no room, take
+ * ordinary memory.  No counterpart in fastnn. */
+void *fnn_hip_host_alloc(size_t bytes);
+void fnn_hip_host_free(void *ptr);
+
 /* ---- weights: get_or_cache_packed + packed_tensor_from_meta,
  * src/backend/cpu/mod.rs:62-89, src/backend/cpu/matmul.rs:81-152.
  * Uploads the packed words once; `key` identifies the weight the way the CPU

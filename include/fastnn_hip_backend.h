@@ -114,6 +114,16 @@ int fnn_plan_describe(const fnn_plan *p, uint64_t instruction, char *buf, uint64
  * dispatches skip the uploads and replay the instruction stream as one HIP graph, the static-shape plan
  * reuse of src/backend/executor.rs:639-667 (see fnn_backend_set_graph_replay). */
 int fnn_backend_dispatch(fnn_backend *b, fnn_plan *p);
+/* write_arena of every input, dispatch (empty ShapeEnv), read_arena of every output, as GraphExecutor::execute_internal
+ * does them (src/backend/executor.rs:599-858), in one call that waits once, at its end.  Outputs in memory from
+ * fnn_hip_host_alloc need no copy by the host. */
+typedef struct {
+    uint64_t offset;   /* in the arena */
+    uint64_t size;     /* bytes */
+    void *data;        /* host memory, read (inputs) or written (outputs) */
+} fnn_host_slice;
+int fnn_backend_forward(fnn_backend *b, fnn_plan *p, const fnn_host_slice *inputs, uint64_t n_inputs,
+                        const fnn_host_slice *outputs, uint64_t n_outputs);
 /* Backend::dispatch with its ShapeEnv argument (src/backend/mod.rs:167-176, src/ir/node.rs:347-391): n_symbols
  * (name, value) bindings, valid for this dispatch; fnn_backend_dispatch is the same with an empty environment.  A
  * name bound twice to different values is refused, as ShapeEnv::bind does.  A resident plan replays its graph only
