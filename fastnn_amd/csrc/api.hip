@@ -187,10 +187,10 @@ int ensure(fnn_hip_ctx *ctx, Staging &s, size_t bytes)
 }
 
 // A call on host pointers: its inputs and outputs go through pinned memory (host_io.h); finish() ends it.
-int stage_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t bytes)
+int stage_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t bytes, size_t at1 = 0, const void *src1 = nullptr, size_t bytes1 = 0)
 {
     if (ctx->capturing) return fail(ctx, FNN_ERR_DISPATCH, "transfer from host memory during graph capture");
-    HIP_TRY(ctx, FNN_ERR_MEMORY, ctx->io.in(ctx->stream, dst_dev, src, bytes));
+    HIP_TRY(ctx, FNN_ERR_MEMORY, ctx->io.in2(ctx->stream, dst_dev, src, bytes, at1, src1, bytes1));
     return FNN_OK;
 }
 
@@ -591,14 +591,11 @@ int fnn_hip_qmatmul(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *a, i
             int rc;
             // one staging buffer for the activations and the bias; a small result is stored by the kernel itself into
             // pinned memory (every element once; 64 KB cross the link in 2 us)
-            const size_t abytes = (size_t)(m * k) * 4, obytes = (size_t)(m * n) * 4, boff = (abytes + 255) / 256 * 256;
-            if ((rc = ensure(ctx, ctx->st_a, boff + (bias ? (size_t)n * 4 : 0)))) return rc;
-            if ((rc = stage_in(ctx, ctx->st_a.ptr, a, abytes))) return rc;
+            const size_t abytes = (size_t)(m * k) * 4, obytes = (size_t)(m * n) * 4, boff = (abytes + 255) / 256 * 256, bbytes = bias ? (size_t)n * 4 : 0;
+            if ((rc = ensure(ctx, ctx->st_a, boff + bbytes))) return rc;
+            if ((rc = stage_in(ctx, ctx->st_a.ptr, a, abytes, boff, bias, bbytes))) return rc;
             da = (const float *)ctx->st_a.ptr;
-            if (bias) {
-                dbias = (const float *)((const char *)ctx->st_a.ptr + boff);
-                if ((rc = stage_in(ctx, (void *)dbias, bias, (size_t)n * 4))) return rc;
-            }
+            if (bias) dbias = (const float *)((const char *)ctx->st_a.ptr + boff);
             if (obytes <= kResultSlot) dout = slot = (float *)ctx->io.result_slot(out, obytes);
             if (!slot) {
                 if ((rc = ensure(ctx, ctx->st_out, obytes))) return rc;

@@ -28,6 +28,8 @@ struct FnnHostIo {
     void destroy();
     // enqueues host -> device; `src` may be reused on return, the transfer is done when the stream gets there
     hipError_t in(hipStream_t s, void *dst, const void *src, size_t bytes);
+    // two inputs into one allocation, the second at offset at1 >= bytes0 (small ones: in one launch)
+    hipError_t in2(hipStream_t s, void *dst, const void *src0, size_t bytes0, size_t at1, const void *src1, size_t bytes1);
     // enqueues device -> host; `dst` holds the result after wait()
     hipError_t out(hipStream_t s, void *dst, const void *src, size_t bytes);
     // staging memory that kernels of the stream may write results to and that wait() copies to `dst`; null: too large

@@ -14,9 +14,9 @@
 namespace {
 
 constexpr size_t kPinnedLive = 1u << 30, kPinnedKept = 256u << 20;
-constexpr size_t kBlock = 1u << 20;                // of a large input: one task of the copying threads, one engine transfer
+constexpr size_t kBlock = 512u << 10;              // of a large input: one task of the copying threads
 constexpr size_t kLargeStaging = 256u << 20;       // larger inputs are left to the runtime
-constexpr int kCopyThreads = 6;                    // (one thread copies 31 GB/s from memory, the engine moves 57)
+constexpr int kCopyThreads = 8;                    // (one thread copies 31 GB/s from memory, the engine moves 57)
 constexpr auto kSpin = std::chrono::microseconds(200);
 
 // T = the widest access that source, destination and size allow
@@ -141,6 +141,20 @@ hipError_t FnnHostIo::take_small(hipStream_t s, size_t bytes, size_t align_like,
     return hipSuccess;
 }
 
+hipError_t FnnHostIo::in2(hipStream_t s, void *dst, const void *src0, size_t bytes0, size_t at1, const void *src1, size_t bytes1)
+{
+    if (!bytes1 || at1 + bytes1 > kSmallTransfer) {
+        const hipError_t e = in(s, dst, src0, bytes0);
+        return e != hipSuccess || !bytes1 ? e : in(s, (unsigned char *)dst + at1, src1, bytes1);
+    }
+    unsigned char *p;
+    const hipError_t e = take_small(s, at1 + bytes1, reinterpret_cast<uintptr_t>(dst), &p);
+    if (e != hipSuccess) return e;
+    std::memcpy(p, src0, bytes0);
+    std::memcpy(p + at1, src1, bytes1);
+    return device_copy(s, dst, p, at1 + bytes1);
+}
+
 hipError_t FnnHostIo::in(hipStream_t s, void *dst, const void *src, size_t bytes)
 {
     if (!bytes) return hipSuccess;
@@ -182,12 +196,17 @@ hipError_t FnnHostIo::in_large(hipStream_t s, unsigned char *dst, const unsigned
         c.done[(size_t)i].store(1, std::memory_order_release);
     }, &copy);
     job.begin(std::min(fnn_host_threads(), kCopyThreads));
+    // Every transfer costs the engine 9 us beside its bytes (78 MB in blocks of 1 MB: 2.1 ms, of 8 MB: 1.48 ms), so they
+    // grow: 8 MB, then as much as the one before took time for the threads to stage.
     hipError_t e = hipSuccess;
-    for (int64_t i = 0; i < blocks && e == hipSuccess;) {
-        if (copy.done[(size_t)i].load(std::memory_order_acquire)) {
-            const size_t at = (size_t)i * kBlock;
-            e = hipMemcpyAsync(dst + at, stage + at, std::min(kBlock, bytes - at), hipMemcpyHostToDevice, s);
-            i++;
+    int64_t ready = 0;
+    for (size_t sent = 0, want = 8u << 20; sent < bytes && e == hipSuccess;) {
+        while (ready < blocks && copy.done[(size_t)ready].load(std::memory_order_acquire)) ready++;
+        const size_t have = ready == blocks ? bytes : (size_t)ready * kBlock;
+        if (have - sent >= std::min(want, bytes - sent)) {
+            e = hipMemcpyAsync(dst + sent, stage + sent, have - sent, hipMemcpyHostToDevice, s);
+            sent = have;
+            want = 16u << 20;
         } else if (!job.run_one()) {
             _mm_pause();
         }

@@ -238,7 +238,7 @@ def _prototype(l):
 
 
 def _np_ptr(a: Optional[np.ndarray]):
-    return None if a is None else a.ctypes.data_as(_vp)
+    return None if a is None else a.ctypes.data
 
 
 class _PinnedBlock:
@@ -266,6 +266,17 @@ def result_array(shape, dtype=np.float32) -> np.ndarray:
         if p:
             return np.asarray(_PinnedBlock(p, nbytes)).view(dtype).reshape(shape)
     return np.empty(shape, dtype)
+
+
+_byte = C.c_ubyte
+
+
+def _ref(a: np.ndarray):
+    """_np_ptr for the calls where microseconds count (0.4 instead of 1.1 us)."""
+    try:
+        return C.byref(_byte.from_buffer(a))
+    except (TypeError, ValueError):   # read-only or empty
+        return a.ctypes.data
 
 
 def _as_ptr(x):
@@ -434,8 +445,11 @@ class HipContext:
         a = np.ascontiguousarray(a, dtype=np.float32)
         m = a.shape[0]
         out = result_array((m, n))
-        b = None if bias is None else np.ascontiguousarray(bias, dtype=np.float32)
-        self._check(self.lib.fnn_hip_qmatmul(self.handle, wh, _np_ptr(a), m, _np_ptr(b), act, _np_ptr(out), flags))
+        if bias is not None:
+            bias = np.ascontiguousarray(bias, dtype=np.float32)
+        rc = self.lib.fnn_hip_qmatmul(self.handle, wh, _ref(a), m, None if bias is None else _ref(bias), act, _ref(out), flags)
+        if rc:
+            self._check(rc)
         return out
 
     def qmatmul_dev(self, wh, a_ptr: int, m: int, out_ptr: int, bias_ptr: int = 0, act: int = ACT_NONE,
