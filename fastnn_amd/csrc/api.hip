@@ -159,6 +159,7 @@ const OptionSpec kOptions[FNN_OPT_COUNT] = {
     {0, 0, 0xffff},   // FNN_OPT_STREAM_SHAPE
     {0, 0, 4},        // FNN_OPT_DIGIT_PLANES
     {1, 0, 1},        // FNN_OPT_GEMV_TILE_MAJOR
+    {0, -1, 0xffff},  // FNN_OPT_FRAGMENT
 };
 
 #define HIP_TRY(ctx, code, expr)                                                              \
@@ -242,6 +243,7 @@ void free_weight(fnn_hip_weight *w)
     if (w->umean) (void)hipFree(w->umean);
     if (w->words4) (void)hipFree(w->words4);
     if (w->words_tm) (void)hipFree(w->words_tm);
+    if (w->words_fr) (void)hipFree(w->words_fr);
     if (w->dense16) (void)hipFree(w->dense16);
     delete w;
 }
@@ -648,7 +650,11 @@ int fnn_hip_qmatmul(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *a, i
         bool handled = false;
         if (!(flags & FNN_FLAG_FORCE_GENERIC)) {
             const bool fma_first = (flags & FNN_FLAG_PREFER_FMA) || w->dtype == FNN_DT_I4CB;
-            if (fma_first) HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_qgemv(w->dtype, p, ctx->stream, &handled));
+            {   // (small aligned M declined by rule)
+                int rc = fnn_frag_qmatmul(ctx, ctx->stream, w, p, flags, &handled);
+                if (rc) return rc;
+            }
+            if (fma_first && !handled) HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_qgemv(w->dtype, p, ctx->stream, &handled));
             if (!handled) {   // (17 <= M <= 32 and, for a long K over few columns, from M = 9 or 5)
                 int rc = fnn_stream_qmatmul(ctx, ctx->stream, w, p, flags, &handled);
                 if (rc) return rc;

@@ -39,6 +39,8 @@ constexpr int FNN_STREAM_COUNTERS = 4096;
 uint32_t *fnn_ctx_stream_counters(fnn_hip_ctx *ctx);
 // int8 matrix-core GEMM over exact activation digit planes (qgemm_digits.hip): M >= 17, I8 / I4 / U4 weights
 int fnn_digits_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
+// a middle number of activation rows, per-channel types: both operands in the order the matrix cores take them (qgemm_frag.hip)
+int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
 int fnn_tiled_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p,
                       int flags, bool *handled);
 // FNN_FLAG_ACT_QUANT with F8 weights: activations rounded to E4M3 (one power-of-two scale per row), fp8 matrix cores

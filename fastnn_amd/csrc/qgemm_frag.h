@@ -1,0 +1,61 @@
+// Launch interface of the fragment-major MatMul kernels (qgemm_frag_impl.h; one translation unit per weight type).
+#pragma once
+#include <cstdint>
+
+#include "common.h"
+
+constexpr int FRAG_NW = 8;        // waves per workgroup, each with an eighth of the workgroup's K range (a segment)
+
+// How K is dealt out: `splits` workgroups of kb_per_split k blocks (64 bytes of a weight row), each in FRAG_NW segments.
+struct FragSplit {
+    int kblocks, splits, kb_per_split;
+    int seg, seg_last;           // k blocks per segment: of the last split (seg_last) and of those before it
+    int piece, pieces;           // a segment in `pieces` pieces of `piece` k blocks: what shares a power of two per row
+    // segment wv of split z: blocks [b0, b1), empty where b0 >= b1
+    __host__ __device__ void segment(int z, int wv, int *b0, int *b1) const
+    {
+        const int kb0 = z * kb_per_split, kb1 = kb0 + kb_per_split < kblocks ? kb0 + kb_per_split : kblocks;
+        const int per = z == splits - 1 ? seg_last : seg;
+        *b0 = kb0 + wv * per;
+        *b1 = *b0 + per < kb1 ? *b0 + per : kb1;
+    }
+    // piece i of all pieces, segment by segment
+    __host__ __device__ void piece_at(int i, int *b0, int *b1) const
+    {
+        const int s = i / pieces;
+        segment(s / FRAG_NW, s % FRAG_NW, b0, b1);
+        *b0 += (i - s * pieces) * piece;
+        *b1 = *b0 + piece < *b1 ? *b0 + piece : *b1;
+    }
+};
+
+// A row's values of a piece of K: the power of two applied to them, and their sum (for the zero-point term).
+struct FragRow { int e; float sum; };
+
+struct FragArgs {
+    const uint32_t *wf;          // weight fragments [row block of 16][k block][q 0..3][row][16 bytes]
+    const _Float16 *af;          // activation fragments [row block of 16][step of 32 k][hi, lo][q 0..3][row][8 f16]
+    const float *a;              // non-null: the f32 activations [m,k], converted in the kernel (splits == 1; af, rows unused)
+    int64_t k;
+    const FragRow *rows;         // [segment][piece][m_pad]
+    const float *scales, *zeros, *bias;
+    float *out;
+    float *part;                 // non-null: [split][m][n] sums with scale and zero applied, no bias or activation
+    const float *residual;       // non-null (no part): sum_out[m,n] = out[m,n] + residual[m,n] as well
+    float *sum_out;
+    int64_t m, n, m_pad;
+    int act;
+    FragSplit ks;
+    FastDiv by_mtiles, by_splits;
+    int mtiles, ntiles, rblocks; // rblocks: blocks of 16 weight rows
+    int vec4;                    // 16-byte accesses along n: n % 4 == 0 and aligned tensors
+};
+
+// mb x 16 activation rows and nb x 16 weight rows per workgroup of eight waves
+hipError_t fnn_frag_launch_i8(int mb, int nb, const FragArgs &p, hipStream_t s);
+hipError_t fnn_frag_launch_i4(int mb, int nb, const FragArgs &p, hipStream_t s);
+hipError_t fnn_frag_launch_u8(int mb, int nb, const FragArgs &p, hipStream_t s);
+hipError_t fnn_frag_launch_u4(int mb, int nb, const FragArgs &p, hipStream_t s);
+hipError_t fnn_frag_launch_f8(int mb, int nb, const FragArgs &p, hipStream_t s);
+hipError_t fnn_frag_launch_f8r(int mb, int nb, const FragArgs &p, hipStream_t s);
+hipError_t fnn_frag_launch_f4(int mb, int nb, const FragArgs &p, hipStream_t s);

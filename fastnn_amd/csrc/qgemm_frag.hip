@@ -1,0 +1,511 @@
+// Host side of the fragment-major MatMul (kernels: qgemm_frag_impl.h): the weight's fragment-major copy, the activation
+// operand, the shape of the launch, the reduction of a K split.
+//
+// Launches: frag_prep_kernel (f32 rows -> f16 hi + lo fragments, row exponents and sums), qgemm_frag_kernel, and with K
+// split over workgroups frag_reduce_kernel (partials added in split order: results do not depend on scheduling).
+#include "mfma.h"
+#include "qgemm_frag.h"
+#include "range_io.h"
+
+namespace {
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));   // rows of any K: 16-byte loads from 4-byte aligned addresses
+
+constexpr float LO_UP = 2048.0f;
+
+__global__ void __launch_bounds__(256) frag_words_kernel(const uint32_t *src, int64_t rows, int64_t kp, int64_t kblocks, u32x4 *dst)
+{
+    const int64_t total = (rows + 15) / 16 * kblocks * 64;   // 16-byte pieces
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+        const int64_t blk = i >> 6, rb = blk / kblocks, kb = blk - rb * kblocks;
+        const int q = (int)((i >> 4) & 3);
+        const int64_t row = rb * 16 + (i & 15), w0 = kb * 16 + q * 4;
+        u32x4 v = {0u, 0u, 0u, 0u};
+        if (row < rows) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (w0 + j < kp) v[j] = src[row * kp + w0 + j];
+        }
+        dst[i] = v;
+    }
+}
+
+struct FragPrepArgs {
+    const float *a;              // [m,k], or
+    FragArgs prev;               // the MatMul whose partial tiles are reduced here: its result (k columns) is what is converted
+    int use_sum;                 // ... or that result plus prev.residual
+    _Float16 *af;
+    FragRow *rows;
+    int64_t m, k, m_pad;
+    FragSplit ks;
+    int four_bit, interleaved;
+};
+
+// eight results of a MatMul from its partial tiles, columns n .. n + 7 of row m: split order, bias, activation
+__device__ __forceinline__ void reduce8(const FragArgs &p, int64_t m, int64_t n, float(&v)[8])
+{
+    const int64_t total = p.m * p.n;
+    const float4 *pp = reinterpret_cast<const float4 *>(p.part + m * p.n + n);
+    float4 t0 = pp[0], t1 = pp[1];
+    for (int z = 1; z < p.ks.splits; z++) {
+        const float4 u0 = pp[(int64_t)z * (total / 4)], u1 = pp[(int64_t)z * (total / 4) + 1];
+        t0.x += u0.x; t0.y += u0.y; t0.z += u0.z; t0.w += u0.w;
+        t1.x += u1.x; t1.y += u1.y; t1.z += u1.z; t1.w += u1.w;
+    }
+    v[0] = t0.x; v[1] = t0.y; v[2] = t0.z; v[3] = t0.w; v[4] = t1.x; v[5] = t1.y; v[6] = t1.z; v[7] = t1.w;
+    if (p.bias) {
+        const float4 b0 = *reinterpret_cast<const float4 *>(p.bias + n), b1 = *reinterpret_cast<const float4 *>(p.bias + n + 4);
+        v[0] = v[0] + b0.x; v[1] = v[1] + b0.y; v[2] = v[2] + b0.z; v[3] = v[3] + b0.w;
+        v[4] = v[4] + b1.x; v[5] = v[5] + b1.y; v[6] = v[6] + b1.z; v[7] = v[7] + b1.w;
+    }
+    if (p.act != FNN_ACT_NONE) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = fnn_activation(v[j], p.act);
+    }
+}
+
+// Activation fragments: one workgroup per block of 16 rows and piece of K.  A row's values of a piece share a power of
+// two, so a workgroup needs nothing from the others; its waves take the piece's steps in turn, lane r + 16 q the eight values of row r that lane will hold as an operand:
+// every store is one contiguous KB.  STEPS: steps per wave that stay in registers between the row maxima and the
+// conversion; longer pieces read their values twice (never with CHAIN).
+// CHAIN: the values are the result of the MatMul before, reduced from its partial tiles and stored here (with its sum
+// with a residual), so that the reduction and the preparation of the next MatMul are one launch.
+template <bool CHAIN, int STEPS, int NW>
+__global__ void __launch_bounds__(NW * 64) frag_prep_kernel(FragPrepArgs p)
+{
+    __shared__ float red[2][NW][16];
+    __shared__ float part[STEPS == 1 ? 2 * NW : 1][64];   // one step per wave: its two half sums per lane
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r = lane & 15, q = lane >> 4;
+    int b0, b1;
+    p.ks.piece_at((int)blockIdx.x, &b0, &b1);
+    if (b0 >= b1) {   // an empty piece: its row sums are read all the same
+        if (tid < 16) p.rows[(int64_t)blockIdx.x * p.m_pad + (int64_t)blockIdx.y * 16 + tid] = FragRow{0, 0.0f};
+        return;
+    }
+    const int64_t m = (int64_t)blockIdx.y * 16 + r, K = p.k;
+    const int sh = p.four_bit ? 2 : 1;                       // log2 of the steps per k block
+    const int s0 = b0 << sh, s1 = b1 << sh, nsteps = p.ks.kblocks << sh;
+    auto first_k = [&](int s) { return ((((int64_t)(s >> sh) << 2) + q) << (sh + 3)) + ((s & ((1 << sh) - 1)) << 3); };
+    auto load8 = [&](int s, float(&v)[8]) {
+        const int64_t k0 = first_k(s);
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = 0.0f;
+        if (s >= s1 || m >= p.m || k0 >= K) return;
+        if constexpr (CHAIN) {   // (K % 8 == 0)
+            reduce8(p.prev, m, k0, v);
+            const int64_t at = m * K + k0;
+            *reinterpret_cast<float4 *>(p.prev.out + at) = make_float4(v[0], v[1], v[2], v[3]);
+            *reinterpret_cast<float4 *>(p.prev.out + at + 4) = make_float4(v[4], v[5], v[6], v[7]);
+            if (p.prev.residual) {
+                const float4 r0 = *reinterpret_cast<const float4 *>(p.prev.residual + at), r1 = *reinterpret_cast<const float4 *>(p.prev.residual + at + 4);
+                const float4 s0_ = make_float4(v[0] + r0.x, v[1] + r0.y, v[2] + r0.z, v[3] + r0.w);
+                const float4 s1_ = make_float4(v[4] + r1.x, v[5] + r1.y, v[6] + r1.z, v[7] + r1.w);
+                *reinterpret_cast<float4 *>(p.prev.sum_out + at) = s0_;
+                *reinterpret_cast<float4 *>(p.prev.sum_out + at + 4) = s1_;
+                if (p.use_sum) { v[0] = s0_.x; v[1] = s0_.y; v[2] = s0_.z; v[3] = s0_.w; v[4] = s1_.x; v[5] = s1_.y; v[6] = s1_.z; v[7] = s1_.w; }
+            }
+        } else {
+            const float *x = p.a + m * K + k0;
+            if (k0 + 8 <= K) {
+                const f4u t0 = *reinterpret_cast<const f4u *>(x), t1 = *reinterpret_cast<const f4u *>(x + 4);
+                v[0] = t0[0]; v[1] = t0[1]; v[2] = t0[2]; v[3] = t0[3];
+                v[4] = t1[0]; v[5] = t1[1]; v[6] = t1[2]; v[7] = t1[3];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    if (k0 + j < K) v[j] = x[j];
+            }
+        }
+    };
+    float keep[STEPS][8];
+    float mx = 0.0f, sum = 0.0f;
+    auto stats = [&](const float(&v)[8]) {
+        mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))),
+                             fmaxf(fmaxf(fabsf(v[4]), fabsf(v[5])), fmaxf(fabsf(v[6]), fabsf(v[7])))));
+        sum += (v[0] + v[1]) + (v[2] + v[3]);
+        sum += (v[4] + v[5]) + (v[6] + v[7]);
+    };
+    const bool in_regs = CHAIN || s1 - s0 <= NW * STEPS;
+    if (in_regs) {
+#pragma unroll
+        for (int t = 0; t < STEPS; t++) load8(s0 + wv + NW * t, keep[t]);
+#pragma unroll
+        for (int t = 0; t < STEPS; t++) stats(keep[t]);
+    } else {
+        for (int s = s0 + wv; s < s1; s += NW) { load8(s, keep[0]); stats(keep[0]); }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if constexpr (STEPS == 1) {
+        part[2 * wv][lane] = (keep[0][0] + keep[0][1]) + (keep[0][2] + keep[0][3]);
+        part[2 * wv + 1][lane] = (keep[0][4] + keep[0][5]) + (keep[0][6] + keep[0][7]);
+        if (q == 0) red[0][wv][r] = mx;
+    } else {
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        if (q == 0) { red[0][wv][r] = mx; red[1][wv][r] = sum; }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w2 = 0; w2 < NW; w2++) mx = fmaxf(mx, red[0][w2][r]);
+    int e = 0;
+    if (mx > 0.0f && mx < __builtin_huge_valf()) {
+        int ex;
+        (void)frexpf(mx, &ex);
+        e = 15 - ex;            // mx * 2^e in [2^14, 2^15)
+    }
+    auto convert = [&](int s, const float(&v)[8]) {
+        f16x8 h, l;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int src = p.interleaved ? ((j & 1) * 4 + (j >> 1)) : j;   // the nibble decoders deliver k = 0,4,1,5,2,6,3,7
+            const float xs = ldexpf(v[src], e);
+            const _Float16 hh = (_Float16)xs;
+            h[j] = hh;
+            l[j] = (_Float16)((xs - (float)hh) * LO_UP);
+        }
+        _Float16 *d = p.af + (((int64_t)blockIdx.y * nsteps + s) * 2) * 512 + lane * 8;
+        *reinterpret_cast<f16x8 *>(d) = h;
+        *reinterpret_cast<f16x8 *>(d + 512) = l;
+    };
+    if (in_regs) {
+#pragma unroll
+        for (int t = 0; t < STEPS; t++)
+            if (s0 + wv + NW * t < s1) convert(s0 + wv + NW * t, keep[t]);
+    } else {
+        for (int s = s0 + wv; s < s1; s += NW) { load8(s, keep[0]); convert(s, keep[0]); }
+    }
+    if (wv != 0) return;
+    float t = 0.0f;
+    if constexpr (STEPS == 1) {   // in the order of the kernel that converts for itself: the two give the same bits
+#pragma unroll
+        for (int h = 0; h < 2 * NW; h++) t += part[h][lane];
+        t += __shfl_xor(t, 16, 64);
+        t += __shfl_xor(t, 32, 64);
+    } else {
+#pragma unroll
+        for (int w2 = 0; w2 < NW; w2++) t += red[1][w2][r];
+    }
+    if (q == 0) p.rows[(int64_t)blockIdx.x * p.m_pad + (int64_t)blockIdx.y * 16 + r] = FragRow{e, t};
+}
+
+template <bool CHAIN>
+hipError_t launch_frag_prep(const FragPrepArgs &a, hipStream_t s)
+{
+    const int steps = a.ks.piece << (a.four_bit ? 2 : 1);
+    const dim3 grid((unsigned)(a.ks.splits * FRAG_NW * a.ks.pieces), (unsigned)((a.m + 15) / 16));
+    if (steps <= 4) hipLaunchKernelGGL((frag_prep_kernel<CHAIN, 1, 4>), grid, dim3(256), 0, s, a);
+    else if (steps <= 8) hipLaunchKernelGGL((frag_prep_kernel<CHAIN, 1, 8>), grid, dim3(512), 0, s, a);
+    else if (steps <= 16) hipLaunchKernelGGL((frag_prep_kernel<CHAIN, 2, 8>), grid, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((frag_prep_kernel<CHAIN, 4, 8>), grid, dim3(512), 0, s, a);
+    return hipGetLastError();
+}
+
+// sum of the K-split partial tiles in split order + bias / activation; four columns per thread
+__global__ void __launch_bounds__(256) frag_reduce_kernel(FragArgs p)
+{
+    const int64_t total = p.m * p.n;
+    if (p.vec4) {
+        const int64_t i4 = (int64_t)blockIdx.x * 256 + threadIdx.x;
+        if (i4 * 4 >= total) return;
+        const int64_t n = i4 * 4 % p.n;
+        const float4 *pp = reinterpret_cast<const float4 *>(p.part) + i4;
+        float4 d = pp[0];
+        for (int z = 1; z < p.ks.splits; z++) {
+            const float4 t = pp[(int64_t)z * (total / 4)];
+            d.x += t.x; d.y += t.y; d.z += t.z; d.w += t.w;
+        }
+        float r[4] = {d.x, d.y, d.z, d.w};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (p.bias) r[j] = r[j] + p.bias[n + j];
+            r[j] = fnn_activation(r[j], p.act);
+        }
+        reinterpret_cast<float4 *>(p.out)[i4] = make_float4(r[0], r[1], r[2], r[3]);
+        if (p.residual) {
+            const float4 q = reinterpret_cast<const float4 *>(p.residual)[i4];
+            reinterpret_cast<float4 *>(p.sum_out)[i4] = make_float4(r[0] + q.x, r[1] + q.y, r[2] + q.z, r[3] + q.w);
+        }
+        return;
+    }
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= total) return;
+    const int64_t n = i % p.n;
+    float d = p.part[i];
+    for (int z = 1; z < p.ks.splits; z++) d += p.part[(int64_t)z * total + i];
+    if (p.bias) d = d + p.bias[n];
+    d = fnn_activation(d, p.act);
+    p.out[i] = d;
+    if (p.residual) p.sum_out[i] = d + p.residual[i];
+}
+
+// fragment-major copy of the packed words; null when it does not exist and this call may not build it
+int frag_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, int64_t kblocks, const uint32_t **out)
+{
+    *out = nullptr;
+    fnn_hip_weight *wm = const_cast<fnn_hip_weight *>(w);
+    if (!wm->words_fr && !fnn_ctx_no_alloc(ctx)) {
+        const int64_t pieces = (w->rows + 15) / 16 * kblocks * 64;
+        if (hipMalloc((void **)&wm->words_fr, (size_t)pieces * 16) != hipSuccess)
+            return fnn_ctx_fail(ctx, FNN_ERR_MEMORY, "out of device memory (fragment-major weight rows)");
+        int64_t blocks = (pieces + 255) / 256;
+        if (blocks > 4096) blocks = 4096;
+        hipLaunchKernelGGL(frag_words_kernel, dim3((unsigned)blocks), dim3(256), 0, s, w->words, w->rows, w->kp, kblocks,
+                           reinterpret_cast<u32x4 *>(wm->words_fr));
+        if (hipGetLastError() != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, "building the fragment-major weight rows failed");
+    }
+    *out = wm->words_fr;
+    return FNN_OK;
+}
+
+struct FragPlan {
+    int mb, nb, rblocks;
+    int op_mb, op_nb;            // the tiles when the operand is in place (the same unless direct)
+    FragSplit ks;
+    int64_t m_pad;
+    bool four_bit, direct;       // direct: activations converted by the MatMul kernel (then mb, nb, tiles are that kernel's)
+    size_t op_bytes, ws_bytes;   // activation fragments; with the row tables behind them
+};
+
+// Microseconds a launch form takes: least squares over 6 500 drawn shapes (M 5..2048, K 256..8192, N 256..16384, every type;
+// 7 to 9 % mean error, and the form they choose is 3.5 % off the best one on average).  R: rounds of workgroups over the
+// 256 CUs (tiles of more than four 16 x 16 blocks fill a CU's registers alone, smaller ones overlap); then, per workgroup,
+// operand bytes through the L1 (64 B/clk) and matrix-core time; per call the preparation, the K split's second launch and
+// partials, output and weight bytes, and what an activation operand beyond an XCD's L2 (4 MB) costs to read again.
+struct FragShape { int mb, nb; };
+constexpr FragShape kTwoLaunch[] = {{1, 1}, {1, 2}, {2, 2}, {2, 4}, {3, 4}, {4, 4}};
+constexpr FragShape kDirect[] = {{1, 1}, {1, 2}, {1, 4}};
+
+float two_launch_us(FragShape t, int splits, int64_t m, int64_t n, int kblocks, bool four)
+{
+    const float kpb = four ? 128.f : 64.f, spb = four ? 4.f : 2.f, area = (float)(t.mb * t.nb);
+    const float wgs = (float)((m + 16 * t.mb - 1) / (16 * t.mb)) * (float)((n + 16 * t.nb - 1) / (16 * t.nb)) * (float)splits, x = wgs / 256.f;
+    const float cx = (float)(int)(x + 0.99999f);
+    float r = area > 4.f ? cx : (x <= 4.f ? 0.5f * (cx + x) : x + 0.25f);
+    if (r < 1.f) r = 1.f;
+    const int kps = (kblocks + splits - 1) / splits;
+    const float seg = (float)((kps + FRAG_NW - 1) / FRAG_NW), mn = (float)m * (float)n;
+    const float bytes = seg * 8.f * ((float)t.mb * 64.f * kpb + (float)t.nb * 1024.f) / 1e5f, mfma = seg * spb * area * 64.f / 2400.f;
+    const float operand = 4.f * (float)m * (float)kblocks * kpb;
+    const float again = operand > 4e6f ? wgs * seg * 8.f * (float)t.mb * 64.f * kpb / 1e8f * (1.f - 4e6f / operand) : 0.f;
+    return 7.223f + r * (0.4467f * bytes + 0.8562f * mfma + 0.0369f * area) + 0.4663f * (float)m * (float)kblocks * kpb * 8.f / 1e6f +
+           (splits > 1 ? 2.559f + 0.0702f * mn * 8.f * (float)splits / 1e6f : 0.f) + 0.7313f * mn * 4.f / 1e6f +
+           0.0576f * (float)n * (float)kblocks * 64.f / 1e6f + 3.519f * again;
+}
+
+// negative: the form does not apply.  Its eight-step variant (K of 1025 .. 2048) needs a CU's registers per workgroup and
+// pays only for small tiles in about one round; from there on the second launch is the better form at every size.
+float direct_us(FragShape t, int64_t m, int64_t n, int kblocks, bool four)
+{
+    const int steps = (kblocks + FRAG_NW - 1) / FRAG_NW * (four ? 4 : 2), padded = steps <= 2 ? 2 : (steps <= 4 ? 4 : 8);
+    const int64_t wgs = ((m + 16 * t.mb - 1) / (16 * t.mb)) * ((n + 16 * t.nb - 1) / (16 * t.nb));
+    if (steps > 8 || (steps > 4 && (wgs > 320 || t.mb * t.nb > 2))) return -1.f;
+    const float x = (float)wgs / 256.f, cx = (float)(int)(x + 0.99999f);
+    float r = padded * t.mb >= 8 || t.mb * t.nb >= 8 ? cx : (x <= 4.f ? 0.5f * (cx + x) : x + 0.25f);
+    if (r < 1.f) r = 1.f;
+    const float kpb = four ? 128.f : 64.f, seg = (float)((kblocks + FRAG_NW - 1) / FRAG_NW);
+    const float bytes = seg * 8.f * ((float)t.mb * 64.f * kpb + (float)t.nb * 1024.f) / 1e5f;
+    return 4.04f + r * (0.8454f * bytes + 0.032f * (float)(padded * t.mb * t.nb)) + 0.5851f * (float)m * (float)n * 4.f / 1e6f + 0.1147f * (float)(padded * t.mb);
+}
+
+// ... and what the LDS-tiled kernels (digit planes, f16 tiles) take at M >= 33: the same kind of fit, 9 % mean error.  A row
+// length that their 16-byte pieces do not fit (ragged) costs them a re-strided operand.
+float tiled_us(bool integer, bool ragged, int64_t m, int64_t n, int64_t k)
+{
+    static const float c[4][6] = {{10.163f, 4.064f, 1.418f, 0.096f, 1.893f, 1.114f},   // other types
+                                  {9.871f, 3.847f, 1.779f, 0.193f, 3.608f, 1.908f},    //   ragged rows
+                                  {10.38f, 2.553f, 2.196f, 0.051f, 2.142f, 1.186f},    // I8, I4, U4
+                                  {10.507f, 2.434f, 2.295f, 0.019f, 3.81f, 1.786f}};   //   ragged rows
+    const float *q = c[(integer ? 2 : 0) + (ragged ? 1 : 0)], fm = (float)m, fn = (float)n, fk = (float)k;
+    return q[0] + q[1] * fm * fn * fk / 1e9f + q[2] * fm * fn / 1e6f + q[3] * fn * fk / 1e6f + q[4] * fm * fk / 1e6f + q[5] * fk / 1e3f;
+}
+
+// an option that names another kernel or its shape keeps the calls with that kernel
+bool options_untouched(fnn_hip_ctx *ctx)
+{
+    static const int opts[][2] = {{FNN_OPT_TILE_SHAPE, -1}, {FNN_OPT_TILE_SPLIT, 0}, {FNN_OPT_TILE_STAGES, 0}, {FNN_OPT_TILE_MIN_M, 5}, {FNN_OPT_GEMM_INT8, 1},
+                                  {FNN_OPT_GEMM_INT8_MIN_M, 17}, {FNN_OPT_DIGIT_PLANES, 0}, {FNN_OPT_STREAM_MIN_M, 17}, {FNN_OPT_STREAM_MAX_M, 32},
+                                  {FNN_OPT_STREAM_SHAPE, 0}, {FNN_OPT_ROWS16_ROW_TILES, 0}, {FNN_OPT_ROWS16_MIN_M, 9}, {FNN_OPT_GEMV_ROW_TILES, 0},
+                                  {FNN_OPT_GEMV_INT8, 1}, {FNN_OPT_GEMV_INT8_MAX_M, 8}};
+    for (const auto &o : opts)
+        if (fnn_ctx_option(ctx, o[0]) != o[1]) return false;
+    return true;
+}
+
+// The launch for an [M, K] x [N, K]^T product with this weight; false: the call is not this kernel's.  The same for every
+// call of the same sizes, so that the MatMul before can prepare the operand.
+bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, FragPlan *out)
+{
+    const int64_t opt = fnn_ctx_option(ctx, FNN_OPT_FRAGMENT);
+    if (opt < 0 || (flags & (FNN_FLAG_ACT_F16_SINGLE | FNN_FLAG_ACT_QUANT | FNN_FLAG_FORCE_GENERIC | FNN_FLAG_PREFER_FMA))) return false;
+    const int dt = w->dtype;
+    const int64_t n = w->rows, k = w->inner;
+    if (dt < FNN_DT_I8 || dt > FNN_DT_F4 || m < 1 || m > (1 << 16) || n < 1 || n > (1 << 22) || k < 1 || k > (1 << 20)) return false;
+    FragPlan f = {};
+    f.four_bit = dt == FNN_DT_I4 || dt == FNN_DT_U4 || dt == FNN_DT_F4;
+    f.ks.kblocks = (int)((w->kp + 15) / 16);
+    const bool integer = dt == FNN_DT_I8 || dt == FNN_DT_I4 || dt == FNN_DT_U4;
+    const int direct_steps = (f.ks.kblocks + FRAG_NW - 1) / FRAG_NW * (f.four_bit ? 4 : 2);
+    const bool direct_ok = m * k < (int64_t)1 << 29;   // (32-bit buffer offsets)
+    int splits = 1;
+    if (opt > 0) {
+        f.mb = (int)(opt & 15); f.nb = (int)((opt >> 4) & 15);
+        splits = (int)((opt >> 8) & 15) > 0 ? (int)((opt >> 8) & 15) : 1;
+        f.direct = (opt >> 15) & 1;
+        bool known = false;
+        if (f.direct) {
+            for (FragShape t : kDirect) known |= t.mb == f.mb && t.nb == f.nb;
+            known &= direct_ok && direct_steps <= 8 && (direct_steps <= 4 || f.mb * f.nb <= 2);
+            splits = 1;
+        } else {
+            for (FragShape t : kTwoLaunch) known |= t.mb == f.mb && t.nb == f.nb && !(f.four_bit && t.mb * t.nb > 12);
+        }
+        if (!known) return false;
+    } else {
+        // Up to 16 rows of whole 16-byte pieces the one-launch kernels for few rows are ahead (up to four rows everywhere,
+        // beyond where a segment is longer than four steps: 5 .. 8 rows F8 832 x 5749 5.4 us either way, 9 .. 16 rows
+        // 960 x 5454 U8 7.4 against 5.7); ragged rows have no such kernel (2 x 4728 x 11904 F4: 233 us there, 14 here).
+        const bool ragged = w->kp % 4 != 0 || k % 8 != 0;
+        if (m > 2048 || !options_untouched(ctx)) return false;
+        if (m <= 16 && !ragged && (m <= 4 || direct_steps > 4 || (m <= 8 && integer))) return false;
+        float best = 1e30f;
+        if (direct_ok)
+            for (FragShape t : kDirect) {
+                const float us = direct_us(t, m, n, f.ks.kblocks, f.four_bit);
+                if (us >= 0.f && us < best) { best = us; f.mb = t.mb; f.nb = t.nb; f.direct = true; }
+            }
+        if (m > 16 || ragged)
+            for (FragShape t : kTwoLaunch) {
+                if ((t.mb - 1) * 16 >= m || (f.four_bit && t.mb * t.nb > 12)) continue;   // (a nibble block's four steps and that tile do not fit the registers)
+                const int64_t wgs = ((m + 16 * t.mb - 1) / (16 * t.mb)) * ((n + 16 * t.nb - 1) / (16 * t.nb));
+                for (int sp : {1, 2, 4, 8}) {
+                    if (sp > 1 && (wgs * sp > 1024 || sp * 8 > f.ks.kblocks)) break;
+                    const float us = two_launch_us(t, sp, m, n, f.ks.kblocks, f.four_bit);
+                    if (us < best) { best = us; f.mb = t.mb; f.nb = t.nb; f.direct = false; splits = sp; }
+                }
+            }
+        // (the margin: where the two are about equal the fits decide at random, and what was there stays)
+        if (best > 1e29f || (m >= 33 && best > 0.93f * tiled_us(integer, ragged, m, n, k))) return false;
+    }
+    if (splits > f.ks.kblocks) splits = f.ks.kblocks;
+    f.ks.kb_per_split = (f.ks.kblocks + splits - 1) / splits;
+    f.ks.splits = (f.ks.kblocks + f.ks.kb_per_split - 1) / f.ks.kb_per_split;
+    f.ks.seg = (f.ks.kb_per_split + FRAG_NW - 1) / FRAG_NW;
+    f.ks.seg_last = (f.ks.kblocks - (f.ks.splits - 1) * f.ks.kb_per_split + FRAG_NW - 1) / FRAG_NW;
+    f.rblocks = (int)((n + 15) / 16);
+    f.op_mb = f.mb; f.op_nb = f.nb;
+    if (f.direct) {
+        float best = 1e30f;
+        for (FragShape t : kTwoLaunch) {
+            const float us = (t.mb - 1) * 16 >= m || (f.four_bit && t.mb * t.nb > 12) ? 1e30f : two_launch_us(t, 1, m, n, f.ks.kblocks, f.four_bit);
+            if (us < best) { best = us; f.op_mb = t.mb; f.op_nb = t.nb; }
+        }
+    }
+    f.m_pad = (m + f.op_mb * 16 - 1) / (f.op_mb * 16) * (f.op_mb * 16);
+    // pieces of eight steps (256 k-values): a preparation workgroup per piece and row block
+    const int seg = f.ks.seg > f.ks.seg_last ? f.ks.seg : f.ks.seg_last, eight = f.four_bit ? 2 : 4;
+    f.ks.piece = f.op_mb * f.op_nb <= 8 && seg > eight ? eight : seg;
+    f.ks.pieces = (seg + f.ks.piece - 1) / f.ks.piece;
+    f.op_bytes = (size_t)f.m_pad * f.ks.kblocks * (f.four_bit ? 128 : 64) * 4;
+    f.ws_bytes = f.op_bytes + (size_t)f.ks.splits * FRAG_NW * f.ks.pieces * f.m_pad * sizeof(FragRow);
+    *out = f;
+    return true;
+}
+
+FragPrepArgs prep_args(const FragPlan &f, const fnn_hip_weight *w, int64_t m, void *ws)
+{
+    FragPrepArgs a = {};
+    a.af = (_Float16 *)ws;
+    a.rows = (FragRow *)((char *)ws + f.op_bytes);
+    a.m = m; a.k = w->inner; a.m_pad = f.m_pad;
+    a.ks = f.ks;
+    a.four_bit = f.four_bit ? 1 : 0;
+    a.interleaved = w->dtype == FNN_DT_I4 || w->dtype == FNN_DT_U4 ? 1 : 0;
+    return a;
+}
+
+}  // namespace
+
+int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, bool *handled)
+{
+    *handled = false;
+    FragPlan f;
+    if (q.words != w->words || q.n != w->rows || q.k != w->inner || !frag_plan(ctx, w, q.m, flags, &f)) return FNN_OK;
+    FragArgs p = {};
+    int rc;
+    if ((rc = frag_words(ctx, s, w, f.ks.kblocks, &p.wf))) return rc;
+    if (!p.wf) return FNN_OK;
+    p.ks = f.ks; p.rblocks = f.rblocks; p.m_pad = f.m_pad; p.k = q.k;
+    p.scales = q.scales; p.zeros = q.zeros; p.bias = q.bias; p.out = q.out;
+    p.m = q.m; p.n = q.n; p.act = q.act;
+    if (FnnResidualIo *res = fnn_ctx_residual_io(ctx); res->residual && res->of_out == q.out && res->elems == (uint64_t)(q.m * q.n)) {
+        p.residual = res->residual; p.sum_out = res->sum_out;
+        res->used = 1;
+    }
+    p.vec4 = q.n % 4 == 0 && !((reinterpret_cast<uintptr_t>(p.out) | reinterpret_cast<uintptr_t>(p.residual) | reinterpret_cast<uintptr_t>(p.sum_out) |
+                                reinterpret_cast<uintptr_t>(p.scales) | reinterpret_cast<uintptr_t>(p.zeros) | reinterpret_cast<uintptr_t>(p.bias)) & 15);
+
+    // What travels between the MatMuls of a plan (range_io.h): the operand may be in place, and the next one's may be asked
+    // for.  From 33 rows on: below, the MatMuls that convert for themselves are ahead of a reduction launch each.  (Integer
+    // weights as the next ones: their MatMul prepares its own operand.)
+    FnnPrepIo *pio = fnn_ctx_prep_io(ctx);
+    FnnPreparedOperand *have = fnn_ctx_prepared(ctx);
+    const int interleaved = w->dtype == FNN_DT_I4 || w->dtype == FNN_DT_U4 ? 1 : 0;
+    const bool handed = pio->offered && have->buffer && have->fragments == 1 + (f.four_bit ? 1 : 0) && have->a == q.a && have->m == q.m && have->k == q.k &&
+                        have->rows_pad == f.m_pad && have->kpad == f.ks.kb_per_split && have->interleaved == interleaved;
+    const bool direct = f.direct && !handed;
+    const int mb = direct ? f.mb : f.op_mb, nb = direct ? f.nb : f.op_nb;
+    p.mtiles = (int)((q.m + mb * 16 - 1) / (mb * 16));
+    p.ntiles = (int)((q.n + nb * 16 - 1) / (nb * 16));
+    p.by_mtiles = fast_div((uint32_t)p.mtiles);
+    p.by_splits = fast_div((uint32_t)f.ks.splits);
+    const int own_slot = handed ? have->slot : 0, next_slot = own_slot == 0 ? 4 : 0;
+    void *ws0 = handed ? have->buffer : nullptr, *ws1 = nullptr, *next_ws = nullptr;
+    FragPlan nf;
+    const bool chain = pio->next_w && q.m >= 33 && p.vec4 && q.n % 8 == 0 && (pio->next_a == q.out || (p.residual && pio->next_a == p.sum_out)) &&
+                       pio->next_w->inner == q.n && !fnn_ctx_static_mode(ctx) &&
+                       (pio->next_w->dtype == FNN_DT_U8 || pio->next_w->dtype == FNN_DT_F8 || pio->next_w->dtype == FNN_DT_F8R || pio->next_w->dtype == FNN_DT_F4) &&
+                       frag_plan(ctx, pio->next_w, q.m, pio->next_flags, &nf) && nf.ks.piece << (nf.four_bit ? 2 : 1) <= 32 &&
+                       fnn_ctx_ensure_tmp(ctx, next_slot, nf.ws_bytes, &next_ws) == FNN_OK && next_ws;
+    if (!handed && !direct && (rc = fnn_ctx_ensure_tmp(ctx, 0, f.ws_bytes, &ws0))) return rc;
+    if ((chain || f.ks.splits > 1) && (rc = fnn_ctx_ensure_tmp(ctx, 1, (size_t)f.ks.splits * q.m * q.n * 4, &ws1))) return rc;
+    *have = FnnPreparedOperand{};   // (whatever was there is used by this call or stale)
+    pio->consumed = handed ? 1 : 0;
+
+    if (direct) p.a = q.a;
+    else if (!ws0) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, "fragment MatMul: no operand buffer");
+    FragPrepArgs a = prep_args(f, w, q.m, ws0);
+    a.a = q.a;
+    hipError_t e = handed || direct ? hipSuccess : launch_frag_prep<false>(a, s);
+    if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
+    p.af = a.af; p.rows = a.rows;
+    p.part = (float *)ws1;
+    switch (w->dtype) {
+    case FNN_DT_I8: e = fnn_frag_launch_i8(mb, nb, p, s); break;
+    case FNN_DT_I4: e = fnn_frag_launch_i4(mb, nb, p, s); break;
+    case FNN_DT_U8: e = fnn_frag_launch_u8(mb, nb, p, s); break;
+    case FNN_DT_U4: e = fnn_frag_launch_u4(mb, nb, p, s); break;
+    case FNN_DT_F8: e = fnn_frag_launch_f8(mb, nb, p, s); break;
+    case FNN_DT_F8R: e = fnn_frag_launch_f8r(mb, nb, p, s); break;
+    default: e = fnn_frag_launch_f4(mb, nb, p, s); break;
+    }
+    if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
+    if (chain) {
+        FragPrepArgs na = prep_args(nf, pio->next_w, q.m, next_ws);
+        na.prev = p;
+        na.use_sum = pio->next_a == q.out ? 0 : 1;
+        e = launch_frag_prep<true>(na, s);
+        if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
+        have->a = pio->next_a; have->buffer = next_ws; have->slot = next_slot;
+        have->m = q.m; have->k = q.n; have->kpad = nf.ks.kb_per_split; have->rows_pad = nf.m_pad;
+        have->fragments = 1 + (nf.four_bit ? 1 : 0); have->interleaved = na.interleaved;
+        pio->produced = 1;
+    } else if (p.part) {
+        const int64_t items = p.vec4 ? q.m * q.n / 4 : q.m * q.n;
+        hipLaunchKernelGGL(frag_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, p);
+        if ((e = hipGetLastError()) != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
+    }
+    *handled = true;
+    return FNN_OK;
+}

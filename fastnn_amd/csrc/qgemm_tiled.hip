@@ -596,7 +596,7 @@ int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QM
     FnnPrepIo *pio = fnn_ctx_prep_io(ctx);
     FnnPreparedOperand *have = fnn_ctx_prepared(ctx);
     constexpr int kInterleaved = DecH<DT>::INTERLEAVED ? 1 : 0;
-    const bool handed = pio->offered && !dense && have->buffer && have->a == q.a && have->m == M && have->k == K && have->kpad == kpad &&
+    const bool handed = pio->offered && !dense && have->buffer && !have->fragments && have->a == q.a && have->m == M && have->k == K && have->kpad == kpad &&
                         have->rows_pad == rows_pad && have->precise == (precise ? 1 : 0) && have->interleaved == kInterleaved;
     const int own_slot = handed ? have->slot : 0;
     void *ws0 = handed ? have->buffer : nullptr, *ws1 = nullptr;

@@ -72,6 +72,7 @@ struct FnnPreparedOperand {
     int slot = -1;                  // workspace slot of buffer
     long long m = 0, k = 0, kpad = 0, rows_pad = 0;
     int precise = 0, interleaved = 0;
+    int fragments = 0;              // 0: rows for the LDS tiles; 1, 2: fragments for weights of 8, 4 bits (then kpad = k blocks per split)
 };
 FnnPreparedOperand *fnn_ctx_prepared(fnn_hip_ctx *ctx);
 

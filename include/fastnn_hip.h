@@ -164,7 +164,13 @@ enum {
                                   /* 4096 x 4096 5.90 -> 5.40), built on the weight's first such call and kept with it (once more  */
                                   /* the packed bytes; rows of whole 64-byte blocks only; a call that may not allocate uses the    */
                                   /* row-major words until the copy exists); 0 = row-major words only                              */
-    FNN_OPT_COUNT = 24
+    FNN_OPT_FRAGMENT = 24,        /* the MatMul kernels on fragment-major operands (per-channel types; both operands lie in memory  */
+                                  /* in the order the matrix cores take them; a second device copy of the packed words, built on  */
+                                  /* the weight's first such call): 0 (default) = by rule (any M with rows of ragged length, from   */
+                                  /* M = 17, or 5 to 9 for short rows, with aligned ones, as far up as it is the faster form), -1 =  */
+                                  /* off, else the shape, (direct << 15) | (K splits << 8) | (16-column blocks << 4) | (16-row       */
+                                  /* blocks); a shape that does not exist for the call is ignored                                   */
+    FNN_OPT_COUNT = 25
 };
 int fnn_hip_set_option(fnn_hip_ctx *ctx, int option, int64_t value);
 int fnn_hip_get_option(fnn_hip_ctx *ctx, int option, int64_t *value);

@@ -1,0 +1,44 @@
+"""The MatMul kernels on fragment-major operands (FNN_OPT_FRAGMENT) against the oracle, at the edges of their tiles: rows and
+columns around multiples of 16, K around the k blocks (64 or 128 values), the pieces of 256 values and the eight waves."""
+import numpy as np
+import pytest
+
+import fastnn_amd
+from fastnn_amd import lib as flib
+from gpu_common import assert_close, to_oracle
+
+pytestmark = pytest.mark.gpu
+TYPES = [flib.DT_I8, flib.DT_I4, flib.DT_U8, flib.DT_U4, flib.DT_F8, flib.DT_F8R, flib.DT_F4]
+SHAPES = [(mb, nb, sp, 0) for mb, nb in ((1, 1), (1, 2), (2, 2), (2, 4), (3, 4), (4, 4)) for sp in (1, 3)] + [(1, nb, 1, 1) for nb in (1, 2, 4)]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    with fastnn_amd.HipContext(0) as c:
+        yield c
+
+
+@pytest.mark.parametrize("dt", TYPES)
+@pytest.mark.parametrize("m,k,n", [(1, 63, 15), (16, 128, 16), (17, 1000, 33), (31, 1025, 64), (49, 2048, 130), (65, 2600, 257), (130, 515, 68)])
+def test_every_shape_of_the_fragment_kernels(ctx, orc, dt, m, k, n):
+    rng = np.random.default_rng(9000 + dt * 7 + m)
+    pw = fastnn_amd.quantize_weights(dt, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    a[:, ::61] *= 100.0
+    a[m // 2] = 0.0
+    bias = (rng.standard_normal(n) * 0.1).astype(np.float32)
+    want = orc.qmatmul(to_oracle(orc, pw), a, order=2, bias=bias, act=flib.ACT_SILU)
+    h = ctx.register(pw)
+    try:
+        results = []
+        for mb, nb, sp, direct in [(0, 0, 0, 0)] + SHAPES:
+            ctx.set_option(flib.OPT_FRAGMENT, direct << 15 | sp << 8 | nb << 4 | mb)
+            got = ctx.qmatmul(h, a, n, bias=bias, act=flib.ACT_SILU)
+            assert_close(got, want, 2e-5, f"{mb}x{nb} splits {sp} direct {direct}")
+            if sp == 1 and (direct or mb * nb <= 4) and k <= 1024:
+                results.append(got)
+        for r in results[1:]:      # the same segments of K: the same bits, whoever converts the activations
+            assert np.array_equal(r, results[0])
+    finally:
+        ctx.set_option(flib.OPT_FRAGMENT, 0)
+        ctx.release(h)
