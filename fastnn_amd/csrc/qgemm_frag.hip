@@ -240,25 +240,6 @@ __global__ void __launch_bounds__(256) frag_reduce_kernel(FragArgs p)
     if (p.residual) p.sum_out[i] = d + p.residual[i];
 }
 
-// fragment-major copy of the packed words; null when it does not exist and this call may not build it
-int frag_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, int64_t kblocks, const uint32_t **out)
-{
-    *out = nullptr;
-    fnn_hip_weight *wm = const_cast<fnn_hip_weight *>(w);
-    if (!wm->words_fr && !fnn_ctx_no_alloc(ctx)) {
-        const int64_t pieces = (w->rows + 15) / 16 * kblocks * 64;
-        if (hipMalloc((void **)&wm->words_fr, (size_t)pieces * 16) != hipSuccess)
-            return fnn_ctx_fail(ctx, FNN_ERR_MEMORY, "out of device memory (fragment-major weight rows)");
-        int64_t blocks = (pieces + 255) / 256;
-        if (blocks > 4096) blocks = 4096;
-        hipLaunchKernelGGL(frag_words_kernel, dim3((unsigned)blocks), dim3(256), 0, s, w->words, w->rows, w->kp, kblocks,
-                           reinterpret_cast<u32x4 *>(wm->words_fr));
-        if (hipGetLastError() != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, "building the fragment-major weight rows failed");
-    }
-    *out = wm->words_fr;
-    return FNN_OK;
-}
-
 struct FragPlan {
     int mb, nb, rblocks;
     int op_mb, op_nb;            // the tiles when the operand is in place (the same unless direct)
@@ -427,6 +408,25 @@ FragPrepArgs prep_args(const FragPlan &f, const fnn_hip_weight *w, int64_t m, vo
 
 }  // namespace
 
+// fragment-major copy of the packed words; null when it does not exist and this call may not build it
+int fnn_fragment_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, int64_t kblocks, const uint32_t **out)
+{
+    *out = nullptr;
+    fnn_hip_weight *wm = const_cast<fnn_hip_weight *>(w);
+    if (!wm->words_fr && !fnn_ctx_no_alloc(ctx)) {
+        const int64_t pieces = (w->rows + 15) / 16 * kblocks * 64;
+        if (hipMalloc((void **)&wm->words_fr, (size_t)pieces * 16) != hipSuccess)
+            return fnn_ctx_fail(ctx, FNN_ERR_MEMORY, "out of device memory (fragment-major weight rows)");
+        int64_t blocks = (pieces + 255) / 256;
+        if (blocks > 4096) blocks = 4096;
+        hipLaunchKernelGGL(frag_words_kernel, dim3((unsigned)blocks), dim3(256), 0, s, w->words, w->rows, w->kp, kblocks,
+                           reinterpret_cast<u32x4 *>(wm->words_fr));
+        if (hipGetLastError() != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, "building the fragment-major weight rows failed");
+    }
+    *out = wm->words_fr;
+    return FNN_OK;
+}
+
 int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, bool *handled)
 {
     *handled = false;
@@ -434,7 +434,7 @@ int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, c
     if (q.words != w->words || q.n != w->rows || q.k != w->inner || !frag_plan(ctx, w, q.m, flags, &f)) return FNN_OK;
     FragArgs p = {};
     int rc;
-    if ((rc = frag_words(ctx, s, w, f.ks.kblocks, &p.wf))) return rc;
+    if ((rc = fnn_fragment_words(ctx, s, w, f.ks.kblocks, &p.wf))) return rc;
     if (!p.wf) return FNN_OK;
     p.ks = f.ks; p.rblocks = f.rblocks; p.m_pad = f.m_pad; p.k = q.k;
     p.scales = q.scales; p.zeros = q.zeros; p.bias = q.bias; p.out = q.out;

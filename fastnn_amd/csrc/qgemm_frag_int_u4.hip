@@ -1,0 +1,4 @@
+// Fragment-major MatMul on the int8 matrix cores (qgemm_frag_int_impl.h), weight type U4.
+#include "mfma.h"
+#include "qgemm_frag_int_impl.h"
+hipError_t fnn_frag_int_launch_u4(int mb, int nb, bool digits, const FragIntArgs &p, hipStream_t s) { return frag_int_launch<FNN_DT_U4>(mb, nb, digits, p, s); }

@@ -463,9 +463,10 @@ namespace {
 template <int DT>
 hipError_t run_i8_gemm(const uint32_t *words, int64_t kp, int64_t rows_total, int64_t n0, int64_t n, const int8_t *a8, int64_t m,
                        int64_t rows_pad, int64_t kpad, int32_t *c, int64_t ldc, hipStream_t s, int splits = 1, const TileArgs *conv = nullptr,
-                       bool small_tiles = false, int form = 0)
+                       bool small_tiles = false, int form = 0, const TileArgs *formula = nullptr)
 {
     TileArgs t = {};
+    if (formula) t = *formula;   // (c is null: the I8-activation formula runs in the kernel)
     if (conv) { t.cv = conv->cv; t.scales = conv->scales; t.zeros = conv->zeros; t.bias = conv->bias; t.act = conv->act; }
     t.words = words + n0 * kp;
     t.zero_chunk = words + rows_total * kp;   // the zeroed margin behind the last row
@@ -667,9 +668,24 @@ int fnn_fp8_actquant_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weig
     return FNN_OK;
 }
 
+int fnn_row_qsum(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const int32_t **qsum)
+{
+    fnn_hip_weight *wm = const_cast<fnn_hip_weight *>(w);
+    if (!wm->row_qsum) {
+        if (fnn_ctx_no_alloc(ctx)) return fnn_ctx_fail(ctx, FNN_ERR_MEMORY, "first use of re-strided weight rows while allocation is not allowed (graph capture, fnn_hip_qmatmul_static)");
+        if (hipMalloc((void **)&wm->row_qsum, (size_t)w->rows * 4 + 64) != hipSuccess)
+            return fnn_ctx_fail(ctx, FNN_ERR_MEMORY, "out of device memory (row sums)");
+        hipError_t e = launch_row_qsum(w, wm->row_qsum, s);
+        if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
+    }
+    *qsum = wm->row_qsum;
+    return FNN_OK;
+}
+
 int fnn_i8_tiled_matmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const I8ActArgs &p, bool *handled)
 {
     *handled = false;
+    if (int rc0 = fnn_frag_i8act(ctx, s, w, p, handled); rc0 || *handled) return rc0;
     if (w->dtype != FNN_DT_I8 && w->dtype != FNN_DT_I4) return FNN_OK;
     if (reinterpret_cast<uintptr_t>(p.words) & 15) return FNN_OK;
     if (p.m < 1 || p.m > (1 << 22) || p.n > (1 << 24) || p.k > (1 << 20)) return FNN_OK;
@@ -698,15 +714,9 @@ int fnn_i8_tiled_matmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w
     if (splits > 16) splits = 16;
     if (splits < 1) splits = 1;
     if ((rc = fnn_ctx_ensure_tmp(ctx, 0, q_off + (size_t)rows_pad * 4 + 256, &ws0))) return rc;
-    if ((rc = fnn_ctx_ensure_tmp(ctx, 1, (size_t)splits * p.m * p.n * 4 + 256, &ws1))) return rc;
-    fnn_hip_weight *wm = const_cast<fnn_hip_weight *>(w);
-    if (!wm->row_qsum) {
-        if (fnn_ctx_no_alloc(ctx)) return fnn_ctx_fail(ctx, FNN_ERR_MEMORY, "first use of re-strided weight rows while allocation is not allowed (graph capture, fnn_hip_qmatmul_static)");
-        if (hipMalloc((void **)&wm->row_qsum, (size_t)w->rows * 4 + 64) != hipSuccess)
-            return fnn_ctx_fail(ctx, FNN_ERR_MEMORY, "out of device memory (row sums)");
-        hipError_t e = launch_row_qsum(w, wm->row_qsum, s);
-        if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
-    }
+    if (splits > 1 && (rc = fnn_ctx_ensure_tmp(ctx, 1, (size_t)splits * p.m * p.n * 4 + 256, &ws1))) return rc;
+    const int32_t *wsum;
+    if ((rc = fnn_row_qsum(ctx, s, w, &wsum))) return rc;
     const uint32_t *words;
     int64_t kp;
     if ((rc = fnn_aligned_rows(ctx, s, w, &words, &kp))) return rc;
@@ -720,18 +730,25 @@ int fnn_i8_tiled_matmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w
     else
         hipLaunchKernelGGL(i8_rows_operand_kernel<false>, dim3((unsigned)rows_pad), dim3(256), 0, s,
                            reinterpret_cast<const int8_t *>(p.payload + 8), p.m, p.k, kpad, rows_pad, a8, qsum);
+    TileArgs formula = {};
+    if (splits == 1) {   // (with one K range a tile holds whole sums)
+        c = nullptr;
+        formula.act_q = reinterpret_cast<const float *>(p.payload);
+        formula.code_sum = qsum; formula.word_sum = wsum; formula.acc_out = p.acc_out; formula.k_values = p.k;
+        formula.scales = p.scales; formula.zeros = p.zeros; formula.bias = p.bias; formula.act = p.act; formula.out = p.out;
+    }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
-        e = w->dtype == FNN_DT_I8 ? run_i8_gemm<FNN_DT_I8>(words, kp, w->rows, 0, p.n, a8, p.m, rows_pad, kpad, c, p.n, s, splits, nullptr, false, form)
-                                  : run_i8_gemm<FNN_DT_I4>(words, kp, w->rows, 0, p.n, a8, p.m, rows_pad, kpad, c, p.n, s, splits, nullptr, false, form);
-    if (e == hipSuccess) {
+        e = w->dtype == FNN_DT_I8 ? run_i8_gemm<FNN_DT_I8>(words, kp, w->rows, 0, p.n, a8, p.m, rows_pad, kpad, c, p.n, s, splits, nullptr, false, form, splits == 1 ? &formula : nullptr)
+                                  : run_i8_gemm<FNN_DT_I4>(words, kp, w->rows, 0, p.n, a8, p.m, rows_pad, kpad, c, p.n, s, splits, nullptr, false, form, splits == 1 ? &formula : nullptr);
+    if (e == hipSuccess && c) {
         const int ips = (iters + splits - 1) / splits;
         splits = (iters + ips - 1) / ips;   // as run_i8_gemm rounds it
         const int64_t colb = (p.n + 255) / 256;
         int64_t rowb = (4096 + colb - 1) / colb;   // about 4096 workgroups
         if (rowb > p.m) rowb = p.m;
         if (rowb > 65535) rowb = 65535;
-        hipLaunchKernelGGL(i8_matmul_epilogue_kernel, dim3((unsigned)colb, (unsigned)rowb), dim3(256), 0, s, c, p.payload, qsum, wm->row_qsum,
+        hipLaunchKernelGGL(i8_matmul_epilogue_kernel, dim3((unsigned)colb, (unsigned)rowb), dim3(256), 0, s, c, p.payload, qsum, wsum,
                            p.scales, p.zeros, p.m, p.n, p.k, p.out, p.acc_out, splits, p.bias, p.act);
         e = hipGetLastError();
     }

@@ -19,7 +19,13 @@ struct TileArgs {
     float *out, *part;
     const float *residual;        // split-K reduction only: non-null = sum_out[m,n] = out[m,n] + residual[m,n] as well
     float *sum_out;
-    int32_t *c_i32;               // int8 mode: raw accumulators [m][ldc]
+    int32_t *c_i32;               // int8 mode: raw accumulators [m][ldc], or null:
+    // the I8-activation formula is applied here (out, scales, zeros, bias, act above; activation scale and zero, row sums of
+    // the codes, sums of the weight rows' integers, the exact sums as a second result)
+    const float *act_q = nullptr;
+    const int32_t *code_sum = nullptr, *word_sum = nullptr;
+    int32_t *acc_out = nullptr;
+    int64_t k_values = 0;
     int64_t ldc;
     int64_t m, n, kp, kpad, rows_pad;
     int act, splits, iters, ips, mtiles, ntiles;
@@ -760,6 +766,49 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
         return;
     } else if constexpr (INT8) {
         const int64_t mrow = ((int64_t)mt * (BM / 32) + wm * TM) * 32;
+        if (!FP8 && !p.c_i32) {   // (uniform) one pass instead of a matrix of sums written and read again
+            const float sa = p.act_q[0], za = p.act_q[1], kza = (float)p.k_values * za;
+            float sw[TN], zw[TN], zws[TN], bs[TN];
+#pragma unroll
+            for (int tn = 0; tn < TN; tn++) {
+                int64_t n = n0 + (wn * TN + tn) * 32 + lr;
+                if (n > p.n - 1) n = p.n - 1;
+                sw[tn] = p.scales[n];
+                zw[tn] = p.zeros[n];
+                zws[tn] = za * (float)p.word_sum[n];
+                bs[tn] = p.bias ? p.bias[n] : 0.0f;
+            }
+            const bool has_bias = p.bias != nullptr;
+#pragma unroll
+            for (int tm = 0; tm < TM; tm++) {
+                int qs[16];
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    int64_t m = mrow + tm * 32 + (i / 4) * 8 + h * 4 + (i % 4);
+                    qs[i] = p.code_sum[m > p.m - 1 ? p.m - 1 : m];
+                }
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int64_t m = mrow + tm * 32 + (i / 4) * 8 + h * 4 + (i % 4);
+                    if (m >= p.m) continue;
+                    const float input_sum = (float)qs[i] * sa + kza;
+#pragma unroll
+                    for (int tn = 0; tn < TN; tn++) {
+                        const int64_t n = n0 + (wn * TN + tn) * 32 + lr;
+                        if (n >= p.n) continue;
+                        const float bits = acc[tm][tn][i];
+                        int a = __float_as_int(bits);
+                        if constexpr (DT == FNN_DT_I4) a >>= 4;
+                        const float dot = za != 0.0f ? (float)a * sa + zws[tn] : (float)a * sa;
+                        float v = dot * sw[tn] + zw[tn] * input_sum;
+                        if (has_bias) v = v + bs[tn];
+                        p.out[m * p.n + n] = fnn_activation(v, p.act);
+                        if (p.acc_out) p.acc_out[m * p.n + n] = za != 0.0f ? 0 : a;
+                    }
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int tm = 0; tm < TM; tm++)
 #pragma unroll
