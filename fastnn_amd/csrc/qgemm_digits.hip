@@ -21,6 +21,7 @@
 // depending on the weights' signs and zeros).
 #include "mfma.h"
 #include "dech.h"
+#include "qgemm_wave.h"
 #include "range_io.h"
 
 #include <type_traits>
@@ -40,6 +41,7 @@ struct DigitArgs {
     int *rexp;         // [m_pad] exponent applied to the row, INT_MIN for a row with a non-finite value
     float *xsum;       // [m_pad] sum_k A[m,k]
     int64_t m, k, kpad, rows_pad;
+    int nsteps = 0;    // fragment order (qgemm_wave.h): steps of 32 k-values per operand row
 };
 
 // 4x4 byte transpose: o[j] = byte j of a, b, c, d (selector bytes 0-3 pick from the second operand of v_perm_b32)
@@ -59,17 +61,28 @@ __device__ __forceinline__ void transpose4(uint32_t a, uint32_t b, uint32_t c, u
 // operand layout.  Operand row of (activation row m, plane j): (m / RPB) * 32 + j * RPB + m % RPB, RPB = 32 / DIG, for
 // two and four planes; with three planes ((m / 8) * 3 + j) * 8 + m % 8 (groups of 24 rows: 8 activation rows x 3 planes).
 // IL: the nibble decoders deliver k = 0,2,4,6,1,3,5,7 of each 8, and the activations are stored in that order.
-template <int DIG, bool IL>
+// FRAG (three planes): the fragment order of qgemm_wave_impl.h instead of tile-major rows.
+template <int DIG, bool IL, bool FRAG = false>
 __global__ void __launch_bounds__(256) digit_prep_kernel(DigitArgs p)
 {
     constexpr int RPB = DIG == 3 ? 8 : 32 / DIG;
     constexpr uint32_t BIAS = DIG == 4 ? 0x80808080u : (DIG == 3 ? 0x00808080u : 0x00008080u);
     __shared__ float red[2][4];
-    const int64_t m = blockIdx.x;
+    // (fragment order: eight activation rows share 128-byte lines of a plane; their workgroups go to one XCD)
+    const int64_t m = FRAG && (blockIdx.x | 63u) < gridDim.x ? (blockIdx.x & ~63u) + (blockIdx.x & 7) * 8 + ((blockIdx.x >> 3) & 7) : blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int64_t nchunks = p.kpad / 16;
     const int64_t row0 = DIG == 3 ? (m / 8) * 24 + m % 8 : (m / RPB) * 32 + m % RPB;
-    auto chunk_at = [&](int j, int64_t c) { return p.planes + (((c >> 3) * p.rows_pad + row0 + j * RPB) * KB + (c & 7) * 16); };
+    auto chunk_at = [&](int j, int64_t c) {
+        if constexpr (FRAG) {
+            // chunk of 16 k-values -> (step, half): 32 s + 16 h, or for nibbles 128 b + 64 p + 32 h + 16 t with step 4 b + 2 p + t
+            const int64_t step = IL ? (c >> 3) * 4 + ((c >> 1) & 2) + (c & 1) : c >> 1;
+            const int half = IL ? (int)(c >> 1) & 1 : (int)c & 1;
+            const int64_t r = row0 + j * RPB;
+            return p.planes + (((r >> 5) * p.nsteps + step) * 64 + half * 32 + (r & 31)) * 16;
+        }
+        return p.planes + (((c >> 3) * p.rows_pad + row0 + j * RPB) * KB + (c & 7) * 16);
+    };
     if (m >= p.m) {   // padding rows of the last tile
         const uint4 z = make_uint4(0, 0, 0, 0);
         for (int64_t c = tid; c < nchunks; c += 256)
@@ -166,6 +179,57 @@ __global__ void __launch_bounds__(256) digit_prep_kernel(DigitArgs p)
         p.rexp[m] = all_finite ? e : INT_MIN;
         p.xsum[m] = sum;
     }
+}
+
+// Three planes on the wave tiles (qgemm_wave_impl.h); wk: waves that share a tile.
+template <int DT>
+int run_digits_wave(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int wk, bool *handled)
+{
+    constexpr bool IL = DecI<DT>::INTERLEAVED, W8 = DecI<DT>::WPS == 4;
+    constexpr int RING = WAVE_RING(W8);
+    WaveArgs p = {};
+    int rc;
+    p.kblocks = (int)((w->kp + 15) / 16);
+    if ((rc = fnn_fragment_words(ctx, s, w, p.kblocks, &p.wf))) return rc;
+    if (!p.wf) return FNN_OK;
+    const int64_t kstep = (int64_t)p.kblocks * (W8 ? 2 : 4);        // steps that hold weights
+    p.units = (int)((kstep + RING - 1) / RING);
+    p.units_per_wave = (p.units + wk - 1) / wk;
+    p.nsteps = p.units * RING;
+    const int act_rows = wk == 1 ? 2 * WAVE_ROWS : WAVE_ROWS, cols = wk == 4 ? WAVE_COLS : 2 * WAVE_COLS;
+    p.mtiles = (int)((q.m + act_rows - 1) / act_rows);
+    p.ntiles = (int)((q.n + cols - 1) / cols);
+    p.rblocks = (int)((q.n + 15) / 16);
+    p.tiles = (unsigned)p.mtiles * (unsigned)p.ntiles;
+    p.by_stripe = fast_div((uint32_t)p.ntiles * 4);
+    const int64_t m_pad = (int64_t)p.mtiles * act_rows;
+    const size_t a_bytes = (size_t)m_pad * 3 * p.nsteps * 32;
+    void *ws0 = nullptr;
+    if ((rc = fnn_ctx_ensure_tmp(ctx, 0, a_bytes + (size_t)m_pad * 8, &ws0))) return rc;
+    *fnn_ctx_prepared(ctx) = FnnPreparedOperand{};
+    DigitArgs d;
+    d.a = q.a;
+    d.planes = (int8_t *)ws0;
+    d.rexp = (int *)((char *)ws0 + a_bytes);
+    d.xsum = (float *)(d.rexp + m_pad);
+    d.m = q.m; d.k = q.k; d.kpad = (int64_t)p.nsteps * 32; d.rows_pad = 0;
+    d.nsteps = p.nsteps;
+    hipLaunchKernelGGL((digit_prep_kernel<3, IL, true>), dim3((unsigned)m_pad), dim3(256), 0, s, d);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
+    p.af = d.planes; p.rexp = d.rexp; p.xsum = d.xsum;
+    p.scales = q.scales; p.zeros = q.zeros; p.bias = q.bias; p.out = q.out;
+    p.m = q.m; p.n = q.n; p.act = q.act;
+    if (FnnResidualIo *res = fnn_ctx_residual_io(ctx); res->residual && res->of_out == q.out && res->elems == (uint64_t)(q.m * q.n)) {
+        p.residual = res->residual; p.sum_out = res->sum_out;
+        res->used = 1;
+    }
+    if constexpr (DT == FNN_DT_I8) e = fnn_wave_launch_i8(wk, p, s);
+    else if constexpr (DT == FNN_DT_I4) e = fnn_wave_launch_i4(wk, p, s);
+    else e = fnn_wave_launch_u4(wk, p, s);
+    if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
+    *handled = true;
+    return FNN_OK;
 }
 
 template <int DT, int WGM, int WGN, int TM, int TN, int NS, int DIG>
@@ -316,6 +380,41 @@ int run_digits(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const Q
 // traffic than four planes for 2e-5 of max|ref| stated (about 3e-6 measured on rows with 200x outliers; the four-plane
 // form holds 4e-6).  Operand rows come in groups of 24, so a wave owns three MFMA blocks: tiles of 192 operand rows
 // (64 activation rows) x 128 weight rows on four waves, x 256 on eight for 4-bit weights with many column tiles.
+// Tile form and K split of run_digits3 by rule.
+// Tile forms: 0 = 192 x 128 on four waves, 1 = 192 x 256 on eight (4-bit weights), 2 = 192 x 128 on eight (twice the
+// waves requesting the operands).  By shape: 4-bit weights take the wide tiles while those still cover the chip,
+// or where they save a round of workgroups (a wide tile takes about 1.4 times as long as a narrow one:
+// 4096 x 4096 at M = 513, 144 wide tiles against 288 narrow ones; 4096 x 11008 at M = 129 ... 192, 129 against 258).
+// K split: as many workgroups as fit one round over the 256 CUs, never more (4096 x 11008 at M = 256, 172 tiles:
+// 47 us unsplit, 66 us in two splits; 4096 x 4096 at M = 128, 64 tiles: 23 us in four splits, 31 us unsplit), and four
+// stages or more per workgroup.
+struct Digits3Form { int form, wide, mtiles, ntiles, splits, ips; int64_t tiles; };
+
+Digits3Form digits3_form(bool w4, int64_t m, int64_t n, int64_t k, int64_t opt_form = -1, int opt_split = 0)
+{
+    Digits3Form f;
+    const int iters = (int)((k + KB - 1) / KB);
+    f.form = 2;
+    f.mtiles = (int)((m + 63) / 64);
+    if (w4) {
+        const int64_t wide_tiles = (n + 255) / 256 * f.mtiles, narrow_tiles = (n + 127) / 128 * f.mtiles;
+        if (wide_tiles >= 160 || 1.4 * (double)((wide_tiles + 255) / 256) < (double)((narrow_tiles + 255) / 256)) f.form = 1;
+    }
+    if (opt_form >= 0 && opt_form <= 2 && (opt_form != 1 || w4)) f.form = (int)opt_form;
+    f.wide = f.form == 1;
+    const int bn = f.wide ? 256 : 128;
+    f.ntiles = (int)((n + bn - 1) / bn);
+    f.tiles = (int64_t)f.mtiles * f.ntiles;
+    f.splits = (int)(256 / f.tiles);
+    if (f.splits > iters / 4) f.splits = iters / 4;
+    if (f.splits < 1) f.splits = 1;
+    if (opt_split > 0) f.splits = opt_split;
+    if (f.splits > iters) f.splits = iters;
+    f.ips = (iters + f.splits - 1) / f.splits;
+    f.splits = (iters + f.ips - 1) / f.ips;   // no empty split
+    return f;
+}
+
 template <int DT>
 int run_digits3(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q)
 {
@@ -325,31 +424,8 @@ int run_digits3(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const 
     const int64_t kpad = (K + KB - 1) / KB * KB;
     const int iters = (int)(kpad / KB);
     const int bm = 192, act_rows = 64;
-    // tile forms: 0 = 192 x 128 on four waves, 1 = 192 x 256 on eight (4-bit weights), 2 = 192 x 128 on eight (twice the
-    // waves requesting the operands).  By shape: 4-bit weights take the wide tiles while those still cover the chip.
-    // ... or where they save a round of workgroups (a wide tile takes about 1.4 times as long as a narrow one:
-    // 4096 x 4096 at M = 513, 144 wide tiles against 288 narrow ones; 4096 x 11008 at M = 129 ... 192, 129 against 258)
-    int form = 2;
-    if (W4) {
-        const int64_t mt = (M + 63) / 64, wide_tiles = (N + 255) / 256 * mt, narrow_tiles = (N + 127) / 128 * mt;
-        if (wide_tiles >= 160 || 1.4 * (double)((wide_tiles + 255) / 256) < (double)((narrow_tiles + 255) / 256)) form = 1;
-    }
-    const int64_t opt_cfg = fnn_ctx_option(ctx, FNN_OPT_TILE_SHAPE);
-    if (opt_cfg >= 0 && opt_cfg <= 2 && (opt_cfg != 1 || W4)) form = (int)opt_cfg;
-    const int wide = form == 1;
-    const int bn = wide ? 256 : 128;
-    const int mtiles = (int)((M + act_rows - 1) / act_rows), ntiles = (int)((N + bn - 1) / bn);
-    const int64_t tiles = (int64_t)mtiles * ntiles;
-    // K split: as many workgroups as fit one round over the 256 CUs, never more (4096 x 11008 at M = 256, 172 tiles:
-    // 47 us unsplit, 66 us in two splits; 4096 x 4096 at M = 128, 64 tiles: 23 us in four splits, 31 us unsplit)
-    int splits = (int)(256 / tiles);
-    if (splits > iters / 4) splits = iters / 4;   // four stages or more per workgroup
-    if (splits < 1) splits = 1;
-    const int opt_split = (int)fnn_ctx_option(ctx, FNN_OPT_TILE_SPLIT);
-    if (opt_split > 0) splits = opt_split;
-    if (splits > iters) splits = iters;
-    const int ips = (iters + splits - 1) / splits;
-    splits = (iters + ips - 1) / ips;   // no empty split
+    const Digits3Form f = digits3_form(W4, M, N, K, fnn_ctx_option(ctx, FNN_OPT_TILE_SHAPE), (int)fnn_ctx_option(ctx, FNN_OPT_TILE_SPLIT));
+    const int form = f.form, mtiles = f.mtiles, ntiles = f.ntiles, splits = f.splits, ips = f.ips;
     const int64_t rows_pad = (int64_t)mtiles * bm, m_pad = (int64_t)mtiles * act_rows;
 
     const size_t a_bytes = (size_t)rows_pad * kpad;
@@ -406,6 +482,40 @@ int run_digits3(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const 
 
 }  // namespace
 
+// Microseconds of preparation + MatMul on the wave tiles and on the LDS tiles of run_digits3, least squares over 126 shapes
+// (M 40 .. 2048, K 1000 .. 8192, N 2048 .. 12288; mean error 2.4 % and 2.6 %).  Both count whole rounds of workgroups over the
+// 256 CUs: which one ends with the emptier round decides more than their rates do.  Taken from 96 rows on (8-bit weights below
+// have four planes), up to the rows that were measured, where it is ahead by more than 5 %.
+int fnn_wave_choice(int dtype, int64_t m, int64_t n, int64_t k, float *us)
+{
+    static const float kWave[2][3][5] = {   // [8-bit][wk 1, 2, 4]: launch, 100 steps of a round, round, M N / 1e6, M K / 1e6
+        {{9.38f, 20.78f, 7.21f, 1.66f, 1.98f}, {7.74f, 22.4f, 5.07f, 1.6f, 1.86f}, {7.42f, 24.47f, 3.72f, 1.78f, 1.91f}},
+        {{8.74f, 22.71f, 6.56f, 2.06f, 2.03f}, {6.99f, 26.77f, 5.33f, 1.82f, 1.96f}, {7.22f, 30.76f, 3.75f, 1.99f, 1.92f}}};
+    if (dtype != FNN_DT_I8 && dtype != FNN_DT_I4 && dtype != FNN_DT_U4) return 0;
+    if (m < 96 || m > 2048 || n * k <= (int64_t)2048 * 2048) return 0;
+    const bool w8 = dtype == FNN_DT_I8;
+    const float mn = (float)m * (float)n / 1e6f, mk = (float)m * (float)k / 1e6f;
+    auto ceil_div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+    const int ring = WAVE_RING(w8), units = (int)ceil_div(w8 ? ceil_div(k, 64) * 2 : ceil_div(k, 128) * 4, ring);
+    int wk = 0;
+    float best = 1e30f;
+    for (int i = 0; i < 3; i++) {
+        const int64_t rows = i == 0 ? 2 * WAVE_ROWS : WAVE_ROWS, cols = i == 2 ? WAVE_COLS : 2 * WAVE_COLS;
+        const float *c = kWave[w8][i], rounds = (float)ceil_div(ceil_div(m, rows) * ceil_div(n, cols), 256);
+        const float t = c[0] + c[1] * rounds * (float)(ceil_div(units, 1 << i) * ring) / 100.f + c[2] * rounds + c[3] * mn + c[4] * mk;
+        if (t < best) { best = t; wk = 1 << i; }
+    }
+    const Digits3Form f = digits3_form(!w8, m, n, k);
+    static const float kTile[3][7] = {   // launch, stage of a round, round, M N / 1e6 written per split, M N / 1e6, M K / 1e6, second launch
+        {10.991f, 0.533f, 0.f, 0.859f, 1.08f, 1.834f, 3.562f},       // 4-bit, 192 x 128
+        {8.574f, 0.978f, 2.738f, 0.f, 1.497f, 1.405f, 0.f},          // 4-bit, 192 x 256
+        {8.014f, 0.671f, 1.524f, 1.369f, 2.179f, 1.583f, 3.103f}};   // 8-bit, 192 x 128
+    const float *c = kTile[w8 ? 2 : f.wide], rounds = (float)ceil_div(f.tiles * f.splits, 256);
+    const float tiles = c[0] + rounds * (c[1] * (float)f.ips + c[2]) + (f.splits > 1 ? c[3] * (float)f.splits * mn + c[6] : 0.f) + c[4] * mn + c[5] * mk;
+    *us = best;
+    return best < 0.95f * tiles ? wk : 0;
+}
+
 int fnn_digits_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, bool *handled)
 {
     *handled = false;
@@ -416,6 +526,18 @@ int fnn_digits_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w,
     // exact i32 sums: |digit| <= 128, |lane| <= 128 (16*q for 4-bit signed lanes) -> K * 2^14 < 2^31
     if (q.m > (1 << 22) || q.n > (1 << 24) || q.k > (1 << 16)) return FNN_OK;
     if (q.words != w->words) return FNN_OK;   // (a row slice of a weight: the zero margin behind the last row is not behind the slice)
+    if (const int64_t opt = fnn_ctx_option(ctx, FNN_OPT_FRAGMENT); opt >= 0 && !(flags & FNN_FLAG_ACT_F16_SINGLE) && q.n == w->rows && q.k == w->inner) {
+        float us;
+        int wk = 0, rc = FNN_OK;
+        if (opt & FRAG_OPT_WAVE) wk = (int)(opt & 7);
+        else if (opt == 0 && fnn_frag_options_untouched(ctx)) wk = fnn_wave_choice(dt, q.m, q.n, q.k, &us);
+        if (wk == 1 || wk == 2 || wk == 4) {
+            if (dt == FNN_DT_I8) rc = run_digits_wave<FNN_DT_I8>(ctx, s, w, q, wk, handled);
+            else if (dt == FNN_DT_I4) rc = run_digits_wave<FNN_DT_I4>(ctx, s, w, q, wk, handled);
+            else rc = run_digits_wave<FNN_DT_U4>(ctx, s, w, q, wk, handled);
+        }
+        if (rc || *handled) return rc;
+    }
     QMatmulArgs qa = q;
     int rc;
     if ((rc = fnn_aligned_rows(ctx, s, w, &qa.words, &qa.kp))) return rc;

@@ -4,6 +4,10 @@
 
 #include "common.h"
 
+constexpr int64_t FRAG_OPT_WAVE = 1 << 14;   // FNN_OPT_FRAGMENT names a form of qgemm_wave_impl.h
+struct fnn_hip_ctx;
+bool fnn_frag_options_untouched(fnn_hip_ctx *ctx);
+
 constexpr int FRAG_NW = 8;        // waves per workgroup, each with an eighth of the workgroup's K range (a segment)
 
 // How K is dealt out: `splits` workgroups of kb_per_split k blocks (64 bytes of a weight row), each in FRAG_NW segments.

@@ -5,6 +5,7 @@
 // split over workgroups frag_reduce_kernel (partials added in split order: results do not depend on scheduling).
 #include "mfma.h"
 #include "qgemm_frag.h"
+#include "qgemm_wave.h"
 #include "range_io.h"
 
 namespace {
@@ -302,18 +303,6 @@ float tiled_us(bool integer, bool ragged, int64_t m, int64_t n, int64_t k)
     return q[0] + q[1] * fm * fn * fk / 1e9f + q[2] * fm * fn / 1e6f + q[3] * fn * fk / 1e6f + q[4] * fm * fk / 1e6f + q[5] * fk / 1e3f;
 }
 
-// an option that names another kernel or its shape keeps the calls with that kernel
-bool options_untouched(fnn_hip_ctx *ctx)
-{
-    static const int opts[][2] = {{FNN_OPT_TILE_SHAPE, -1}, {FNN_OPT_TILE_SPLIT, 0}, {FNN_OPT_TILE_STAGES, 0}, {FNN_OPT_TILE_MIN_M, 5}, {FNN_OPT_GEMM_INT8, 1},
-                                  {FNN_OPT_GEMM_INT8_MIN_M, 17}, {FNN_OPT_DIGIT_PLANES, 0}, {FNN_OPT_STREAM_MIN_M, 17}, {FNN_OPT_STREAM_MAX_M, 32},
-                                  {FNN_OPT_STREAM_SHAPE, 0}, {FNN_OPT_ROWS16_ROW_TILES, 0}, {FNN_OPT_ROWS16_MIN_M, 9}, {FNN_OPT_GEMV_ROW_TILES, 0},
-                                  {FNN_OPT_GEMV_INT8, 1}, {FNN_OPT_GEMV_INT8_MAX_M, 8}};
-    for (const auto &o : opts)
-        if (fnn_ctx_option(ctx, o[0]) != o[1]) return false;
-    return true;
-}
-
 // The launch for an [M, K] x [N, K]^T product with this weight; false: the call is not this kernel's.  The same for every
 // call of the same sizes, so that the MatMul before can prepare the operand.
 bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, FragPlan *out)
@@ -331,6 +320,7 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
     const bool direct_ok = m * k < (int64_t)1 << 29;   // (32-bit buffer offsets)
     int splits = 1;
     if (opt > 0) {
+        if (opt & FRAG_OPT_WAVE) return false;
         f.mb = (int)(opt & 15); f.nb = (int)((opt >> 4) & 15);
         splits = (int)((opt >> 8) & 15) > 0 ? (int)((opt >> 8) & 15) : 1;
         f.direct = (opt >> 15) & 1;
@@ -348,7 +338,7 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
         // beyond where a segment is longer than four steps: 5 .. 8 rows F8 832 x 5749 5.4 us either way, 9 .. 16 rows
         // 960 x 5454 U8 7.4 against 5.7); ragged rows have no such kernel (2 x 4728 x 11904 F4: 233 us there, 14 here).
         const bool ragged = w->kp % 4 != 0 || k % 8 != 0;
-        if (m > 2048 || !options_untouched(ctx)) return false;
+        if (m > 2048 || !fnn_frag_options_untouched(ctx)) return false;
         if (m <= 16 && !ragged && (m <= 4 || direct_steps > 4 || (m <= 8 && integer))) return false;
         float best = 1e30f;
         if (direct_ok)
@@ -368,6 +358,7 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
             }
         // (the margin: where the two are about equal the fits decide at random, and what was there stays)
         if (best > 1e29f || (m >= 33 && best > 0.93f * tiled_us(integer, ragged, m, n, k))) return false;
+        if (float us; !(flags & FNN_FLAG_ACT_F16_SINGLE) && fnn_wave_choice(w->dtype, m, n, k, &us) && us < best) return false;
     }
     if (splits > f.ks.kblocks) splits = f.ks.kblocks;
     f.ks.kb_per_split = (f.ks.kblocks + splits - 1) / splits;
@@ -407,6 +398,18 @@ FragPrepArgs prep_args(const FragPlan &f, const fnn_hip_weight *w, int64_t m, vo
 }
 
 }  // namespace
+
+// an option that names another kernel or its shape keeps the calls with that kernel
+bool fnn_frag_options_untouched(fnn_hip_ctx *ctx)
+{
+    static const int opts[][2] = {{FNN_OPT_TILE_SHAPE, -1}, {FNN_OPT_TILE_SPLIT, 0}, {FNN_OPT_TILE_STAGES, 0}, {FNN_OPT_TILE_MIN_M, 5}, {FNN_OPT_GEMM_INT8, 1},
+                                  {FNN_OPT_GEMM_INT8_MIN_M, 17}, {FNN_OPT_DIGIT_PLANES, 0}, {FNN_OPT_STREAM_MIN_M, 17}, {FNN_OPT_STREAM_MAX_M, 32},
+                                  {FNN_OPT_STREAM_SHAPE, 0}, {FNN_OPT_ROWS16_ROW_TILES, 0}, {FNN_OPT_ROWS16_MIN_M, 9}, {FNN_OPT_GEMV_ROW_TILES, 0},
+                                  {FNN_OPT_GEMV_INT8, 1}, {FNN_OPT_GEMV_INT8_MAX_M, 8}};
+    for (const auto &o : opts)
+        if (fnn_ctx_option(ctx, o[0]) != o[1]) return false;
+    return true;
+}
 
 // fragment-major copy of the packed words; null when it does not exist and this call may not build it
 int fnn_fragment_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, int64_t kblocks, const uint32_t **out)

@@ -167,7 +167,7 @@ int fnn_frag_i8act(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, con
         else hipLaunchKernelGGL(frag_codes_kernel<false>, grid, dim3(256), 0, s, q.payload, q.m, q.k, nsteps, (uint4 *)ws0);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
     }
-    hipError_t e = four ? fnn_frag_int_launch_i4(mb, nb, false, p, s) : fnn_frag_int_launch_i8(mb, nb, false, p, s);
+    hipError_t e = four ? fnn_frag_int_launch_i4(mb, nb, p, s) : fnn_frag_int_launch_i8(mb, nb, p, s);
     if (e == hipSuccess && p.part) {
         hipLaunchKernelGGL(frag_codes_reduce_kernel, dim3((unsigned)((q.m * q.n + 255) / 256)), dim3(256), 0, s, p);
         e = hipGetLastError();

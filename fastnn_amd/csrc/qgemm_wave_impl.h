@@ -1,0 +1,241 @@
+// Int8 MatMul for many activation rows: one wave per SIMD with a large register tile, operands straight from memory.
+//
+// Bound: the matrix cores (v_mfma_i32_32x32x32_i8, 32 clocks each; 3.6 to 4.4 POP/s sustained by themselves, by the data's
+// power) and, close behind, the 64 B/clk that a CU's L1 delivers: a wave tile of 96 x 128 (three digit planes of 32 activation
+// rows) asks for 224 bytes per k-value with 8-bit and 160 with 4-bit weights against 12 clocks of its SIMD's matrix core, so
+// the four waves of a CU need 14 and 10 clocks of L1 time in the same 12.  No LDS, no barrier: the operands lie in memory in
+// fragment order, a wave's load is contiguous, and RING steps of 32 k-values are in flight per wave.  What is left at large M
+// is the epilogue, which nothing overlaps at one wave per SIMD (10 to 15 us per round of tiles), and a matrix core that is
+// busy half the time (counters: 48 %, 23 % of the clocks waiting for memory).
+// Measured against the LDS tiles of qgemm_digits.hip: I8 4096 x 4096 M = 256 29.6 -> 27.4 us, M = 1024 72.5 -> 65.5,
+// M = 2048 130.6 -> 122; I8 4096 x 11008 M = 700 131 -> 111; I4 4096 x 4096 M = 256 27.2 -> 23.6.  Row blocks an odd number
+// of pieces apart, to spread them over the L2's channels, gained nothing (122 -> 127 us).
+#pragma once
+#include <climits>
+#include <type_traits>
+
+#include "dech.h"
+#include "qgemm_wave.h"
+
+namespace {
+
+using namespace dech;
+typedef int wi32x4 __attribute__((ext_vector_type(4)));
+typedef int wi32x16 __attribute__((ext_vector_type(16)));
+
+// Operand rows in groups of 24 = 8 activation rows x 3 planes (plane j in rows [8j, 8j + 8) of the group).  WK: waves of the
+// four that share an output tile and split K (they meet in LDS at the end); the others lie side by side (WK = 1: 2 x 2,
+// WK = 2: 1 x 2).
+template <int DT, int WK>
+__global__ void __launch_bounds__(256, 1) qgemm_wave_kernel(WaveArgs p)
+{
+    using D = DecI<DT>;
+    constexpr int TM = WAVE_ROWS * 3 / 32, TN = WAVE_COLS / 32;   // blocks of 32 x 32
+    constexpr bool W8 = D::WPS == 4;
+    constexpr int RING = WAVE_RING(W8);                // steps in flight, and the unit in which K is dealt out
+    constexpr int SHIFT = DT == FNN_DT_I4 ? 4 : 0;     // 4-bit signed lanes enter as 16 q
+    constexpr int WL = W8 ? RING : RING / 2;           // weight loads per ring: a 16-byte piece is one step or two
+    extern __shared__ __attribute__((aligned(16))) float wred[];   // [wave][value][lane]
+    __shared__ int2 row_const[4][WAVE_ROWS];
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, h = lane >> 5;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = WK == 1 ? 0 : (WK == 2 ? wv >> 1 : wv);
+    const int wm = WK == 1 ? wv >> 1 : 0, wn = WK == 4 ? 0 : wv & 1;
+    constexpr int WM = WK == 1 ? 2 : 1, WN = WK == 4 ? 1 : 2;
+
+    // Workgroup id -> tile.  Ids are dealt round-robin over the 8 XCDs; each XCD takes a contiguous share of the tiles, walked
+    // in stripes of four row tiles, so that the workgroups resident on it read few different operand rows.
+    const unsigned per_xcd = (p.tiles + 7) / 8;
+    const unsigned T = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((blockIdx.x >> 3) >= per_xcd || T >= p.tiles) return;
+    const unsigned stripe = p.by_stripe.div(T), first_m = stripe * 4, in_stripe = T - stripe * 4 * (unsigned)p.ntiles;
+    const unsigned height = (unsigned)p.mtiles - first_m < 4 ? (unsigned)p.mtiles - first_m : 4;
+    const unsigned nt = height == 4 ? in_stripe >> 2 : in_stripe / height, mt = first_m + (in_stripe - nt * height);
+
+    const int rb0 = (int)(mt * WM + wm) * TM;              // first block of 32 operand rows
+    const int64_t m0 = (int64_t)(mt * WM + wm) * WAVE_ROWS;     // first activation row
+    const int64_t n0 = (int64_t)(nt * WN + wn) * WAVE_COLS;
+    const int u0 = wk * p.units_per_wave, u1 = u0 + p.units_per_wave < p.units ? u0 + p.units_per_wave : p.units;
+
+    wi32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[i][j][e] = 0;
+
+    // Row and column constants of the outputs: requested before the last unit, so that the epilogue, which nothing overlaps
+    // on this SIMD, does not begin with a trip to memory.
+    auto slot_row = [&](int r) { return (r >> 2) * 8 + h * 4 + (r & 3); };   // of a lane's 16 row slots
+    float sc[TN], zp[TN], bi[TN];
+    int rexp = 0;
+    float xsum = 0.0f;
+    auto load_constants = [&] {
+        rexp = p.rexp[m0 + lr];   // (rows past M lie inside the tables)
+        xsum = p.xsum[m0 + lr];
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            int64_t n = n0 + j * 32 + lr;
+            if (n > p.n - 1) n = p.n - 1;
+            sc[j] = p.scales[n];
+            zp[j] = p.zeros[n];
+            bi[j] = p.bias ? p.bias[n] : 0.0f;
+        }
+    };
+
+    if (u0 < u1) {
+        const wi32x4 *a0 = reinterpret_cast<const wi32x4 *>(p.af) + (int64_t)rb0 * p.nsteps * 64 + lane;
+        const u32x4 *w0[TN];   // [row block of 16][k block][q][row]: two row blocks and a pair of q per load
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            int rb = (int)(n0 >> 4) + 2 * j + (lr >> 4);
+            if (rb > p.rblocks - 1) rb = p.rblocks - 1;
+            w0[j] = reinterpret_cast<const u32x4 *>(p.wf) + (int64_t)rb * p.kblocks * 64 + h * 16 + (lr & 15);
+        }
+        wi32x4 a[RING][TM];
+        u32x4 w[WL][TN];
+        auto load_a = [&](int s, int i) { return a0[((int64_t)i * p.nsteps + s) * 64]; };
+        // piece x of a row: k block x / 2, q = 2 (x & 1) + h
+        auto load_w = [&](int x, int j) {
+            int kb = x >> 1;
+            if (kb > p.kblocks - 1) kb = p.kblocks - 1;   // (past the last block the activations are zero)
+            return w0[j][kb * 64 + (x & 1) * 32];
+        };
+        auto decode = [&](int st, int j) {
+            uint32_t ww[4];
+#pragma unroll
+            for (int e = 0; e < D::WPS; e++) ww[e] = W8 ? w[W8 ? st : 0][j][e] : w[W8 ? 0 : st / 2][j][2 * (st & 1) + (e & 1)];
+            return __builtin_bit_cast(wi32x4, D::step(ww));
+        };
+        // One ring of steps.  A step's matrix instructions carry, one by one between them, the requests that refill what the
+        // step before has used up and the decoding of the next step's weights: issued in a bunch they leave the matrix core
+        // idle while the four waves' requests queue for the L1 (2048 x 4096 x 4096 I8: 113 us).
+        wi32x4 wd[2][TN];
+        auto unit = [&](int u, auto last) {
+            constexpr bool LAST = decltype(last)::value;
+#pragma unroll
+            for (int st = 0; st < RING; st++) {
+                constexpr int NM = TM * TN;
+                const bool want_a = !LAST || st == 0;
+                const bool want_w = want_a && (W8 || st % 2 == 0);
+                const int sp = (st + RING - 1) % RING, step = (st == 0 ? u : u + 1) * RING + sp;   // slot to refill, its step
+                const int wp = W8 ? sp : sp / 2, piece = W8 ? step : step / 2;
+#pragma unroll
+                for (int x = 0; x < NM; x++) {
+                    const int i = x / TN, j = x % TN;
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[st][i], wd[st & 1][j], acc[i][j], 0, 0, 0);
+                    // requests 0 .. TM + TN - 1 at equal distances, then the next step's decoding
+#pragma unroll
+                    for (int r = 0; r < TM + TN; r++)
+                        if (r * NM / (TM + TN) == x) {
+                            if (r < TM) { if (want_a) a[sp][r] = load_a(step, r); }
+                            else if (want_w) w[wp][r - TM] = load_w(piece, r - TM);
+                        }
+                    if (x >= NM - TN && (!LAST || st < RING - 1)) wd[(st + 1) & 1][x - (NM - TN)] = decode((st + 1) % RING, x - (NM - TN));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        };
+#pragma unroll
+        for (int st = 0; st < RING - 1; st++) {
+#pragma unroll
+            for (int i = 0; i < TM; i++) a[st][i] = load_a(u0 * RING + st, i);
+            if (W8 || st % 2 == 0)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    if (W8 || st / 2 < WL - 1) w[W8 ? st : st / 2][j] = load_w(W8 ? u0 * RING + st : u0 * WL + st / 2, j);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < TN; j++) wd[0][j] = decode(0, j);
+        for (int u = u0; u < u1 - 1; u++) unit(u, std::false_type{});
+        load_constants();
+        unit(u1 - 1, std::true_type{});
+    } else {
+        load_constants();
+    }
+
+    // D: acc[i][j][e] is operand row 32 i + (e / 4) * 8 + h * 4 + e % 4, column 32 j + lr.
+    // A value of this lane, (row slot r, column block j): the three planes of one activation row combined
+    auto value = [&](int r, int j) {
+        float v = 0.0f;
+#pragma unroll
+        for (int d = 2; d >= 0; d--) {
+            const int slab = 3 * (r >> 2) + d;
+            v = fmaf(v, 256.0f, (float)acc[slab >> 2][j][(slab & 3) * 4 + (r & 3)]);
+        }
+        return v;
+    };
+    if (h == 0) row_const[wv][lr] = make_int2(rexp, __float_as_int(xsum));
+    const bool has_bias = p.bias != nullptr;
+    // row slot r, its TN values
+    auto finish = [&](int r, const float (&v)[TN]) {
+        const int64_t m = m0 + slot_row(r);
+        if (m >= p.m) return;
+        float o[TN];
+        const int2 rc = row_const[wv][slot_row(r)];
+        const bool bad = rc.x == INT_MIN;   // a non-finite row
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const float d = bad ? __builtin_nanf("") : ldexpf(v[j], -rc.x - SHIFT);
+            o[j] = d * sc[j] + zp[j] * __int_as_float(rc.y);
+        }
+        if (has_bias)
+#pragma unroll
+            for (int j = 0; j < TN; j++) o[j] = o[j] + bi[j];
+        if (p.act != FNN_ACT_NONE)
+#pragma unroll
+            for (int j = 0; j < TN; j++) o[j] = fnn_activation(o[j], p.act);
+        const int64_t at = m * p.n + n0 + lr;
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            if (n0 + j * 32 + lr >= p.n) continue;
+            p.out[at + j * 32] = o[j];
+            if (p.residual) p.sum_out[at + j * 32] = o[j] + p.residual[at + j * 32];
+        }
+    };
+    // The sums go through LDS and the formula runs in a loop over them: unrolled over the registers it is some 40 KB of code
+    // that every wave runs once, and fetching that took 10 us.
+    constexpr int VALUES = 16 * TN, OWN = 16 / WK;
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) wred[(wv * VALUES + r * TN + j) * 64 + lane] = value(r, j);
+    __syncthreads();
+    // wave wk finishes its share of the slots; its partners' values lie WN waves apart
+    const float *q = wred + ((WK == 1 ? wv : wn) * VALUES + wk * OWN * TN) * 64 + lane;
+#pragma unroll 2
+    for (int x = 0; x < OWN; x++, q += TN * 64) {
+        float v[TN];
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            v[j] = q[j * 64];
+#pragma unroll
+            for (int y = 1; y < WK; y++) v[j] += q[(y * WN * VALUES + j) * 64];
+        }
+        finish(wk * OWN + x, v);
+    }
+}
+
+template <int DT, int WK>
+hipError_t wave_launch_one(const WaveArgs &p, hipStream_t s)
+{
+    constexpr int lds = 4 * 16 * WAVE_COLS / 32 * 256;
+    auto kern = qgemm_wave_kernel<DT, WK>;
+    static std::atomic<uint64_t> raised{0};
+    const hipError_t e = fnn_raise_lds_limit(raised, reinterpret_cast<const void *>(kern), lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kern, dim3((p.tiles + 7) / 8 * 8), dim3(256), lds, s, p);
+    return hipGetLastError();
+}
+
+template <int DT>
+hipError_t wave_launch(int wk, const WaveArgs &p, hipStream_t s)
+{
+    if (wk == 1) return wave_launch_one<DT, 1>(p, s);
+    if (wk == 2) return wave_launch_one<DT, 2>(p, s);
+    return wave_launch_one<DT, 4>(p, s);
+}
+
+}  // namespace

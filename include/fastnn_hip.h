@@ -169,7 +169,9 @@ enum {
                                   /* the weight's first such call): 0 (default) = by rule (any M with rows of ragged length, from   */
                                   /* M = 17, or 5 to 9 for short rows, with aligned ones, as far up as it is the faster form), -1 =  */
                                   /* off, else the shape, (direct << 15) | (K splits << 8) | (16-column blocks << 4) | (16-row       */
-                                  /* blocks); a shape that does not exist for the call is ignored                                   */
+                                  /* blocks); a shape that does not exist for the call is ignored;                                  */
+                                  /* (1 << 14) | w, w = 1, 2 or 4: I8, I4 and U4 weights on the large register tiles of three     */
+                                  /* digit planes, w waves of a workgroup sharing a tile                                            */
     FNN_OPT_COUNT = 25
 };
 int fnn_hip_set_option(fnn_hip_ctx *ctx, int option, int64_t value);

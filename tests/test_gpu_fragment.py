@@ -42,3 +42,45 @@ def test_every_shape_of_the_fragment_kernels(ctx, orc, dt, m, k, n):
     finally:
         ctx.set_option(flib.OPT_FRAGMENT, 0)
         ctx.release(h)
+
+
+@pytest.mark.parametrize("dt", [flib.DT_I8, flib.DT_I4, flib.DT_U4])
+@pytest.mark.parametrize("m,k,n", [(17, 63, 15), (31, 200, 129), (33, 1000, 257), (65, 2600, 260), (130, 515, 140)])
+def test_every_form_of_the_wave_tiles(ctx, orc, dt, m, k, n):
+    """Rows around 32 and 64, columns around 128 and 256, K around the rings of six or eight steps of 32 and their split."""
+    rng = np.random.default_rng(9100 + dt * 7 + m)
+    pw = fastnn_amd.quantize_weights(dt, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    a[:, ::61] *= 100.0
+    a[m // 2] = 0.0
+    bias = (rng.standard_normal(n) * 0.1).astype(np.float32)
+    want = orc.qmatmul(to_oracle(orc, pw), a, order=2, bias=bias, act=flib.ACT_SILU)
+    h = ctx.register(pw)
+    try:
+        for waves in (1, 2, 4):
+            ctx.set_option(flib.OPT_FRAGMENT, 1 << 14 | waves)
+            assert_close(ctx.qmatmul(h, a, n, bias=bias, act=flib.ACT_SILU), want, 2e-5, f"{waves} waves a tile")
+    finally:
+        ctx.set_option(flib.OPT_FRAGMENT, 0)
+        ctx.release(h)
+
+
+@pytest.mark.parametrize("dt", [flib.DT_I8, flib.DT_I4])
+@pytest.mark.parametrize("m,k,n", [(1, 63, 15), (17, 1000, 33), (31, 1026, 64), (65, 2600, 257), (130, 515, 68)])
+def test_every_shape_of_the_integer_fragment_kernels(ctx, orc, dt, m, k, n):
+    rng = np.random.default_rng(9200 + dt * 7 + m)
+    pw = fastnn_amd.quantize_weights(dt, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    payload = orc.quantize_activations(rng.standard_normal((m, k)).astype(np.float32))
+    want, want_acc = orc.qmatmul_i8act(to_oracle(orc, pw), payload, m, want_acc=True)
+    h = ctx.register(pw)
+    try:
+        for mb, nb in ((1, 1), (1, 2), (2, 2), (2, 4), (4, 4)):
+            for sp in (1, 3):
+                for direct in (0, 1):
+                    ctx.set_option(flib.OPT_FRAGMENT, direct << 15 | sp << 8 | nb << 4 | mb)
+                    got, acc = ctx.qmatmul_i8act(h, payload, m, n, want_acc=True)
+                    assert np.array_equal(acc, want_acc), f"{mb}x{nb} splits {sp} direct {direct}"
+                    assert_close(got, want, 2e-5, f"{mb}x{nb} splits {sp} direct {direct}")
+    finally:
+        ctx.set_option(flib.OPT_FRAGMENT, 0)
+        ctx.release(h)
