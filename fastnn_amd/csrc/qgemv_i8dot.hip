@@ -25,6 +25,7 @@
 // 13.9, M = 16 16.2 against 14.2), so M <= 8 is the default range.
 // Algorithmic bytes per launch: N*K*bits/8 + side tables + 4*M*(K+N).
 #include "mfma.h"
+#include "range_io.h"
 
 #include <climits>
 
@@ -34,6 +35,10 @@ struct DotArgs {
     const uint32_t *words;
     const float *scales, *zeros, *a, *bias;
     float *out;
+    // a plan's Add behind this MatMul, sum_out[i] = out[i] + residual[i], or null: as an instruction of its own it is a launch
+    // of 2 us and a gap of 2 to 4 behind a MatMul of 4
+    const float *residual;
+    float *sum_out;
     int64_t m, n, k, kp;
     int act;
     int nslice;   // slices of 512 k-values covering K
@@ -130,18 +135,19 @@ __global__ void __launch_bounds__(NW * 64) qgemv_i8dot_kernel(DotArgs p)
     int e_r[OPT], e_m[OPT], e_c[OPT];
     int64_t e_n[OPT];
     bool finisher[OPT];
-    float e_scale[OPT], e_zero[OPT], e_bias[OPT];
+    float e_scale[OPT], e_zero[OPT], e_bias[OPT], e_res[OPT];
 #pragma unroll
     for (int o = 0; o < OPT; o++) {
         const int idx = tid + o * NW * 64;
         e_r[o] = idx / (MT * 16); e_m[o] = (idx >> 4) % MT; e_c[o] = idx & 15;
         e_n[o] = n0 + e_r[o] * 16 + e_c[o];
         finisher[o] = idx < OUTS && e_m[o] < mreal && e_n[o] < N;
-        e_scale[o] = e_zero[o] = e_bias[o] = 0.0f;
+        e_scale[o] = e_zero[o] = e_bias[o] = e_res[o] = 0.0f;
         if (finisher[o]) {
             e_scale[o] = p.scales[e_n[o]];
             e_zero[o] = p.zeros[e_n[o]];
             e_bias[o] = p.bias ? p.bias[e_n[o]] : 0.0f;
+            if (p.residual) e_res[o] = p.residual[(int64_t)e_m[o] * N + e_n[o]];
         }
     }
 
@@ -312,7 +318,9 @@ __global__ void __launch_bounds__(NW * 64) qgemv_i8dot_kernel(DotArgs p)
             for (int w = 0; w < NW; w++) { dot += red[w][e_r[o]][e_m[o]][e_c[o]]; xs += xred[w][e_m[o]]; }
             dot *= W::POST;
             const float v = dot * e_scale[o] + e_zero[o] * xs;
-            p.out[(int64_t)e_m[o] * N + e_n[o]] = fnn_activation(p.bias ? v + e_bias[o] : v, p.act);
+            const float r = fnn_activation(p.bias ? v + e_bias[o] : v, p.act);
+            p.out[(int64_t)e_m[o] * N + e_n[o]] = r;
+            if (p.residual) p.sum_out[(int64_t)e_m[o] * N + e_n[o]] = r + e_res[o];
         }
     }
 }
@@ -421,6 +429,8 @@ int fnn_i8dot_qgemv(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, co
             if (best < 0 || cost < best) { best = cost; rt = c; }
         }
     }
+    p.residual = nullptr; p.sum_out = nullptr;
+    fnn_take_residual(ctx, q.out, q.m * q.n, &p.residual, &p.sum_out);
     hipError_t e;
     switch (w->dtype) {
     case FNN_DT_I8: e = launch_dt<FNN_DT_I8>(p, rt, s, handled); break;

@@ -26,6 +26,7 @@
 // Algorithmic bytes per launch: N*K*bits/8 + side tables + 4*M*(K+N).
 #include "dech.h"
 #include "mfma.h"
+#include "range_io.h"
 
 #include <cstdlib>
 
@@ -38,6 +39,10 @@ struct GemvArgs {
     const float *scales, *zeros, *a, *bias;
     const float *umean;   // single-f16 mode: mean lane value per weight row, or null
     float *out;
+    // a plan's Add behind this MatMul, sum_out[i] = out[i] + residual[i], or null: as an instruction of its own it is a launch
+    // of 2 us and a gap of 2 to 4 behind a MatMul of 4
+    const float *residual;
+    float *sum_out;
     int64_t m, n, k, kp;
     int act;
     const uint32_t *words_tm;   // non-null: the words in blocks of 16 rows x 64 bytes ([row block][k block][row][64 bytes]),
@@ -94,6 +99,7 @@ __global__ void __launch_bounds__(NW * 64) qgemv_mfma_kernel(GemvArgs p)
     if (e_n > N - 1) e_n = N - 1;
     const float e_scale = p.scales[e_n], e_zero = p.zeros[e_n];
     const float e_bias = p.bias ? p.bias[e_n] : 0.0f;
+    const float e_res = p.residual && e_ok ? p.residual[(int64_t)e_m * N + e_n] : 0.0f;
     const float e_umean = (SINGLE && p.umean) ? p.umean[e_n] : 0.0f;
 
     f32x4 tot[RT];
@@ -249,7 +255,9 @@ __global__ void __launch_bounds__(NW * 64) qgemv_mfma_kernel(GemvArgs p)
         }
         if (SINGLE) dot = dot - e_umean * es;
         const float v = dot * e_scale + e_zero * xs + e_bias;   // fnn_epilogue with preloaded operands
-        p.out[(int64_t)e_m * N + e_n] = fnn_activation(p.bias ? v : dot * e_scale + e_zero * xs, p.act);
+        const float r = fnn_activation(p.bias ? v : dot * e_scale + e_zero * xs, p.act);
+        p.out[(int64_t)e_m * N + e_n] = r;
+        if (p.residual) p.sum_out[(int64_t)e_m * N + e_n] = r + e_res;
     }
 }
 
@@ -344,6 +352,8 @@ int fnn_mfma_qgemv(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, con
         if (rc) return rc;
     }
     const int rt = (int)fnn_ctx_option(ctx, FNN_OPT_GEMV_ROW_TILES);   // 0: by the cost model
+    p.residual = nullptr; p.sum_out = nullptr;
+    fnn_take_residual(ctx, q.out, q.m * q.n, &p.residual, &p.sum_out);
     hipError_t e;
     switch (w->dtype) {
     case FNN_DT_I8: e = launch_gemv<FNN_DT_I8>(p, single, rt, s); break;

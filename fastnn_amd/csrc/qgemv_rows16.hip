@@ -22,6 +22,7 @@
 // Algorithmic bytes per launch: N*K*bits/8 + side tables + 4*M*(K+N).
 #include "dech.h"
 #include "mfma.h"
+#include "range_io.h"
 
 #include <cstdlib>
 
@@ -34,6 +35,10 @@ struct Rows16Args {
     const float *scales, *zeros, *a, *bias;
     const float *umean;   // single-f16 mode: mean lane value per weight row, or null
     float *out;
+    // a plan's Add behind this MatMul, sum_out[i] = out[i] + residual[i], or null: as an instruction of its own it is a launch
+    // of 2 us and a gap of 2 to 4 behind a MatMul of 4
+    const float *residual;
+    float *sum_out;
     int64_t m, n, k, kp;
     int act;
     const uint32_t *words_tm;   // non-null: the words in blocks of 16 rows x 64 bytes ([row block][k block][row][64 bytes]),
@@ -260,7 +265,9 @@ __global__ void __launch_bounds__(NW * 64) qgemv_rows16_kernel(Rows16Args p)
         }
         // single-f16 mode, first-order correction of the rounding: dot -= mean_k u[n,k] * sum_k (hi - x)
         if (SINGLE && p.umean) dot = dot - p.umean[n] * es;
-        p.out[(int64_t)m * N + n] = fnn_epilogue(dot, p.scales[n], p.zeros[n], xs, p.bias, n, p.act);
+        const float v = fnn_epilogue(dot, p.scales[n], p.zeros[n], xs, p.bias, n, p.act);
+        p.out[(int64_t)m * N + n] = v;
+        if (p.residual) p.sum_out[(int64_t)m * N + n] = v + p.residual[(int64_t)m * N + n];
     }
 }
 
@@ -337,6 +344,8 @@ int fnn_mfma_rows16(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, co
         return rc;
     }
     const int rt = (int)fnn_ctx_option(ctx, FNN_OPT_ROWS16_ROW_TILES);   // 0: by the cost model
+    p.residual = nullptr; p.sum_out = nullptr;
+    fnn_take_residual(ctx, q.out, q.m * q.n, &p.residual, &p.sum_out);
     hipError_t e;
     switch (w->dtype) {
     case FNN_DT_I8: e = launch_rows16<FNN_DT_I8>(p, single, rt, s); break;

@@ -46,6 +46,16 @@ struct FnnResidualIo {
     int used = 0;
 };
 FnnResidualIo *fnn_ctx_residual_io(fnn_hip_ctx *ctx);
+// the request for an output of `elems` values at `out`, taken: the kernel to be launched stores the sum
+inline bool fnn_take_residual(fnn_hip_ctx *ctx, const float *out, int64_t elems, const float **residual, float **sum_out)
+{
+    FnnResidualIo *res = fnn_ctx_residual_io(ctx);
+    if (!res->residual || res->of_out != out || res->elems != (uint64_t)elems) return false;
+    *residual = res->residual;
+    *sum_out = res->sum_out;
+    res->used = 1;
+    return true;
+}
 
 // A prepared MatMul operand that travels from one MatMul call to the next: at 17 <= M the f16 matrix-core path
 // first turns its f32 activations into scaled f16 hi + lo operand rows (a launch of its own).  When the caller knows

@@ -1418,3 +1418,30 @@ def test_dispatch_profile_runs_under_the_shape_environment_it_is_given(be, orc):
     with pytest.raises(flib.FnnError) as e:
         be.dispatch_profile(sym)
     assert "DimExpr::Symbol 'T' is not bound" in e.value.message
+
+
+@pytest.mark.parametrize("wdt,kname", [(flib.DT_I8, "matmul_i8"), (flib.DT_U4, "matmul_u4_relu"), (flib.DT_F8, "matmul_f8")])
+@pytest.mark.parametrize("m,k,n", [(1, 512, 33), (2, 2048, 200), (8, 2560, 129), (16, 1024, 5000)])
+def test_residual_add_behind_a_matmul_of_few_rows(be, wdt, kname, m, k, n):
+    """The GEMV kernels store the sum of the Add behind them: bit for bit what two instructions give."""
+    rng = np.random.default_rng(7100 + m)
+    x, r = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    pw = fastnn_amd.quantize_weights(wdt, _w(rng, n, k))
+    a = Arena()
+    s_x, s_w, s_r, s_y, s_s = a.take(x.nbytes), a.take(pw.words.nbytes), a.take(r.nbytes), a.take(r.nbytes), a.take(r.nbytes)
+    plan = ExecutablePlan(a.top).write_const(s_w[0], pw.words)
+    plan.call_kernel(kname, [s_x, s_w], s_y, [m, k, n], meta_of(pw)).call_kernel("add_f32", [s_r, s_y], s_s, [m * n])
+    be.allocate_arena(a.top)
+    be.write_arena(s_x[0], x)
+    be.write_arena(s_r[0], r)
+    got = {}
+    try:
+        for fuse in (1, 0):
+            be.set_option(flib.OPT_FUSE_RESIDUAL, fuse)
+            be.dispatch(plan)
+            assert plan.residuals_fused == fuse
+            got[fuse] = be.read_arena(*s_s, np.float32).copy()
+            assert np.array_equal(got[fuse], (be.read_arena(*s_y, np.float32) + r.reshape(-1)).astype(np.float32))
+    finally:
+        be.set_option(flib.OPT_FUSE_RESIDUAL, 1)
+    assert np.array_equal(got[0], got[1])
