@@ -34,11 +34,14 @@ inline hipError_t fnn_raise_lds_limit(std::atomic<uint64_t> &done, const void *k
 // 17 <= M <= 32: one launch, weights streamed into the MFMA operand registers, activations converted in the kernel,
 // K split over workgroups and reduced by the last one to arrive (qgemm_stream.hip)
 int fnn_stream_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
+bool fnn_stream_takes(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QMatmulArgs &p, int flags);
 // arrival counters of that kernel's column tiles: FNN_STREAM_COUNTERS words of device memory, zero between launches
 constexpr int FNN_STREAM_COUNTERS = 4096;
 uint32_t *fnn_ctx_stream_counters(fnn_hip_ctx *ctx);
 // int8 matrix-core GEMM over exact activation digit planes (qgemm_digits.hip): M >= 17, I8 / I4 / U4 weights
 int fnn_digits_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
+// digit planes that path would multiply the call with by rule and options (3, 4); 0: the call is another kernel's
+int fnn_digits_planes(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags);
 // a middle number of activation rows, per-channel types: both operands in the order the matrix cores take them (qgemm_frag.hip)
 int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
 int fnn_frag_i8act(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const I8ActArgs &p, bool *handled);

@@ -516,15 +516,43 @@ int fnn_wave_choice(int dtype, int64_t m, int64_t n, int64_t k, float *us)
     return best < 0.95f * tiles ? wk : 0;
 }
 
+// what the kernels of this file can multiply at all
+static bool digits_possible(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k)
+{
+    if (fnn_ctx_option(ctx, FNN_OPT_GEMM_INT8) == 0 || m < fnn_ctx_option(ctx, FNN_OPT_GEMM_INT8_MIN_M)) return false;
+    if (dt != FNN_DT_I8 && dt != FNN_DT_I4 && dt != FNN_DT_U4) return false;
+    // exact i32 sums: |digit| <= 128, |lane| <= 128 (16*q for 4-bit signed lanes) -> K * 2^14 < 2^31
+    return m <= (1 << 22) && n <= (1 << 24) && k <= (1 << 16);
+}
+
+int fnn_digits_planes(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags)
+{
+    if (!digits_possible(ctx, dt, m, n, k)) return 0;
+    // The single-rounding mode stays with the f16 tiles: two digit planes (15 bits below the row maximum) were 15 %
+    // faster than one f16 row but measured 1.9e-3 on rows with a few 200x outliers, where a float rounding per
+    // element keeps 2.4e-4; three planes cost what the f16 row costs.
+    if (flags & FNN_FLAG_ACT_F16_SINGLE) return 0;
+    // Small weights stay with the f16 tiles as well (by rule; FNN_OPT_DIGIT_PLANES = 3 or 4 or FNN_OPT_GEMM_INT8_MIN_M
+    // below its default still bring them here): 1024 x 1024 I4 at M = 48 / 256 / 1024 14.6 / 16.2 / 22.3 us here against 12.9 / 13.6 / 15.9 there, 2048 x 2048 I8
+    // at M = 64 / 512 16.4 / 26.6 against 15.1 / 22.0; from 3072 x 3072 and 8192 x 1024 on this path is ahead
+    int planes = (int)fnn_ctx_option(ctx, FNN_OPT_DIGIT_PLANES);
+    if (planes != 3 && planes != 4 && n * k <= (int64_t)2048 * 2048 && fnn_ctx_option(ctx, FNN_OPT_GEMM_INT8_MIN_M) >= 17) return 0;
+    // Planes by shape: three wherever they measured faster than four, i.e. 4-bit weights at every M (4096 x 11008: M = 64
+    // 26.3 against 29.3 us, M = 128 30.9 against 40.2, M = 256 47.2 against 54.9, M = 1024 139 against 168) and 8-bit
+    // weights from M = 96 (4096 x 4096: M = 64 21.6 against 19.1, M = 128 23.1 against 24.2, M = 512 40.7 against 49.7).
+    if (planes != 3 && planes != 4) planes = (dt == FNN_DT_I8 && m < 96) ? 4 : 3;
+    // 8-bit weights decode to f16 with one permute per pair, so at four planes the int8 form only ties the f16 tiles
+    // (hi + lo rows) and falls 4-5 % behind them from M = 1024 on (4096 x 4096: 93 vs 89 us, M = 2048: 172 vs 164); at
+    // three planes it stays ahead (M = 1024: 70 against 86 us, M = 2048: 128 against 160)
+    if (planes == 4 && dt == FNN_DT_I8 && m >= 768 && fnn_ctx_option(ctx, FNN_OPT_GEMM_INT8_MIN_M) <= 17) return 0;
+    return planes;
+}
+
 int fnn_digits_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, bool *handled)
 {
     *handled = false;
-    if (fnn_ctx_option(ctx, FNN_OPT_GEMM_INT8) == 0) return FNN_OK;
-    if (q.m < fnn_ctx_option(ctx, FNN_OPT_GEMM_INT8_MIN_M)) return FNN_OK;
     const int dt = w->dtype;
-    if (dt != FNN_DT_I8 && dt != FNN_DT_I4 && dt != FNN_DT_U4) return FNN_OK;
-    // exact i32 sums: |digit| <= 128, |lane| <= 128 (16*q for 4-bit signed lanes) -> K * 2^14 < 2^31
-    if (q.m > (1 << 22) || q.n > (1 << 24) || q.k > (1 << 16)) return FNN_OK;
+    if (!digits_possible(ctx, dt, q.m, q.n, q.k)) return FNN_OK;
     if (q.words != w->words) return FNN_OK;   // (a row slice of a weight: the zero margin behind the last row is not behind the slice)
     if (const int64_t opt = fnn_ctx_option(ctx, FNN_OPT_FRAGMENT); opt >= 0 && !(flags & FNN_FLAG_ACT_F16_SINGLE) && q.n == w->rows && q.k == w->inner) {
         float us;
@@ -538,27 +566,12 @@ int fnn_digits_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w,
         }
         if (rc || *handled) return rc;
     }
+    const int planes = fnn_digits_planes(ctx, dt, q.m, q.n, q.k, flags);
+    if (!planes) return FNN_OK;
     QMatmulArgs qa = q;
     int rc;
     if ((rc = fnn_aligned_rows(ctx, s, w, &qa.words, &qa.kp))) return rc;
     if (qa.kp % 4 != 0 || (reinterpret_cast<uintptr_t>(qa.words) & 15)) return FNN_OK;
-    // The single-rounding mode stays with the f16 tiles: two digit planes (15 bits below the row maximum) were 15 %
-    // faster than one f16 row but measured 1.9e-3 on rows with a few 200x outliers, where a float rounding per
-    // element keeps 2.4e-4; three planes cost what the f16 row costs.
-    if (flags & FNN_FLAG_ACT_F16_SINGLE) return FNN_OK;
-    // Small weights stay with the f16 tiles as well (by rule; FNN_OPT_DIGIT_PLANES = 3 or 4 or FNN_OPT_GEMM_INT8_MIN_M
-    // below its default still bring them here): 1024 x 1024 I4 at M = 48 / 256 / 1024 14.6 / 16.2 / 22.3 us here against 12.9 / 13.6 / 15.9 there, 2048 x 2048 I8
-    // at M = 64 / 512 16.4 / 26.6 against 15.1 / 22.0; from 3072 x 3072 and 8192 x 1024 on this path is ahead
-    int64_t planes = fnn_ctx_option(ctx, FNN_OPT_DIGIT_PLANES);
-    if (planes != 3 && planes != 4 && q.n * q.k <= (int64_t)2048 * 2048 && fnn_ctx_option(ctx, FNN_OPT_GEMM_INT8_MIN_M) >= 17) return FNN_OK;
-    // Planes by shape: three wherever they measured faster than four, i.e. 4-bit weights at every M (4096 x 11008: M = 64
-    // 26.3 against 29.3 us, M = 128 30.9 against 40.2, M = 256 47.2 against 54.9, M = 1024 139 against 168) and 8-bit
-    // weights from M = 96 (4096 x 4096: M = 64 21.6 against 19.1, M = 128 23.1 against 24.2, M = 512 40.7 against 49.7).
-    if (planes != 3 && planes != 4) planes = (dt == FNN_DT_I8 && q.m < 96) ? 4 : 3;
-    // 8-bit weights decode to f16 with one permute per pair, so at four planes the int8 form only ties the f16 tiles
-    // (hi + lo rows) and falls 4-5 % behind them from M = 1024 on (4096 x 4096: 93 vs 89 us, M = 2048: 172 vs 164); at
-    // three planes it stays ahead (M = 1024: 70 against 86 us, M = 2048: 128 against 160)
-    if (planes == 4 && dt == FNN_DT_I8 && q.m >= 768 && fnn_ctx_option(ctx, FNN_OPT_GEMM_INT8_MIN_M) <= 17) return FNN_OK;
     if (planes == 3) {
         switch (dt) {
         case FNN_DT_I8: rc = run_digits3<FNN_DT_I8>(ctx, s, w, qa); break;

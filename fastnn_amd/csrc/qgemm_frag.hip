@@ -304,8 +304,8 @@ float tiled_us(bool integer, bool ragged, int64_t m, int64_t n, int64_t k)
 }
 
 // The launch for an [M, K] x [N, K]^T product with this weight; false: the call is not this kernel's.  The same for every
-// call of the same sizes, so that the MatMul before can prepare the operand.
-bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, FragPlan *out)
+// call of the same sizes, so that the MatMul before can prepare the operand (q null: the call is not there yet).
+bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, const QMatmulArgs *q, FragPlan *out)
 {
     const int64_t opt = fnn_ctx_option(ctx, FNN_OPT_FRAGMENT);
     if (opt < 0 || (flags & (FNN_FLAG_ACT_F16_SINGLE | FNN_FLAG_ACT_QUANT | FNN_FLAG_FORCE_GENERIC | FNN_FLAG_PREFER_FMA))) return false;
@@ -340,6 +340,9 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
         const bool ragged = w->kp % 4 != 0 || k % 8 != 0;
         if (m > 2048 || !fnn_frag_options_untouched(ctx)) return false;
         if (m <= 16 && !ragged && (m <= 4 || direct_steps > 4 || (m <= 8 && integer))) return false;
+        // Four digit planes keep 30 bits of an activation and exact sums, hi + lo f16 rows 22 bits and f32 sums: the product of
+        // 4096 x 4096 I8 is 6.2e-8 off (2-norm, against 64 bits) there and 1.3e-7 here, so those calls stay there at any time.
+        if (q && fnn_digits_planes(ctx, dt, m, n, k, flags) == 4 && !(m <= 32 && fnn_stream_takes(ctx, w, *q, flags))) return false;
         float best = 1e30f;
         if (direct_ok)
             for (FragShape t : kDirect) {
@@ -434,7 +437,7 @@ int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, c
 {
     *handled = false;
     FragPlan f;
-    if (q.words != w->words || q.n != w->rows || q.k != w->inner || !frag_plan(ctx, w, q.m, flags, &f)) return FNN_OK;
+    if (q.words != w->words || q.n != w->rows || q.k != w->inner || !frag_plan(ctx, w, q.m, flags, &q, &f)) return FNN_OK;
     FragArgs p = {};
     int rc;
     if ((rc = fnn_fragment_words(ctx, s, w, f.ks.kblocks, &p.wf))) return rc;
@@ -469,7 +472,7 @@ int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, c
     const bool chain = pio->next_w && q.m >= 33 && p.vec4 && q.n % 8 == 0 && (pio->next_a == q.out || (p.residual && pio->next_a == p.sum_out)) &&
                        pio->next_w->inner == q.n && !fnn_ctx_static_mode(ctx) &&
                        (pio->next_w->dtype == FNN_DT_U8 || pio->next_w->dtype == FNN_DT_F8 || pio->next_w->dtype == FNN_DT_F8R || pio->next_w->dtype == FNN_DT_F4) &&
-                       frag_plan(ctx, pio->next_w, q.m, pio->next_flags, &nf) && nf.ks.piece << (nf.four_bit ? 2 : 1) <= 32 &&
+                       frag_plan(ctx, pio->next_w, q.m, pio->next_flags, nullptr, &nf) && nf.ks.piece << (nf.four_bit ? 2 : 1) <= 32 &&
                        fnn_ctx_ensure_tmp(ctx, next_slot, nf.ws_bytes, &next_ws) == FNN_OK && next_ws;
     if (!handed && !direct && (rc = fnn_ctx_ensure_tmp(ctx, 0, f.ws_bytes, &ws0))) return rc;
     if ((chain || f.ks.splits > 1) && (rc = fnn_ctx_ensure_tmp(ctx, 1, (size_t)f.ks.splits * q.m * q.n * 4, &ws1))) return rc;

@@ -55,11 +55,8 @@ bool plan_stream(int bits, int max_tiles, int max_mb, int64_t m, int64_t n, int6
     return true;
 }
 
-}  // namespace
-
-int fnn_stream_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, bool *handled)
+bool stream_plan_for(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, StreamPlan *pl)
 {
-    *handled = false;
     int64_t lo = fnn_ctx_option(ctx, FNN_OPT_STREAM_MIN_M), hi = fnn_ctx_option(ctx, FNN_OPT_STREAM_MAX_M);
     const int dt = w->dtype;
     const bool cb = dt == FNN_DT_I4CB;
@@ -85,24 +82,39 @@ int fnn_stream_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w,
         if (q.k >= 4 * q.n || (q.k >= 2 * q.n && q.k >= 8192)) lo = lo < 9 ? lo : 9;
         if (q.n <= 2048 && q.k >= 4 * q.n && q.k >= (int_type ? 16384 : 8192)) lo = lo < 5 ? lo : 5;
     }
-    if (q.m < lo || q.m > hi || q.m > (cb ? 64 : 32) || q.n < 1) return FNN_OK;
-    if (flags & FNN_FLAG_ACT_F16_SINGLE) return FNN_OK;
-    if (cb && fnn_ctx_option(ctx, FNN_OPT_CODEBOOK_EXPANDED) != 0) return FNN_OK;   // (the option names a form of the tiled path)
+    if (q.m < lo || q.m > hi || q.m > (cb ? 64 : 32) || q.n < 1) return false;
+    if (flags & FNN_FLAG_ACT_F16_SINGLE) return false;
+    if (cb && fnn_ctx_option(ctx, FNN_OPT_CODEBOOK_EXPANDED) != 0) return false;   // (the option names a form of the tiled path)
     if (cb && (q.as_written || q.qblock != 32 || q.k % 128 != 0 || q.bpr != q.k / 32 || (reinterpret_cast<uintptr_t>(q.scales) & 15) ||
-               q.bpr * 4 * 256 >= (int64_t)1 << 31)) return FNN_OK;
-    if (dt < FNN_DT_I8 || (dt > FNN_DT_F4 && !cb)) return FNN_OK;
-    if (int_type && fnn_ctx_option(ctx, FNN_OPT_GEMM_INT8) == 0) return FNN_OK;
-    if (q.kp % 4 != 0 || q.k % 8 != 0 || q.k < 8) return FNN_OK;
+               q.bpr * 4 * 256 >= (int64_t)1 << 31)) return false;
+    if (dt < FNN_DT_I8 || (dt > FNN_DT_F4 && !cb)) return false;
+    if (int_type && fnn_ctx_option(ctx, FNN_OPT_GEMM_INT8) == 0) return false;
+    if (q.kp % 4 != 0 || q.k % 8 != 0 || q.k < 8) return false;
     // the f16 types multiply whatever bytes a lane load holds: every load must lie wholly inside or wholly past K
-    if (!int_type && q.k % (dt == FNN_DT_F4 ? 128 : 64) != 0) return FNN_OK;
-    if ((reinterpret_cast<uintptr_t>(q.a) & 15) || (reinterpret_cast<uintptr_t>(q.words) & 15)) return FNN_OK;
+    if (!int_type && q.k % (dt == FNN_DT_F4 ? 128 : 64) != 0) return false;
+    if ((reinterpret_cast<uintptr_t>(q.a) & 15) || (reinterpret_cast<uintptr_t>(q.words) & 15)) return false;
     // 32-bit buffer offsets: a column tile of 256 rows, the activation block
-    if (q.kp * 4 * 256 >= (int64_t)1 << 31 || q.m * q.k * 4 >= (int64_t)0xFFFFFF00 || q.k >= (int64_t)1 << 28) return FNN_OK;
-    StreamPlan pl;
+    if (q.kp * 4 * 256 >= (int64_t)1 << 31 || q.m * q.k * 4 >= (int64_t)0xFFFFFF00 || q.k >= (int64_t)1 << 28) return false;
     const int64_t forced = fnn_ctx_option(ctx, FNN_OPT_STREAM_SHAPE);
     const int bits = (dt == FNN_DT_I4 || dt == FNN_DT_U4 || dt == FNN_DT_F4 || cb) ? 4 : 8;
-    if (!plan_stream(bits, int_type ? 4 : (cb ? 6 : 8), cb ? 4 : 2, q.m, q.n, q.k, forced, &pl)) return FNN_OK;
-    if (pl.ntiles > FNN_STREAM_COUNTERS) return FNN_OK;
+    return plan_stream(bits, int_type ? 4 : (cb ? 6 : 8), cb ? 4 : 2, q.m, q.n, q.k, forced, pl) && pl->ntiles <= FNN_STREAM_COUNTERS;
+}
+
+}  // namespace
+
+bool fnn_stream_takes(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QMatmulArgs &q, int flags)
+{
+    StreamPlan pl;
+    return stream_plan_for(ctx, w, q, flags, &pl);
+}
+
+int fnn_stream_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, bool *handled)
+{
+    *handled = false;
+    StreamPlan pl;
+    if (!stream_plan_for(ctx, w, q, flags, &pl)) return FNN_OK;
+    const int dt = w->dtype;
+    const bool cb = dt == FNN_DT_I4CB;
     StreamArgs p;
     p.words = q.words; p.scales = q.scales; p.zeros = q.zeros; p.a = q.a; p.bias = q.bias; p.out = q.out;
     p.codebook = cb ? q.codebook : nullptr; p.bpr = cb ? q.bpr : 0;

@@ -84,3 +84,24 @@ def test_every_shape_of_the_integer_fragment_kernels(ctx, orc, dt, m, k, n):
     finally:
         ctx.set_option(flib.OPT_FRAGMENT, 0)
         ctx.release(h)
+
+
+@pytest.mark.parametrize("m,k,n", [(17, 2050, 2100), (33, 4096, 1100), (64, 2050, 2100), (95, 4096, 1100)])
+def test_int8_weights_keep_four_digit_planes(ctx, m, k, n):
+    """The sizes whose activations are four digit planes: exact sums, so what is left is the rounding of the recombination
+    (four conversions, three multiply-adds, the scale, the K split's additions: at most 14 roundings of 2.4e-8 rms each,
+    9e-8 in all).  f16 hi + lo rows with f32 sums are 1.2e-7 off and more."""
+    rng = np.random.default_rng(9300 + m)
+    pw = fastnn_amd.quantize_weights(flib.DT_I8, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    pw.zeros = np.zeros(0, np.float32)
+    lanes = pw.words[:n * (-(-k // 4))].view(np.int8).reshape(n, -1)[:, :k].astype(np.float64)
+    h = ctx.register(pw)
+    try:
+        for scale in (1.0, 100.0):
+            a = rng.standard_normal((m, k)).astype(np.float32)
+            a[:, ::61] *= scale
+            want = a.astype(np.float64) @ lanes.T * pw.scales.astype(np.float64)
+            got = ctx.qmatmul(h, a, n)
+            assert np.linalg.norm(got - want) <= 9e-8 * np.linalg.norm(want), (scale, np.linalg.norm(got - want) / np.linalg.norm(want))
+    finally:
+        ctx.release(h)
