@@ -35,6 +35,10 @@ struct FragSplit {
 
 // A row's values of a piece of K: the power of two applied to them, and their sum (for the zero-point term).
 struct FragRow { int e; float sum; };
+__device__ __forceinline__ double frag_sum8(const float(&v)[8])
+{
+    return (double)(((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
+}
 
 struct FragArgs {
     const uint32_t *wf;          // weight fragments [row block of 16][k block][q 0..3][row][16 bytes]

@@ -75,8 +75,10 @@ __device__ __forceinline__ void reduce8(const FragArgs &p, int64_t m, int64_t n,
 template <bool CHAIN, int STEPS, int NW>
 __global__ void __launch_bounds__(NW * 64) frag_prep_kernel(FragPrepArgs p)
 {
-    __shared__ float red[2][NW][16];
-    __shared__ float part[STEPS == 1 ? 2 * NW : 1][64];   // one step per wave: its two half sums per lane
+    // Row sums in double from eight values on: chained in f32 over a lane's steps, the waves and the pieces they were 1.1e-7 off
+    // (2-norm, K = 1000 .. 6000; now 5e-8), and with a large zero point that is the error of the result.
+    __shared__ float red[NW][16];
+    __shared__ double part[NW][STEPS == 1 ? 64 : 16];   // one step per wave: per lane
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r = lane & 15, q = lane >> 4;
     int b0, b1;
     p.ks.piece_at((int)blockIdx.x, &b0, &b1);
@@ -120,12 +122,12 @@ __global__ void __launch_bounds__(NW * 64) frag_prep_kernel(FragPrepArgs p)
         }
     };
     float keep[STEPS][8];
-    float mx = 0.0f, sum = 0.0f;
+    float mx = 0.0f;
+    double sum = 0.0;
     auto stats = [&](const float(&v)[8]) {
         mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))),
                              fmaxf(fmaxf(fabsf(v[4]), fabsf(v[5])), fmaxf(fabsf(v[6]), fabsf(v[7])))));
-        sum += (v[0] + v[1]) + (v[2] + v[3]);
-        sum += (v[4] + v[5]) + (v[6] + v[7]);
+        sum += frag_sum8(v);
     };
     const bool in_regs = CHAIN || s1 - s0 <= NW * STEPS;
     if (in_regs) {
@@ -139,17 +141,16 @@ __global__ void __launch_bounds__(NW * 64) frag_prep_kernel(FragPrepArgs p)
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     if constexpr (STEPS == 1) {
-        part[2 * wv][lane] = (keep[0][0] + keep[0][1]) + (keep[0][2] + keep[0][3]);
-        part[2 * wv + 1][lane] = (keep[0][4] + keep[0][5]) + (keep[0][6] + keep[0][7]);
-        if (q == 0) red[0][wv][r] = mx;
+        part[wv][lane] = sum;
     } else {
         sum += __shfl_xor(sum, 16, 64);
         sum += __shfl_xor(sum, 32, 64);
-        if (q == 0) { red[0][wv][r] = mx; red[1][wv][r] = sum; }
+        if (q == 0) part[wv][r] = sum;
     }
+    if (q == 0) red[wv][r] = mx;
     __syncthreads();
 #pragma unroll
-    for (int w2 = 0; w2 < NW; w2++) mx = fmaxf(mx, red[0][w2][r]);
+    for (int w2 = 0; w2 < NW; w2++) mx = fmaxf(mx, red[w2][r]);
     int e = 0;
     if (mx > 0.0f && mx < __builtin_huge_valf()) {
         int ex;
@@ -178,17 +179,14 @@ __global__ void __launch_bounds__(NW * 64) frag_prep_kernel(FragPrepArgs p)
         for (int s = s0 + wv; s < s1; s += NW) { load8(s, keep[0]); convert(s, keep[0]); }
     }
     if (wv != 0) return;
-    float t = 0.0f;
-    if constexpr (STEPS == 1) {   // in the order of the kernel that converts for itself: the two give the same bits
+    double t = 0.0;
 #pragma unroll
-        for (int h = 0; h < 2 * NW; h++) t += part[h][lane];
+    for (int w2 = 0; w2 < NW; w2++) t += part[w2][STEPS == 1 ? lane : r];
+    if constexpr (STEPS == 1) {   // in the order of the kernel that converts for itself: the two give the same bits
         t += __shfl_xor(t, 16, 64);
         t += __shfl_xor(t, 32, 64);
-    } else {
-#pragma unroll
-        for (int w2 = 0; w2 < NW; w2++) t += red[1][w2][r];
     }
-    if (q == 0) p.rows[(int64_t)blockIdx.x * p.m_pad + (int64_t)blockIdx.y * 16 + r] = FragRow{e, t};
+    if (q == 0) p.rows[(int64_t)blockIdx.x * p.m_pad + (int64_t)blockIdx.y * 16 + r] = FragRow{e, (float)t};
 }
 
 template <bool CHAIN>

@@ -23,14 +23,14 @@ constexpr float FRAG_LO_DOWN = 1.0f / 2048.0f;   // the lo activation term is st
 // sum[i]: sum of A[m,k] over this wave's segment, m = row 16 i + (lane & 15).
 template <int MB, int NB>
 __device__ __forceinline__ void frag_finish(const FragArgs &p, unsigned mt, unsigned nt, unsigned z, const f32x4 (&total)[MB][NB],
-                                            const float (&sum)[MB])
+                                            const double (&sum)[MB])
 {
     extern __shared__ __attribute__((aligned(16))) f32x4 red[];   // [wave][tile][lane]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     // D: column (lane & 15) = activation row, rows 4 (lane >> 4) + i = weight rows
     constexpr int TILES = MB * NB;
-    __shared__ float xsum[FRAG_NW][MB * 16];
+    __shared__ double xsum[FRAG_NW][MB * 16];
     if (lane < 16) {
 #pragma unroll
         for (int i = 0; i < MB; i++) xsum[wv][i * 16 + lane] = sum[i];
@@ -70,9 +70,10 @@ __device__ __forceinline__ void frag_finish(const FragArgs &p, unsigned mt, unsi
 #pragma unroll
         for (int q = 1; q < FRAG_NW; q++) v += red[q * TILES * 64 + c];
         const int lrow = (c >> 6) / NB * 16 + (c & 15);
-        float xs = xsum[0][lrow];
+        double xd = xsum[0][lrow];
 #pragma unroll
-        for (int q = 1; q < FRAG_NW; q++) xs += xsum[q][lrow];
+        for (int q = 1; q < FRAG_NW; q++) xd += xsum[q][lrow];
+        const float xs = (float)xd;
         float d[4] = {v[0] * sc[r].x + zp[r].x * xs, v[1] * sc[r].y + zp[r].y * xs, v[2] * sc[r].z + zp[r].z * xs, v[3] * sc[r].w + zp[r].w * xs};
         float *o = p.out + om[r] * p.n + on[r];
         if (split) {
@@ -134,7 +135,7 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_kernel(FragArgs p)
     // largest tiles have no registers for a second set of sums, their segments are one piece.
     constexpr bool PIECES = MB * NB <= 8;
     f32x4 total[MB][NB];
-    float xsum[MB];
+    double xsum[MB];
     FragRow row[MB];   // of this lane's activation rows (lane & 15) in the current piece
     const FragRow *rows = p.rows + ((int64_t)z * FRAG_NW + wv) * p.ks.pieces * p.m_pad + (int64_t)mt * MB * 16 + (lane & 15);
     auto next_rows = [&] {
@@ -162,7 +163,7 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_kernel(FragArgs p)
     };
 #pragma unroll
     for (int i = 0; i < MB; i++) {
-        xsum[i] = 0.0f;
+        xsum[i] = 0.0;
         if constexpr (PIECES)
 #pragma unroll
             for (int j = 0; j < NB; j++) total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -311,14 +312,14 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_direct_kernel(FragArg
         }
 #pragma unroll
         for (int i = 0; i < MB; i++) {
-            float mx = 0.0f, sum = 0.0f;
+            float mx = 0.0f;
+            double sum = 0.0;
 #pragma unroll
             for (int s = 0; s < STEPS; s++) {
                 const float(&v)[8] = x[i][s];
                 mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))),
                                      fmaxf(fmaxf(fabsf(v[4]), fabsf(v[5])), fmaxf(fabsf(v[6]), fabsf(v[7])))));
-                sum += (v[0] + v[1]) + (v[2] + v[3]);
-                sum += (v[4] + v[5]) + (v[6] + v[7]);
+                sum += frag_sum8(v);
             }
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
@@ -330,7 +331,7 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_direct_kernel(FragArg
                 (void)frexpf(mx, &ex);
                 e = 15 - ex;
             }
-            row[i] = FragRow{e, sum};
+            row[i] = FragRow{e, (float)sum};
         }
 #pragma unroll
         for (int s = 0; s < STEPS; s++) {
@@ -361,10 +362,10 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_direct_kernel(FragArg
         }
     }
     f32x4 total[MB][NB];
-    float xsum[MB];
+    double xsum[MB];
 #pragma unroll
     for (int i = 0; i < MB; i++) {
-        xsum[i] = 0.0f + row[i].sum;
+        xsum[i] = row[i].sum;
 #pragma unroll
         for (int j = 0; j < NB; j++)
 #pragma unroll

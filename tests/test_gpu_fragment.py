@@ -105,3 +105,25 @@ def test_int8_weights_keep_four_digit_planes(ctx, m, k, n):
             assert np.linalg.norm(got - want) <= 9e-8 * np.linalg.norm(want), (scale, np.linalg.norm(got - want) / np.linalg.norm(want))
     finally:
         ctx.release(h)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 301, 40), (16, 1003, 72), (33, 1003, 72), (64, 6005, 72), (48, 2048, 64)])
+def test_row_sums_of_the_fragment_kernels(ctx, m, k, n):
+    """The zero-point term alone (scale 0, zero 1): every column is its row's sum.  Three levels of f32 additions per eight
+    values, the sum of a piece of K and the result: five roundings of 2.4e-8 rms, 5.4e-8 of sqrt(K) times the rms of a value."""
+    rng = np.random.default_rng(9400 + m)
+    pw = fastnn_amd.quantize_weights(flib.DT_U8, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    pw.scales, pw.zeros = np.zeros(n, np.float32), np.ones(n, np.float32)
+    h = ctx.register(pw)
+    try:
+        for shape in (0, 1 << 8 | 1 << 4 | 1, 2 << 8 | 2 << 4 | 2, 1 << 8 | 4 << 4 | 4):
+            ctx.set_option(flib.OPT_FRAGMENT, shape)
+            square = 0.0
+            for _ in range(64 // m + 8):
+                a = rng.standard_normal((m, k)).astype(np.float32)
+                off = ctx.qmatmul(h, a, n)[:, 0] - a.astype(np.float64).sum(1)
+                square += (off ** 2).mean() / k / (64 // m + 8)
+            assert square ** 0.5 <= 7e-8, (hex(shape), square ** 0.5)
+    finally:
+        ctx.set_option(flib.OPT_FRAGMENT, 0)
+        ctx.release(h)
