@@ -1259,12 +1259,19 @@ int fnn_hip_graph_destroy(fnn_hip_ctx *ctx, fnn_hip_graph *g)
 }  // extern "C"
 
 // staging access for the matrix-core translation units
+// 0: prepared operands, 1: partial tiles / accumulators, 2 and 3: conv operand, transient weight expansion,
+// 4: the prepared operand one MatMul call leaves for the next
+static Staging &tmp_slot(fnn_hip_ctx *ctx, int which)
+{
+    return which == 0 ? ctx->st_tmp : (which == 1 ? ctx->st_tmp2 : (which == 4 ? ctx->st_tmp4 : ctx->st_tmp3));
+}
+// fnn_hip_qmatmul_static: fixed regions of the static workspace, nothing grows
+static size_t static_room(int which) { return which == 0 ? kStaticOperandBytes : (which == 1 ? kStaticPartialBytes : 0); }
+
 int fnn_ctx_ensure_tmp(fnn_hip_ctx *ctx, int which, size_t bytes, void **ptr)
 {
     if (ctx->static_mode) {
-        // fnn_hip_qmatmul_static: fixed regions of the static workspace, nothing grows
-        const size_t off = which == 0 ? 0 : kStaticOperandBytes;
-        const size_t cap = which == 0 ? kStaticOperandBytes : (which == 1 ? kStaticPartialBytes : 0);
+        const size_t off = which == 0 ? 0 : kStaticOperandBytes, cap = static_room(which);
         if (bytes > cap)
             return fail(ctx, FNN_ERR_MEMORY,
                         "fnn_hip_qmatmul_static: this shape needs %zu bytes of %s workspace, the static buffer holds %zu: use fnn_hip_qmatmul",
@@ -1272,13 +1279,24 @@ int fnn_ctx_ensure_tmp(fnn_hip_ctx *ctx, int which, size_t bytes, void **ptr)
         *ptr = ctx->static_ws + off;
         return FNN_OK;
     }
-    // 0: prepared operands, 1: partial tiles / accumulators, 2 and 3: conv operand, transient weight expansion,
-    // 4: the prepared operand one MatMul call leaves for the next
-    Staging &s = which == 0 ? ctx->st_tmp : (which == 1 ? ctx->st_tmp2 : (which == 4 ? ctx->st_tmp4 : ctx->st_tmp3));
+    Staging &s = tmp_slot(ctx, which);
     int rc = ensure(ctx, s, bytes);
     if (rc) return rc;
     *ptr = s.ptr;
     return FNN_OK;
+}
+
+bool fnn_ctx_tmp_fits(fnn_hip_ctx *ctx, int which, size_t bytes)
+{
+    if (ctx->static_mode) return bytes <= static_room(which);
+    return !ctx->capturing || bytes <= tmp_slot(ctx, which).cap;
+}
+
+bool fnn_ctx_operand_allowed(fnn_hip_ctx *ctx, int64_t m, int64_t k, size_t bytes)
+{
+    // (the limit that the header names: sizes within it run the same kernel with either entry point)
+    const bool promised = m <= FNN_STATIC_MAX_M && 4 * ((m + 15) / 16 * 16) * ((k + 63) / 64 * 64) + 12 * m <= (int64_t)kStaticOperandBytes;
+    return bytes <= kStaticOperandBytes || (!promised && !ctx->static_mode);
 }
 
 bool fnn_ctx_capturing(fnn_hip_ctx *ctx) { return ctx->capturing; }

@@ -190,8 +190,6 @@ int run_digits_wave(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, co
     WaveArgs p = {};
     int rc;
     p.kblocks = (int)((w->kp + 15) / 16);
-    if ((rc = fnn_fragment_words(ctx, s, w, p.kblocks, &p.wf))) return rc;
-    if (!p.wf) return FNN_OK;
     const int64_t kstep = (int64_t)p.kblocks * (W8 ? 2 : 4);        // steps that hold weights
     p.units = (int)((kstep + RING - 1) / RING);
     p.units_per_wave = (p.units + wk - 1) / wk;
@@ -204,8 +202,12 @@ int run_digits_wave(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, co
     p.by_stripe = fast_div((uint32_t)p.ntiles * 4);
     const int64_t m_pad = (int64_t)p.mtiles * act_rows;
     const size_t a_bytes = (size_t)m_pad * 3 * p.nsteps * 32;
+    const size_t op_bytes = a_bytes + (size_t)m_pad * 8;
+    if (!fnn_ctx_operand_allowed(ctx, q.m, q.k, op_bytes) || !fnn_ctx_tmp_fits(ctx, 0, op_bytes)) return FNN_OK;
+    if ((rc = fnn_fragment_words(ctx, s, w, p.kblocks, &p.wf))) return rc;
+    if (!p.wf) return FNN_OK;
     void *ws0 = nullptr;
-    if ((rc = fnn_ctx_ensure_tmp(ctx, 0, a_bytes + (size_t)m_pad * 8, &ws0))) return rc;
+    if ((rc = fnn_ctx_ensure_tmp(ctx, 0, op_bytes, &ws0))) return rc;
     *fnn_ctx_prepared(ctx) = FnnPreparedOperand{};
     DigitArgs d;
     d.a = q.a;

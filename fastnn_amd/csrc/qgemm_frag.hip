@@ -301,6 +301,23 @@ float tiled_us(bool integer, bool ragged, int64_t m, int64_t n, int64_t k)
     return q[0] + q[1] * fm * fn * fk / 1e9f + q[2] * fm * fn / 1e6f + q[3] * fn * fk / 1e6f + q[4] * fm * fk / 1e6f + q[5] * fk / 1e3f;
 }
 
+// K dealt out over `splits` and the bytes of the operand, for the plan's tiles
+void frag_sizes(FragPlan *f, int64_t m, int splits)
+{
+    if (splits > f->ks.kblocks) splits = f->ks.kblocks;
+    f->ks.kb_per_split = (f->ks.kblocks + splits - 1) / splits;
+    f->ks.splits = (f->ks.kblocks + f->ks.kb_per_split - 1) / f->ks.kb_per_split;
+    f->ks.seg = (f->ks.kb_per_split + FRAG_NW - 1) / FRAG_NW;
+    f->ks.seg_last = (f->ks.kblocks - (f->ks.splits - 1) * f->ks.kb_per_split + FRAG_NW - 1) / FRAG_NW;
+    f->m_pad = (m + f->op_mb * 16 - 1) / (f->op_mb * 16) * (f->op_mb * 16);
+    // pieces of eight steps (256 k-values): a preparation workgroup per piece and row block
+    const int seg = f->ks.seg > f->ks.seg_last ? f->ks.seg : f->ks.seg_last, eight = f->four_bit ? 2 : 4;
+    f->ks.piece = f->op_mb * f->op_nb <= 8 && seg > eight ? eight : seg;
+    f->ks.pieces = (seg + f->ks.piece - 1) / f->ks.piece;
+    f->op_bytes = (size_t)f->m_pad * f->ks.kblocks * (f->four_bit ? 128 : 64) * 4;
+    f->ws_bytes = f->op_bytes + (size_t)f->ks.splits * FRAG_NW * f->ks.pieces * f->m_pad * sizeof(FragRow);
+}
+
 // The launch for an [M, K] x [N, K]^T product with this weight; false: the call is not this kernel's.  The same for every
 // call of the same sizes, so that the MatMul before can prepare the operand (q null: the call is not there yet).
 bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, const QMatmulArgs *q, FragPlan *out)
@@ -354,18 +371,18 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
                 for (int sp : {1, 2, 4, 8}) {
                     if (sp > 1 && (wgs * sp > 1024 || sp * 8 > f.ks.kblocks)) break;
                     const float us = two_launch_us(t, sp, m, n, f.ks.kblocks, f.four_bit);
-                    if (us < best) { best = us; f.mb = t.mb; f.nb = t.nb; f.direct = false; splits = sp; }
+                    if (us >= best) continue;
+                    FragPlan c = f;
+                    c.op_mb = t.mb; c.op_nb = t.nb;
+                    frag_sizes(&c, m, sp);
+                    if (!fnn_ctx_operand_allowed(ctx, m, k, c.ws_bytes)) continue;
+                    best = us; f.mb = t.mb; f.nb = t.nb; f.direct = false; splits = sp;
                 }
             }
         // (the margin: where the two are about equal the fits decide at random, and what was there stays)
         if (best > 1e29f || (m >= 33 && best > 0.93f * tiled_us(integer, ragged, m, n, k))) return false;
         if (float us; !(flags & FNN_FLAG_ACT_F16_SINGLE) && fnn_wave_choice(w->dtype, m, n, k, &us) && us < best) return false;
     }
-    if (splits > f.ks.kblocks) splits = f.ks.kblocks;
-    f.ks.kb_per_split = (f.ks.kblocks + splits - 1) / splits;
-    f.ks.splits = (f.ks.kblocks + f.ks.kb_per_split - 1) / f.ks.kb_per_split;
-    f.ks.seg = (f.ks.kb_per_split + FRAG_NW - 1) / FRAG_NW;
-    f.ks.seg_last = (f.ks.kblocks - (f.ks.splits - 1) * f.ks.kb_per_split + FRAG_NW - 1) / FRAG_NW;
     f.rblocks = (int)((n + 15) / 16);
     f.op_mb = f.mb; f.op_nb = f.nb;
     if (f.direct) {
@@ -375,13 +392,7 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
             if (us < best) { best = us; f.op_mb = t.mb; f.op_nb = t.nb; }
         }
     }
-    f.m_pad = (m + f.op_mb * 16 - 1) / (f.op_mb * 16) * (f.op_mb * 16);
-    // pieces of eight steps (256 k-values): a preparation workgroup per piece and row block
-    const int seg = f.ks.seg > f.ks.seg_last ? f.ks.seg : f.ks.seg_last, eight = f.four_bit ? 2 : 4;
-    f.ks.piece = f.op_mb * f.op_nb <= 8 && seg > eight ? eight : seg;
-    f.ks.pieces = (seg + f.ks.piece - 1) / f.ks.piece;
-    f.op_bytes = (size_t)f.m_pad * f.ks.kblocks * (f.four_bit ? 128 : 64) * 4;
-    f.ws_bytes = f.op_bytes + (size_t)f.ks.splits * FRAG_NW * f.ks.pieces * f.m_pad * sizeof(FragRow);
+    frag_sizes(&f, m, splits);
     *out = f;
     return true;
 }
@@ -436,6 +447,18 @@ int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, c
     *handled = false;
     FragPlan f;
     if (q.words != w->words || q.n != w->rows || q.k != w->inner || !frag_plan(ctx, w, q.m, flags, &q, &f)) return FNN_OK;
+    // What travels between the MatMuls of a plan (range_io.h): the operand may be in place, and the next one's may be asked
+    // for.  From 33 rows on: below, the MatMuls that convert for themselves are ahead of a reduction launch each.  (Integer
+    // weights as the next ones: their MatMul prepares its own operand.)
+    FnnPrepIo *pio = fnn_ctx_prep_io(ctx);
+    FnnPreparedOperand *have = fnn_ctx_prepared(ctx);
+    const int interleaved = w->dtype == FNN_DT_I4 || w->dtype == FNN_DT_U4 ? 1 : 0;
+    const bool handed = pio->offered && have->buffer && have->fragments == 1 + (f.four_bit ? 1 : 0) && have->a == q.a && have->m == q.m && have->k == q.k &&
+                        have->rows_pad == f.m_pad && have->kpad == f.ks.kb_per_split && have->interleaved == interleaved;
+    const bool direct = f.direct && !handed;
+    // what does not fit is left to the kernels behind this one
+    if ((!handed && !direct && !fnn_ctx_tmp_fits(ctx, 0, f.ws_bytes)) ||
+        (f.ks.splits > 1 && !fnn_ctx_tmp_fits(ctx, 1, (size_t)f.ks.splits * q.m * q.n * 4))) return FNN_OK;
     FragArgs p = {};
     int rc;
     if ((rc = fnn_fragment_words(ctx, s, w, f.ks.kblocks, &p.wf))) return rc;
@@ -449,16 +472,6 @@ int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, c
     }
     p.vec4 = q.n % 4 == 0 && !((reinterpret_cast<uintptr_t>(p.out) | reinterpret_cast<uintptr_t>(p.residual) | reinterpret_cast<uintptr_t>(p.sum_out) |
                                 reinterpret_cast<uintptr_t>(p.scales) | reinterpret_cast<uintptr_t>(p.zeros) | reinterpret_cast<uintptr_t>(p.bias)) & 15);
-
-    // What travels between the MatMuls of a plan (range_io.h): the operand may be in place, and the next one's may be asked
-    // for.  From 33 rows on: below, the MatMuls that convert for themselves are ahead of a reduction launch each.  (Integer
-    // weights as the next ones: their MatMul prepares its own operand.)
-    FnnPrepIo *pio = fnn_ctx_prep_io(ctx);
-    FnnPreparedOperand *have = fnn_ctx_prepared(ctx);
-    const int interleaved = w->dtype == FNN_DT_I4 || w->dtype == FNN_DT_U4 ? 1 : 0;
-    const bool handed = pio->offered && have->buffer && have->fragments == 1 + (f.four_bit ? 1 : 0) && have->a == q.a && have->m == q.m && have->k == q.k &&
-                        have->rows_pad == f.m_pad && have->kpad == f.ks.kb_per_split && have->interleaved == interleaved;
-    const bool direct = f.direct && !handed;
     const int mb = direct ? f.mb : f.op_mb, nb = direct ? f.nb : f.op_nb;
     p.mtiles = (int)((q.m + mb * 16 - 1) / (mb * 16));
     p.ntiles = (int)((q.n + nb * 16 - 1) / (nb * 16));

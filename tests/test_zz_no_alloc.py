@@ -107,3 +107,26 @@ def test_static_entry_point_refuses_what_does_not_fit(orc):
         ctx.qmatmul_static(h, d64.ptr, 64, o64.ptr)
         ctx.sync()
         assert_close(o64.download(np.float32, 64 * n).reshape(64, n), orc.qmatmul(to_oracle(orc, pw), a), 2e-5, "after refusals")
+
+
+@pytest.mark.parametrize("dt,m,k,n,within", [(flib.DT_I8, 97, 16384, 2048, True), (flib.DT_I8, 112, 16384, 2048, True), (flib.DT_I8, 128, 16384, 2048, False),
+                                             (flib.DT_U8, 97, 16384, 2048, True), (flib.DT_I4, 112, 16384, 2048, True), (flib.DT_F8, 49, 32000, 512, True),
+                                             (flib.DT_I4, 128, 16384, 2048, False)])
+def test_static_entry_point_takes_what_its_limits_allow(dt, m, k, n, within):
+    """Sizes close to the operand limit, on a weight that fnn_hip_qmatmul has run (so that every copy of it exists): inside the
+    limit the two entry points run the same kernel; three digit planes past it fit the buffer too and are accepted."""
+    rng = np.random.default_rng(16)
+    pw = fastnn_amd.quantize_weights(dt, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    assert within == (4 * (-(-m // 16) * 16) * (-(-k // 64) * 64) + 12 * m <= 8 << 20)
+    with fastnn_amd.HipContext(0) as ctx:
+        h = ctx.register(pw)
+        want = a.astype(np.float64) @ ctx.dequant(h, n, k).T.astype(np.float64)
+        da, d_ref, d_got = ctx.to_device(a), ctx.alloc(m * n * 4), ctx.alloc(m * n * 4)
+        ctx.qmatmul_dev(h, da.ptr, m, d_ref.ptr)
+        ctx.qmatmul_static(h, da.ptr, m, d_got.ptr)
+        ctx.sync()
+        got = d_got.download(np.float32, m * n).reshape(m, n)
+        assert_close(got, want, 2e-5, f"dt={dt} M={m} K={k}")
+        if within:
+            assert np.array_equal(got, d_ref.download(np.float32, m * n).reshape(m, n))
