@@ -52,6 +52,8 @@ int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, c
 int fnn_frag_i8act(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const I8ActArgs &p, bool *handled);
 // fragment-major copy of a weight's packed words, built on first use; null when it does not exist and this call may not build it
 int fnn_fragment_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, int64_t kblocks, const uint32_t **words);
+// that copy (kp 0) or the registered rows
+int fnn_frag_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, int64_t kblocks, const uint32_t **words, int *kp);
 // sum of the integer lanes per weight row (I8, I4), built on first use
 int fnn_row_qsum(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const int32_t **qsum);
 int fnn_tiled_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p,

@@ -197,15 +197,13 @@ int run_digits_wave(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, co
     const int act_rows = wk == 1 ? 2 * WAVE_ROWS : WAVE_ROWS, cols = wk == 4 ? WAVE_COLS : 2 * WAVE_COLS;
     p.mtiles = (int)((q.m + act_rows - 1) / act_rows);
     p.ntiles = (int)((q.n + cols - 1) / cols);
-    p.rblocks = (int)((q.n + 15) / 16);
     p.tiles = (unsigned)p.mtiles * (unsigned)p.ntiles;
     p.by_stripe = fast_div((uint32_t)p.ntiles * 4);
     const int64_t m_pad = (int64_t)p.mtiles * act_rows;
     const size_t a_bytes = (size_t)m_pad * 3 * p.nsteps * 32;
     const size_t op_bytes = a_bytes + (size_t)m_pad * 8;
     if (!fnn_ctx_operand_allowed(ctx, q.m, q.k, op_bytes) || !fnn_ctx_tmp_fits(ctx, 0, op_bytes)) return FNN_OK;
-    if ((rc = fnn_fragment_words(ctx, s, w, p.kblocks, &p.wf))) return rc;
-    if (!p.wf) return FNN_OK;
+    if ((rc = fnn_frag_words(ctx, s, w, p.kblocks, &p.wf, &p.words_kp))) return rc;
     void *ws0 = nullptr;
     if ((rc = fnn_ctx_ensure_tmp(ctx, 0, op_bytes, &ws0))) return rc;
     *fnn_ctx_prepared(ctx) = FnnPreparedOperand{};

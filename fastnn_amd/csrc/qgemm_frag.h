@@ -40,8 +40,22 @@ __device__ __forceinline__ double frag_sum8(const float(&v)[8])
     return (double)(((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
 }
 
+// The packed words as the kernels read them: the fragment-major copy [row block of 16][k block][q 0..3][row][16 bytes] (kp 0),
+// or the registered rows of kp words where there is no copy (the same values, so the same results; a wave load is then 16
+// pieces of 64 bytes instead of one contiguous KB).  This: 16 bytes `piece` of row r of row block rb in its first k block (past
+// the last of `rows`: that row's; never stored).
+__device__ __forceinline__ const uint32_t *frag_row_at(const uint32_t *w, int kp, int rows, int kblocks, int rb, int r, int piece)
+{
+    const int last_rb = (rows - 1) >> 4;
+    if (rb > last_rb) rb = last_rb;
+    if (!kp) return w + (int64_t)rb * kblocks * 256 + piece * 64 + r * 4;
+    const int last = rows - 1 - rb * 16;
+    return w + (int64_t)rb * 16 * kp + (uint32_t)((r < last ? r : last) * kp + piece * 4);
+}
+typedef uint32_t frag_u32x4 __attribute__((ext_vector_type(4), aligned(4)));   // (registered rows of any length: 4-byte aligned)
+
 struct FragArgs {
-    const uint32_t *wf;          // weight fragments [row block of 16][k block][q 0..3][row][16 bytes]
+    const uint32_t *wf;          // weight words: frag_row_at.  (Fields are dear here: 48 bytes more cost 0.25 us a launch)
     const _Float16 *af;          // activation fragments [row block of 16][step of 32 k][hi, lo][q 0..3][row][8 f16]
     const float *a;              // non-null: the f32 activations [m,k], converted in the kernel (splits == 1; af, rows unused)
     int64_t k;
@@ -55,7 +69,7 @@ struct FragArgs {
     int act;
     FragSplit ks;
     FastDiv by_mtiles, by_splits;
-    int mtiles, ntiles, rblocks; // rblocks: blocks of 16 weight rows
+    int mtiles, ntiles, words_kp;
     int vec4;                    // 16-byte accesses along n: n % 4 == 0 and aligned tensors
 };
 

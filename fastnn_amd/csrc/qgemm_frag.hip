@@ -240,7 +240,7 @@ __global__ void __launch_bounds__(256) frag_reduce_kernel(FragArgs p)
 }
 
 struct FragPlan {
-    int mb, nb, rblocks;
+    int mb, nb;
     int op_mb, op_nb;            // the tiles when the operand is in place (the same unless direct)
     FragSplit ks;
     int64_t m_pad;
@@ -383,7 +383,6 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
         if (best > 1e29f || (m >= 33 && best > 0.93f * tiled_us(integer, ragged, m, n, k))) return false;
         if (float us; !(flags & FNN_FLAG_ACT_F16_SINGLE) && fnn_wave_choice(w->dtype, m, n, k, &us) && us < best) return false;
     }
-    f.rblocks = (int)((n + 15) / 16);
     f.op_mb = f.mb; f.op_nb = f.nb;
     if (f.direct) {
         float best = 1e30f;
@@ -423,11 +422,11 @@ bool fnn_frag_options_untouched(fnn_hip_ctx *ctx)
     return true;
 }
 
-// fragment-major copy of the packed words; null when it does not exist and this call may not build it
 int fnn_fragment_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, int64_t kblocks, const uint32_t **out)
 {
     *out = nullptr;
     fnn_hip_weight *wm = const_cast<fnn_hip_weight *>(w);
+    if (fnn_ctx_option(ctx, FNN_OPT_GEMV_TILE_MAJOR) != 1) return FNN_OK;
     if (!wm->words_fr && !fnn_ctx_no_alloc(ctx)) {
         const int64_t pieces = (w->rows + 15) / 16 * kblocks * 64;
         if (hipMalloc((void **)&wm->words_fr, (size_t)pieces * 16) != hipSuccess)
@@ -439,6 +438,14 @@ int fnn_fragment_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w,
         if (hipGetLastError() != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, "building the fragment-major weight rows failed");
     }
     *out = wm->words_fr;
+    return FNN_OK;
+}
+
+int fnn_frag_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, int64_t kblocks, const uint32_t **words, int *kp)
+{
+    if (int rc = fnn_fragment_words(ctx, s, w, kblocks, words)) return rc;
+    *kp = *words ? 0 : (int)w->kp;
+    if (!*words) *words = w->words;   // (a load past the last registered row stays inside the zeroed margin behind it)
     return FNN_OK;
 }
 
@@ -461,9 +468,8 @@ int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, c
         (f.ks.splits > 1 && !fnn_ctx_tmp_fits(ctx, 1, (size_t)f.ks.splits * q.m * q.n * 4))) return FNN_OK;
     FragArgs p = {};
     int rc;
-    if ((rc = fnn_fragment_words(ctx, s, w, f.ks.kblocks, &p.wf))) return rc;
-    if (!p.wf) return FNN_OK;
-    p.ks = f.ks; p.rblocks = f.rblocks; p.m_pad = f.m_pad; p.k = q.k;
+    if ((rc = fnn_frag_words(ctx, s, w, f.ks.kblocks, &p.wf, &p.words_kp))) return rc;
+    p.ks = f.ks; p.m_pad = f.m_pad; p.k = q.k;
     p.scales = q.scales; p.zeros = q.zeros; p.bias = q.bias; p.out = q.out;
     p.m = q.m; p.n = q.n; p.act = q.act;
     if (FnnResidualIo *res = fnn_ctx_residual_io(ctx); res->residual && res->of_out == q.out && res->elems == (uint64_t)(q.m * q.n)) {

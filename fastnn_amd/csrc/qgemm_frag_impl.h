@@ -21,9 +21,9 @@ constexpr float FRAG_LO_DOWN = 1.0f / 2048.0f;   // the lo activation term is st
 
 // The eight partial tiles of a workgroup meet in LDS; scale, zero point, bias, activation, stores.
 // sum[i]: sum of A[m,k] over this wave's segment, m = row 16 i + (lane & 15).
-template <int MB, int NB>
+template <int MB, int NB, class SUM>
 __device__ __forceinline__ void frag_finish(const FragArgs &p, unsigned mt, unsigned nt, unsigned z, const f32x4 (&total)[MB][NB],
-                                            const double (&sum)[MB])
+                                            const SUM (&sum)[MB])
 {
     extern __shared__ __attribute__((aligned(16))) f32x4 red[];   // [wave][tile][lane]
     const int tid = threadIdx.x, lane = tid & 63;
@@ -106,7 +106,29 @@ __device__ __forceinline__ void frag_finish(const FragArgs &p, unsigned mt, unsi
     }
 }
 
-template <int DT, int MB, int NB>
+// of the 16 bytes `piece` of a row's last k block, the words that belong to the row
+__device__ __forceinline__ void frag_own_words(u32x4 &w, int tail, int piece)
+{
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (piece * 4 + e >= tail) w[e] = 0u;
+}
+
+// ROWS: the registered rows instead of the fragment-major copy (strides and ends that are known only at run time cost the
+// others 1 %)
+template <bool ROWS>
+__device__ __forceinline__ const uint32_t *frag_row(const FragArgs &p, int rb, int lane)
+{
+    return frag_row_at(p.wf, ROWS ? p.words_kp : 0, (int)p.n, p.ks.kblocks, rb, lane & 15, lane >> 4);
+}
+template <bool ROWS>
+__device__ __forceinline__ u32x4 frag_load(const FragArgs &p, const uint32_t *w0, int b)
+{
+    if constexpr (ROWS) return *reinterpret_cast<const frag_u32x4 *>(w0 + (int64_t)b * 16);
+    return *reinterpret_cast<const u32x4 *>(w0 + (int64_t)b * 256);
+}
+
+template <int DT, int MB, int NB, bool ROWS>
 __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_kernel(FragArgs p)
 {
     using D = DecH<DT>;
@@ -135,7 +157,7 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_kernel(FragArgs p)
     // largest tiles have no registers for a second set of sums, their segments are one piece.
     constexpr bool PIECES = MB * NB <= 8;
     f32x4 total[MB][NB];
-    double xsum[MB];
+    std::conditional_t<PIECES, double, float> xsum[MB];
     FragRow row[MB];   // of this lane's activation rows (lane & 15) in the current piece
     const FragRow *rows = p.rows + ((int64_t)z * FRAG_NW + wv) * p.ks.pieces * p.m_pad + (int64_t)mt * MB * 16 + (lane & 15);
     auto next_rows = [&] {
@@ -163,7 +185,7 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_kernel(FragArgs p)
     };
 #pragma unroll
     for (int i = 0; i < MB; i++) {
-        xsum[i] = 0.0;
+        xsum[i] = 0;
         if constexpr (PIECES)
 #pragma unroll
             for (int j = 0; j < NB; j++) total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -172,13 +194,9 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_kernel(FragArgs p)
     if (b0 < b1) {
         const int nsteps = p.ks.kblocks * SPB;
         const f16x8 *a0 = reinterpret_cast<const f16x8 *>(p.af) + (int64_t)mt * MB * nsteps * 128 + lane;
-        const u32x4 *w0[NB];
+        const uint32_t *w0[NB];
 #pragma unroll
-        for (int j = 0; j < NB; j++) {
-            int rb = (int)nt * NB + j;
-            if (rb > p.rblocks - 1) rb = p.rblocks - 1;   // (a column tile past the last row block repeats it; never stored)
-            w0[j] = reinterpret_cast<const u32x4 *>(p.wf) + (int64_t)rb * p.ks.kblocks * 64 + lane;
-        }
+        for (int j = 0; j < NB; j++) w0[j] = frag_row<ROWS>(p, (int)nt * NB + j, lane);
         f16x8 a[AR][MB][2];
         u32x4 w[NB], wn[NB];
         auto load_a = [&](int s, f16x8(&d)[MB][2]) {
@@ -191,7 +209,7 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_kernel(FragArgs p)
         };
         auto load_w = [&](int b, u32x4(&d)[NB]) {
 #pragma unroll
-            for (int j = 0; j < NB; j++) d[j] = w0[j][(int64_t)b * 64];
+            for (int j = 0; j < NB; j++) d[j] = frag_load<ROWS>(p, w0[j], b);
         };
         // one k block; `last`: no requests past it
         auto block = [&](int b, auto last) {
@@ -236,6 +254,10 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_kernel(FragArgs p)
                 left = p.ks.piece;
             }
         }
+        if (ROWS && b1 == p.ks.kblocks) {   // (wave-uniform) words of the next row: not a number, they would not vanish
+#pragma unroll
+            for (int j = 0; j < NB; j++) frag_own_words(w[j], p.words_kp - (b1 - 1) * 16, lane >> 4);
+        }
         block(b1 - 1, std::true_type{});
     }
     if (!PIECES) next_rows();
@@ -246,7 +268,7 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_kernel(FragArgs p)
 // The same product with the f32 activations converted by the waves that multiply them: one launch instead of two, for
 // products so small that a second launch costs more than converting a row block once per column tile.  A wave holds its
 // whole segment (at most STEPS steps of 32 k-values) in registers, every load of it in flight at once.
-template <int DT, int MB, int NB, int STEPS>
+template <int DT, int MB, int NB, int STEPS, bool ROWS>
 __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_direct_kernel(FragArgs p)
 {
     using D = DecH<DT>;
@@ -274,11 +296,9 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_direct_kernel(FragArg
         u32x4 w[BLOCKS][NB];
 #pragma unroll
         for (int j = 0; j < NB; j++) {
-            int rb = (int)nt * NB + j;
-            if (rb > p.rblocks - 1) rb = p.rblocks - 1;
-            const u32x4 *w0 = reinterpret_cast<const u32x4 *>(p.wf) + (int64_t)rb * p.ks.kblocks * 64 + lane;
+            const uint32_t *w0 = frag_row<ROWS>(p, (int)nt * NB + j, lane);
 #pragma unroll
-            for (int b = 0; b < BLOCKS; b++) w[b][j] = w0[(int64_t)(b0 + b < b1 ? b0 + b : b1 - 1) * 64];
+            for (int b = 0; b < BLOCKS; b++) w[b][j] = frag_load<ROWS>(p, w0, b0 + b < b1 ? b0 + b : b1 - 1);
         }
         // a row past M asks for offset ~0, which the buffer's range check answers with zeros, like everything past the tensor
         const uint32_t K = (uint32_t)p.k;
@@ -299,6 +319,13 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_direct_kernel(FragArg
                     x[i][s][4 + j] = __uint_as_float(t1[j]);
                 }
             }
+        }
+        if (ROWS && b1 == p.ks.kblocks) {   // (wave-uniform; past the last block it is repeated)
+#pragma unroll
+            for (int b = 0; b < BLOCKS; b++)
+                if (b0 + b >= b1 - 1)
+#pragma unroll
+                    for (int j = 0; j < NB; j++) frag_own_words(w[b][j], p.words_kp - (b1 - 1) * 16, q);
         }
         if (K % 8 != 0 && b1 == p.ks.kblocks) {   // (wave-uniform) the last values of a row run into the next row: they do not count
 #pragma unroll
@@ -362,7 +389,7 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_direct_kernel(FragArg
         }
     }
     f32x4 total[MB][NB];
-    double xsum[MB];
+    float xsum[MB];
 #pragma unroll
     for (int i = 0; i < MB; i++) {
         xsum[i] = row[i].sum;
@@ -374,7 +401,7 @@ __global__ void __launch_bounds__(FRAG_NW * 64) qgemm_frag_direct_kernel(FragArg
     frag_finish<MB, NB>(p, mt, nt, 0, total, xsum);
 }
 
-template <int DT, int MB, int NB>
+template <int DT, int MB, int NB, bool ROWS>
 hipError_t frag_launch_direct(const FragArgs &p, hipStream_t s)
 {
     constexpr int SPB = DecH<DT>::WPS == 1 ? 4 : 2;
@@ -382,18 +409,18 @@ hipError_t frag_launch_direct(const FragArgs &p, hipStream_t s)
     const dim3 grid(((unsigned)p.ntiles + 7) / 8 * 8 * (unsigned)p.mtiles), block(FRAG_NW * 64);
     constexpr int lds = FRAG_NW * MB * NB * 1024;
     if constexpr (SPB == 2)
-        if (steps <= 2) { hipLaunchKernelGGL((qgemm_frag_direct_kernel<DT, MB, NB, 2>), grid, block, lds, s, p); return hipGetLastError(); }
-    if (steps <= 4) { hipLaunchKernelGGL((qgemm_frag_direct_kernel<DT, MB, NB, 4>), grid, block, lds, s, p); return hipGetLastError(); }
+        if (steps <= 2) { hipLaunchKernelGGL((qgemm_frag_direct_kernel<DT, MB, NB, 2, ROWS>), grid, block, lds, s, p); return hipGetLastError(); }
+    if (steps <= 4) { hipLaunchKernelGGL((qgemm_frag_direct_kernel<DT, MB, NB, 4, ROWS>), grid, block, lds, s, p); return hipGetLastError(); }
     if constexpr (MB * NB <= 2)
-        if (steps <= 8) { hipLaunchKernelGGL((qgemm_frag_direct_kernel<DT, MB, NB, 8>), grid, block, lds, s, p); return hipGetLastError(); }
+        if (steps <= 8) { hipLaunchKernelGGL((qgemm_frag_direct_kernel<DT, MB, NB, 8, ROWS>), grid, block, lds, s, p); return hipGetLastError(); }
     return hipErrorInvalidValue;
 }
 
-template <int DT, int MB, int NB>
+template <int DT, int MB, int NB, bool ROWS>
 hipError_t frag_launch_one(const FragArgs &p, hipStream_t s)
 {
     constexpr int lds = FRAG_NW * MB * NB * 1024;
-    auto kern = qgemm_frag_kernel<DT, MB, NB>;
+    auto kern = qgemm_frag_kernel<DT, MB, NB, ROWS>;
     if constexpr (lds > 64 * 1024) {
         static std::atomic<uint64_t> raised{0};
         const hipError_t e = fnn_raise_lds_limit(raised, reinterpret_cast<const void *>(kern), lds);
@@ -404,28 +431,34 @@ hipError_t frag_launch_one(const FragArgs &p, hipStream_t s)
     return hipGetLastError();
 }
 
-template <int DT>
-hipError_t frag_launch(int mb, int nb, const FragArgs &p, hipStream_t s)
+template <int DT, bool ROWS>
+hipError_t frag_launch_words(int mb, int nb, const FragArgs &p, hipStream_t s)
 {
     if (p.a) {
         switch (mb * 16 + nb) {
-        case 1 * 16 + 1: return frag_launch_direct<DT, 1, 1>(p, s);
-        case 1 * 16 + 2: return frag_launch_direct<DT, 1, 2>(p, s);
-        case 1 * 16 + 4: return frag_launch_direct<DT, 1, 4>(p, s);
+        case 1 * 16 + 1: return frag_launch_direct<DT, 1, 1, ROWS>(p, s);
+        case 1 * 16 + 2: return frag_launch_direct<DT, 1, 2, ROWS>(p, s);
+        case 1 * 16 + 4: return frag_launch_direct<DT, 1, 4, ROWS>(p, s);
         default: return hipErrorInvalidValue;
         }
     }
     switch (mb * 16 + nb) {
-    case 1 * 16 + 1: return frag_launch_one<DT, 1, 1>(p, s);
-    case 1 * 16 + 2: return frag_launch_one<DT, 1, 2>(p, s);
-    case 2 * 16 + 2: return frag_launch_one<DT, 2, 2>(p, s);
-    case 2 * 16 + 4: return frag_launch_one<DT, 2, 4>(p, s);
-    case 3 * 16 + 4: return frag_launch_one<DT, 3, 4>(p, s);
+    case 1 * 16 + 1: return frag_launch_one<DT, 1, 1, ROWS>(p, s);
+    case 1 * 16 + 2: return frag_launch_one<DT, 1, 2, ROWS>(p, s);
+    case 2 * 16 + 2: return frag_launch_one<DT, 2, 2, ROWS>(p, s);
+    case 2 * 16 + 4: return frag_launch_one<DT, 2, 4, ROWS>(p, s);
+    case 3 * 16 + 4: return frag_launch_one<DT, 3, 4, ROWS>(p, s);
     case 4 * 16 + 4:
-        if constexpr (DecH<DT>::WPS == 2) return frag_launch_one<DT, 4, 4>(p, s);   // (the four steps of a nibble block do not fit the registers beside it)
+        if constexpr (DecH<DT>::WPS == 2) return frag_launch_one<DT, 4, 4, ROWS>(p, s);   // (the four steps of a nibble block do not fit the registers beside it)
         return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
     }
+}
+
+template <int DT>
+hipError_t frag_launch(int mb, int nb, const FragArgs &p, hipStream_t s)
+{
+    return p.words_kp ? frag_launch_words<DT, true>(mb, nb, p, s) : frag_launch_words<DT, false>(mb, nb, p, s);
 }
 
 }  // namespace

@@ -8,7 +8,7 @@ constexpr int WAVE_RING(bool w8) { return w8 ? 6 : 8; }
 constexpr int WAVE_ROWS = 32, WAVE_COLS = 128;   // activation rows (three planes each) and columns of a wave's tile
 
 struct WaveArgs {
-    const uint32_t *wf;          // weight fragments as in FragArgs, kblocks blocks of 64 bytes per row of fragments
+    const uint32_t *wf;          // weight words (frag_row_at), kblocks blocks of 64 bytes per row
     const int8_t *af;            // [block of 32 operand rows][step][h 0..1][row][16 bytes]
     const int *rexp;             // [m_pad] power of two applied to the row, INT_MIN: a non-finite row
     const float *xsum;           // [m_pad] sum_k A[m,k]
@@ -17,7 +17,7 @@ struct WaveArgs {
     const float *residual;       // sum_out = out + residual as well
     float *sum_out;
     int64_t m, n;
-    int act, kblocks, mtiles, ntiles, rblocks;
+    int act, kblocks, mtiles, ntiles, words_kp;
     int nsteps;                  // steps per operand row, whole units
     int units, units_per_wave;   // a unit is a ring of steps
     unsigned tiles;

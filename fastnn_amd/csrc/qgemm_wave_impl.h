@@ -86,13 +86,10 @@ __global__ void __launch_bounds__(256, 1) qgemm_wave_kernel(WaveArgs p)
 
     if (u0 < u1) {
         const wi32x4 *a0 = reinterpret_cast<const wi32x4 *>(p.af) + (int64_t)rb0 * p.nsteps * 64 + lane;
-        const u32x4 *w0[TN];   // [row block of 16][k block][q][row]: two row blocks and a pair of q per load
+        const int block_words = p.words_kp ? 16 : 256, pair_words = p.words_kp ? 8 : 128;
+        const uint32_t *w0[TN];   // two row blocks and a pair of pieces per load
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            int rb = (int)(n0 >> 4) + 2 * j + (lr >> 4);
-            if (rb > p.rblocks - 1) rb = p.rblocks - 1;
-            w0[j] = reinterpret_cast<const u32x4 *>(p.wf) + (int64_t)rb * p.kblocks * 64 + h * 16 + (lr & 15);
-        }
+        for (int j = 0; j < TN; j++) w0[j] = frag_row_at(p.wf, p.words_kp, (int)p.n, p.kblocks, (int)(n0 >> 4) + 2 * j + (lr >> 4), lr & 15, h);
         wi32x4 a[RING][TM];
         u32x4 w[WL][TN];
         auto load_a = [&](int s, int i) { return a0[((int64_t)i * p.nsteps + s) * 64]; };
@@ -100,7 +97,7 @@ __global__ void __launch_bounds__(256, 1) qgemm_wave_kernel(WaveArgs p)
         auto load_w = [&](int x, int j) {
             int kb = x >> 1;
             if (kb > p.kblocks - 1) kb = p.kblocks - 1;   // (past the last block the activations are zero)
-            return w0[j][kb * 64 + (x & 1) * 32];
+            return (u32x4)*reinterpret_cast<const frag_u32x4 *>(w0[j] + (int64_t)kb * block_words + (x & 1) * pair_words);
         };
         auto decode = [&](int st, int j) {
             uint32_t ww[4];

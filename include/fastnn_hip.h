@@ -163,10 +163,12 @@ enum {
                                   /* (one contiguous KB per wave load: same bits, C1 M=1 5.97 -> 5.15 us, C2 6.70 -> 6.41, FP8     */
                                   /* 4096 x 4096 5.90 -> 5.40), built on the weight's first such call and kept with it (once more  */
                                   /* the packed bytes; rows of whole 64-byte blocks only; a call that may not allocate uses the    */
-                                  /* row-major words until the copy exists); 0 = row-major words only                              */
+                                  /* row-major words until the copy exists); 0 = row-major words only, for these kernels and those */
+                                  /* of FNN_OPT_FRAGMENT.  The same results either way                                             */
     FNN_OPT_FRAGMENT = 24,        /* the MatMul kernels on fragment-major operands (per-channel types; both operands lie in memory  */
                                   /* in the order the matrix cores take them; a second device copy of the packed words, built on  */
-                                  /* the weight's first such call): 0 (default) = by rule (any M with rows of ragged length, from   */
+                                  /* the weight's first such call; a call that may not allocate reads the registered words until   */
+                                  /* that exists, with the same results): 0 (default) = by rule (any M with rows of ragged length, from   */
                                   /* M = 17, or 5 to 9 for short rows, with aligned ones, as far up as it is the faster form), -1 =  */
                                   /* off, else the shape, (direct << 15) | (K splits << 8) | (16-column blocks << 4) | (16-row       */
                                   /* blocks); a shape that does not exist for the call is ignored;                                  */
@@ -227,7 +229,8 @@ int fnn_hip_qmatmul(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *a, i
  *     that with FNN_FLAG_ACT_F16_SINGLE), split-K partials splits*M*N*4 bytes <= 24 MiB;
  *   - per-weight side tables that fnn_hip_qmatmul builds on first use (the f16 expansion of a codebook weight at
  *     M >= 5, row means for FNN_FLAG_ACT_F16_SINGLE, re-strided rows when ceil(K/ITEMS) % 4 != 0) must exist
- *     already: call fnn_hip_qmatmul once per weight and flag combination beforehand.
+ *     already: call fnn_hip_qmatmul once per weight and flag combination beforehand.  (The copies of the packed words
+ *     in other orders are not among them: without one a call reads the registered words, slower, with the same result.)
  * Every GPU the library runs on holds its copy of the array until the process ends, and every call on a GPU, from
  * any context, uses that one copy: calls that overlap in time on one GPU (two contexts, two threads) race; calls
  * on one context are ordered by its stream.  Nothing in the array needs to start at zero. */

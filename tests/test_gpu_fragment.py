@@ -127,3 +127,36 @@ def test_row_sums_of_the_fragment_kernels(ctx, m, k, n):
     finally:
         ctx.set_option(flib.OPT_FRAGMENT, 0)
         ctx.release(h)
+
+
+@pytest.mark.parametrize("dt", TYPES)
+@pytest.mark.parametrize("m,k,n", [(1, 63, 15), (17, 1000, 33), (33, 1025, 70), (65, 2600, 257), (40, 2048, 2112)])
+def test_results_do_not_depend_on_the_copy_of_the_weight(ctx, dt, m, k, n):
+    """The registered rows instead of the fragment-major copy: the same bits, for every form, K that ends inside a 64-byte block
+    and rows of not-a-number next to others (the last block's words past a row are the next row's)."""
+    rng = np.random.default_rng(9500 + dt * 7 + m)
+    pw = fastnn_amd.quantize_weights(dt, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    if dt == flib.DT_F8:
+        pw.words[n // 2 * (-(-k // 4))] = 0x7f
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    forms = [0, 1 << 8 | 1 << 4 | 1, 3 << 8 | 2 << 4 | 2, 1 << 8 | 4 << 4 | 4] + [1 << 15 | nb << 4 | 1 for nb in (1, 2, 4)]
+    if dt in (flib.DT_I8, flib.DT_I4, flib.DT_U4):
+        forms += [1 << 14 | w for w in (1, 2, 4)]
+    h = ctx.register(pw)
+    try:
+        results = []
+        for copy in (0, 1):
+            ctx.set_option(flib.OPT_GEMV_TILE_MAJOR, copy)
+            for i, form in enumerate(forms):
+                ctx.set_option(flib.OPT_FRAGMENT, form)
+                got = ctx.qmatmul(h, a, n)
+                if copy == 0:
+                    results.append(got)
+                else:
+                    assert got.tobytes() == results[i].tobytes(), hex(form)
+        if dt == flib.DT_F8:
+            assert np.isnan(results[0][:, n // 2]).all() and np.isnan(results[0]).sum() == m
+    finally:
+        ctx.set_option(flib.OPT_FRAGMENT, 0)
+        ctx.set_option(flib.OPT_GEMV_TILE_MAJOR, 1)
+        ctx.release(h)

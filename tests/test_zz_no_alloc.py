@@ -130,3 +130,27 @@ def test_static_entry_point_takes_what_its_limits_allow(dt, m, k, n, within):
         assert_close(got, want, 2e-5, f"dt={dt} M={m} K={k}")
         if within:
             assert np.array_equal(got, d_ref.download(np.float32, m * n).reshape(m, n))
+
+
+@pytest.mark.parametrize("dt,m,k,n", [(flib.DT_I8, 1, 1003, 700), (flib.DT_U8, 12, 512, 1024), (flib.DT_F8, 24, 2048, 2048), (flib.DT_I4, 64, 1003, 3333),
+                                      (flib.DT_U4, 130, 4096, 4096), (flib.DT_I8, 256, 4096, 4096), (flib.DT_F4, 64, 2048, 8192), (flib.DT_I8, 64, 4096, 4096)])
+def test_static_entry_point_first_on_a_weight_gives_the_same_bits(dt, m, k, n):
+    """No call has built a copy of the weight yet: the static entry point and a captured call read the registered rows, with the
+    kernels and the results that calls after them have."""
+    rng = np.random.default_rng(17)
+    pw = fastnn_amd.quantize_weights(dt, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    with fastnn_amd.HipContext(0) as ctx:
+        warm, fresh = ctx.register(pw), ctx.register(pw)
+        da, out = ctx.to_device(a), [ctx.alloc(m * n * 4) for _ in range(4)]
+        ctx.qmatmul_dev(warm, da.ptr, m, out[0].ptr)           # (workspaces for the captured call)
+        ctx.qmatmul_static(fresh, da.ptr, m, out[1].ptr)
+        ctx.graph_begin()
+        ctx.qmatmul_dev(fresh, da.ptr, m, out[2].ptr)
+        g = ctx.graph_end()
+        ctx.graph_launch(g)
+        ctx.qmatmul_dev(fresh, da.ptr, m, out[3].ptr)
+        ctx.sync()
+        got = [o.download(np.float32, m * n).tobytes() for o in out]
+        ctx.graph_destroy(g)
+        assert got[1] == got[0] and got[2] == got[0] and got[3] == got[0]
