@@ -158,7 +158,7 @@ const OptionSpec kOptions[FNN_OPT_COUNT] = {
     {32, 0, 32},      // FNN_OPT_STREAM_MAX_M
     {0, 0, 0xffff},   // FNN_OPT_STREAM_SHAPE
     {0, 0, 4},        // FNN_OPT_DIGIT_PLANES
-    {1, 0, 1},        // FNN_OPT_GEMV_TILE_MAJOR
+    {1, 0, 2},        // FNN_OPT_GEMV_TILE_MAJOR
     {0, -1, 0xffff},  // FNN_OPT_FRAGMENT
 };
 
@@ -1297,6 +1297,15 @@ bool fnn_ctx_operand_allowed(fnn_hip_ctx *ctx, int64_t m, int64_t k, size_t byte
     // (the limit that the header names: sizes within it run the same kernel with either entry point)
     const bool promised = m <= FNN_STATIC_MAX_M && 4 * ((m + 15) / 16 * 16) * ((k + 63) / 64 * 64) + 12 * m <= (int64_t)kStaticOperandBytes;
     return bytes <= kStaticOperandBytes || (!promised && !ctx->static_mode);
+}
+
+void *fnn_ctx_copy_memory(fnn_hip_ctx *ctx, size_t bytes)
+{
+    if (ctx->capturing || ctx->static_mode || ctx->options[FNN_OPT_GEMV_TILE_MAJOR] != 1) return nullptr;
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
 }
 
 bool fnn_ctx_capturing(fnn_hip_ctx *ctx) { return ctx->capturing; }

@@ -17,6 +17,9 @@ bool fnn_ctx_capturing(fnn_hip_ctx *ctx);
 // true while device memory must not be allocated: graph capture, or a call through fnn_hip_qmatmul_static
 bool fnn_ctx_no_alloc(fnn_hip_ctx *ctx);
 bool fnn_ctx_static_mode(fnn_hip_ctx *ctx);
+// memory for a copy of packed words in another order: null where this call may not allocate or the device has no room (the
+// kernels read the registered words then)
+void *fnn_ctx_copy_memory(fnn_hip_ctx *ctx, size_t bytes);
 // value of a per-context option (FNN_OPT_*, set through fnn_hip_set_option)
 int64_t fnn_ctx_option(const fnn_hip_ctx *ctx, int option);
 

@@ -426,11 +426,9 @@ int fnn_fragment_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w,
 {
     *out = nullptr;
     fnn_hip_weight *wm = const_cast<fnn_hip_weight *>(w);
-    if (fnn_ctx_option(ctx, FNN_OPT_GEMV_TILE_MAJOR) != 1) return FNN_OK;
-    if (!wm->words_fr && !fnn_ctx_no_alloc(ctx)) {
-        const int64_t pieces = (w->rows + 15) / 16 * kblocks * 64;
-        if (hipMalloc((void **)&wm->words_fr, (size_t)pieces * 16) != hipSuccess)
-            return fnn_ctx_fail(ctx, FNN_ERR_MEMORY, "out of device memory (fragment-major weight rows)");
+    if (fnn_ctx_option(ctx, FNN_OPT_GEMV_TILE_MAJOR) == 0) return FNN_OK;
+    const int64_t pieces = (w->rows + 15) / 16 * kblocks * 64;
+    if (!wm->words_fr && (wm->words_fr = (uint32_t *)fnn_ctx_copy_memory(ctx, (size_t)pieces * 16))) {
         int64_t blocks = (pieces + 255) / 256;
         if (blocks > 4096) blocks = 4096;
         hipLaunchKernelGGL(frag_words_kernel, dim3((unsigned)blocks), dim3(256), 0, s, w->words, w->rows, w->kp, kblocks,

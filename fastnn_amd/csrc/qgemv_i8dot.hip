@@ -381,12 +381,10 @@ int fnn_tile_major_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *
 {
     *words_tm = nullptr;
     *kb64 = 0;
-    if (fnn_ctx_option(ctx, FNN_OPT_GEMV_TILE_MAJOR) != 1 || q.words != w->words || q.kp != w->kp || q.kp % 16 != 0 || q.n != w->rows) return FNN_OK;
+    if (fnn_ctx_option(ctx, FNN_OPT_GEMV_TILE_MAJOR) == 0 || q.words != w->words || q.kp != w->kp || q.kp % 16 != 0 || q.n != w->rows) return FNN_OK;
     fnn_hip_weight *wm = const_cast<fnn_hip_weight *>(w);
-    if (!wm->words_tm && !fnn_ctx_no_alloc(ctx)) {
-        const int64_t nwords = (w->rows + 15) / 16 * 16 * w->kp;
-        if (hipMalloc((void **)&wm->words_tm, (size_t)nwords * 4 + 256) != hipSuccess)
-            return fnn_ctx_fail(ctx, FNN_ERR_MEMORY, "out of device memory (tile-major weight rows)");
+    const int64_t nwords = (w->rows + 15) / 16 * 16 * w->kp;
+    if (!wm->words_tm && (wm->words_tm = (uint32_t *)fnn_ctx_copy_memory(ctx, (size_t)nwords * 4 + 256))) {
         int64_t blocks = (nwords / 4 + 255) / 256;
         if (blocks > 4096) blocks = 4096;
         hipLaunchKernelGGL(tile_major_kernel, dim3((unsigned)blocks), dim3(256), 0, s, w->words, w->rows, w->kp, w->kp / 16,

@@ -164,7 +164,8 @@ enum {
                                   /* 4096 x 4096 5.90 -> 5.40), built on the weight's first such call and kept with it (once more  */
                                   /* the packed bytes; rows of whole 64-byte blocks only; a call that may not allocate uses the    */
                                   /* row-major words until the copy exists); 0 = row-major words only, for these kernels and those */
-                                  /* of FNN_OPT_FRAGMENT.  The same results either way                                             */
+                                  /* of FNN_OPT_FRAGMENT; 2 = copies that exist, but none is built (as when the device has no       */
+                                  /* memory for one).  The same results in every case                                              */
     FNN_OPT_FRAGMENT = 24,        /* the MatMul kernels on fragment-major operands (per-channel types; both operands lie in memory  */
                                   /* in the order the matrix cores take them; a second device copy of the packed words, built on  */
                                   /* the weight's first such call; a call that may not allocate reads the registered words until   */

@@ -145,7 +145,7 @@ def test_results_do_not_depend_on_the_copy_of_the_weight(ctx, dt, m, k, n):
     h = ctx.register(pw)
     try:
         results = []
-        for copy in (0, 1):
+        for copy in (0, 2, 1, 2):   # none; none built (as without memory for one); built; the built one
             ctx.set_option(flib.OPT_GEMV_TILE_MAJOR, copy)
             for i, form in enumerate(forms):
                 ctx.set_option(flib.OPT_FRAGMENT, form)
