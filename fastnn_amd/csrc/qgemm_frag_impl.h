@@ -119,7 +119,9 @@ __device__ __forceinline__ void frag_own_words(u32x4 &w, int tail, int piece)
 template <bool ROWS>
 __device__ __forceinline__ const uint32_t *frag_row(const FragArgs &p, int rb, int lane)
 {
-    return frag_row_at(p.wf, ROWS ? p.words_kp : 0, (int)p.n, p.ks.kblocks, rb, lane & 15, lane >> 4);
+    if constexpr (ROWS) return frag_row_at(p.wf, p.words_kp, (int)p.n, p.ks.kblocks, rb, lane & 15, lane >> 4);
+    const int last_rb = ((int)p.n - 1) >> 4;
+    return p.wf + ((int64_t)(rb < last_rb ? rb : last_rb) * p.ks.kblocks * 64 + lane) * 4;
 }
 template <bool ROWS>
 __device__ __forceinline__ u32x4 frag_load(const FragArgs &p, const uint32_t *w0, int b)
