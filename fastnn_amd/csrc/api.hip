@@ -242,7 +242,6 @@ void free_weight(fnn_hip_weight *w)
     if (w->row_qsum) (void)hipFree(w->row_qsum);
     if (w->umean) (void)hipFree(w->umean);
     if (w->words4) (void)hipFree(w->words4);
-    if (w->words_tm) (void)hipFree(w->words_tm);
     if (w->words_fr) (void)hipFree(w->words_fr);
     if (w->dense16) (void)hipFree(w->dense16);
     delete w;

@@ -14,7 +14,7 @@ struct StreamArgs {
     uint32_t *count;         // splits > 1: one arrival counter per column tile, zero between launches
     int64_t m, n, k, kp;
     int act, splits, rounds, ntiles;
-    const uint32_t *words_tm;   // non-null: the words in blocks of 16 rows x 64 bytes ([row block][k block][row][64 bytes]),
+    const uint32_t *words_fr;   // non-null: the words fragment-major ([block of 16 rows][k block][g 0..3][row][16 bytes]),
     int64_t kb64;               // kb64 k blocks per row: a wave load is one contiguous KB
 };
 

@@ -7,9 +7,9 @@
 
 struct TileArgs {
     const uint32_t *words;
-    // non-null (weight types with 64 bytes per row and stage only): the words in blocks of 16 rows x 64 bytes,
-    // [row block][k block][row][64 bytes], kb64 k blocks per row: a wave's 64 chunk loads of a stage are one contiguous KB
-    const uint32_t *words_tm = nullptr;
+    // non-null (weight types with 64 bytes per row and stage only): the words fragment-major,
+    // [block of 16 rows][k block][piece 0..3][row][16 bytes], kb64 k blocks per row: a wave's 64 chunk loads of a stage are one contiguous KB
+    const uint32_t *words_fr = nullptr;
     int64_t kb64 = 0;
     const uint32_t *zero_chunk;   // 16 zero bytes: source of weight chunks past the end of a row
     const float *scales, *zeros, *umean, *bias;
@@ -247,23 +247,26 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
         a_src[j] = p.ap + ((int64_t)mt * BM + row) * 64 + g * 8 - (j & 3) * 512;   // (biased: see load_group_to_lds16)
     }
     // weights: chunk (row, c) lives at slot row*WC + (c ^ swz(row)); rows past N repeat the last row
-    // tile-major copy: 64 bytes per row and stage = one block per stage (WC == 4); 32 bytes = half a block (WC == 2)
-    const bool tmaj = (WC == 4 || WC == 2) && !CB && p.words_tm != nullptr;   // (uniform)
+    // fragment-major copy: 64 bytes per row and stage = one block per stage (WC == 4); 32 bytes = half a block (WC == 2).  The
+    // LDS holds it in the copy's order, [row block][c][row]: sixteen rows' chunks fill a window by themselves, and every four
+    // lanes ask for 64 contiguous bytes (in the order above, a row's chunks being 256 bytes apart, they ask for four lines:
+    // U8 4096 x 11008 at M = 256 74.7 against 65.3 us)
+    const bool frag = (WC == 4 || WC == 2) && !CB && p.words_fr != nullptr;   // (uniform)
     const uint32_t *w_src[W_LPW];
     int w_chunk[W_LPW];
 #pragma unroll
     for (int j = 0; j < W_LPW; j++) {
         const int slot = (wv * W_LPW + j) * 64 + lane;
-        const int row = slot / WC;
+        const int row = frag ? slot / (16 * WC) * 16 + (slot & 15) : slot / WC;
         const int sw = (WC == 2) ? ((row >> 3) & 1) : (WC == 4 ? ((row >> 2) & 3) : ((row >> 1) & 7));
-        const int c = (slot % WC) ^ sw;
+        const int c = frag ? (slot >> 4) % WC : (slot % WC) ^ sw;
         int64_t grow = n0 + row;
         if (grow > p.n - 1) grow = p.n - 1;
         w_src[j] = p.words + grow * p.kp + c * 4 - (j & 3) * 256;                  // (biased likewise)
-        if (tmaj) w_src[j] = p.words_tm + (((grow >> 4) * p.kb64) << 8) + ((grow & 15) << 4) + c * 4 - (j & 3) * 256;
+        if (frag) w_src[j] = p.words_fr + (((grow >> 4) * p.kb64) << 8) + ((grow & 15) << 2) + c * 64 - (j & 3) * 256;
         w_chunk[j] = c * 4;
     }
-    const int w_stride = tmaj ? 256 : WC * 4;   // words between consecutive stages of a row (tile-major, WC == 4: one block on)
+    const int w_stride = frag ? WC * 64 : WC * 4;   // words between consecutive stages of a row (copy: a block or half of one on)
     const int64_t a_step = p.rows_pad * 64;   // elements between consecutive k blocks
     const unsigned a_dst = __builtin_amdgcn_readfirstlane(lds0 + wv * A_LPW * 1024);
     const unsigned w_dst = __builtin_amdgcn_readfirstlane(lds0 + A_BYTES + wv * W_LPW * 1024);
@@ -276,7 +279,7 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
 #pragma unroll
     for (int j = 0; j < A_LPW; j++) a_src[j] += (int64_t)(DENSE ? it0 % p.a_wrap : it0) * a_step;
 #pragma unroll
-    for (int j = 0; j < W_LPW; j++) w_src[j] += (tmaj && WC == 2) ? (int64_t)(it0 >> 1) * 256 + (it0 & 1) * 8 : (int64_t)it0 * w_stride;
+    for (int j = 0; j < W_LPW; j++) w_src[j] += (int64_t)it0 * w_stride;
     int a_pos = DENSE ? it0 % p.a_wrap : 0;       // position inside the activation sweep
     const bool ragged = !DENSE && (p.kp % (WC * 4)) != 0;
     bool w_past[W_LPW];   // this lane's chunk of the last stage lies behind the end of the row
@@ -320,8 +323,7 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
             a_pos = 0;
             astep = -(int64_t)(p.a_wrap - 1) * a_step;
         }
-        // (half blocks: from the even half to the odd half of a block 32 bytes, from there to the next block 1024 - 32)
-        const int wstep = !more ? 0 : ((tmaj && WC == 2) ? ((it & 1) ? 248 : 8) : w_stride);
+        const int wstep = !more ? 0 : w_stride;
 #pragma unroll
         for (int j = 0; j < A_LPW; j++) a_src[j] += astep;
 #pragma unroll
@@ -337,15 +339,20 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
             for (int i = 0; i < 16; i++) acc[tm][tn][i] = 0.0f;
 
     // operand read offsets inside a stage
-    int a_off[TM], w_off[TN];
+    constexpr int CPH = WC == 2 ? 1 : WC / 2;   // chunks per lane half: 2 (8-bit types) or 4 (f16)
+    int a_off[TM], w_off[TN], w_at[CPH];        // w_at: chunk CPH*h + c of the wave's first weight rows (not the codebook type)
+#pragma unroll
+    for (int c = 0; c < CPH; c++) {
+        const int row = wn * TN * 32 + lr, ch = CPH * h + c;
+        const int sw = (WC == 2) ? ((row >> 3) & 1) : (WC == 4 ? ((row >> 2) & 3) : ((row >> 1) & 7));
+        w_at[c] = A_BYTES + (frag ? ((row >> 4) * WC + ch) * 256 + (row & 15) * 16 : (row * WC + (ch ^ sw)) * 16);
+    }
 #pragma unroll
     for (int tm = 0; tm < TM; tm++) a_off[tm] = ((wm * TM + tm) * 32 + lr) * 128;
 #pragma unroll
     for (int tn = 0; tn < TN; tn++) {
         const int row = (wn * TN + tn) * 32 + lr;
-        if constexpr (CB) w_off[tn] = A_BYTES + row * 32;   // both chunks of the row are read
-        else if constexpr (WC == 2) w_off[tn] = A_BYTES + (row * 2 + (h ^ ((row >> 3) & 1))) * 16;
-        else w_off[tn] = A_BYTES + row * (WC * 16);   // chunk index added per read
+        w_off[tn] = A_BYTES + row * 32;   // codebook type: both chunks of the row are read
     }
     const int asw = (lr >> 1) & 7;   // (row >> 1) & 7 of every activation row this lane reads
 
@@ -367,16 +374,10 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
                     const u32x4 t1 = *reinterpret_cast<const u32x4 *>(sbase + w_off[tn] + (1 ^ sw) * 16);
                     wq[tn][0] = t0[0]; wq[tn][1] = t0[1]; wq[tn][2] = t0[2]; wq[tn][3] = t0[3];
                     wq[tn][4] = t1[0]; wq[tn][5] = t1[1]; wq[tn][6] = t1[2]; wq[tn][7] = t1[3];
-                } else if constexpr (WC == 2) {
-                    const u32x4 t = *reinterpret_cast<const u32x4 *>(sbase + w_off[tn]);
-                    wq[tn][0] = t[0]; wq[tn][1] = t[1]; wq[tn][2] = t[2]; wq[tn][3] = t[3];
                 } else {
-                    constexpr int CPH = WC / 2;   // chunks per lane half: 2 (8-bit types) or 4 (f16)
-                    const int row = (wn * TN + tn) * 32 + lr;
-                    const int sw = (WC == 4) ? ((row >> 2) & 3) : ((row >> 1) & 7);
 #pragma unroll
-                    for (int c = 0; c < CPH; c++) {
-                        const u32x4 t = *reinterpret_cast<const u32x4 *>(sbase + w_off[tn] + (((CPH * h + c) ^ sw) * 16));
+                    for (int c = 0; c < CPH; c++) {   // (32 rows on: the same swizzle)
+                        const u32x4 t = *reinterpret_cast<const u32x4 *>(sbase + w_at[c] + tn * (32 * WC * 16));
                         wq[tn][4 * c + 0] = t[0]; wq[tn][4 * c + 1] = t[1]; wq[tn][4 * c + 2] = t[2]; wq[tn][4 * c + 3] = t[3];
                     }
                 }

@@ -159,11 +159,11 @@ enum {
                                   /* I8 / I4 / U4 / U8 / F8 / F8R weights; 9 <= M <= 32: every per-channel type)                   */
                                   /* and the tile kernels of the types with 64 or 32 bytes per row and stage (I4 / U4 digit        */
                                   /* planes, U8 / F8 / F8R / F4):                                                                  */
-                                  /* 1 (default) = read them from a second device copy laid out in blocks of 16 rows x 64 bytes    */
-                                  /* (one contiguous KB per wave load: same bits, C1 M=1 5.97 -> 5.15 us, C2 6.70 -> 6.41, FP8     */
-                                  /* 4096 x 4096 5.90 -> 5.40), built on the weight's first such call and kept with it (once more  */
-                                  /* the packed bytes; rows of whole 64-byte blocks only; a call that may not allocate uses the    */
-                                  /* row-major words until the copy exists); 0 = row-major words only, for these kernels and those */
+                                  /* 1 (default) = read them from a second device copy in the order of those registers, the one that */
+                                  /* FNN_OPT_FRAGMENT's kernels read (one contiguous KB per wave load: same bits, C1 M=1 5.97 ->   */
+                                  /* 5.15 us, C2 6.70 -> 6.41, FP8 4096 x 4096 5.90 -> 5.40), built on the weight's first such     */
+                                  /* call and kept with it (once more the packed bytes; here rows of whole 64-byte blocks only; a  */
+                                  /* call that may not allocate uses the row-major words until the copy exists); 0 = row-major words only, for these kernels and those */
                                   /* of FNN_OPT_FRAGMENT; 2 = copies that exist, but none is built (as when the device has no       */
                                   /* memory for one).  The same results in every case                                              */
     FNN_OPT_FRAGMENT = 24,        /* the MatMul kernels on fragment-major operands (per-channel types; both operands lie in memory  */
