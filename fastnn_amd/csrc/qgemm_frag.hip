@@ -15,20 +15,32 @@ typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));   // rows of 
 
 constexpr float LO_UP = 2048.0f;
 
-__global__ void __launch_bounds__(256) frag_words_kernel(const uint32_t *src, int64_t rows, int64_t kp, int64_t kblocks, u32x4 *dst)
+// Registered rows -> fragment-major copy.  Bound: memory (a weight read and written once).  A wave moves COPY_BLOCKS
+// blocks of 1 KB, all of its loads in flight: lane r + 16 q the piece q of row r, every store one contiguous KB.  Rows start on any
+// word: 16-byte loads from 4-byte aligned addresses (the last row's may reach into the zeroed margin behind it), and what lies
+// past the end of a row is cleared.
+constexpr int COPY_BLOCKS = 4;
+__global__ void __launch_bounds__(256) frag_words_kernel(const uint32_t *src, int64_t rows, int64_t kp, uint32_t kblocks, FastDiv by_kblocks, uint32_t blocks,
+                                                         u32x4 *dst)
 {
-    const int64_t total = (rows + 15) / 16 * kblocks * 64;   // 16-byte pieces
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-        const int64_t blk = i >> 6, rb = blk / kblocks, kb = blk - rb * kblocks;
-        const int q = (int)((i >> 4) & 3);
-        const int64_t row = rb * 16 + (i & 15), w0 = kb * 16 + q * 4;
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (row < rows) {
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    const uint32_t first = (blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * COPY_BLOCKS;
+    u32x4 v[COPY_BLOCKS];
+    int left[COPY_BLOCKS];   // words of the piece that belong to the row
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (w0 + j < kp) v[j] = src[row * kp + w0 + j];
-        }
-        dst[i] = v;
+    for (int i = 0; i < COPY_BLOCKS; i++) {
+        const uint32_t blk = first + i < blocks ? first + i : blocks - 1;   // (past the end: the last one again)
+        const uint32_t rb = by_kblocks.div(blk), kb = blk - rb * kblocks;
+        const int64_t row = (int64_t)rb * 16 + r, w0 = (int64_t)kb * 16 + q * 4;
+        left[i] = row < rows ? (int)(kp - w0) : 0;
+        v[i] = *reinterpret_cast<const frag_u32x4 *>(src + (row < rows ? row : rows - 1) * kp + w0);
+    }
+#pragma unroll
+    for (int i = 0; i < COPY_BLOCKS; i++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (e >= left[i]) v[i][e] = 0u;
+        if (first + i < blocks) dst[(int64_t)(first + i) * 64 + lane] = v[i];
     }
 }
 
@@ -427,13 +439,15 @@ int fnn_fragment_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w,
     *out = nullptr;
     fnn_hip_weight *wm = const_cast<fnn_hip_weight *>(w);
     if (fnn_ctx_option(ctx, FNN_OPT_GEMV_TILE_MAJOR) == 0) return FNN_OK;
-    const int64_t pieces = (w->rows + 15) / 16 * kblocks * 64;
-    if (!wm->words_fr && (wm->words_fr = (uint32_t *)fnn_ctx_copy_memory(ctx, (size_t)pieces * 16))) {
-        int64_t blocks = (pieces + 255) / 256;
-        if (blocks > 4096) blocks = 4096;
-        hipLaunchKernelGGL(frag_words_kernel, dim3((unsigned)blocks), dim3(256), 0, s, w->words, w->rows, w->kp, kblocks,
-                           reinterpret_cast<u32x4 *>(wm->words_fr));
-        if (hipGetLastError() != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, "building the fragment-major weight rows failed");
+    const int64_t blocks = (w->rows + 15) / 16 * kblocks;   // of 1 KB
+    if (!wm->words_fr && blocks < (int64_t)1 << 31 && (wm->words_fr = (uint32_t *)fnn_ctx_copy_memory(ctx, (size_t)blocks * 1024 + 256))) {
+        hipLaunchKernelGGL(frag_words_kernel, dim3((unsigned)((blocks + 4 * COPY_BLOCKS - 1) / (4 * COPY_BLOCKS))), dim3(256), 0, s, w->words, w->rows, w->kp,
+                           (uint32_t)kblocks, fast_div((uint32_t)kblocks), (uint32_t)blocks, reinterpret_cast<u32x4 *>(wm->words_fr));
+        if (hipGetLastError() != hipSuccess) {
+            (void)hipFree(wm->words_fr);
+            wm->words_fr = nullptr;
+            return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, "building the fragment-major weight rows failed");
+        }
     }
     *out = wm->words_fr;
     return FNN_OK;

@@ -1,5 +1,7 @@
 """The MatMul kernels on fragment-major operands (FNN_OPT_FRAGMENT) against the oracle, at the edges of their tiles: rows and
 columns around multiples of 16, K around the k blocks (64 or 128 values), the pieces of 256 values and the eight waves."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -165,14 +167,18 @@ def test_results_do_not_depend_on_the_copy_of_the_weight(ctx, dt, m, k, n):
 def test_a_weight_has_one_copy_beside_its_words(ctx):
     """Decode, few-row, tile and prefill kernels read the same fragment-major copy: a weight of 32 MB that has served them all
     takes 64 MB and its side tables."""
-    import torch
+    def free():      # (the runtime that the library is linked with)
+        f, t = C.c_size_t(), C.c_size_t()
+        assert ctx.lib.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
     n = k = 8192
     pw = fastnn_amd.quantize_weights(flib.DT_I4, np.tile(np.random.default_rng(9600).standard_normal((n, 64)).astype(np.float32) * 0.05, (1, k // 64)))
     a, out = ctx.to_device(np.ones((512, k), np.float32)), ctx.alloc(512 * n * 4)
     taken = []
     for _ in range(2):      # (the first one grows the workspaces)
         ctx.sync()
-        before = torch.cuda.mem_get_info()[0]
+        before = free()
         h = ctx.register(pw)
         for m in (1, 8, 16, 24, 64, 512):
             ctx.qmatmul_dev(h, a.ptr, m, out.ptr)
@@ -181,5 +187,5 @@ def test_a_weight_has_one_copy_beside_its_words(ctx):
             ctx.qmatmul_dev(h, a.ptr, m, out.ptr)
         ctx.set_option(flib.OPT_FRAGMENT, 0)
         ctx.sync()
-        taken.append(before - torch.cuda.mem_get_info()[0])
+        taken.append(before - free())
     assert taken[1] < 80 << 20, [t >> 20 for t in taken]
