@@ -62,6 +62,7 @@ struct fnn_hip_ctx {
     uint64_t ws_epoch = 0;     // bumped whenever a staging buffer is re-allocated (captured graphs go stale)
     unsigned char *static_ws = nullptr;   // this device's copy of the library's static workspace
     bool static_mode = false;             // inside fnn_hip_qmatmul_static: workspaces come from static_ws, nothing allocates
+    size_t static_operand_room = 0;       // ... and as much of its operand region as that call may use
     FnnRangeIo range;                     // value ranges handed from one call to the next (range_io.h)
     FnnResidualIo residual;               // a residual addition handed to the next MatMul call (range_io.h)
     FnnPrepIo prep;                       // a prepared operand handed from one MatMul call to the next (range_io.h)
@@ -70,10 +71,12 @@ struct fnn_hip_ctx {
 };
 
 // Workspace of fnn_hip_qmatmul_static, part of the library's device image: every GPU the library runs on holds one
-// copy (32 MiB) until the process ends.  Region 0: prepared activation operands + row tables; region 1: split-K
-// partial tiles.  Host code never passes the array's name to a kernel: the device address of each GPU's copy is
+// copy (44 MiB) until the process ends.  Region 0: prepared activation operands + row tables; region 1: split-K
+// partial tiles.  Sizes within the limit that fnn_hip.h names may use all of region 0 (a kernel pads the rows to its tiles and K
+// to its steps: up to twice the limit and the tables), others as much as the limit.  Host code never passes the array's name to a kernel: the device address of each GPU's copy is
 // looked up once per device (static_workspace_of) and kept.
-constexpr size_t kStaticOperandBytes = 8u << 20;
+constexpr size_t kStaticOperandLimit = 8u << 20;
+constexpr size_t kStaticOperandBytes = 20u << 20;
 constexpr size_t kStaticPartialBytes = 24u << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticOperandBytes + kStaticPartialBytes];
 
@@ -702,9 +705,11 @@ int fnn_hip_qmatmul_static(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const floa
     // duration of the call, and everything that would allocate fails instead
     struct Mode {
         fnn_hip_ctx *c;
-        explicit Mode(fnn_hip_ctx *c_) : c(c_) { c->static_mode = true; }
+        Mode(fnn_hip_ctx *c_, size_t room) : c(c_) { c->static_mode = true; c->static_operand_room = room; }
         ~Mode() { c->static_mode = false; }
-    } mode(ctx);
+    };
+    const bool within = 4 * ((m + 15) / 16 * 16) * ((w->inner + 63) / 64 * 64) + 12 * m <= (int64_t)kStaticOperandLimit;
+    const Mode mode(ctx, within ? kStaticOperandBytes : kStaticOperandLimit);
     return fnn_hip_qmatmul(ctx, w, a_dev, m, bias_dev, act, out_dev, flags | FNN_FLAG_DEVICE_PTRS);
 }
 
@@ -1265,12 +1270,12 @@ static Staging &tmp_slot(fnn_hip_ctx *ctx, int which)
     return which == 0 ? ctx->st_tmp : (which == 1 ? ctx->st_tmp2 : (which == 4 ? ctx->st_tmp4 : ctx->st_tmp3));
 }
 // fnn_hip_qmatmul_static: fixed regions of the static workspace, nothing grows
-static size_t static_room(int which) { return which == 0 ? kStaticOperandBytes : (which == 1 ? kStaticPartialBytes : 0); }
+static size_t static_room(const fnn_hip_ctx *ctx, int which) { return which == 0 ? ctx->static_operand_room : (which == 1 ? kStaticPartialBytes : 0); }
 
 int fnn_ctx_ensure_tmp(fnn_hip_ctx *ctx, int which, size_t bytes, void **ptr)
 {
     if (ctx->static_mode) {
-        const size_t off = which == 0 ? 0 : kStaticOperandBytes, cap = static_room(which);
+        const size_t off = which == 0 ? 0 : kStaticOperandBytes, cap = static_room(ctx, which);
         if (bytes > cap)
             return fail(ctx, FNN_ERR_MEMORY,
                         "fnn_hip_qmatmul_static: this shape needs %zu bytes of %s workspace, the static buffer holds %zu: use fnn_hip_qmatmul",
@@ -1287,15 +1292,8 @@ int fnn_ctx_ensure_tmp(fnn_hip_ctx *ctx, int which, size_t bytes, void **ptr)
 
 bool fnn_ctx_tmp_fits(fnn_hip_ctx *ctx, int which, size_t bytes)
 {
-    if (ctx->static_mode) return bytes <= static_room(which);
+    if (ctx->static_mode) return bytes <= static_room(ctx, which);
     return !ctx->capturing || bytes <= tmp_slot(ctx, which).cap;
-}
-
-bool fnn_ctx_operand_allowed(fnn_hip_ctx *ctx, int64_t m, int64_t k, size_t bytes)
-{
-    // (the limit that the header names: sizes within it run the same kernel with either entry point)
-    const bool promised = m <= FNN_STATIC_MAX_M && 4 * ((m + 15) / 16 * 16) * ((k + 63) / 64 * 64) + 12 * m <= (int64_t)kStaticOperandBytes;
-    return bytes <= kStaticOperandBytes || (!promised && !ctx->static_mode);
 }
 
 void *fnn_ctx_copy_memory(fnn_hip_ctx *ctx, size_t bytes)

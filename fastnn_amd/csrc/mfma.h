@@ -9,9 +9,6 @@
 int fnn_ctx_ensure_tmp(fnn_hip_ctx *ctx, int which, size_t bytes, void **ptr);
 // whether fnn_ctx_ensure_tmp would give this call the bytes (a kernel that has others behind it leaves the call to them)
 bool fnn_ctx_tmp_fits(fnn_hip_ctx *ctx, int which, size_t bytes);
-// whether a rule may choose a kernel with this much of workspace 0 for activations of [m, k]: not where fnn_hip_qmatmul_static
-// takes the sizes and its buffer does not hold it
-bool fnn_ctx_operand_allowed(fnn_hip_ctx *ctx, int64_t m, int64_t k, size_t bytes);
 int fnn_ctx_fail(fnn_hip_ctx *ctx, int code, const char *msg);
 bool fnn_ctx_capturing(fnn_hip_ctx *ctx);
 // true while device memory must not be allocated: graph capture, or a call through fnn_hip_qmatmul_static

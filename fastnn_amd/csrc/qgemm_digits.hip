@@ -202,7 +202,7 @@ int run_digits_wave(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, co
     const int64_t m_pad = (int64_t)p.mtiles * act_rows;
     const size_t a_bytes = (size_t)m_pad * 3 * p.nsteps * 32;
     const size_t op_bytes = a_bytes + (size_t)m_pad * 8;
-    if (!fnn_ctx_operand_allowed(ctx, q.m, q.k, op_bytes) || !fnn_ctx_tmp_fits(ctx, 0, op_bytes)) return FNN_OK;
+    if (!fnn_ctx_tmp_fits(ctx, 0, op_bytes)) return FNN_OK;
     if ((rc = fnn_frag_words(ctx, s, w, p.kblocks, &p.wf, &p.words_kp))) return rc;
     void *ws0 = nullptr;
     if ((rc = fnn_ctx_ensure_tmp(ctx, 0, op_bytes, &ws0))) return rc;

@@ -384,10 +384,6 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
                     if (sp > 1 && (wgs * sp > 1024 || sp * 8 > f.ks.kblocks)) break;
                     const float us = two_launch_us(t, sp, m, n, f.ks.kblocks, f.four_bit);
                     if (us >= best) continue;
-                    FragPlan c = f;
-                    c.op_mb = t.mb; c.op_nb = t.nb;
-                    frag_sizes(&c, m, sp);
-                    if (!fnn_ctx_operand_allowed(ctx, m, k, c.ws_bytes)) continue;
                     best = us; f.mb = t.mb; f.nb = t.nb; f.direct = false; splits = sp;
                 }
             }

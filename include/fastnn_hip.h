@@ -223,11 +223,12 @@ int fnn_hip_qmatmul(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *a, i
  * loops, harnesses that forbid hipMalloc.  No counterpart in fastnn.  Same kernels and the same result as
  * fnn_hip_qmatmul with FNN_FLAG_DEVICE_PTRS (a, bias, out are device pointers; the call only enqueues work on the
  * context's stream), but the workspaces of the M >= 17 path (prepared activation operands, split-K partial tiles)
- * come from a 32 MiB array inside the library's device image instead of hipMalloc, and the call makes no
+ * come from a 44 MiB array inside the library's device image instead of hipMalloc, and the call makes no
  * allocation of any kind.  Limits, refused with FNN_ERR_MEMORY and a message that names them:
  *   - M <= FNN_STATIC_MAX_M;
  *   - operand workspace 2*ceil16(M)*ceil64(K)*2 + 12*M bytes <= 8 MiB (M = 256 at K = 4096 uses 4 MiB; half of
- *     that with FNN_FLAG_ACT_F16_SINGLE), split-K partials splits*M*N*4 bytes <= 24 MiB;
+ *     that with FNN_FLAG_ACT_F16_SINGLE; sizes beyond that are taken where a kernel needs no more than 8 MiB, then perhaps
+ *     not the kernel of fnn_hip_qmatmul), split-K partials splits*M*N*4 bytes <= 24 MiB;
  *   - per-weight side tables that fnn_hip_qmatmul builds on first use (the f16 expansion of a codebook weight at
  *     M >= 5, row means for FNN_FLAG_ACT_F16_SINGLE, re-strided rows when ceil(K/ITEMS) % 4 != 0) must exist
  *     already: call fnn_hip_qmatmul once per weight and flag combination beforehand.  (The copies of the packed words

@@ -110,7 +110,7 @@ def test_static_entry_point_refuses_what_does_not_fit(orc):
 
 
 @pytest.mark.parametrize("dt,m,k,n,within", [(flib.DT_I8, 97, 16384, 2048, True), (flib.DT_I8, 112, 16384, 2048, True), (flib.DT_I8, 128, 16384, 2048, False),
-                                             (flib.DT_U8, 97, 16384, 2048, True), (flib.DT_I4, 112, 16384, 2048, True), (flib.DT_F8, 49, 32000, 512, True),
+                                             (flib.DT_U8, 97, 16384, 2048, True), (flib.DT_I4, 112, 16384, 2048, True), (flib.DT_F8, 49, 32000, 512, True), (flib.DT_F8R, 491, 4096, 2048, True),
                                              (flib.DT_I4, 128, 16384, 2048, False)])
 def test_static_entry_point_takes_what_its_limits_allow(dt, m, k, n, within):
     """Sizes close to the operand limit, on a weight that fnn_hip_qmatmul has run (so that every copy of it exists): inside the
