@@ -39,7 +39,8 @@ inline hipError_t fnn_raise_lds_limit(std::atomic<uint64_t> &done, const void *k
 // 17 <= M <= 32: one launch, weights streamed into the MFMA operand registers, activations converted in the kernel,
 // K split over workgroups and reduced by the last one to arrive (qgemm_stream.hip)
 int fnn_stream_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
-bool fnn_stream_takes(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QMatmulArgs &p, int flags);
+// whether it takes the call, and the microseconds that it is expected to take
+bool fnn_stream_takes(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, float *us);
 // arrival counters of that kernel's column tiles: FNN_STREAM_COUNTERS words of device memory, zero between launches
 constexpr int FNN_STREAM_COUNTERS = 4096;
 uint32_t *fnn_ctx_stream_counters(fnn_hip_ctx *ctx);
@@ -47,6 +48,7 @@ uint32_t *fnn_ctx_stream_counters(fnn_hip_ctx *ctx);
 int fnn_digits_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
 // digit planes that path would multiply the call with by rule and options (3, 4); 0: the call is another kernel's
 int fnn_digits_planes(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags);
+float fnn_digits3_us(int dt, int64_t m, int64_t n, int64_t k);   // microseconds expected of three planes
 // a middle number of activation rows, per-channel types: both operands in the order the matrix cores take them (qgemm_frag.hip)
 int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
 int fnn_frag_i8act(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const I8ActArgs &p, bool *handled);
@@ -56,6 +58,8 @@ int fnn_fragment_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w,
 int fnn_frag_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, int64_t kblocks, const uint32_t **words, int *kp);
 // sum of the integer lanes per weight row (I8, I4), built on first use
 int fnn_row_qsum(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const int32_t **qsum);
+// microseconds expected of the f16 tiles (per-channel types)
+float fnn_tiled_us(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags);
 int fnn_tiled_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p,
                       int flags, bool *handled);
 // FNN_FLAG_ACT_QUANT with F8 weights: activations rounded to E4M3 (one power-of-two scale per row), fp8 matrix cores

@@ -482,6 +482,22 @@ int run_digits3(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const 
 
 }  // namespace
 
+// Microseconds of preparation + three planes on the LDS tiles: least squares over 690 drawn calls (M 17 .. 2048, K 256 .. 16384,
+// N 16 .. 16384; 4 to 9 % mean error)
+float fnn_digits3_us(int dt, int64_t m, int64_t n, int64_t k)
+{
+    static const float kFit[3][9] = {   // launch, stage of a round, round, M N / 1e6 per split, second launch, M N, M K, M K of ragged rows, N K / 1e6
+        {0.f, 0.440f, 9.22f, 1.810f, 3.40f, 0.205f, 2.173f, 3.171f, 0.1245f},      // 4-bit, 192 x 128
+        {6.31f, 1.026f, 2.63f, 0.f, 0.f, 1.507f, 0.929f, 2.695f, 0.0455f},         // 4-bit, 192 x 256
+        {3.21f, 0.725f, 5.57f, 2.441f, 4.14f, 0.601f, 1.477f, 1.522f, 0.0310f}};   // 8-bit, 192 x 128
+    const bool w8 = dt == FNN_DT_I8;
+    const Digits3Form f = digits3_form(!w8, m, n, k);
+    const float *c = kFit[w8 ? 2 : f.wide], rounds = (float)((f.tiles * f.splits + 255) / 256), mn = (float)m * (float)n / 1e6f, mk = (float)m * (float)k / 1e6f;
+    const bool ragged = (w8 ? (k + 3) / 4 : (k + 7) / 8) % 4 != 0;
+    return c[0] + rounds * (c[1] * (float)f.ips + c[2]) + (f.splits > 1 ? c[3] * (float)f.splits * mn + c[4] : 0.f) + c[5] * mn +
+           (c[6] + (ragged ? c[7] : 0.f)) * mk + c[8] * (float)n * (float)k / 1e6f;
+}
+
 // Microseconds of preparation + MatMul on the wave tiles and on the LDS tiles of run_digits3, least squares over 126 shapes
 // (M 40 .. 2048, K 1000 .. 8192, N 2048 .. 12288; mean error 2.4 % and 2.6 %).  Both count whole rounds of workgroups over the
 // 256 CUs: which one ends with the emptier round decides more than their rates do.  Taken from 96 rows on (8-bit weights below

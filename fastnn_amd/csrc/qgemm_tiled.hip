@@ -542,6 +542,30 @@ bool tile_layout_of(fnn_hip_ctx *ctx, int dtype, int64_t M, int64_t N, int64_t K
     }
 }
 
+// Split K over workgroups when the tiles alone do not fill the 256 CUs.  The factor minimises a
+// small cost model in microseconds, fitted to sweeps over the split factor on the benchmark shapes:
+// stages per workgroup x time a CU needs per stage x workgroups per CU (a CU gets through
+// stages at the same rate with one or several workgroups resident, but a lone workgroup cannot
+// hide its load latency: factor 1.5), plus, for s > 1, the write + read of s partial [M,N] tiles.
+// t_bits: the time of a 128 x 128 stage.  lone_rounds: one workgroup per CU, rounds do not overlap (the dense operand's 128 x 128
+// stages take 96 KB of LDS).
+int tile_splits(double t_bits, int cfg, int base, int iters, int64_t M, int64_t N, bool lone_rounds)
+{
+    const double t_stage = t_bits * (cfg == 3 ? 2.0 : (cfg == 0 ? 1.0 : (cfg == 1 ? 0.5 : 0.25)));
+    const double part_us = (double)M * (double)N * 8.0 / 3.0e6;
+    int splits = 1;
+    double best = 1e30;
+    for (int sp = 1; sp <= 32 && sp <= (iters / 4 > 0 ? iters / 4 : 1); sp++) {
+        const int per = (iters + sp - 1) / sp;
+        const double r = (double)base * sp / 256.0;
+        const double wgs = lone_rounds ? 1.5 * (double)(int64_t)(r + 0.999)
+                                       : (r <= 1.0 ? 1.5 : (double)(int64_t)(r + 0.95));
+        const double cost = per * t_stage * wgs + (sp > 1 ? 2.0 * sp * part_us : 0.0);
+        if (cost < best * 0.995) { best = cost; splits = sp; }   // on a tie the coarser split wins
+    }
+    return splits;
+}
+
 template <int DT>
 int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags,
               const DenseOperand *dense = nullptr)
@@ -554,28 +578,11 @@ int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QM
     const int mtiles = L.mtiles, ntiles = L.ntiles;
     const int passes = dense ? 2 : 1;
     const int iters = (int)(kpad / BK) * passes;
-    // Split K over workgroups when the tiles alone do not fill the 256 CUs.  The factor minimises a
-    // small cost model in microseconds, fitted to sweeps over the split factor on the benchmark shapes:
-    // stages per workgroup x time a CU needs per stage x workgroups per CU (a CU gets through
-    // stages at the same rate with one or several workgroups resident, but a lone workgroup cannot
-    // hide its load latency: factor 1.5), plus, for s > 1, the write + read of s partial [M,N] tiles.
     const int env_split = (int)fnn_ctx_option(ctx, FNN_OPT_TILE_SPLIT);
     const int base = mtiles * ntiles;
     // (codebook weights decoded in the kernel: two MFMAs per step and the table look-ups)
     const double t_bits = DT == FNN_DT_I4CB ? 0.9 : (DecH<DT>::WPS == 1 ? 0.4 : (DecH<DT>::WPS == 2 ? 0.7 : 1.0));
-    const double t_stage = t_bits * (cfg == 3 ? 2.0 : (cfg == 0 ? 1.0 : (cfg == 1 ? 0.5 : 0.25)));
-    const double part_us = (double)M * (double)N * 8.0 / 3.0e6;
-    int splits = 1;
-    double best = 1e30;
-    for (int sp = 1; sp <= 32 && sp <= (iters / 4 > 0 ? iters / 4 : 1); sp++) {
-        const int per = (iters + sp - 1) / sp;
-        const double r = (double)base * sp / 256.0;
-        // (the dense operand's 128x128 stages take 96 KB of LDS: one workgroup per CU, rounds do not overlap)
-        const double wgs = (dense && cfg == 0) ? 1.5 * (double)(int64_t)(r + 0.999)
-                                               : (r <= 1.0 ? 1.5 : (double)(int64_t)(r + 0.95));
-        const double cost = per * t_stage * wgs + (sp > 1 ? 2.0 * sp * part_us : 0.0);
-        if (cost < best * 0.995) { best = cost; splits = sp; }   // on a tie the coarser split wins
-    }
+    int splits = tile_splits(t_bits, cfg, base, iters, M, N, dense && cfg == 0);
     // the dense operand (128 x 128 tiles, one workgroup per CU): as many splits as fill one round, no more (measured on
     // 4096 x 4096: 96 tiles 58.0 us with 2 splits against 71.6 with the model's choice, 192 tiles 82.1 with none against 110)
     if (dense && cfg == 0) splits = base >= 256 ? 1 : 256 / base;
@@ -837,6 +844,23 @@ int fnn_row_means(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, cons
     }
     *umean = wm->umean;
     return FNN_OK;
+}
+
+// Least squares over 3260 drawn calls (M 17 .. 2048, K 256 .. 16384, N 16 .. 16384; 6.5 % mean error): a CU's stages, rounds of
+// resident workgroups, the K split's second launch and partials, output, operand and weight bytes, the longest row, ragged rows.
+float fnn_tiled_us(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags)
+{
+    static const float kFit[2][10] = {{6.35f, 0.332f, 1.544f, 2.757f, 1.217f, 2.056f, 1.619f, 0.172f, 0.826f, 4.50f},    // 8-bit
+                                      {8.08f, 0.345f, 0.f, 2.411f, 1.183f, 1.975f, 2.246f, 0.098f, 0.772f, 3.36f}};      // 4-bit
+    const bool four = dt == FNN_DT_I4 || dt == FNN_DT_U4 || dt == FNN_DT_F4;
+    const TileLayout L = four ? tile_layout<FNN_DT_F4>(ctx, m, n, k, flags, false) : tile_layout<FNN_DT_U8>(ctx, m, n, k, flags, false);
+    const int iters = (int)(L.kpad / BK), base = L.mtiles * L.ntiles;
+    const int sp0 = tile_splits(four ? 0.4 : 0.7, L.cfg, base, iters, m, n, false), ips = (iters + sp0 - 1) / sp0, sp = (iters + ips - 1) / ips;
+    const int load = (base * sp + 255) / 256, per_cu = L.bm == 32 ? 4 : (L.bm == 64 ? 3 : 2);
+    const float *c = kFit[four], mn = (float)m * (float)n / 1e6f, mk = (float)m * (float)k / 1e6f;
+    const bool ragged = (four ? (k + 7) / 8 : (k + 3) / 4) % 4 != 0;
+    return c[0] + c[1] * (float)(load * ips) * (float)L.bm / 128.f + c[2] * (float)((load + per_cu - 1) / per_cu) +
+           (sp > 1 ? c[3] + c[4] * mn * (float)sp : 0.f) + c[5] * mn + (c[6] + (ragged ? c[9] : 0.f)) * mk + c[7] * (float)n * (float)k / 1e6f + c[8] * (float)k / 1e3f;
 }
 
 int fnn_tiled_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, bool *handled)
