@@ -131,7 +131,10 @@ template <class F>
 int guarded(fnn_hip_ctx *ctx, const char *fn, F &&body) noexcept
 {
     const int rc = guarded_body(ctx, fn, body);
-    if (rc && ctx) ctx->io.pending.clear();   // results of a call that failed half way go nowhere
+    if (rc && ctx) {
+        if (ctx->capturing) ctx->io.pending.clear();   // (no wait inside a capture; the call around it ends what it began)
+        else ctx->io.abandon(ctx->stream);
+    }
     return rc;
 }
 
@@ -190,11 +193,12 @@ int ensure(fnn_hip_ctx *ctx, Staging &s, size_t bytes)
     return FNN_OK;
 }
 
-// A call on host pointers: its inputs and outputs go through pinned memory (host_io.h); finish() ends it.
-int stage_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t bytes, size_t at1 = 0, const void *src1 = nullptr, size_t bytes1 = 0)
+// A call on host pointers: its inputs and outputs go through pinned memory (host_io.h); finish() ends it, until then its
+// arrays are held.
+int stage_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t bytes, size_t at1 = 0, const void *src1 = nullptr, size_t bytes1 = 0, bool held = true)
 {
     if (ctx->capturing) return fail(ctx, FNN_ERR_DISPATCH, "transfer from host memory during graph capture");
-    HIP_TRY(ctx, FNN_ERR_MEMORY, ctx->io.in2(ctx->stream, dst_dev, src, bytes, at1, src1, bytes1));
+    HIP_TRY(ctx, FNN_ERR_MEMORY, ctx->io.in2(ctx->stream, dst_dev, src, bytes, at1, src1, bytes1, held));
     return FNN_OK;
 }
 
@@ -278,7 +282,6 @@ int fnn_hip_create(int device, fnn_hip_ctx **out)
         fnn_hip_ctx *ctx = new (std::nothrow) fnn_hip_ctx();
         if (!ctx) return fail(nullptr, FNN_ERR_MEMORY, "fnn_hip_create: out of host memory");
         ctx->device = device;
-        ctx->io.device = device;
         for (int i = 0; i < FNN_OPT_COUNT; i++) ctx->options[i] = kOptions[i].dflt;
         if ((e = hipSetDevice(device)) != hipSuccess ||
             (e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking)) != hipSuccess ||
@@ -1312,10 +1315,13 @@ bool fnn_ctx_no_alloc(fnn_hip_ctx *ctx) { return ctx->capturing || ctx->static_m
 int fnn_ctx_fail(fnn_hip_ctx *ctx, int code, const char *msg) { return fail(ctx, code, "%s", msg); }
 
 int64_t fnn_ctx_option(const fnn_hip_ctx *ctx, int option) { return ctx->options[option]; }
-int fnn_ctx_copy_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t bytes) { return guarded(ctx, "copy in", [&] { return stage_in(ctx, dst_dev, src, bytes); }); }
+int fnn_ctx_copy_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t bytes, bool held)
+{
+    return guarded(ctx, "copy in", [&] { return stage_in(ctx, dst_dev, src, bytes, 0, nullptr, 0, held); });
+}
 int fnn_ctx_copy_out(fnn_hip_ctx *ctx, void *dst, const void *src_dev, size_t bytes) { return guarded(ctx, "copy out", [&] { return stage_out(ctx, dst, src_dev, bytes); }); }
 int fnn_ctx_wait(fnn_hip_ctx *ctx) { return guarded(ctx, "wait", [&] { return finish(ctx); }); }
-void fnn_ctx_drop(fnn_hip_ctx *ctx) { ctx->io.pending.clear(); }
+void fnn_ctx_drop(fnn_hip_ctx *ctx) { ctx->io.abandon(ctx->stream); }
 uint32_t *fnn_ctx_stream_counters(fnn_hip_ctx *ctx) { return ctx->stream_counters; }
 FnnRangeIo *fnn_ctx_range_io(fnn_hip_ctx *ctx) { return &ctx->range; }
 FnnResidualIo *fnn_ctx_residual_io(fnn_hip_ctx *ctx) { return &ctx->residual; }

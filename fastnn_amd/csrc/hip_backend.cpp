@@ -201,15 +201,18 @@ int lift(fnn_backend *b, int st) noexcept
 template <class F>
 int guarded(fnn_backend *b, const char *fn, F &&body) noexcept
 {
+    int rc;
     try {
         return body();
     } catch (const std::bad_alloc &) {
-        return fail(b, FNN_ERR_MEMORY, "%s: out of host memory", fn);
+        rc = fail(b, FNN_ERR_MEMORY, "%s: out of host memory", fn);
     } catch (const std::exception &e) {
-        return fail(b, FNN_ERR_DISPATCH, "%s: %s", fn, e.what());
+        rc = fail(b, FNN_ERR_DISPATCH, "%s: %s", fn, e.what());
     } catch (...) {
-        return fail(b, FNN_ERR_DISPATCH, "%s: unknown C++ exception", fn);
+        rc = fail(b, FNN_ERR_DISPATCH, "%s: unknown C++ exception", fn);
     }
+    if (b && b->ctx) fnn_ctx_drop(b->ctx);   // (a body that returns a failure has done so itself)
+    return rc;
 }
 
 // One more write to `s` that plans must notice: the entry of the same range takes the new sequence number, a new
@@ -1220,8 +1223,8 @@ int dispatch_impl(fnn_backend *b, fnn_plan *p, uint64_t *elapsed_ns, uint64_t n_
     return st;
 }
 
-// write_arena without the wait: the copy is ordered by the stream
-int write_slice(fnn_backend *b, uint64_t offset, const void *data, uint64_t size)
+// write_arena without the wait: the copy is ordered by the stream (held: `data` stays as it is until the call's wait)
+int write_slice(fnn_backend *b, uint64_t offset, const void *data, uint64_t size, bool held)
 {
     fnn_slice s{offset, size};
     if (!b->arena || !in_arena(b, s)) return fail(b, FNN_ERR_MEMORY, "write_arena: %llu bytes at %llu outside the arena of %llu bytes", (unsigned long long)size, (unsigned long long)offset, (unsigned long long)b->arena_bytes);
@@ -1230,7 +1233,7 @@ int write_slice(fnn_backend *b, uint64_t offset, const void *data, uint64_t size
     drop_weights_overlapping(b, s);
     b->write_seq++;
     log_write(b, s);
-    return lift(b, fnn_ctx_copy_in(b->ctx, b->arena + offset, data, size));
+    return lift(b, fnn_ctx_copy_in(b->ctx, b->arena + offset, data, size, held));
 }
 
 int read_slice(fnn_backend *b, uint64_t offset, void *out, uint64_t size)
@@ -1340,7 +1343,7 @@ int fnn_backend_write_arena(fnn_backend *b, uint64_t offset, const void *data, u
 {
     return guarded(b, "fnn_backend_write_arena", [&]() -> int {
         if (!b) return fail(nullptr, FNN_ERR_DISPATCH, "fnn_backend_write_arena: NULL backend");
-        return write_slice(b, offset, data, size);
+        return write_slice(b, offset, data, size, false);
     });
 }
 
@@ -1532,7 +1535,7 @@ int fnn_backend_forward(fnn_backend *b, fnn_plan *p, const fnn_host_slice *input
         b->shape_env.clear();
         b->shape_env_sig.clear();
         int st = FNN_OK;
-        for (uint64_t i = 0; i < n_inputs && !st; i++) st = write_slice(b, inputs[i].offset, inputs[i].data, inputs[i].size);
+        for (uint64_t i = 0; i < n_inputs && !st; i++) st = write_slice(b, inputs[i].offset, inputs[i].data, inputs[i].size, true);
         if (!st) st = dispatch_impl(b, p, nullptr, 0, 0, nullptr, false);
         for (uint64_t i = 0; i < n_outputs && !st; i++) st = read_slice(b, outputs[i].offset, outputs[i].data, outputs[i].size);
         if (!st) return lift(b, fnn_ctx_wait(b->ctx));

@@ -16,7 +16,6 @@
 constexpr size_t kSmallTransfer = 1u << 20;
 
 struct FnnHostIo {
-    int device = 0;
     unsigned char *small = nullptr;     // kSmallTransfer bytes of pinned memory handed out from the start between two waits
     size_t small_used = 0;
     std::vector<void *> borrowed;       // staging blocks of large inputs, given back by wait()
@@ -25,17 +24,22 @@ struct FnnHostIo {
     struct Pending { void *dst; const void *src; size_t bytes; };
     std::vector<Pending> pending;       // results in staging memory, copied out when the stream has reached them
 
+    bool touched = false;               // transfers from or to the caller's own (pinned) memory may be under way
+
     void destroy();
-    // enqueues host -> device; `src` may be reused on return, the transfer is done when the stream gets there
-    hipError_t in(hipStream_t s, void *dst, const void *src, size_t bytes);
+    // enqueues host -> device; the transfer is done when the stream gets there.  held: the caller leaves `src` alone until the
+    // wait that ends its call (also one that fails: abandon); else it may be reused on return
+    hipError_t in(hipStream_t s, void *dst, const void *src, size_t bytes, bool held);
     // two inputs into one allocation, the second at offset at1 >= bytes0 (small ones: in one launch)
-    hipError_t in2(hipStream_t s, void *dst, const void *src0, size_t bytes0, size_t at1, const void *src1, size_t bytes1);
+    hipError_t in2(hipStream_t s, void *dst, const void *src0, size_t bytes0, size_t at1, const void *src1, size_t bytes1, bool held);
     // enqueues device -> host; `dst` holds the result after wait()
     hipError_t out(hipStream_t s, void *dst, const void *src, size_t bytes);
     // staging memory that kernels of the stream may write results to and that wait() copies to `dst`; null: too large
     void *result_slot(void *dst, size_t bytes);
     // waits until the stream has done everything enqueued and finishes the outputs
     hipError_t wait(hipStream_t s);
+    // instead of wait() where a call fails half way: its results go nowhere, and nothing touches the caller's memory any more
+    void abandon(hipStream_t s);
 
 private:
     hipError_t take_small(hipStream_t s, size_t bytes, size_t align_like, unsigned char **p);

@@ -141,11 +141,11 @@ hipError_t FnnHostIo::take_small(hipStream_t s, size_t bytes, size_t align_like,
     return hipSuccess;
 }
 
-hipError_t FnnHostIo::in2(hipStream_t s, void *dst, const void *src0, size_t bytes0, size_t at1, const void *src1, size_t bytes1)
+hipError_t FnnHostIo::in2(hipStream_t s, void *dst, const void *src0, size_t bytes0, size_t at1, const void *src1, size_t bytes1, bool held)
 {
     if (!bytes1 || at1 + bytes1 > kSmallTransfer) {
-        const hipError_t e = in(s, dst, src0, bytes0);
-        return e != hipSuccess || !bytes1 ? e : in(s, (unsigned char *)dst + at1, src1, bytes1);
+        const hipError_t e = in(s, dst, src0, bytes0, held);
+        return e != hipSuccess || !bytes1 ? e : in(s, (unsigned char *)dst + at1, src1, bytes1, held);
     }
     unsigned char *p;
     const hipError_t e = take_small(s, at1 + bytes1, reinterpret_cast<uintptr_t>(dst), &p);
@@ -155,12 +155,13 @@ hipError_t FnnHostIo::in2(hipStream_t s, void *dst, const void *src0, size_t byt
     return device_copy(s, dst, p, at1 + bytes1);
 }
 
-hipError_t FnnHostIo::in(hipStream_t s, void *dst, const void *src, size_t bytes)
+hipError_t FnnHostIo::in(hipStream_t s, void *dst, const void *src, size_t bytes, bool held)
 {
     if (!bytes) return hipSuccess;
-    if (fnn_is_pinned(src, bytes)) {               // a result array of an earlier call: no staging, but the caller may reuse it
+    if ((held || bytes > kSmallTransfer) && fnn_is_pinned(src, bytes)) {   // a result array of an earlier call: no staging
+        touched = true;
         const hipError_t e = bytes <= kSmallTransfer ? device_copy(s, dst, src, bytes) : hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
-        return e != hipSuccess ? e : hipStreamSynchronize(s);
+        return e != hipSuccess || held ? e : hipStreamSynchronize(s);
     }
     if (bytes > kSmallTransfer) return in_large(s, (unsigned char *)dst, (const unsigned char *)src, bytes);
     unsigned char *p;
@@ -218,8 +219,14 @@ hipError_t FnnHostIo::in_large(hipStream_t s, unsigned char *dst, const unsigned
 hipError_t FnnHostIo::out(hipStream_t s, void *dst, const void *src, size_t bytes)
 {
     if (!bytes) return hipSuccess;
-    if (bytes > kSmallTransfer) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
-    if (fnn_is_pinned(dst, bytes)) return device_copy(s, dst, src, bytes);
+    if (bytes > kSmallTransfer) {
+        touched = true;
+        return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+    }
+    if (fnn_is_pinned(dst, bytes)) {
+        touched = true;
+        return device_copy(s, dst, src, bytes);
+    }
     unsigned char *p;
     const hipError_t e = take_small(s, bytes, reinterpret_cast<uintptr_t>(src), &p);
     if (e != hipSuccess) return e;
@@ -266,5 +273,13 @@ hipError_t FnnHostIo::wait(hipStream_t s)
     for (void *b : borrowed) fnn_pinned_free(b);
     borrowed.clear();
     small_used = 0;
+    touched = false;
     return e;
+}
+
+void FnnHostIo::abandon(hipStream_t s)
+{
+    if (touched) (void)hipStreamSynchronize(s);
+    touched = false;
+    pending.clear();   // (what it staged stays taken until the next wait)
 }

@@ -87,9 +87,9 @@ struct FnnPreparedOperand {
 FnnPreparedOperand *fnn_ctx_prepared(fnn_hip_ctx *ctx);
 
 // Transfers between host memory and the context's stream (host_io.h) without the wait that ends a host-pointer call:
-// copy_in returns when the source may be reused, copy_out's destination holds the result after fnn_ctx_wait, and
-// fnn_ctx_drop forgets results that nobody waits for any more.
-int fnn_ctx_copy_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t bytes);
+// copy_in returns when the source may be reused (held: that is after fnn_ctx_wait or fnn_ctx_drop), copy_out's destination holds
+// the result after fnn_ctx_wait, and fnn_ctx_drop ends a call that failed: its results go nowhere, its arrays are free again.
+int fnn_ctx_copy_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t bytes, bool held);
 int fnn_ctx_copy_out(fnn_hip_ctx *ctx, void *dst, const void *src_dev, size_t bytes);
 int fnn_ctx_wait(fnn_hip_ctx *ctx);
 void fnn_ctx_drop(fnn_hip_ctx *ctx);
