@@ -243,15 +243,16 @@ def _np_ptr(a: Optional[np.ndarray]):
 
 
 class _PinnedBlock:
-    """Pinned memory that a result array keeps alive through its base."""
-    __slots__ = ("ptr", "__array_interface__")
+    """Pinned memory that a result array keeps alive through its base (and that may be the last to go when Python ends: it
+    holds what it needs for that)."""
+    __slots__ = ("ptr", "free", "__array_interface__")
 
-    def __init__(self, ptr: int, nbytes: int):
-        self.ptr = ptr
+    def __init__(self, ptr: int, nbytes: int, free):
+        self.ptr, self.free = ptr, free
         self.__array_interface__ = {"data": (ptr, False), "shape": (nbytes,), "typestr": "|u1", "version": 3}
 
     def __del__(self):
-        _lib.fnn_hip_host_free(self.ptr)
+        self.free(self.ptr)
 
 
 _PINNED_MIN = 1 << 15   # (smaller results are cheaper to copy out of the staging memory)
@@ -263,9 +264,10 @@ def result_array(shape, dtype=np.float32) -> np.ndarray:
     shape = (shape,) if isinstance(shape, (int, np.integer)) else tuple(shape)
     nbytes = math.prod(shape) * dtype.itemsize
     if nbytes >= _PINNED_MIN:
-        p = load_library().fnn_hip_host_alloc(nbytes)
+        lib = load_library()
+        p = lib.fnn_hip_host_alloc(nbytes)
         if p:
-            return np.asarray(_PinnedBlock(p, nbytes)).view(dtype).reshape(shape)
+            return np.asarray(_PinnedBlock(p, nbytes, lib.fnn_hip_host_free)).view(dtype).reshape(shape)
     return np.empty(shape, dtype)
 
 

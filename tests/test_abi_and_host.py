@@ -3,6 +3,8 @@ public header declares, and the host-side weight packers are bit-identical to th
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -174,3 +176,14 @@ def test_transpose_kn(orc):
     po = orc.quantize_kn(orc.I8, w)
     assert pw.rows == 45 and pw.inner == 70
     assert np.array_equal(pw.words, po.words)
+
+
+def test_a_result_array_may_outlive_the_module():
+    """When Python ends, a module's globals may be gone before the last array in pinned memory is: without a word on stderr."""
+    code = ("import numpy as np, fastnn_amd\nfrom fastnn_amd import lib\nfreed = []\n"
+            "data = np.zeros(64, np.uint8)\n"
+            "class Fake:\n    def fnn_hip_host_alloc(self, n): return data.ctypes.data\n    def fnn_hip_host_free(self, p): freed.append(p)\n"
+            "lib._lib = Fake()\nlib._PINNED_MIN = 0\nlib.load_library = lambda: lib._lib\n"
+            "x = lib.result_array(8)\nlib._lib = None\ndel x\nassert freed == [data.ctypes.data]\n")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert r.returncode == 0 and "Exception ignored" not in r.stderr, r.stderr
