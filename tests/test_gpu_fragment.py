@@ -208,3 +208,48 @@ def test_calls_that_the_other_kernels_do_faster_stay_with_them(ctx, dt, m, k, n)
     finally:
         ctx.set_option(flib.OPT_FRAGMENT, 0)
         ctx.release(h)
+
+
+@pytest.mark.parametrize("dt", [flib.DT_I8, flib.DT_I4, flib.DT_U4])
+@pytest.mark.parametrize("m,k,n", [(330, 1024, 2300), (600, 640, 5000)])
+def test_wave_tiles_over_many_tiles(ctx, dt, m, k, n):
+    """Tiles by the hundred, in stripes of four row tiles with a shorter last one, dealt to eight XCDs in unequal shares; rows of
+    infinity and not-a-number come out as such in every column and touch no other row."""
+    rng = np.random.default_rng(9800 + dt + m)
+    pw = fastnn_amd.quantize_weights(dt, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    h = ctx.register(pw)
+    try:
+        want = a.astype(np.float64) @ ctx.dequant(h, n, k).T.astype(np.float64)
+        bad = a.copy()
+        bad[3, k // 2], bad[m - 1, 0] = np.inf, np.nan
+        good = np.setdiff1d(np.arange(m), [3, m - 1])
+        for waves in (1, 2, 4):
+            ctx.set_option(flib.OPT_FRAGMENT, 1 << 14 | waves)
+            got = ctx.qmatmul(h, a, n)
+            assert_close(got, want, 2e-5, f"{waves} waves a tile")
+            off = ctx.qmatmul(h, bad, n)
+            assert not np.isfinite(off[[3, m - 1]]).any() and off[good].tobytes() == got[good].tobytes()
+    finally:
+        ctx.set_option(flib.OPT_FRAGMENT, 0)
+        ctx.release(h)
+
+
+@pytest.mark.parametrize("dt", TYPES)
+@pytest.mark.parametrize("m,k,n", [(20, 1000, 70), (33, 512, 4000)])
+def test_rows_that_are_not_finite_in_the_fragment_kernels(ctx, dt, m, k, n):
+    rng = np.random.default_rng(9900 + dt + m)
+    pw = fastnn_amd.quantize_weights(dt, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    bad = a.copy()
+    bad[3, k // 2], bad[17, k - 1], bad[m - 1, 0] = np.inf, -np.inf, np.nan
+    good = np.setdiff1d(np.arange(m), [3, 17, m - 1])
+    h = ctx.register(pw)
+    try:
+        for form in [1 << 8 | 1 << 4 | 1, 2 << 8 | 2 << 4 | 2, 1 << 8 | 4 << 4 | 3] + [1 << 15 | nb << 4 | 1 for nb in (1, 2, 4)]:
+            ctx.set_option(flib.OPT_FRAGMENT, form)
+            got, off = ctx.qmatmul(h, a, n), ctx.qmatmul(h, bad, n)
+            assert not np.isfinite(off[[3, 17, m - 1]]).any() and off[good].tobytes() == got[good].tobytes(), hex(form)
+    finally:
+        ctx.set_option(flib.OPT_FRAGMENT, 0)
+        ctx.release(h)
