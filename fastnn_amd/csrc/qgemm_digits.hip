@@ -220,10 +220,7 @@ int run_digits_wave(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, co
     p.af = d.planes; p.rexp = d.rexp; p.xsum = d.xsum;
     p.scales = q.scales; p.zeros = q.zeros; p.bias = q.bias; p.out = q.out;
     p.m = q.m; p.n = q.n; p.act = q.act;
-    if (FnnResidualIo *res = fnn_ctx_residual_io(ctx); res->residual && res->of_out == q.out && res->elems == (uint64_t)(q.m * q.n)) {
-        p.residual = res->residual; p.sum_out = res->sum_out;
-        res->used = 1;
-    }
+    fnn_take_residual(ctx, q.out, q.m * q.n, &p.residual, &p.sum_out);
     if constexpr (DT == FNN_DT_I8) e = fnn_wave_launch_i8(wk, p, s);
     else if constexpr (DT == FNN_DT_I4) e = fnn_wave_launch_i4(wk, p, s);
     else e = fnn_wave_launch_u4(wk, p, s);
@@ -339,10 +336,7 @@ int run_digits(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const Q
     t.ap = reinterpret_cast<const _Float16 *>(d.planes);
     t.rexp = d.rexp; t.xsum = d.xsum;
     t.out = q.out; t.part = (float *)ws1;
-    if (FnnResidualIo *res = fnn_ctx_residual_io(ctx); splits > 1 && res->residual && res->of_out == q.out && res->elems == (uint64_t)(M * N)) {
-        t.residual = res->residual; t.sum_out = res->sum_out;
-        res->used = 1;
-    }
+    if (splits > 1) fnn_take_residual(ctx, q.out, M * N, &t.residual, &t.sum_out);
     t.m = M; t.n = N; t.kp = q.kp; t.kpad = kpad; t.rows_pad = rows_pad;
     t.act = q.act; t.splits = splits; t.iters = iters; t.ips = ips; t.mtiles = mtiles; t.ntiles = ntiles;
     // ring depth: a stage is requested NS - 2 stages before it is consumed, and what is in flight has to cover the
@@ -455,10 +449,7 @@ int run_digits3(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const 
     t.ap = reinterpret_cast<const _Float16 *>(d.planes);
     t.rexp = d.rexp; t.xsum = d.xsum;
     t.out = q.out; t.part = (float *)ws1;
-    if (FnnResidualIo *res = fnn_ctx_residual_io(ctx); splits > 1 && res->residual && res->of_out == q.out && res->elems == (uint64_t)(M * N)) {
-        t.residual = res->residual; t.sum_out = res->sum_out;
-        res->used = 1;
-    }
+    if (splits > 1) fnn_take_residual(ctx, q.out, M * N, &t.residual, &t.sum_out);
     t.m = M; t.n = N; t.kp = q.kp; t.kpad = kpad; t.rows_pad = rows_pad;
     t.act = q.act; t.splits = splits; t.iters = iters; t.ips = ips; t.mtiles = mtiles; t.ntiles = ntiles;
     // ring depth: four stages (24 KB of planes + 8 or 16 KB of weights each; the 8-bit and the wide forms fill the LDS)

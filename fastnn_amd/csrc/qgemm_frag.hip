@@ -487,10 +487,7 @@ int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, c
     p.ks = f.ks; p.m_pad = f.m_pad; p.k = q.k;
     p.scales = q.scales; p.zeros = q.zeros; p.bias = q.bias; p.out = q.out;
     p.m = q.m; p.n = q.n; p.act = q.act;
-    if (FnnResidualIo *res = fnn_ctx_residual_io(ctx); res->residual && res->of_out == q.out && res->elems == (uint64_t)(q.m * q.n)) {
-        p.residual = res->residual; p.sum_out = res->sum_out;
-        res->used = 1;
-    }
+    fnn_take_residual(ctx, q.out, q.m * q.n, &p.residual, &p.sum_out);
     p.vec4 = q.n % 4 == 0 && !((reinterpret_cast<uintptr_t>(p.out) | reinterpret_cast<uintptr_t>(p.residual) | reinterpret_cast<uintptr_t>(p.sum_out) |
                                 reinterpret_cast<uintptr_t>(p.scales) | reinterpret_cast<uintptr_t>(p.zeros) | reinterpret_cast<uintptr_t>(p.bias)) & 15);
     const int mb = direct ? f.mb : f.op_mb, nb = direct ? f.nb : f.op_nb;

@@ -138,10 +138,7 @@ int fnn_stream_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w,
         if (rc) return rc;
         p.part = (float *)ws;
     }
-    if (FnnResidualIo *res = fnn_ctx_residual_io(ctx); res->residual && res->of_out == q.out && res->elems == (uint64_t)(q.m * q.n)) {
-        p.residual = res->residual; p.sum_out = res->sum_out;
-        res->used = 1;
-    }
+    fnn_take_residual(ctx, q.out, q.m * q.n, &p.residual, &p.sum_out);
     hipError_t e;
     switch (dt) {
     case FNN_DT_I8: e = fnn_stream_launch_i8(pl, p, s); break;
