@@ -1,4 +1,5 @@
-// Quantised MatMul with f32 activations on the int8 matrix cores, M >= 17, I8 / I4 / U4 weights.
+// Quantised MatMul with f32 activations on the int8 matrix cores, M >= 17, I8 / I4 / U4 weights: host side of the register
+// tiles of qgemm_wave_impl.h (three planes, from 96 rows on, where they are expected to finish first) and of the LDS tiles.
 //
 //   out[m,n] = act((sum_k A[m,k]*u(W[n,k]))*scale[n] + zero[n]*sum_k A[m,k] + bias[n])
 //   (gemm_batch_packed_simd + apply_affine_dot, src/backend/cpu/microkernels/gemm.rs:1982-2088,
@@ -473,31 +474,38 @@ int run_digits3(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const 
 
 }  // namespace
 
-// Microseconds of preparation + three planes on the LDS tiles: least squares over 690 drawn calls (M 17 .. 2048, K 256 .. 16384,
-// N 16 .. 16384; 4 to 9 % mean error)
+// Microseconds of preparation + three planes on the LDS tiles: least squares over 1480 drawn calls (M 17 .. 2048, K 256 .. 16384,
+// N 16 .. 16384, weights from memory and from cache; 4 to 7 % mean error)
 float fnn_digits3_us(int dt, int64_t m, int64_t n, int64_t k)
 {
-    static const float kFit[3][9] = {   // launch, stage of a round, round, M N / 1e6 per split, second launch, M N, M K, M K of ragged rows, N K / 1e6
-        {0.f, 0.440f, 9.22f, 1.810f, 3.40f, 0.205f, 2.173f, 3.171f, 0.1245f},      // 4-bit, 192 x 128
-        {6.31f, 1.026f, 2.63f, 0.f, 0.f, 1.507f, 0.929f, 2.695f, 0.0455f},         // 4-bit, 192 x 256
-        {3.21f, 0.725f, 5.57f, 2.441f, 4.14f, 0.601f, 1.477f, 1.522f, 0.0310f}};   // 8-bit, 192 x 128
+    static const float kFit[3][11] = {   // launch, stage of a round, round, M N / 1e6 per split, second launch, M N, M K, M K of ragged rows, N K / 1e6,
+                                         // workgroups / 256, K / 1e3
+        {7.48f, 0.457f, 0.f, 1.157f, 3.00f, 1.151f, 1.160f, 3.593f, 0.0564f, 2.443f, 0.495f},      // 4-bit, 192 x 128
+        {6.41f, 1.075f, 1.72f, 0.f, 0.f, 0.097f, 0.597f, 3.272f, 0.f, 6.814f, 0.f},                // 4-bit, 192 x 256
+        {3.68f, 0.714f, 2.17f, 0.425f, 4.77f, 0.417f, 1.060f, 1.826f, 0.0286f, 6.016f, 0.265f}};   // 8-bit, 192 x 128
     const bool w8 = dt == FNN_DT_I8;
     const Digits3Form f = digits3_form(!w8, m, n, k);
     const float *c = kFit[w8 ? 2 : f.wide], rounds = (float)((f.tiles * f.splits + 255) / 256), mn = (float)m * (float)n / 1e6f, mk = (float)m * (float)k / 1e6f;
     const bool ragged = (w8 ? (k + 3) / 4 : (k + 7) / 8) % 4 != 0;
     return c[0] + rounds * (c[1] * (float)f.ips + c[2]) + (f.splits > 1 ? c[3] * (float)f.splits * mn + c[4] : 0.f) + c[5] * mn +
-           (c[6] + (ragged ? c[7] : 0.f)) * mk + c[8] * (float)n * (float)k / 1e6f;
+           (c[6] + (ragged ? c[7] : 0.f)) * mk + c[8] * (float)n * (float)k / 1e6f + c[9] * (float)(f.tiles * f.splits) / 256.f + c[10] * (float)k / 1e3f;
 }
 
-// Microseconds of preparation + MatMul on the wave tiles and on the LDS tiles of run_digits3, least squares over 126 shapes
-// (M 40 .. 2048, K 1000 .. 8192, N 2048 .. 12288; mean error 2.4 % and 2.6 %).  Both count whole rounds of workgroups over the
-// 256 CUs: which one ends with the emptier round decides more than their rates do.  Taken from 96 rows on (8-bit weights below
-// have four planes), up to the rows that were measured, where it is ahead by more than 5 %.
+// Microseconds of preparation + MatMul on the wave tiles, against the LDS tiles of run_digits3: least squares over 950 drawn calls
+// (M 96 .. 2048, K 256 .. 16384, N 257 .. 16384, weights from memory and from cache; 8 % mean error for 8-bit, 4 to 6 % for 4-bit
+// weights).  Both count whole rounds of workgroups over the 256 CUs: which one ends with the emptier round decides more than
+// their rates do; with few rows the weight's bytes and the steps that a wave walks alone count beside them (without those two
+// 15 % of the I8 calls of 96 .. 160 rows lost more than 3 %, 119 x 6016 x 8704 51.8 us against 42.8; now none, at 0.87 of the LDS tiles'
+// time on average, the best choice 0.86).  Taken from 96 rows on (8-bit weights below have four planes), up to the rows that
+// were measured, where it is ahead by more than 5 %.
 int fnn_wave_choice(int dtype, int64_t m, int64_t n, int64_t k, float *us)
 {
-    static const float kWave[2][3][5] = {   // [8-bit][wk 1, 2, 4]: launch, 100 steps of a round, round, M N / 1e6, M K / 1e6
-        {{9.38f, 20.78f, 7.21f, 1.66f, 1.98f}, {7.74f, 22.4f, 5.07f, 1.6f, 1.86f}, {7.42f, 24.47f, 3.72f, 1.78f, 1.91f}},
-        {{8.74f, 22.71f, 6.56f, 2.06f, 2.03f}, {6.99f, 26.77f, 5.33f, 1.82f, 1.96f}, {7.22f, 30.76f, 3.75f, 1.99f, 1.92f}}};
+    static const float kWave[2][3][8] = {   // [8-bit][wk 1, 2, 4]: launch, 100 steps of a round, round, M N / 1e6, M K / 1e6, weight MB, 100 steps of all
+                                            // tiles / 256, 100 steps of a wave
+        {{6.26f, 22.15f, 5.061f, 1.073f, 1.556f, 0.1649f, 1.445f, 0.f}, {4.91f, 21.54f, 5.071f, 0.766f, 1.519f, 0.1213f, 3.563f, 2.75f},
+         {4.99f, 24.77f, 4.294f, 0.165f, 1.970f, 0.1820f, 2.357f, 2.19f}},
+        {{1.21f, 15.25f, 8.626f, 0.664f, 0.519f, 0.2031f, 8.724f, 12.22f}, {3.00f, 18.95f, 6.416f, 0.212f, 0.532f, 0.0494f, 14.53f, 14.06f},
+         {2.92f, 22.45f, 4.955f, 0.034f, 1.345f, 0.1360f, 11.79f, 15.26f}}};
     if (dtype != FNN_DT_I8 && dtype != FNN_DT_I4 && dtype != FNN_DT_U4) return 0;
     if (m < 96 || m > 2048 || n * k <= (int64_t)2048 * 2048) return 0;
     const bool w8 = dtype == FNN_DT_I8;
@@ -508,19 +516,14 @@ int fnn_wave_choice(int dtype, int64_t m, int64_t n, int64_t k, float *us)
     float best = 1e30f;
     for (int i = 0; i < 3; i++) {
         const int64_t rows = i == 0 ? 2 * WAVE_ROWS : WAVE_ROWS, cols = i == 2 ? WAVE_COLS : 2 * WAVE_COLS;
-        const float *c = kWave[w8][i], rounds = (float)ceil_div(ceil_div(m, rows) * ceil_div(n, cols), 256);
-        const float t = c[0] + c[1] * rounds * (float)(ceil_div(units, 1 << i) * ring) / 100.f + c[2] * rounds + c[3] * mn + c[4] * mk;
+        const int64_t tiles = ceil_div(m, rows) * ceil_div(n, cols);
+        const float *c = kWave[w8][i], rounds = (float)ceil_div(tiles, 256), steps = (float)(ceil_div(units, 1 << i) * ring) / 100.f;
+        const float t = c[0] + c[1] * rounds * steps + c[2] * rounds + c[3] * mn + c[4] * mk + c[5] * (float)n * (float)k * (w8 ? 1.f : 0.5f) / 1e6f +
+                        c[6] * (float)tiles / 256.f * steps + c[7] * steps;
         if (t < best) { best = t; wk = 1 << i; }
     }
-    const Digits3Form f = digits3_form(!w8, m, n, k);
-    static const float kTile[3][7] = {   // launch, stage of a round, round, M N / 1e6 written per split, M N / 1e6, M K / 1e6, second launch
-        {10.991f, 0.533f, 0.f, 0.859f, 1.08f, 1.834f, 3.562f},       // 4-bit, 192 x 128
-        {8.574f, 0.978f, 2.738f, 0.f, 1.497f, 1.405f, 0.f},          // 4-bit, 192 x 256
-        {8.014f, 0.671f, 1.524f, 1.369f, 2.179f, 1.583f, 3.103f}};   // 8-bit, 192 x 128
-    const float *c = kTile[w8 ? 2 : f.wide], rounds = (float)ceil_div(f.tiles * f.splits, 256);
-    const float tiles = c[0] + rounds * (c[1] * (float)f.ips + c[2]) + (f.splits > 1 ? c[3] * (float)f.splits * mn + c[6] : 0.f) + c[4] * mn + c[5] * mk;
     *us = best;
-    return best < 0.95f * tiles ? wk : 0;
+    return best < 0.95f * fnn_digits3_us(dtype, m, n, k) ? wk : 0;
 }
 
 // what the kernels of this file can multiply at all

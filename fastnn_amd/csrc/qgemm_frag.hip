@@ -260,8 +260,10 @@ struct FragPlan {
     size_t op_bytes, ws_bytes;   // activation fragments; with the row tables behind them
 };
 
-// Microseconds a launch form takes: least squares over 47 000 measurements of 5 400 drawn calls (M 17 .. 2048, K 256 .. 16384,
-// N 16 .. 16384, seven types; 6 % mean error, one launch 7 and 12 %; the form they choose is 1.2 % off the best one on average).
+// Microseconds a launch form takes: least squares over 97 000 measurements of 9 600 drawn calls (M 17 .. 2048, K 256 .. 16384,
+// N 16 .. 16384, seven types; 7 % mean error, one launch 6 and 7 %; the form they choose is 0.5 to 2 % off the best one on average up
+// to 160 rows).  The calls read their weights from the Infinity Cache (up to 300 MB of them in turn), those with weights of more
+// than 4 MB also from memory (640 MB in turn): a fragment kernel loses 1.5 to 2.5 us on 17 MB from memory, the streaming kernel 0.5.
 // What decides is the load of the busiest CU: the row tiles of a column tile and split go to one XCD (one L2 fetches their
 // weights), so 18 column tiles are three for the 32 CUs of some XCD, not 2.25.  The load counts the operand bytes through the
 // L1 and the matrix instructions, a round of resident workgroups the latency of its k blocks; per call the preparation, the K split's
@@ -274,9 +276,9 @@ int64_t cu_load(int64_t mtiles, int64_t columns) { return ((columns + 7) / 8 * m
 
 float two_launch_us(FragShape t, int splits, int64_t m, int64_t n, int kblocks, bool four)
 {
-    static const float kFit[2][11] = {{5.02f, 0.1164f, 0.0785f, 0.0083f, 0.1017f, 0.1604f, 3.165f, 2.333f, 0.791f, 0.980f, 0.1234f},    // 8-bit
-                                      {5.12f, 0.0993f, 0.0764f, 0.0136f, 0.2221f, 0.0967f, 3.656f, 2.448f, 0.189f, 1.009f, 0.1448f}};   // 4-bit
-    static const float kAgain[2] = {1.53f, 2.51f};
+    static const float kFit[2][11] = {{4.83f, 0.1196f, 0.0985f, 0.0060f, 0.1715f, 0.1674f, 2.914f, 2.452f, 0.858f, 0.717f, 0.1457f},    // 8-bit
+                                      {4.97f, 0.1057f, 0.1036f, 0.0101f, 0.2262f, 0.1137f, 3.695f, 2.346f, 0.587f, 0.721f, 0.1967f}};   // 4-bit
+    static const float kAgain[2] = {0.59f, 1.53f};
     const float *c = kFit[four], kpb = four ? 128.f : 64.f, spb = four ? 4.f : 2.f, mn = (float)m * (float)n / 1e6f;
     const int64_t mt = (m + 16 * t.mb - 1) / (16 * t.mb), nt = (n + 16 * t.nb - 1) / (16 * t.nb);
     const int kps = (kblocks + splits - 1) / splits, sp = (kblocks + kps - 1) / kps;
@@ -292,16 +294,29 @@ float two_launch_us(FragShape t, int splits, int64_t m, int64_t n, int kblocks, 
     return sp > 1 && us < 11.5f ? 11.5f : us;
 }
 
-// Negative: the form does not apply (eight steps, K of 1025 .. 2048, need the registers of the smaller tiles; from a load of
-// eight on, which was not measured, the second launch is the better form).
+// The one launch: the busiest CU's steps, the chain of a wave, weight bytes, and the activations, which every column tile fetches
+// and converts.  Negative: the form does not apply (eight steps, K of 1025 .. 2048, need the registers of the smaller tiles;
+// from a load of eight on, which was not measured, the second launch is the better form).
 float direct_us(FragShape t, int64_t m, int64_t n, int kblocks, bool four)
 {
-    static const float kFit[2][6] = {{2.51f, 0.1563f, 0.2627f, 0.f, 1.57f, 0.196f}, {1.12f, 0.f, 0.1852f, 0.0705f, 0.f, 0.443f}};   // 8-bit, 4-bit
+    static const float kFit[2][5] = {{2.75f, 0.0945f, 0.2591f, 0.0461f, 8.51f}, {1.91f, 0.0692f, 0.3642f, 0.0885f, 9.00f}};   // 8-bit, 4-bit
     const int seg = (kblocks + FRAG_NW - 1) / FRAG_NW, steps = seg * (four ? 4 : 2);
-    const int64_t load = cu_load((m + 16 * t.mb - 1) / (16 * t.mb), (n + 16 * t.nb - 1) / (16 * t.nb));
+    const int64_t mt = (m + 16 * t.mb - 1) / (16 * t.mb), nt = (n + 16 * t.nb - 1) / (16 * t.nb), load = cu_load(mt, nt);
     if (steps > 8 || (steps > 4 && t.mb * t.nb > 2) || (m > 16 && load > 8)) return -1.f;
-    const float *c = kFit[four], l = (float)load, padded = steps <= 2 ? 2.f : (steps <= 4 ? 4.f : 8.f);
-    return c[0] + l * (c[1] * (float)(seg * t.nb) + padded * (c[2] + c[3] * (float)t.nb)) + c[4] * (float)m * (float)n / 1e6f + c[5] * padded;
+    const float *c = kFit[four], padded = steps <= 2 ? 2.f : (steps <= 4 ? 4.f : 8.f);
+    return c[0] + c[1] * (float)load * padded * (float)t.nb + c[2] * padded + c[3] * (float)n * (float)kblocks * 64.f / 1e6f +
+           c[4] * (float)(mt * t.mb * nt) * (float)kblocks * (four ? 128.f : 64.f) * 64.f / 1e8f;
+}
+
+// Which of its shapes: a fit that is twice as far off on average (10 %) but orders them better, 0.7 % off the best shape on average
+// where that one is 1.2 % off.
+float direct_order(FragShape t, int64_t m, int64_t n, int kblocks, bool four)
+{
+    static const float kFit[2][5] = {{0.1563f, 0.2627f, 0.f, 1.57f, 0.196f}, {0.f, 0.1852f, 0.0705f, 0.f, 0.443f}};   // 8-bit, 4-bit
+    const int seg = (kblocks + FRAG_NW - 1) / FRAG_NW, steps = seg * (four ? 4 : 2);
+    const float *c = kFit[four], padded = steps <= 2 ? 2.f : (steps <= 4 ? 4.f : 8.f);
+    const float l = (float)cu_load((m + 16 * t.mb - 1) / (16 * t.mb), (n + 16 * t.nb - 1) / (16 * t.nb));
+    return l * (c[0] * (float)(seg * t.nb) + padded * (c[1] + c[2] * (float)t.nb)) + c[3] * (float)m * (float)n / 1e6f + c[4] * padded;
 }
 
 // ... and what the kernel behind this one takes (from 17 rows on): the streaming kernel, three digit planes or the f16 tiles.
@@ -373,11 +388,11 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
         if (m <= 16 && !ragged && (m <= 4 || direct_steps > 4 || (m <= 8 && integer))) return false;
         const float others = m > 16 ? others_us(ctx, w, m, flags, q) : 1e30f;
         if (others < 0.f) return false;
-        float best = 1e30f;
+        float best = 1e30f, order = 1e30f;
         if (direct_ok)
             for (FragShape t : kDirect) {
-                const float us = direct_us(t, m, n, f.ks.kblocks, f.four_bit);
-                if (us >= 0.f && us < best) { best = us; f.mb = t.mb; f.nb = t.nb; f.direct = true; }
+                const float us = direct_us(t, m, n, f.ks.kblocks, f.four_bit), o = direct_order(t, m, n, f.ks.kblocks, f.four_bit);
+                if (us >= 0.f && o < order) { order = o; best = us; f.mb = t.mb; f.nb = t.nb; f.direct = true; }
             }
         if (m > 16 || ragged)
             for (FragShape t : kTwoLaunch) {
@@ -390,13 +405,15 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
                     best = us; f.mb = t.mb; f.nb = t.nb; f.direct = false; splits = sp;
                 }
             }
-        // (the margin: where the two are about equal the fits decide at random, and what was there stays.  On 3 200 drawn calls of 17
-        // to 1500 rows that are not among the fitted ones the others' time is undercut by 22 % on average, and 1.3 % of the calls lose
-        // more than 3 %, the worst 1.27 times; a wider margin for operands beyond an XCD's L2, where the fit is at its worst, halves
-        // what is lost there.)
-        const float margin = 4.f * (float)m * (float)f.ks.kblocks * (f.four_bit ? 128.f : 64.f) > 4e6f ? 0.90f : 0.95f;
+        // (the margin: where the two are about equal the fits decide at random, and what was there stays.  With one half of the drawn
+        // calls fitted, on the other half, weights of more than 4 MB, from memory / from cache: 17 .. 32 rows take 0.80 / 0.78 of the
+        // others' time on average, 0.6 / 0.2 % of the calls lose more than 3 %; 33 .. 95 rows 0.75 / 0.72, 0.5 / 0.8 %; 161 .. 800 rows 0.95 / 0.95,
+        // 1.6 / 1.5 %, the worst 1.17 times.  Fitted from the cache alone, 3.5 % of the calls of 17 .. 32 rows lost with weights
+        // from memory (32 x 2048 x 8192 F8 12.6 us streamed, 14.1 here; 64 x 4096 x 11008 I4 25.5 on the LDS tiles, 29.4 here).  A wider
+        // margin for operands beyond an XCD's L2 and from 500 rows on, where the fits are at their worst, halves what is lost there.)
+        const float margin = m >= 500 || 4.f * (float)m * (float)f.ks.kblocks * (f.four_bit ? 128.f : 64.f) > 4e6f ? 0.90f : 0.97f;
         if (best > 1e29f || best > margin * others) return false;
-        if (float us; fnn_wave_choice(w->dtype, m, n, k, &us) && us < best) return false;
+        if (float us; fnn_wave_choice(w->dtype, m, n, k, &us) && best > margin * us) return false;
     }
     f.op_mb = f.mb; f.op_nb = f.nb;
     if (f.direct) {

@@ -843,12 +843,13 @@ int fnn_row_means(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, cons
     return FNN_OK;
 }
 
-// Least squares over 3260 drawn calls (M 17 .. 2048, K 256 .. 16384, N 16 .. 16384; 6.5 % mean error): a CU's stages, rounds of
-// resident workgroups, the K split's second launch and partials, output, operand and weight bytes, the longest row, ragged rows.
+// Least squares over 5080 drawn calls (M 17 .. 2048, K 256 .. 16384, N 16 .. 16384, weights from memory and from cache; 8 % mean
+// error): a CU's stages, rounds of resident workgroups, the K split's second launch and partials, output, operand and weight
+// bytes, the longest row, ragged rows.
 float fnn_tiled_us(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags)
 {
-    static const float kFit[2][10] = {{6.35f, 0.332f, 1.544f, 2.757f, 1.217f, 2.056f, 1.619f, 0.172f, 0.826f, 4.50f},    // 8-bit
-                                      {8.08f, 0.345f, 0.f, 2.411f, 1.183f, 1.975f, 2.246f, 0.098f, 0.772f, 3.36f}};      // 4-bit
+    static const float kFit[2][11] = {{5.03f, 0.2922f, 2.760f, 2.696f, 1.447f, 2.021f, 1.363f, 0.194f, 0.841f, 5.68f, 0.0748f},    // 8-bit
+                                      {7.12f, 0.3122f, 0.972f, 2.467f, 1.069f, 1.962f, 2.417f, 0.146f, 0.717f, 3.81f, 0.0050f}};   // 4-bit
     const bool four = dt == FNN_DT_I4 || dt == FNN_DT_U4 || dt == FNN_DT_F4;
     const TileLayout L = four ? tile_layout<FNN_DT_F4>(ctx, m, n, k, flags, false) : tile_layout<FNN_DT_U8>(ctx, m, n, k, flags, false);
     const int iters = (int)(L.kpad / BK), base = L.mtiles * L.ntiles;
@@ -856,7 +857,7 @@ float fnn_tiled_us(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, in
     const int load = (base * sp + 255) / 256, per_cu = L.bm == 32 ? 4 : (L.bm == 64 ? 3 : 2);
     const float *c = kFit[four], mn = (float)m * (float)n / 1e6f, mk = (float)m * (float)k / 1e6f;
     const bool ragged = (four ? (k + 7) / 8 : (k + 3) / 4) % 4 != 0;
-    return c[0] + c[1] * (float)(load * ips) * (float)L.bm / 128.f + c[2] * (float)((load + per_cu - 1) / per_cu) +
+    return c[0] + (c[1] * (float)L.bm / 128.f + c[10]) * (float)(load * ips) + c[2] * (float)((load + per_cu - 1) / per_cu) +
            (sp > 1 ? c[3] + c[4] * mn * (float)sp : 0.f) + c[5] * mn + (c[6] + (ragged ? c[9] : 0.f)) * mk + c[7] * (float)n * (float)k / 1e6f + c[8] * (float)k / 1e3f;
 }
 
