@@ -649,18 +649,18 @@ int fnn_hip_qmatmul(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *a, i
             return FNN_OK;
         }
 
-        // kernel choice: matrix-core kernel for every M (bandwidth-bound at small M); the FMA GEMV
-        // serves the codebook type at M <= 4 and any weight when FNN_FLAG_PREFER_FMA asks for it;
-        // the shape-agnostic kernel takes what is left (ragged rows, unaligned pointers).
+        // kernel choice: each kernel in turn declines or takes the call.  Matrix-core kernels for every M
+        // (bandwidth-bound at small M); the FMA GEMV serves the codebook type at M <= 4 and any weight when
+        // FNN_FLAG_PREFER_FMA asks for it; the shape-agnostic kernel takes what is left (unaligned pointers).
         bool handled = false;
         if (!(flags & FNN_FLAG_FORCE_GENERIC)) {
             const bool fma_first = (flags & FNN_FLAG_PREFER_FMA) || w->dtype == FNN_DT_I4CB;
-            {   // (small aligned M declined by rule)
+            {   // (ragged rows at any M; else from M = 5 or 17 where it is expected to finish before the kernels below)
                 int rc = fnn_frag_qmatmul(ctx, ctx->stream, w, p, flags, &handled);
                 if (rc) return rc;
             }
             if (fma_first && !handled) HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_qgemv(w->dtype, p, ctx->stream, &handled));
-            if (!handled) {   // (17 <= M <= 32 and, for a long K over few columns, from M = 9 or 5)
+            if (!handled) {   // (M <= 32 from 17 on and, for a long K over few columns, from 9 or 5; codebook type 5 .. 64)
                 int rc = fnn_stream_qmatmul(ctx, ctx->stream, w, p, flags, &handled);
                 if (rc) return rc;
             }

@@ -36,20 +36,22 @@ inline hipError_t fnn_raise_lds_limit(std::atomic<uint64_t> &done, const void *k
 
 // M >= 5: activations prepared once as f16 operands, 4-wave output tiles with the
 // activations staged through LDS and optional split of K (deterministic reduction).
-// 17 <= M <= 32: one launch, weights streamed into the MFMA operand registers, activations converted in the kernel,
-// K split over workgroups and reduced by the last one to arrive (qgemm_stream.hip)
+// up to 32 rows (codebook type 64), where the fragment kernels below do not take the call: one launch, weights streamed into the MFMA operand
+// registers, activations converted in the kernel, K split over workgroups and reduced by the last one to arrive (qgemm_stream.hip)
 int fnn_stream_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
 // whether it takes the call, and the microseconds that it is expected to take
 bool fnn_stream_takes(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, float *us);
 // arrival counters of that kernel's column tiles: FNN_STREAM_COUNTERS words of device memory, zero between launches
 constexpr int FNN_STREAM_COUNTERS = 4096;
 uint32_t *fnn_ctx_stream_counters(fnn_hip_ctx *ctx);
-// int8 matrix-core GEMM over exact activation digit planes (qgemm_digits.hip): M >= 17, I8 / I4 / U4 weights
+// int8 matrix-core GEMM over exact activation digit planes (qgemm_digits.hip: LDS tiles, or the register tiles of qgemm_wave_impl.h):
+// M >= 17, I8 / I4 / U4 weights, where the kernels above and below do not take the call
 int fnn_digits_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
 // digit planes that path would multiply the call with by rule and options (3, 4); 0: the call is another kernel's
 int fnn_digits_planes(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags);
 float fnn_digits3_us(int dt, int64_t m, int64_t n, int64_t k);   // microseconds expected of three planes
-// a middle number of activation rows, per-channel types: both operands in the order the matrix cores take them (qgemm_frag.hip)
+// a middle number of activation rows (and any number with ragged weight rows), per-channel types: both operands in the order the
+// matrix cores take them; asked first, takes what it is expected to finish before the kernels it would replace (qgemm_frag.hip)
 int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
 int fnn_frag_i8act(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const I8ActArgs &p, bool *handled);
 // fragment-major copy of a weight's packed words, built on first use; null when it does not exist and this call may not build it

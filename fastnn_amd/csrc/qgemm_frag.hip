@@ -407,7 +407,7 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
             }
         // (the margin: where the two are about equal the fits decide at random, and what was there stays.  With one half of the drawn
         // calls fitted, on the other half, weights of more than 4 MB, from memory / from cache: 17 .. 32 rows take 0.80 / 0.78 of the
-        // others' time on average, 0.6 / 0.2 % of the calls lose more than 3 %; 33 .. 95 rows 0.75 / 0.72, 0.5 / 0.8 %; 161 .. 800 rows 0.95 / 0.95,
+        // others' time on average, 0.3 / 0.2 % of the calls lose more than 3 %; 33 .. 95 rows 0.75 / 0.72, 0.5 / 0.8 %; 161 .. 800 rows 0.95 / 0.95,
         // 1.6 / 1.5 %, the worst 1.17 times.  Fitted from the cache alone, 3.5 % of the calls of 17 .. 32 rows lost with weights
         // from memory (32 x 2048 x 8192 F8 12.6 us streamed, 14.1 here; 64 x 4096 x 11008 I4 25.5 on the LDS tiles, 29.4 here).  A wider
         // margin for operands beyond an XCD's L2 and from 500 rows on, where the fits are at their worst, halves what is lost there.)

@@ -1,5 +1,7 @@
 // Fragment-major MatMul of I8 activations on the int8 matrix cores (exact i32 sums).  The organisation is that of qgemm_frag_impl.h: contiguous wave loads
 // straight into the registers of v_mfma_i32_16x16x64_i8, the eight waves of a workgroup split its K range, one meeting in LDS.
+// Bound: as there, bytes and the chain of a launch.  Against operand kernel + LDS tiles + formula as launches of their own,
+// quantisation included: 64 x 2048 x 2048 19.4 -> 11.7 us, 256 x 4096 x 4096 28.9 -> 21.0.
 #pragma once
 #include <climits>
 #include <type_traits>

@@ -6,7 +6,8 @@
 //     quantisation + integer GEMM + 4-term dequantise, src/backend/cpu/packed_conv.rs:125-232,444-625).
 // An operand kernel writes the int8 activation matrix in the tile-major layout of the GEMM kernel (for conv it
 // evaluates im2col and the quantisation on the fly) and leaves sum_k q_a per row; the shared tiled GEMM kernel
-// produces the i32 accumulators.  MatMul: an epilogue kernel applies the reference's float formula to them.
+// produces the i32 accumulators.  MatMul: the tile kernel applies the reference's float formula where a tile holds whole sums, an
+// epilogue kernel where K is split (products of up to 8e9 MACs run on the kernels of qgemm_frag_int.hip instead).
 // Conv: the same formula, the activation and the NCHW stores run inside the GEMM kernel (or, by option and for
 // the matmul-form epilogue of 4-bit weights on an int8 payload, as a kernel of their own).
 #include "mfma.h"

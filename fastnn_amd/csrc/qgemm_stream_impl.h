@@ -1,4 +1,4 @@
-// Quantised MatMul for up to 32 activation rows (17..32 by default) in ONE launch on the matrix cores (gfx950): the packed weights are
+// Quantised MatMul for up to 32 activation rows (codebook type: 64) in ONE launch on the matrix cores (gfx950): the packed weights are
 // streamed straight into the registers that are the MFMA's weight operand, the f32 activations are converted inside
 // the kernel, K is split over workgroups and the split is reduced inside the same launch.
 //

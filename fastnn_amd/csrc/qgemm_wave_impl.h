@@ -1,12 +1,12 @@
 // Int8 MatMul for many activation rows: one wave per SIMD with a large register tile, operands straight from memory.
 //
-// Bound: the matrix cores (v_mfma_i32_32x32x32_i8, 32 clocks each; 3.6 to 4.4 POP/s sustained by themselves, by the data's
-// power) and, close behind, the 64 B/clk that a CU's L1 delivers: a wave tile of 96 x 128 (three digit planes of 32 activation
+// Bound: the matrix cores (v_mfma_i32_32x32x32_i8, 32 clocks each; MFMAs alone sustain 3.1 to 3.4 POP/s here) and, close behind, the 64 B/clk that a CU's L1 delivers: a wave tile of 96 x 128 (three digit planes of 32 activation
 // rows) asks for 224 bytes per k-value with 8-bit and 160 with 4-bit weights against 12 clocks of its SIMD's matrix core, so
 // the four waves of a CU need 14 and 10 clocks of L1 time in the same 12.  No LDS, no barrier: the operands lie in memory in
 // fragment order, a wave's load is contiguous, and RING steps of 32 k-values are in flight per wave.  What is left at large M
 // is the epilogue, which nothing overlaps at one wave per SIMD (10 to 15 us per round of tiles), and a matrix core that is
-// busy half the time (counters: 48 %, 23 % of the clocks waiting for memory).
+// busy half the time: I8 4096 x 4096 M = 2048 1.88 POP/s, matrix cores busy 47 % of the launch's clocks, waves waiting 24 % of
+// theirs; M = 256 (one tile per CU, a chain of latencies) 21 % and 31 %.
 // Measured against the LDS tiles of qgemm_digits.hip: I8 4096 x 4096 M = 256 29.6 -> 27.4 us, M = 1024 72.5 -> 65.5,
 // M = 2048 130.6 -> 122; I8 4096 x 11008 M = 700 131 -> 111; I4 4096 x 4096 M = 256 27.2 -> 23.6.  Row blocks an odd number
 // of pieces apart, to spread them over the L2's channels, gained nothing (122 -> 127 us).

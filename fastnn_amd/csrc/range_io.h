@@ -57,8 +57,8 @@ inline bool fnn_take_residual(fnn_hip_ctx *ctx, const float *out, int64_t elems,
     return true;
 }
 
-// A prepared MatMul operand that travels from one MatMul call to the next: at 17 <= M the f16 matrix-core path
-// first turns its f32 activations into scaled f16 hi + lo operand rows (a launch of its own).  When the caller knows
+// A prepared MatMul operand that travels from one MatMul call to the next: at 17 <= M the f16 matrix-core paths (LDS
+// tiles, fragment kernels) first turn their f32 activations into scaled f16 hi + lo operand rows (a launch of its own).  When the caller knows
 // that the next call on the context is the MatMul reading this one's result, the split-K reduction of this call can
 // leave that operand behind (it has the whole result row in registers), and the next call skips its preparation.
 // The conversion code is the same, so results are identical.

@@ -117,7 +117,7 @@ enum {
                                   /* mode, and by rule not weights of up to 2048 x 2048 elements, which the f16 tiles    */
                                   /* serve faster: FNN_OPT_DIGIT_PLANES = 3 / 4 or a smaller MIN_M brings them here);     */
                                   /* 0: the f16 tiled GEMM takes them too                                                 */
-    FNN_OPT_GEMM_INT8_MIN_M = 11, /* smallest M of that path (default 17)                                                 */
+    FNN_OPT_GEMM_INT8_MIN_M = 11, /* smallest M of that path (default 17; the streaming and the fragment kernels come first)   */
     FNN_OPT_CODEBOOK_EXPANDED = 12, /* codebook weights with blocks of 32 at M >= 5: 0 (default) = by M (the streaming       */
                                   /* MatMul up to M = 64, beyond it decoded inside the tiled GEMM where that measured      */
                                   /* faster), 1 = always the tiled GEMM on the expanded f16 hi + lo operand                */
@@ -144,7 +144,8 @@ enum {
     FNN_OPT_STREAM_MIN_M = 19,    /* smallest and largest M of the one-launch streaming MatMul (weights straight into the      */
     FNN_OPT_STREAM_MAX_M = 20,    /* matrix-core operand registers, activations converted in the kernel, K split reduced by the  */
                                   /* last workgroup to arrive): defaults 17 and 32, 1..32; MAX_M = 0 switches it off.  By rule   */
-                                  /* it declines shapes with more column tiles x K splits than the chip holds at once.           */
+                                  /* it declines shapes with more column tiles x K splits than the chip holds at once, and of     */
+                                  /* what is left from 17 rows on it runs what FNN_OPT_FRAGMENT's kernels would finish later.      */
                                   /* Codebook weights with blocks of 32 (K % 128 == 0): with MAX_M at 32 the kernel takes        */
                                   /* min(MIN_M, 5) <= M <= 64 (a smaller MAX_M is taken as it is).  A long K over few output     */
                                   /* columns, with MIN_M not above its default: from M = 9 where K >= 4 N (K >= 2 N from         */
@@ -154,7 +155,8 @@ enum {
                                   /* (k-values per round / 256), splits = 0 meaning one round per workgroup                      */
     FNN_OPT_DIGIT_PLANES = 22,    /* int8 matrix-core GEMM (M >= 17, I8 / I4 / U4 weights): activation digit planes, 3 (22 bits     */
                                   /* below the row maximum, 2e-5 of max|ref| stated) or 4 (30 bits, 4e-6, a third more matrix-core */
-                                  /* work and operand traffic); 0 (default) = three wherever they measured faster                  */
+                                  /* work and operand traffic); 0 (default) = three wherever they measured faster (4-bit weights;   */
+                                  /* I8 from 96 rows on)                                                                           */
     FNN_OPT_GEMV_TILE_MAJOR = 23, /* the kernels that stream the packed words straight into matrix-core operand registers (M <= 8: */
                                   /* I8 / I4 / U4 / U8 / F8 / F8R weights; 9 <= M <= 32: every per-channel type)                   */
                                   /* and the tile kernels of the types with 64 or 32 bytes per row and stage (I4 / U4 digit        */
