@@ -166,6 +166,7 @@ const OptionSpec kOptions[FNN_OPT_COUNT] = {
     {0, 0, 4},        // FNN_OPT_DIGIT_PLANES
     {1, 0, 2},        // FNN_OPT_GEMV_TILE_MAJOR
     {0, -1, 0xffff},  // FNN_OPT_FRAGMENT
+    {0, 0, 0xff},     // FNN_OPT_CONV_PATCH
 };
 
 #define HIP_TRY(ctx, code, expr)                                                              \
@@ -246,7 +247,8 @@ void free_weight(fnn_hip_weight *w)
     if (w->scales) (void)hipFree(w->scales);
     if (w->zeros) (void)hipFree(w->zeros);
     if (w->codebook) (void)hipFree(w->codebook);
-    if (w->row_qsum) (void)hipFree(w->row_qsum);
+    if (w->row_qsum && !w->row_qsum_shared) (void)hipFree(w->row_qsum);
+    if (w->conv_words) (void)hipFree(w->conv_words);
     if (w->umean) (void)hipFree(w->umean);
     if (w->words4) (void)hipFree(w->words4);
     if (w->words_fr) (void)hipFree(w->words_fr);
@@ -863,11 +865,7 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
         if (b * groups > 65535) return fail(ctx, FNN_ERR_UNSUPPORTED_OP, "conv2d_i8: batch*groups > 65535");
         const bool dev = (flags & FNN_FLAG_DEVICE_PTRS) != 0;
         fnn_hip_weight *wm = const_cast<fnn_hip_weight *>(w);
-        if (integer_kernel && !wm->row_qsum) {
-            if (ctx->capturing) return fail(ctx, FNN_ERR_MEMORY, "conv2d_i8: first use of a weight during graph capture");
-            HIP_TRY(ctx, FNN_ERR_MEMORY, hipMalloc((void **)&wm->row_qsum, (size_t)oc * 4 + 64));
-            HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_row_qsum(w, wm->row_qsum, ctx->stream));
-        }
+        if (integer_kernel && !wm->row_qsum && ctx->capturing) return fail(ctx, FNN_ERR_MEMORY, "conv2d_i8: first use of a weight during graph capture");
         const size_t xin = (size_t)(b * c * h * wd) * 4, yout = (size_t)(b * oc * ho * wo) * 4;
         const float *dx = x, *dbias = bias;
         float *dy = y;
@@ -923,7 +921,7 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
         }
         if ((rc = ensure(ctx, ctx->st_tmp, (size_t)(b * groups) * (QCONV_NPART * 2 + 4) * 4))) return rc;
         QConvArgs p;
-        p.words = w->words; p.scales = w->scales; p.zeros = w->zeros; p.row_qsum = wm->row_qsum;
+        p.words = w->words; p.scales = w->scales; p.zeros = w->zeros;
         p.x = dx; p.bias = dbias; p.y = dy; p.acc_out = dacc;
         p.minmax_partial = (float *)ctx->st_tmp.ptr;
         p.actq = p.minmax_partial + (size_t)(b * groups) * QCONV_NPART * 2;
@@ -932,6 +930,17 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
         p.wbits = w->dtype == FNN_DT_I4 ? 4 : 8;
         p.x8 = nullptr; p.payload_i4 = 0; p.nparts = 0;
         p.part_stride = QCONV_NPART; p.range_zero = 0; p.range_out = nullptr; p.range_out_stride = 0;
+        // Many groups (depthwise convolutions): the matrix-core paths are one or two launches per group on a few
+        // channels each; the direct kernel covers all groups in one launch (64 groups of one channel at 80 x 80:
+        // 0.25 ms against 0.86-1.14 ms per call from host memory, 8 groups: equal, 4 groups: 0.35 against 0.22).
+        const bool many_groups = groups >= 16;
+        FnnPatchShape shape;
+        const bool patch = !many_groups && !(flags & FNN_FLAG_FORCE_GENERIC) && fnn_patch_conv_takes(ctx, ctx->stream, w, p, &shape);
+        if (!wm->row_qsum) {
+            HIP_TRY(ctx, FNN_ERR_MEMORY, hipMalloc((void **)&wm->row_qsum, (size_t)oc * 4 + 64));
+            HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_row_qsum(w, wm->row_qsum, ctx->stream));
+        }
+        p.row_qsum = wm->row_qsum;
         FnnRangeIo &rio = ctx->range;
         rio.in_used = 0;
         if (flags & FNN_FLAG_FORCE_GENERIC) {
@@ -966,24 +975,18 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
             } else {
                 HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_qconv2d_i8(p, ctx->stream, 3, &nparts));
             }
-            // One implicit-GEMM kernel where it is ahead, else the operand kernel and the int8 GEMM.  Either forms
-            // the scales itself when its workgroups' rows touch at most two images and they are few enough for the
+            // One launch from a patch in LDS, or the operand kernel and the int8 GEMM.  Either forms the scales itself when its
+            // workgroups' pixels belong to at most two images (the patch kernel's: to one) and they are few enough for the
             // repeated reduction to be cheaper than a launch.
-            int wg_rows = 64;
-            int64_t wgs = 0;
-            // Many groups (depthwise convolutions): the matrix-core paths are one or two launches per group on a few
-            // channels each; the direct kernel covers all groups in one launch (64 groups of one channel at 80 x 80:
-            // 0.25 ms against 0.86-1.14 ms per call from host memory, 8 groups: equal, 4 groups: 0.35 against 0.22).
-            const bool many_groups = groups >= 16;
-            const bool implicit = !many_groups && fnn_implicit_conv_takes(w, p, ctx->options[FNN_OPT_CONV_IMPLICIT], &wg_rows, &wgs);
-            if (!implicit) { wg_rows = 64; wgs = fnn_conv_operand_workgroups(p); }
-            const bool fused_scales = !many_groups && ho * wo >= wg_rows && nparts <= 4 * QCONV_NPART && wgs <= 8192;
+            const int64_t wgs = patch ? shape.workgroups(b) : fnn_conv_operand_workgroups(p);
+            const bool fused_scales = !many_groups && (patch || ho * wo >= 64) && nparts <= 4 * QCONV_NPART && wgs <= 8192;
             if (fused_scales) p.nparts = nparts;
             else HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_qconv2d_i8(p, ctx->stream, 4, &nparts));
-            bool handled = false;
-            int rc2 = many_groups ? FNN_OK : (implicit ? fnn_i8_implicit_conv(ctx, ctx->stream, w, p, &handled) : fnn_i8_tiled_conv(ctx, ctx->stream, w, p, &handled));
+            bool handled = patch;
+            int rc2 = FNN_OK;
+            if (patch) rc2 = fnn_patch_conv(ctx, ctx->stream, w, p, shape);
+            else if (!many_groups) rc2 = fnn_i8_tiled_conv(ctx, ctx->stream, w, p, &handled);
             if (rc2) return rc2;
-            if (implicit && !handled) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, "the implicit convolution kernel declined a shape it had accepted");
             if (!handled) {
                 if (fused_scales) HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_qconv2d_i8(p, ctx->stream, 4, &nparts));
                 p.nparts = 0;

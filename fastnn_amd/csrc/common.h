@@ -29,6 +29,9 @@ struct fnn_hip_weight {
     float *zeros;       // device; [rows]
     float *codebook;    // device; 16 floats (I4CB) or nullptr
     int32_t *row_qsum;  // device; [rows] sum of integer lanes per row (I8/I4), for the conv epilogue
+    int8_t *conv_words; // device; a Conv2d's rows as bytes in the operand order of conv_patch_kernel, built on its first call
+    int conv_groups, conv_kh, conv_kw;   // the geometry of that order
+    bool row_qsum_shared;                // row_qsum lies behind conv_words in one allocation
     float *umean;       // device; [rows] mean lane value per row, built on first single-pass GEMM use
     uint32_t *words4;   // device; rows re-strided to kp4 = ceil4(kp) words (+16 zero words) when kp % 4 != 0,
     int64_t kp4;        //         built on first use by a kernel that fetches 16-byte pieces of a row

@@ -68,9 +68,15 @@ int fnn_tiled_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, 
 int fnn_fp8_actquant_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, bool *handled);
 
 int64_t fnn_conv_operand_workgroups(const QConvArgs &p);
-// the implicit-GEMM convolution (qconv_implicit.hip): rows of one of its workgroups for this shape, and the call
-bool fnn_implicit_conv_takes(const fnn_hip_weight *w, const QConvArgs &p, int option, int *wg_rows, int64_t *wgs);
-int fnn_i8_implicit_conv(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QConvArgs &p, bool *handled);
+// the convolution from an int8 patch in LDS (qconv_patch.hip), asked first: rectangles of 32 * wpx pixels, nw waves over pixels (wpx), blocks of 32
+// channels (wch) and K (wks), `per` rectangles a workgroup, gy workgroups over the channels
+struct FnnPatchShape {
+    int nw, wpx, wch, wks, gy, per, twl, th, pw, pp, tiles_x, tiles;
+    size_t lds;
+    int64_t workgroups(int64_t images) const { return images * ((tiles + per - 1) / per) * gy; }
+};
+bool fnn_patch_conv_takes(fnn_hip_ctx *ctx, hipStream_t stream, const fnn_hip_weight *w, const QConvArgs &p, FnnPatchShape *s);
+int fnn_patch_conv(fnn_hip_ctx *ctx, hipStream_t stream, const fnn_hip_weight *w, const QConvArgs &p, const FnnPatchShape &s);
 
 // single-f16 activation mode: mean lane value per weight row (null for types whose lanes have zero mean)
 int fnn_row_means(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const float **umean);

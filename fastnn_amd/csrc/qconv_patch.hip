@@ -1,0 +1,641 @@
+// Quantised Conv2d (I8 or I4 weights, f32 NCHW activations) from an int8 patch in LDS: conv2d_packed_i8x4 /
+// conv2d_packed_i4x8 (src/backend/cpu/packed_conv.rs:125-283,444-841) in one launch.
+//
+// A workgroup of four waves owns a rectangle of output pixels of ONE image.  Phase 1: it loads the input patch under that
+// rectangle (all channels, halo included), quantises every value once with the image's scale and leaves it in LDS, channels
+// innermost: [chunk of 16 channels][patch pixel][16 bytes].  Phase 2: a tap of the kernel is then a fixed LDS offset, and the
+// 16 bytes that a lane (pixel lane & 31, k half lane >> 5) reads there are the A operand of v_mfma_i32_32x32x32_i8 as they
+// are, for k in the order (kernel row, kernel column, channel).  The weights are kept in that order, one KB per block of 32
+// channels and step (conv_words_kernel, built with the row sums on a weight's first call).  The waves share pixel blocks,
+// channel blocks and, where there is little work, the K range; K parts meet in LDS and then share the epilogue.
+//
+// What bounded the kernels that fetched im2col taps was vector instructions and their chain: a 3 x 3 layer fetched and quantised every
+// input value nine times, about 11 instructions a tap; here it is about 1.4 times (18 x 10 pixels under 16 x 8) and the tap arithmetic
+// is gone.  One image: 64 -> 64 channels 3x3 at 40 x 40 10.5 -> 6.6 us (before: operand kernel + GEMM), 128 -> 128 3x3 at 20 x 20 12.0 -> 7.2,
+// 512 -> 256 1x1 at 20 x 20 10.4 -> 7.0, 16 -> 32 3x3 stride 2 at 320 x 320 9.6 -> 7.8; what is left of these is the floor of a dependent launch
+// (2.3) and a chain of memory, LDS and barrier latencies.  Sixteen images: 16 -> 16 3x3 at 160 x 160 34 -> 23.5 us, 3 -> 16 3x3 stride 2 at
+// 640 x 640 63 -> 52 (184 MB), 64 -> 64 1x1 at 80 x 80 17.1 -> 16.1 (52 MB: 3.2 TB/s; loads in flight).  Two blocks of 32 channels a wave (one A
+// operand for two products) measured slower at every size: 130 registers, three waves a SIMD, against 107 and four.
+#include "mfma.h"
+#include "range_io.h"
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+namespace {
+
+struct PatchArgs {
+    // of one group of the convolution
+    const float *x;           // its first channel in image 0
+    const int8_t *cw;         // weights in operand order: [block of 32 channels][step][64 lanes][16 bytes]
+    const float *scales, *zeros, *bias;
+    const int32_t *qsum;
+    const float *actq, *pairs;   // ready-made scales, or npairs partial ranges per image
+    float *y, *sum_out, *range_out;
+    const float *residual;
+    int32_t *acc_out;
+    int64_t x_image, y_image;    // values of an image (all groups)
+    int npairs, pair_stride, actq_stride, range_zero, range_stride;
+    int cg, ocg, act, wbits, vec4;
+    float kk;
+    int hh, ww, ho, wo;       // geometry of a plane (1x1 without padding or stride: one row of all pixels)
+    int kw, stride, pad, dil;
+    int twl, th;              // rectangle: 1 << twl wide, th high
+    int tiles, per, parts;    // rectangles of an image, of a workgroup, workgroups of an image
+    int pw, pp, pgroups;      // patch width, pixels, groups of 64 pixels
+    int split;                // patches of up to 32 pixels: the two halves of a wave take a chunk each
+    int nch;                  // chunks of 16 channels (up to 4 channels: one chunk = 4 pixels of 4 channels)
+    int nsteps, nkc;          // K steps of two chunks, chunks
+    int lnw, lwch, lwks;      // log2 of the waves, of those over channels, over K
+    int w_at, tab_at, red_at; // LDS offsets behind the patch
+    FastDiv dpw, dpg, dparts, dtx, dper, dkw;   // (dper: chunks per tap, or per kernel row of up to 4 channels)
+};
+
+// 64 lanes' 16 bytes each from memory into LDS, without registers: lane i's land at lds + 16 i.  The compiler does not see these loads.
+__device__ __forceinline__ void load_kb(const void *gptr, unsigned lds_wave_base)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_wave_base), "v"(gptr) : "memory");
+}
+
+__device__ __forceinline__ float row16_min(float v)
+{
+    v = fminf(v, dpp_f32<0xB1>(v));
+    v = fminf(v, dpp_f32<0x4E>(v));
+    v = fminf(v, dpp_f32<0x141>(v));
+    return fminf(v, dpp_f32<0x140>(v));
+}
+__device__ __forceinline__ float row16_max(float v)
+{
+    v = fmaxf(v, dpp_f32<0xB1>(v));
+    v = fmaxf(v, dpp_f32<0x4E>(v));
+    v = fmaxf(v, dpp_f32<0x141>(v));
+    return fmaxf(v, dpp_f32<0x140>(v));
+}
+
+constexpr uint32_t NOWHERE = 0x80000000u;   // a buffer offset past every slab (slabs are below 2 GiB)
+constexpr int MAX_WAVES = 8;
+constexpr int MAX_LDS = 152 * 1024;   // beside the static part
+
+// C4: up to four channels in a group.  KS: the K range is shared by 1 << lwks waves.
+template <bool KS, bool C4>
+__global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs p)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    __shared__ float s_mm[2][MAX_WAVES], s_rng[MAX_WAVES][2];
+    __shared__ __attribute__((aligned(16))) int s_qs[MAX_WAVES][32];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 31, hf = lane >> 5;
+    const int nw = 1 << p.lnw, lwks = KS ? p.lwks : 0, wks = 1 << lwks, wch = 1 << p.lwch;
+    const int kw_ = wv & (wks - 1), cw_ = (wv >> lwks) & (wch - 1), px_ = wv >> (lwks + p.lwch);   // this wave's share of K, channels, pixels
+
+    const int nn = __builtin_amdgcn_readfirstlane((int)p.dparts.div(blockIdx.x)), part = (int)blockIdx.x - nn * p.parts;
+    const int t0 = part * p.per, t1 = min(t0 + p.per, p.tiles);
+    const int chstep = p.hh * p.ww * 4;
+    const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.x + nn * p.x_image), 0, p.cg * chstep, 0x00020000);
+
+    // ---- loads of phase 1: a unit is 64 patch pixels of one chunk (or 32 of two); a channel's plane is a scalar offset, so
+    // that only the pixel costs address arithmetic, once for 16 loads
+    const int units = C4 ? p.pgroups : (p.split ? (p.nch + 1) >> 1 : p.pgroups * p.nch);
+    auto unit_at = [&](int u, int &chunk, int &pix) {   // (chunk: uniform but for split patches)
+        if (!C4 && p.split) {
+            chunk = 2 * u + hf;
+            pix = lr;
+        } else {
+            chunk = C4 ? 0 : __builtin_amdgcn_readfirstlane((int)p.dpg.div((uint32_t)u));
+            pix = (u - chunk * p.pgroups) * 64 + lane;
+        }
+    };
+    auto fetch = [&](int u, int t, float(&v)[16]) {
+        const int ty = __builtin_amdgcn_readfirstlane((int)p.dtx.div((uint32_t)t)), tx = t - ty * (int)p.dtx.d;
+        const int iy0 = ty * p.th * p.stride - p.pad, ix0 = (tx << p.twl) * p.stride - p.pad;
+        int chunk, pix;
+        unit_at(u, chunk, pix);
+        const int py = (int)p.dpw.div((uint32_t)pix), iy = iy0 + py, ix = ix0 + pix - py * p.pw;
+        bool ok = pix < p.pp && (unsigned)iy < (unsigned)p.hh && (unsigned)ix < (unsigned)p.ww;
+        uint32_t vo = (uint32_t)(iy * p.ww + ix) * 4u;
+        int chunk0 = 0, wide = 16;   // (uniform) the unit's first chunk, channels from there on that it may touch
+        if (!C4) {
+            chunk0 = p.split ? 2 * u : __builtin_amdgcn_readfirstlane(chunk);
+            if (p.split) {
+                ok = ok && chunk < p.nch;
+                vo += hf ? (uint32_t)(16 * chstep) : 0u;
+                wide = 32;
+            }
+        }
+        vo = ok ? vo : NOWHERE;   // outside the image: zero by the range check
+        int so = chunk0 * 16 * chstep;
+        if (!C4 && chunk0 * 16 + wide <= p.cg) {
+#pragma unroll
+            for (int c = 0; c < 16; c++, so += chstep) v[c] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xbuf, vo, so, 0));
+        } else {
+            const int left = p.cg - chunk * 16, left0 = p.cg - chunk0 * 16;
+#pragma unroll
+            for (int c = 0; c < (C4 ? 4 : 16); c++, so += chstep)
+                v[c] = c < left0 ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xbuf, c < left ? vo : NOWHERE, so, 0)) : 0.0f;
+        }
+    };
+    float v0[16], v1[16];
+    if (wv < units) fetch(wv, t0, v0);
+
+    // ---- this lane's channel: a wave works on one block of 32
+    const bool share = !KS && p.ocg <= 16;   // (uniform) up to 16 channels: the lanes of channels 16 .. 31 take half of
+    const int blk = (int)blockIdx.y * wch + cw_, n = blk * 32 + (share ? (lr & 15) : lr);   // the pixels of the lane 16 below in the epilogue
+    const int ch = n < p.ocg ? n : 0;
+    const float sw = p.scales[ch], zw = p.zeros[ch], bi = p.bias ? p.bias[ch] : 0.0f;
+    const int qw = p.qsum[ch];
+
+    // ---- LDS offset of every chunk of K, relative to a pixel's first tap; bits 24 up: how many of its four words count
+    uint32_t *tab = reinterpret_cast<uint32_t *>(lds + p.tab_at);   // [2 halves][nsteps]
+    for (int kc = tid; kc < 2 * p.nsteps; kc += nw * 64) {
+        uint32_t e = 0;
+        if (kc < p.nkc) {
+            const int tap = (int)p.dper.div((uint32_t)kc), r = kc - tap * (int)p.dper.d;
+            if (C4) {
+                e = (uint32_t)((tap * p.pw + r * 4) * p.dil * 4) | ((uint32_t)min(4, p.kw - r * 4) << 24);
+            } else {
+                const int i = (int)p.dkw.div((uint32_t)tap), j = tap - i * p.kw;
+                e = (uint32_t)((r * p.pp + (i * p.pw + j) * p.dil) * 16) | (4u << 24);
+            }
+        }
+        tab[(kc & 1) * p.nsteps + (kc >> 1)] = e;
+    }
+
+    // ---- the workgroup's weights on their way into LDS, where every rectangle and every wave finds them
+    auto weights = [&]() {
+        const int kbs = p.nsteps << p.lwch;
+        const unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)lds + p.w_at);
+        const char *src = reinterpret_cast<const char *>(p.cw) + (int64_t)blockIdx.y * kbs * 1024 + lane * 16;
+        for (int i = wv; i < kbs; i += nw) load_kb(src + (int64_t)i * 1024, base + i * 1024);
+    };
+
+    // ---- activation scale of the image: from partial ranges, or ready-made
+    float sa, za, inv;
+    weights();
+    if (p.npairs > 0) {
+        float mn = p.range_zero ? 0.0f : INFINITY, mx = p.range_zero ? 0.0f : -INFINITY;
+        conv_fold_partial_ranges(p.pairs + (int64_t)nn * p.pair_stride * 2, p.npairs, tid, nw * 64, mn, mx);
+        mn = wave_min(mn);
+        mx = wave_max(mx);
+        if (lane == 0) { s_mm[0][wv] = mn; s_mm[1][wv] = mx; }
+        __syncthreads();
+        // (every wave by itself: one lane a wave's pair)
+        mn = row16_min(s_mm[0][lane & (nw - 1)]);
+        mx = row16_max(s_mm[1][lane & (nw - 1)]);
+        const float range = mx - mn;
+        if (p.wbits == 4) {
+            sa = (range > 0.0f) ? range / 15.0f : 1.0f;
+            za = mn + 8.0f * sa;
+        } else {
+            sa = (range > 0.0f) ? range / 255.0f : 1.0f;
+            za = (range > 0.0f) ? mn + 128.0f * sa : 0.0f;
+        }
+        inv = (sa != 0.0f) ? 1.0f / sa : 0.0f;
+    } else {
+        const float *q = p.actq + (int64_t)nn * p.actq_stride;
+        sa = q[0]; za = q[1]; inv = q[2];
+    }
+    const float wt = sw * (float)qw;
+    const int bq = p.bias ? conv_bias_q(bi, sa, sw) : 0;
+
+    const int qlo = p.wbits == 4 ? -8 : -128, qhi = p.wbits == 4 ? 7 : 127;
+    auto quantise = [&](int u, const float(&v)[16]) {
+        int chunk, pix;
+        unit_at(u, chunk, pix);
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < (C4 ? 1 : 4); i++) {
+            int q[4];
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                // round half away from zero, then clamp: trunc(x + copysign(0.49999997, x)) equals roundf(x) after the
+                // clamp for every float (the conversion truncates, saturates and maps NaN to 0)
+                const float x = (v[i * 4 + t] - za) * inv;
+                q[t] = max(qlo, min((int)(x + __builtin_copysignf(0.49999997f, x)), qhi));
+            }
+            w[i] = __builtin_amdgcn_perm((uint32_t)q[1], (uint32_t)q[0], 0x0c0c0400u) | __builtin_amdgcn_perm((uint32_t)q[3], (uint32_t)q[2], 0x04000c0cu);
+        }
+        if (C4 || (p.cg & 15)) {   // bytes of channels that do not exist are zero
+            const int left = p.cg - chunk * 16;
+#pragma unroll
+            for (int i = 0; i < (C4 ? 1 : 4); i++)
+                if (left < i * 4 + 4) w[i] = left <= i * 4 ? 0u : w[i] & (0xffffffffu >> (8 * (i * 4 + 4 - left)));
+        }
+        if (pix >= p.pp || (!C4 && p.split && chunk >= p.nch)) return;
+        if (C4) reinterpret_cast<uint32_t *>(lds)[pix] = w[0];
+        else reinterpret_cast<u32x4 *>(lds)[chunk * p.pp + pix] = u32x4{w[0], w[1], w[2], w[3]};
+    };
+
+    const int np = p.ho * p.wo, tw1 = (1 << p.twl) - 1;
+    const int pl = px_ * 32 + lr;
+    const unsigned char *a_lds = lds + ((pl >> p.twl) * p.pw + (pl & tw1)) * p.stride * (C4 ? 4 : 16);
+    const unsigned char *w_lds = lds + p.w_at + cw_ * p.nsteps * 1024 + lane * 16;
+    const int s0 = (p.nsteps * kw_) >> lwks, s1 = (p.nsteps * (kw_ + 1)) >> lwks;
+    int *red = reinterpret_cast<int *>(lds + p.red_at);
+    float mn = INFINITY, mx = -INFINITY;
+
+    for (int t = t0; t < t1; t++) {
+        // ---- phase 1
+        for (int u = wv; u < units; u += 2 * nw) {
+            if (u + nw < units) fetch(u + nw, t, v1);
+            quantise(u, v0);
+            if (u + nw < units) {
+                if (u + 2 * nw < units) fetch(u + 2 * nw, t, v0);
+                quantise(u + nw, v1);
+            }
+        }
+        if (t == t0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the weights are there
+        __syncthreads();
+        if (t + 1 < t1 && wv < units) fetch(wv, t + 1, v0);   // the next patch's first loads pass under phase 2
+
+        // ---- phase 2
+        i32x16 acc;
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[i] = 0;
+        int qs = 0;
+        for (int s = s0; s < s1; s += 4) {
+            uint32_t e[4];
+            i32x4 af[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) e[i] = tab[hf * p.nsteps + min(s + i, s1 - 1)];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const unsigned char *at = a_lds + (e[i] & 0xffffffu);
+                if constexpr (C4) {
+#pragma unroll
+                    for (int q = 0; q < 4; q++) af[i][q] = *reinterpret_cast<const int *>(at + q * p.dil * 4);
+                } else {
+                    af[i] = *reinterpret_cast<const i32x4 *>(at);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                if (s + i >= s1) break;   // (wave-uniform)
+                acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], *reinterpret_cast<const i32x4 *>(w_lds + (s + i) * 1024), acc, 0, 0, 0);
+                if constexpr (C4) {
+#pragma unroll
+                    for (int q = 0; q < 4; q++) qs = __builtin_amdgcn_sdot4(af[i][q], q < (int)(e[i] >> 24) ? 0x01010101 : 0, qs, false);
+                } else {
+                    const int ones = (e[i] >> 24) ? 0x01010101 : 0;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) qs = __builtin_amdgcn_sdot4(af[i][q], ones, qs, false);
+                }
+            }
+        }
+        // ---- the K parts meet (exact integers: any order), and every wave that held one finishes its share of the pixels
+        qs += __shfl_xor(qs, 32, 64);   // the two k halves of a pixel
+        if (hf == 0) s_qs[wv][lr] = qs;
+        if constexpr (KS) {
+#pragma unroll
+            for (int ig = 0; ig < 4; ig++)
+                *reinterpret_cast<i32x4 *>(red + ((wv * 4 + ig) * 64 + lane) * 4) = i32x4{acc[ig * 4], acc[ig * 4 + 1], acc[ig * 4 + 2], acc[ig * 4 + 3]};
+            __syncthreads();
+        } else {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (share) {
+                // rows of 16 lanes: (k half 0, channels 0-15), (0, 16-31), (1, 0-15), (1, 16-31).  Registers 8 .. 15 (pixel
+                // groups 2 and 3) of the even rows move into registers 0 .. 7 of the odd rows above them
+#pragma unroll
+                for (int i = 0; i < 8; i++) acc[i] = (int)__builtin_amdgcn_permlane16_swap((uint32_t)acc[i], (uint32_t)acc[i + 8], false, false)[0];
+            }
+        }
+        const int ty = __builtin_amdgcn_readfirstlane((int)p.dtx.div((uint32_t)t)), oy0 = ty * p.th, ox0 = (t - ty * (int)p.dtx.d) << p.twl;
+        // pixels 8 ig + 4 hf + (0 .. 3) of the block: scale times the sum of their codes, place in a plane (false: outside)
+        auto pixels = [&](int ig, float(&rs)[4], int &at, int &ow) {
+            const int pq = ig * 8 + hf * 4, pt = px_ * 32 + pq, oh = oy0 + (pt >> p.twl);
+            ow = ox0 + (pt & tw1);
+            at = oh * p.wo + ow;
+            i32x4 q4 = *reinterpret_cast<const i32x4 *>(&s_qs[wv - kw_][pq]);
+            if constexpr (KS)
+                for (int k2 = 1; k2 < wks; k2++) {
+                    const i32x4 o4 = *reinterpret_cast<const i32x4 *>(&s_qs[wv - kw_ + k2][pq]);
+#pragma unroll
+                    for (int j = 0; j < 4; j++) q4[j] += o4[j];
+                }
+#pragma unroll
+            for (int j = 0; j < 4; j++) rs[j] = sa * (float)q4[j];
+            return oh < p.ho && ow < p.wo;
+        };
+        auto finish = [&](const i32x4 &a4, const float(&rs)[4], int at, int ow) {
+            if (n >= p.ocg) return;
+            float v[4];
+            int av[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = conv_affine(a4[j], sa, za, rs[j], sw, zw, wt, bq, p.kk, &av[j]);
+            conv_act4(v, p.act);
+            const int64_t o = nn * p.y_image + (uint32_t)(n * np + at);
+            // a residual: the Add behind this convolution; v becomes the sums, whose ranges travel on instead of y's
+            if (p.vec4) {
+                *reinterpret_cast<float4 *>(p.y + o) = make_float4(v[0], v[1], v[2], v[3]);
+                if (p.acc_out) *reinterpret_cast<int4 *>(p.acc_out + o) = make_int4(av[0], av[1], av[2], av[3]);
+                if (p.residual) {
+                    const float4 r4 = *reinterpret_cast<const float4 *>(p.residual + o);
+                    v[0] = v[0] + r4.x; v[1] = v[1] + r4.y; v[2] = v[2] + r4.z; v[3] = v[3] + r4.w;
+                    *reinterpret_cast<float4 *>(p.sum_out + o) = make_float4(v[0], v[1], v[2], v[3]);
+                }
+                mn = fminf(fminf(mn, fminf(v[0], v[1])), fminf(v[2], v[3]));
+                mx = fmaxf(fmaxf(mx, fmaxf(v[0], v[1])), fmaxf(v[2], v[3]));
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if (ow + j >= p.wo) continue;
+                    p.y[o + j] = v[j];
+                    if (p.acc_out) p.acc_out[o + j] = av[j];
+                    if (p.residual) {
+                        v[j] = v[j] + p.residual[o + j];
+                        p.sum_out[o + j] = v[j];
+                    }
+                    mn = fminf(mn, v[j]);
+                    mx = fmaxf(mx, v[j]);
+                }
+            }
+        };
+        float rs[4];
+        int at, ow;
+        if constexpr (KS) {
+            for (int ig = (4 * kw_) >> lwks; ig < (4 * (kw_ + 1)) >> lwks; ig++) {   // (eight parts: every other wave has one)
+                const int *src = red + (((wv - kw_) * 4 + ig) * 64 + lane) * 4;
+                i32x4 a4 = *reinterpret_cast<const i32x4 *>(src);
+                for (int k2 = 1; k2 < wks; k2++) {
+                    const i32x4 o4 = *reinterpret_cast<const i32x4 *>(src + k2 * (4 * 64 * 4));
+#pragma unroll
+                    for (int j = 0; j < 4; j++) a4[j] += o4[j];
+                }
+                if (pixels(ig, rs, at, ow)) finish(a4, rs, at, ow);
+            }
+        } else {
+#pragma unroll
+            for (int t4 = 0; t4 < 4; t4++) {
+                if (share && t4 >= 2) break;
+                if (pixels(share ? t4 + 2 * (lr >> 4) : t4, rs, at, ow))
+                    finish(i32x4{acc[t4 * 4], acc[t4 * 4 + 1], acc[t4 * 4 + 2], acc[t4 * 4 + 3]}, rs, at, ow);
+            }
+        }
+        if (t + 1 < t1) __syncthreads();   // this patch is read before the next one is written
+    }
+
+    if (p.range_out) {
+        // one pair per workgroup and block of 32 channels, [image][block][workgroup]: a convolution that reads whole blocks takes
+        // their pairs
+        mn = wave_min(mn);
+        mx = wave_max(mx);
+        if (lane == 0) { s_rng[wv][0] = mn; s_rng[wv][1] = mx; }
+        __syncthreads();
+        const int b32 = (int)blockIdx.y * wch + tid;
+        if (tid < wch && b32 * 32 < p.ocg) {
+            mn = INFINITY;
+            mx = -INFINITY;
+            for (int w2 = 0; w2 < nw; w2++)
+                if (((w2 >> lwks) & (wch - 1)) == tid) { mn = fminf(mn, s_rng[w2][0]); mx = fmaxf(mx, s_rng[w2][1]); }
+            float *dst = p.range_out + ((int64_t)nn * p.range_stride + (int64_t)b32 * p.parts + part) * 2;
+            dst[0] = mn;
+            dst[1] = mx;
+        }
+    }
+}
+
+// Weight rows in the order of the kernel above, one workgroup per channel (channels past the group's last: zeros), and the
+// sum of a row's integers.
+__global__ void __launch_bounds__(64) conv_words_kernel(const uint32_t *words, int64_t kp, int bits, int ocg, int cg, int kh, int kw, int ncb, int nsteps,
+                                                        int nch, int kwc, int8_t *cw, int32_t *qsum)
+{
+    const int lane = threadIdx.x, nb = ncb * 32, g = blockIdx.x / nb, n = blockIdx.x % nb;
+    const uint32_t *row = words + ((int64_t)g * ocg + n) * kp;
+    const bool c4 = kwc > 0;
+    int sum = 0;
+    for (int kc = lane; kc < 2 * nsteps; kc += 64) {
+        u32x4 o = {0, 0, 0, 0};
+        const int per = c4 ? kwc : nch, tap = kc / per, r = kc - tap * per;
+        if (n < ocg && tap < (c4 ? kh : kh * kw)) {
+#pragma unroll
+            for (int b = 0; b < 16; b++) {
+                const int c = c4 ? b & 3 : r * 16 + b, j = c4 ? r * 4 + (b >> 2) : tap % kw, i = c4 ? tap : tap / kw;
+                if (c >= cg || j >= kw) continue;
+                const int k = (c * kh + i) * kw + j;
+                const int q = bits == 4 ? ((int)(row[k >> 3] << (28 - 4 * (k & 7)))) >> 28 : (int)(int8_t)(row[k >> 2] >> (8 * (k & 3)));
+                o[b >> 2] |= (uint32_t)(q & 255) << (8 * (b & 3));
+                sum += q;
+            }
+        }
+        reinterpret_cast<u32x4 *>(cw)[((int64_t)(g * ncb + n / 32) * nsteps + (kc >> 1)) * 64 + (kc & 1) * 32 + (n & 31)] = o;
+    }
+    sum = wave_sum_i32(sum);
+    if (lane == 0 && n < ocg) qsum[g * ocg + n] = sum;
+}
+
+struct Geometry { int nch, kwc, nkc, nsteps, ncb; };   // ncb: blocks of 32 channels kept
+
+Geometry geometry(int64_t cg, int64_t ocg, int kh, int kw)
+{
+    Geometry q;
+    const bool c4 = cg <= 4;
+    q.nch = (int)((cg + 15) / 16);
+    q.kwc = c4 ? (kw + 3) / 4 : 0;
+    q.nkc = c4 ? kh * q.kwc : kh * kw * q.nch;
+    q.nsteps = (q.nkc + 1) / 2;
+    q.ncb = (int)((ocg + 31) / 32);
+    return q;
+}
+
+typedef FnnPatchShape Shape;
+
+// The rectangle of 32 * wpx pixels with the fewest patch values to load and outputs to finish; false: does not fit the LDS.
+bool place(const QConvArgs &p, const Geometry &q, Shape &s)
+{
+    const bool flat = p.kh == 1 && p.kw == 1 && p.pad == 0 && p.stride == 1;
+    const int64_t cg = p.c / p.groups, ocg = p.oc / p.groups, np = p.ho * p.wo;
+    const int64_t ho = flat ? 1 : p.ho, wo = flat ? np : p.wo;
+    double best = 0;
+    bool found = false;
+    for (int twl = 2; twl <= 9; twl++) {
+        const int tw = 1 << twl, th = 32 * s.wpx / tw;
+        if (th < 1 || (flat && th != 1)) continue;
+        const int64_t pw = (int64_t)(tw - 1) * p.stride + (int64_t)(p.kw - 1) * p.dil + 1, ph = (int64_t)(th - 1) * p.stride + (int64_t)(p.kh - 1) * p.dil + 1;
+        if (pw * ph > 1 << 16) continue;
+        const int64_t pp = pw * ph, tx = (wo + tw - 1) / tw, tiles = tx * ((ho + th - 1) / th);
+        const int64_t patch = cg <= 4 ? (pp * 4 + 4 * 4 * p.dil + 15) / 16 * 16 : pp * q.nch * 16;
+        const int64_t bytes = patch + (int64_t)s.wch * q.nsteps * 1024 + (q.nsteps * 8 + 15) / 16 * 16 + (s.wks > 1 ? 4096 * s.nw : 0);
+        if (bytes > MAX_LDS) continue;
+        // vector instructions: 8 a patch value, 18 an output; narrow rectangles use less of a cache line
+        const double cost = (double)tiles * ((double)((pp + 63) / 64 * 64) * (cg <= 4 ? cg : q.nch * 16) * 8 + 32.0 * s.wpx * ((ocg + 31) / 32 * 32) * 18) * (1 + 0.4 / tw);
+        if (found && cost >= best) continue;
+        best = cost; found = true;
+        s.twl = twl; s.th = th; s.pw = (int)pw; s.pp = (int)pp; s.tiles_x = (int)tx; s.tiles = (int)tiles; s.lds = (size_t)bytes;
+    }
+    return found;
+}
+
+// Microseconds expected of a shape, and of the operand kernel + GEMM pair (qgemm_i8.hip).  Fitted by least squares to kernel times of 239
+// layers (YOLOv8n's at 224 to 640 pixels a side and batches of 1 to 16, ResNet's at 1, 8 and 32) in some 35 shapes each; the shape with the
+// lowest figure is 3 % off the best on average, and 22 % below the kernels that were there before (4052 -> 3141 us over all layers).
+float patch_us(const QConvArgs &p, const Geometry &q, const Shape &s)
+{
+    const int64_t cg = p.c / p.groups, ocg = p.oc / p.groups;
+    const bool c4 = cg <= 4, split = !c4 && s.pp <= 32 && q.nch > 1;
+    const int groups = (s.pp + 63) / 64, units = c4 ? groups : (split ? (q.nch + 1) / 2 : groups * q.nch);
+    const float units_wave = (float)((units + s.nw - 1) / s.nw) * (c4 ? 0.25f : 1.0f);
+    const int steps = (q.nsteps + s.wks - 1) / s.wks, items = s.wks == 1 ? (ocg <= 16 ? 2 : 4) : (s.wks < 4 ? 4 / s.wks : 1);
+    const int64_t wgs = p.b * ((s.tiles + s.per - 1) / s.per) * s.gy, per_cu = (wgs + 255) / 256;
+    const int64_t resident = 160 * 1024 / (int64_t)(s.lds + 1300) < 16 / s.nw ? 160 * 1024 / (int64_t)(s.lds + 1300) : 16 / s.nw;
+    const float seq = (float)((per_cu + resident - 1) / resident) * s.per, all = (float)(per_cu * s.per);
+    const float issue = units_wave * 170 + steps * 12 + items * 75 + 40 + 15 * (s.wks - 1);   // vector instructions of a wave and rectangle
+    return 3.58f + seq * (0.271f + 0.285f * units_wave + 0.432f * ((steps + 3) / 4) + 0.397f * items + (s.wks > 1 ? 0.516f : 0.0f)) +
+           0.0307f * per_cu * s.wch * q.nsteps + 0.0000072f * all * s.pp * cg + 0.000149f * all * s.nw * issue + 0.102f * per_cu * s.nw;
+}
+float pair_us(const QConvArgs &p)
+{
+    const float rows = (float)(p.b * p.ho * p.wo), ocg = (float)(p.oc / p.groups);
+    const float stages = (float)(((p.c / p.groups) * p.kh * p.kw + 127) / 128);
+    const float wgs = ceilf(rows / 64) * ceilf(ocg / 64);
+    return 8.87f + 0.443f * stages + 41.8e-6f * rows * stages + 1.24e-6f * rows * ocg + 0.0741f * ceilf(wgs / 256) * stages + 0.0015625f * wgs * stages;
+}
+
+// false: the pair runs this convolution.  form: FNN_OPT_CONV_PATCH
+bool choose(const QConvArgs &p, const Geometry &q, int option, int form, Shape &best)
+{
+    // waves over pixels and over channels, all of them (the rest share K)
+    static const int8_t shapes[][3] = {{1, 1, 4}, {1, 1, 8}, {1, 2, 4}, {1, 2, 8}, {1, 4, 4}, {1, 4, 8}, {2, 1, 4}, {2, 1, 8}, {2, 2, 4}, {2, 4, 8}, {4, 1, 4}, {4, 1, 8}, {4, 2, 8}, {8, 1, 8}};
+    float us = 0;
+    bool found = false;
+    auto consider = [&](int wpx, int wch, int nw, int per) {
+        Shape s;
+        s.wpx = wpx; s.wch = wch; s.nw = nw; s.wks = nw / (wpx * wch); s.per = per;
+        if (q.ncb % wch) return;
+        s.gy = q.ncb / wch;
+        if (!place(p, q, s)) return;
+        // several rectangles a workgroup only where that leaves work for most CUs
+        for (int k = 1; k <= (per ? 1 : 4); k *= 2) {
+            if (!per) s.per = k;
+            if (!per && k > 1 && p.b * ((s.tiles + k - 1) / k) * s.gy < 200) break;
+            const float t = patch_us(p, q, s);
+            if (!found || t < us) { us = t; best = s; found = true; }
+        }
+    };
+    if (form) {
+        const int wpx = 1 << (form & 3), wch = 1 << ((form >> 2) & 3), nw = 4 << ((form >> 4) & 1);
+        if (wpx * wch <= nw) consider(wpx, wch, nw, 1 << ((form >> 5) & 3));
+        return found;
+    }
+    for (const auto &c : shapes) consider(c[0], c[1], c[2], 0);
+    // many channels and a long K under many pixels: every workgroup loads its channels' weights and quantises the pixels again, the pair does
+    // that once (16 x 128 x 40 x 40 -> 256 3x3 stride 2: 28.8 against 24.6 us; 32 x 256 x 40 x 40: 164 against 64)
+    return found && (option != 0 || us < pair_us(p) * 0.95f);
+}
+
+bool plan(const fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QConvArgs &p, Geometry &q, Shape &s)
+{
+    const int option = (int)fnn_ctx_option(ctx, FNN_OPT_CONV_IMPLICIT);
+    if (option == 2 || (w->dtype != FNN_DT_I8 && w->dtype != FNN_DT_I4) || p.x8 || p.payload_i4) return false;
+    const int64_t cg = p.c / p.groups, ocg = p.oc / p.groups, np = p.ho * p.wo;
+    // 32-bit offsets inside a slab of the input and inside an image of the output, whole tiles in 31 bits
+    if (p.c * p.h * p.w >= 1ll << 29 || p.oc * np >= 1ll << 29 || p.b * np >= 1ll << 30 || p.kh > 64 || p.kw > 64 || cg * p.kh * p.kw > 1 << 20) return false;
+    if (p.pad > 32767 || p.dil > 32767 || p.stride > 32767 || p.h > 1 << 24 || p.w > 1 << 24) return false;
+    q = geometry(cg, ocg, p.kh, p.kw);
+    return choose(p, q, option, (int)fnn_ctx_option(ctx, FNN_OPT_CONV_PATCH), s) && p.b * s.tiles < 1ll << 30;
+}
+
+template <bool KS, bool C4>
+hipError_t launch(const PatchArgs &p, dim3 grid, size_t lds, hipStream_t s)
+{
+    static std::atomic<uint64_t> raised{0};
+    if (lds > 48 * 1024) {
+        const hipError_t e = fnn_raise_lds_limit(raised, (const void *)conv_patch_kernel<KS, C4>, MAX_LDS);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((conv_patch_kernel<KS, C4>), grid, dim3(64u << p.lnw), lds, s, p);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+// What a quantised Conv2d keeps with its weight: the rows in the kernel's order (where this call may have memory for them; false: not
+// there, or in the order of another kernel geometry) and the sums of their integers.
+static bool conv_words(fnn_hip_ctx *ctx, hipStream_t stream, const fnn_hip_weight *w, int groups, int64_t cg, int kh, int kw)
+{
+    fnn_hip_weight *wm = const_cast<fnn_hip_weight *>(w);
+    if (wm->conv_words) return wm->conv_groups == groups && wm->conv_kh == kh && wm->conv_kw == kw;
+    const int64_t ocg = w->rows / groups;
+    const Geometry q = geometry(cg, ocg, kh, kw);
+    const size_t copy = (size_t)groups * q.ncb * q.nsteps * 1024;
+    if ((int64_t)groups * q.ncb * 32 > 1 << 30) return false;
+    // one allocation for the copy and, behind it, the row sums
+    void *mem = fnn_ctx_copy_memory(ctx, copy + (size_t)w->rows * 4 + 64);
+    if (!mem) return false;
+    int32_t *sums = reinterpret_cast<int32_t *>((char *)mem + copy);
+    hipLaunchKernelGGL(conv_words_kernel, dim3((unsigned)(groups * q.ncb * 32)), dim3(64), 0, stream, w->words, w->kp, w->dtype == FNN_DT_I4 ? 4 : 8, (int)ocg,
+                       (int)cg, kh, kw, q.ncb, q.nsteps, q.nch, q.kwc, (int8_t *)mem, sums);
+    if (hipGetLastError() != hipSuccess) {
+        (void)hipFree(mem);
+        return false;
+    }
+    wm->conv_words = (int8_t *)mem;
+    wm->conv_groups = groups; wm->conv_kh = kh; wm->conv_kw = kw;
+    if (!wm->row_qsum) { wm->row_qsum = sums; wm->row_qsum_shared = true; }
+    return true;
+}
+
+// Does the kernel take this convolution, and in which shape?  Builds the weight's copy on first use; where that cannot be had now, the
+// call is left to the pair.
+bool fnn_patch_conv_takes(fnn_hip_ctx *ctx, hipStream_t stream, const fnn_hip_weight *w, const QConvArgs &p, FnnPatchShape *s)
+{
+    Geometry q;
+    return plan(ctx, w, p, q, *s) && conv_words(ctx, stream, w, p.groups, p.c / p.groups, p.kh, p.kw);
+}
+
+// p.range_out: partial ranges of y are left when the pairs fit (ctx's out_parts says so)
+int fnn_patch_conv(fnn_hip_ctx *ctx, hipStream_t stream, const fnn_hip_weight *w, const QConvArgs &p, const FnnPatchShape &s)
+{
+    const Geometry q = geometry(p.c / p.groups, p.oc / p.groups, p.kh, p.kw);
+    const int64_t cg = p.c / p.groups, ocg = p.oc / p.groups, np = p.ho * p.wo;
+    const bool flat = p.kh == 1 && p.kw == 1 && p.pad == 0 && p.stride == 1, c4 = cg <= 4;
+    PatchArgs a;
+    a.kk = (float)(cg * p.kh * p.kw);
+    a.x_image = p.c * p.h * p.w; a.y_image = p.oc * np;
+    a.npairs = p.nparts > 0 ? p.nparts : 0; a.pair_stride = p.part_stride * p.groups; a.actq_stride = 4 * p.groups;
+    a.range_zero = p.range_zero; a.range_stride = p.range_out_stride;
+    a.cg = (int)cg; a.ocg = (int)ocg; a.act = p.act; a.wbits = p.wbits;
+    a.hh = flat ? 1 : (int)p.h; a.ww = flat ? (int)np : (int)p.w;
+    a.ho = flat ? 1 : (int)p.ho; a.wo = flat ? (int)np : (int)p.wo;
+    a.kw = p.kw; a.stride = p.stride; a.pad = p.pad; a.dil = p.dil;
+    a.twl = s.twl; a.th = s.th; a.tiles = s.tiles; a.per = s.per; a.parts = (s.tiles + s.per - 1) / s.per;
+    a.pw = s.pw; a.pp = s.pp; a.pgroups = (s.pp + 63) / 64; a.split = !c4 && s.pp <= 32 && q.nch > 1;
+    a.nch = q.nch; a.nsteps = q.nsteps; a.nkc = q.nkc;
+    auto log2of = [](int v) { int l = 0; while (1 << l < v) l++; return l; };
+    a.lnw = log2of(s.nw); a.lwch = log2of(s.wch); a.lwks = log2of(s.wks);
+    a.w_at = c4 ? (s.pp * 4 + 4 * 4 * p.dil + 15) / 16 * 16 : s.pp * q.nch * 16;
+    a.tab_at = a.w_at + s.wch * q.nsteps * 1024;
+    a.red_at = a.tab_at + (q.nsteps * 8 + 15) / 16 * 16;
+    a.dpw = fast_div((uint32_t)s.pw); a.dpg = fast_div((uint32_t)a.pgroups); a.dparts = fast_div((uint32_t)a.parts);
+    a.dtx = fast_div((uint32_t)s.tiles_x); a.dper = fast_div((uint32_t)(c4 ? q.kwc : q.nch)); a.dkw = fast_div((uint32_t)p.kw);
+    const bool with_sum = p.residual && p.sum_out;
+    a.vec4 = (a.wo % 4 == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 && (!p.acc_out || (reinterpret_cast<uintptr_t>(p.acc_out) & 15) == 0) &&
+              (!with_sum || ((reinterpret_cast<uintptr_t>(p.residual) | reinterpret_cast<uintptr_t>(p.sum_out)) & 15) == 0)) ? 1 : 0;
+    const int64_t parts = (int64_t)q.ncb * a.parts;
+    a.range_out = nullptr;
+    if (p.range_out && p.groups == 1 && parts <= p.range_out_stride) {
+        FnnRangeIo *rio = fnn_ctx_range_io(ctx);
+        rio->out_parts = (int)parts;
+        rio->out_tile_elems = 32 * (uint64_t)np;
+        rio->out_tile_pairs = a.parts;
+        a.range_out = p.range_out;
+    }
+    const dim3 grid((unsigned)(p.b * a.parts), (unsigned)s.gy);
+    for (int g = 0; g < p.groups; g++) {
+        const int64_t oc0 = g * ocg;
+        a.x = p.x + g * cg * p.h * p.w;
+        a.cw = w->conv_words + (int64_t)g * q.ncb * q.nsteps * 1024;
+        a.scales = p.scales + oc0; a.zeros = p.zeros + oc0; a.qsum = p.row_qsum + oc0;
+        a.bias = p.bias ? p.bias + oc0 : nullptr;
+        a.actq = p.actq + g * 4; a.pairs = p.minmax_partial + (int64_t)g * p.part_stride * 2;
+        a.y = p.y + oc0 * np;
+        a.acc_out = p.acc_out ? p.acc_out + oc0 * np : nullptr;
+        a.residual = with_sum ? p.residual + oc0 * np : nullptr;
+        a.sum_out = with_sum ? p.sum_out + oc0 * np : nullptr;
+        hipError_t e;
+        if (s.wks > 1) e = c4 ? launch<true, true>(a, grid, s.lds, stream) : launch<true, false>(a, grid, s.lds, stream);
+        else e = c4 ? launch<false, true>(a, grid, s.lds, stream) : launch<false, false>(a, grid, s.lds, stream);
+        if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
+    }
+    if (with_sum) fnn_ctx_residual_io(ctx)->used = 1;   // the epilogue stored y + residual as well
+    return FNN_OK;
+}

@@ -48,6 +48,7 @@ OPT_STREAM_SHAPE = 21
 OPT_DIGIT_PLANES = 22
 OPT_GEMV_TILE_MAJOR = 23
 OPT_FRAGMENT = 24
+OPT_CONV_PATCH = 25
 
 STATUS_NAMES = {0: "Ok", 1: "Dispatch", 2: "Memory", 3: "UnsupportedOp", 4: "Compilation"}
 

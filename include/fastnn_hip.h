@@ -131,10 +131,10 @@ enum {
     FNN_OPT_CONV_RANGES = 15,     /* plans: 1 (default) = the instruction that writes the input of a quantised Conv2d leaves   */
                                   /* partial (min, max) pairs per image behind and the convolution does not scan its input; 0 = */
                                   /* every convolution scans                                                               */
-    FNN_OPT_CONV_IMPLICIT = 16,   /* quantised Conv2d (I8 / I4 weights, f32 input): 1 = one implicit-GEMM kernel (im2col taps    */
-                                  /* fetched and quantised in the GEMM's operand registers, no int8 operand in memory), 2 = the */
-                                  /* operand kernel + GEMM pair, 3 = the fused kernel (a workgroup quantises 32 pixels once     */
-                                  /* into LDS and runs all output channels against them; K up to 1280), 0 (default) = by shape  */
+    FNN_OPT_CONV_IMPLICIT = 16,   /* quantised Conv2d (I8 / I4 weights, f32 input): 1 or 3 = one launch (a patch of the input        */
+                                  /* quantised once into LDS, no int8 operand in memory) wherever it fits, 2 = the operand kernel + */
+                                  /* GEMM pair, 0 (default) = whichever is expected to finish first.  The launch reads a second      */
+                                  /* device copy of the weight's integers, built with its first such call                            */
     FNN_OPT_FUSE_RESIDUAL = 17,   /* plans: 1 (default) = a MatMul or quantised Conv2d whose output the next instruction adds to  */
                                   /* another tensor stores that sum from its own last kernel where it can (the Add instruction   */
                                   /* is then skipped; same f32 addition, identical results), 0 = every Add runs as its own launch */
@@ -177,7 +177,10 @@ enum {
                                   /* blocks); a shape that does not exist for the call is ignored;                                  */
                                   /* (1 << 14) | w, w = 1, 2 or 4: I8, I4 and U4 weights on the large register tiles of three     */
                                   /* digit planes, w waves of a workgroup sharing a tile                                            */
-    FNN_OPT_COUNT = 25
+    FNN_OPT_CONV_PATCH = 25,      /* shape of that launch: 0 (default) = by rule, else 128 + log2 of the waves over pixels + 4 * log2  */
+                                  /* over channels + 16 (eight waves instead of four) + 32 * log2 of the rectangles of a workgroup; */
+                                  /* a shape that does not fit leaves the call to the pair                                          */
+    FNN_OPT_COUNT = 26
 };
 int fnn_hip_set_option(fnn_hip_ctx *ctx, int option, int64_t value);
 int fnn_hip_get_option(fnn_hip_ctx *ctx, int option, int64_t *value);
