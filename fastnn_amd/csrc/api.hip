@@ -661,6 +661,10 @@ int fnn_hip_qmatmul(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *a, i
                 int rc = fnn_frag_qmatmul(ctx, ctx->stream, w, p, flags, &handled);
                 if (rc) return rc;
             }
+            if (!handled) {
+                int rc = fnn_codebook_qmatmul(ctx, ctx->stream, w, p, flags, &handled);
+                if (rc) return rc;
+            }
             if (fma_first && !handled) HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_qgemv(w->dtype, p, ctx->stream, &handled));
             if (!handled) {   // (M <= 32 from 17 on and, for a long K over few columns, from 9 or 5; codebook type 5 .. 64)
                 int rc = fnn_stream_qmatmul(ctx, ctx->stream, w, p, flags, &handled);

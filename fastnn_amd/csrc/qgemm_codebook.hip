@@ -1,0 +1,285 @@
+// Codebook MatMul for a few activation rows, one launch.
+//
+//   out[m,n] = act(sum_blk scale[n,blk] * sum_{k in blk} table[q[n,k]] * A[m,k] + bias[n])        (blocks of 32 k-values)
+//
+// A workgroup of sixteen waves owns 16 weight rows over all of K, a wave a sixteenth of it, so that nothing is added up outside the
+// workgroup.  The words come as the fragment-major copy holds them, lane r + 16 p with the 16 bytes of row r that are block p of a
+// k block of 128; a 4x4 transpose over the lanes' four rows of 16 (four swaps) turns them into the operand of
+// v_mfma_f32_16x16x32_f16 whose 32 k-values are ONE block, so the block's scale multiplies the four sums of a product instead of
+// every weight.  A nibble looks up (f16 hi, f16 lo) of its table value in LDS (16 words: no bank conflicts), and the activations,
+// scaled by a power of two per row and piece of K, are f16 hi + lo as well: all four products are formed.  Up to eight rows the hi and
+// the lo parts share the 16 columns of the other operand, each lane converts four of its row's eight values and fetches the
+// others' halves from the lane eight on.
+//
+// Bound: bytes into a CU (16 rows of words and scales and all activations: 4096 x 4096 with 8 rows 168 KB a workgroup, 4 us of 11) and
+// vector instructions (720 a wave: look-ups 2.5 a value, conversion 3.5 an activation).  It has no launch or tail for a K split, so
+// it is ahead of the streaming kernel where a round of workgroups covers the rows and K is not long, and of the tile kernels
+// wherever K is ragged.  Eight waves with twice the piece (200 registers) measured the same at 4096 x 4096 and 25 % slower at
+// 1024 x 1024; two or three blocks of rows a workgroup spill.
+#include "dech.h"
+#include "mfma.h"
+#include "qgemm_frag.h"
+#include "range_io.h"
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+namespace {
+
+constexpr int NW = 16;
+constexpr float LO_UP = 2048.0f, LO_DOWN = 1.0f / 2048.0f;   // the lo activation term is stored scaled by 2^11
+
+struct CodebookArgs {
+    const uint32_t *wf;          // weight words: the fragment-major copy (kp 0) or the registered rows of kp words
+    const float *bscales, *codebook, *a, *bias;
+    float *out;
+    const float *residual;       // non-null: sum_out[m,n] = out[m,n] + residual[m,n] as well
+    float *sum_out;
+    int m, n, k, kblocks, bpr, kp, act;
+    int vec4;                    // 16-byte accesses along n
+};
+
+// R16: 9 to 16 activation rows (hi and lo as two operands), else up to 8 (hi in columns 0 - 7, lo in 8 - 15)
+template <bool R16>
+__global__ void __launch_bounds__(NW * 64) qgemm_codebook_kernel(CodebookArgs p)
+{
+    constexpr int PB = R16 ? 1 : 2;            // k blocks of a piece: their activations stay in registers
+    constexpr int STEPS = PB * 4, VALS = R16 ? 8 : 4;
+    __shared__ __attribute__((aligned(16))) uint32_t table[16];   // hi | lo << 16
+    __shared__ int s_exp;
+    __shared__ __attribute__((aligned(16))) float s_sc[NW][PB][64];
+    __shared__ f32x4 red[NW][64];
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nt = (int)blockIdx.x;
+    const int per = (p.kblocks + NW - 1) / NW, b0 = wv * per, b1 = min(b0 + per, p.kblocks);
+
+    const uint32_t *w0 = frag_row_at(p.wf, p.kp, p.n, p.kblocks, nt, r, q);
+    const int wstep = p.kp ? 16 : 256;
+    const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.a), 0, (int)((uint32_t)p.m * (uint32_t)p.k * 4u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t sbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.bscales), 0, (int)((uint32_t)p.n * (uint32_t)p.bpr * 4u), 0x00020000);
+    const int half = R16 ? 0 : r >> 3, row = R16 ? r : r & 7;
+
+    u32x4 w[PB];
+    float sc[PB], x[STEPS][VALS];
+    auto request = [&](int b) {
+#pragma unroll
+        for (int t = 0; t < PB; t++) w[t] = *reinterpret_cast<const frag_u32x4 *>(w0 + (int64_t)min(b + t, b1 - 1) * wstep);
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) {
+            const int k0 = b * 128 + s * 32 + q * 8 + half * 4;
+            const uint32_t at = row < p.m && k0 < p.k && b + s / 4 < b1 ? (uint32_t)(row * p.k + k0) * 4u : 0xffffffe0u;   // (else: zeros)
+            const u32x4 t0 = __builtin_amdgcn_raw_buffer_load_b128(xbuf, at, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) x[s][i] = __uint_as_float(t0[i]);
+            if constexpr (R16) {
+                const u32x4 t1 = __builtin_amdgcn_raw_buffer_load_b128(xbuf, at, 16, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[s][4 + i] = __uint_as_float(t1[i]);
+            }
+        }
+        // one scale a lane and k block: row lane >> 2, block lane & 3
+#pragma unroll
+        for (int t = 0; t < PB; t++) {
+            const int n = nt * 16 + (lane >> 2), blk = (b + t) * 4 + (lane & 3);
+            sc[t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(sbuf, n < p.n && blk < p.bpr ? (uint32_t)(n * p.bpr + blk) * 4u : 0xffffffe0u, 0, 0));
+        }
+    };
+    if (b0 < b1) request(b0);
+    if (wv == NW - 1) {
+        const int ex = dech::codebook_exp(p.codebook);
+        if (lane < 16) {
+            const float v = ldexpf(p.codebook[lane], ex);
+            const _Float16 h = (_Float16)v, l = (_Float16)(v - (float)h);
+            table[lane] = (uint32_t)__builtin_bit_cast(uint16_t, h) | ((uint32_t)__builtin_bit_cast(uint16_t, l) << 16);
+        }
+        if (lane == 0) s_exp = ex;
+    }
+    __syncthreads();
+
+    f32x4 total = {0.f, 0.f, 0.f, 0.f};
+    for (int b = b0; b < b1; b += PB) {
+        if (b > b0) request(b);
+        // ---- the activations of the piece: one power of two per row, f16 hi + lo
+        if (p.k % 4 != 0 && b + PB >= p.kblocks) {   // (uniform) the last values of a row run into the next row: they do not count
+#pragma unroll
+            for (int s = 0; s < STEPS; s++)
+#pragma unroll
+                for (int i = 0; i < VALS; i++) x[s][i] = b * 128 + s * 32 + q * 8 + half * 4 + i < p.k ? x[s][i] : 0.0f;
+        }
+        float mx = 0.0f;
+#pragma unroll
+        for (int s = 0; s < STEPS; s++)
+#pragma unroll
+            for (int i = 0; i < VALS; i += 2) mx = fmaxf(mx, fmaxf(fabsf(x[s][i]), fabsf(x[s][i + 1])));
+        if constexpr (!R16) mx = fmaxf(mx, dpp_f32<0x128>(mx));   // (row_ror:8) the lane with the other half of the values
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        int e = 0;
+        if (mx > 0.0f && mx < __builtin_huge_valf()) {
+            int ex;
+            (void)frexpf(mx, &ex);
+            e = 15 - ex;
+        }
+        f16x8 xh[STEPS], xl[R16 ? STEPS : 1];   // up to eight rows: xh is this lane's operand, hi or lo
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) {
+            f16x2 h[VALS / 2], l[VALS / 2];
+#pragma unroll
+            for (int i = 0; i < VALS / 2; i++) {
+                const f32x2 v = {ldexpf(x[s][2 * i], e), ldexpf(x[s][2 * i + 1], e)};
+                h[i] = __builtin_convertvector(v, f16x2);
+                const f32x2 d = {fmaf((float)h[i][0], -LO_UP, v[0] * LO_UP), fmaf((float)h[i][1], -LO_UP, v[1] * LO_UP)};   // (exact)
+                l[i] = __builtin_convertvector(d, f16x2);
+            }
+            if constexpr (R16) {
+#pragma unroll
+                for (int i = 0; i < 8; i++) { xh[s][i] = h[i / 2][i & 1]; xl[s][i] = l[i / 2][i & 1]; }
+            } else {
+                uint32_t hw[2], lw[2], got[2];
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    hw[i] = __builtin_bit_cast(uint32_t, h[i]);
+                    lw[i] = __builtin_bit_cast(uint32_t, l[i]);
+                    got[i] = (uint32_t)dpp_i32<0x128>((int)(half ? hw[i] : lw[i]));
+                }
+                const u32x4 o = half ? u32x4{got[0], got[1], lw[0], lw[1]} : u32x4{hw[0], hw[1], got[0], got[1]};
+                xh[s] = __builtin_bit_cast(f16x8, o);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < PB; t++) s_sc[wv][t][(lane & 3) * 16 + (lane >> 2)] = sc[t];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < PB; t++) {
+            if (b + t >= b1) break;   // (wave-uniform)
+            // word i of block q  ->  word q of block i
+            const auto a0 = __builtin_amdgcn_permlane32_swap(w[t][0], w[t][2], false, false);
+            const auto a1 = __builtin_amdgcn_permlane32_swap(w[t][1], w[t][3], false, false);
+            const auto c0 = __builtin_amdgcn_permlane16_swap(a0[0], a1[0], false, false);
+            const auto c1 = __builtin_amdgcn_permlane16_swap(a0[1], a1[1], false, false);
+            const uint32_t wd[4] = {c0[0], c0[1], c1[0], c1[1]};
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                uint32_t d[8], hi4[4], lo4[4];
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const uint32_t off = (((i & 1) ? wd[u] >> 2 : wd[u] << 2) & 0x3c3c3c3cu) >> (8 * (i >> 1)) & 0xffu;   // four bytes an entry
+                    d[i] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(table) + off);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    hi4[i] = __builtin_amdgcn_perm(d[2 * i + 1], d[2 * i], 0x05040100u);
+                    lo4[i] = __builtin_amdgcn_perm(d[2 * i + 1], d[2 * i], 0x07060302u);
+                }
+                if ((b + t + 1) * 128 > p.k) {   // (uniform) nibbles past the row: no table value, it might be not a number
+                    const int left = p.k - ((b + t) * 128 + u * 32 + q * 8);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t keep = left >= 2 * i + 2 ? ~0u : (left == 2 * i + 1 ? 0xffffu : 0u);
+                        hi4[i] &= keep;
+                        lo4[i] &= keep;
+                    }
+                }
+                const f16x8 wh = __builtin_bit_cast(f16x8, u32x4{hi4[0], hi4[1], hi4[2], hi4[3]});
+                const f16x8 wl = __builtin_bit_cast(f16x8, u32x4{lo4[0], lo4[1], lo4[2], lo4[3]});
+                f32x4 v = __builtin_amdgcn_mfma_f32_16x16x32_f16(wl, xh[t * 4 + u], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                v = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh, xh[t * 4 + u], v, 0, 0, 0);
+                if constexpr (R16) {
+                    f32x4 v2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(wl, xl[t * 4 + u], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    v2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh, xl[t * 4 + u], v2, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) v[i] = fmaf(v2[i], LO_DOWN, v[i]);
+                }
+                const f32x4 s4 = *reinterpret_cast<const f32x4 *>(&s_sc[wv][t][u * 16 + 4 * q]);   // weight rows 4 q + (0 .. 3)
+#pragma unroll
+                for (int i = 0; i < 4; i++) sum[i] = fmaf(s4[i], v[i], sum[i]);
+            }
+            __builtin_amdgcn_sched_barrier(0);   // (else the look-ups of all blocks are hoisted, and spill)
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) total[i] += ldexpf(sum[i], -e);
+    }
+
+    // ---- the parts of K meet; lane: activation row (column of the product) r, weight rows 4 q + (0 .. 3)
+    red[wv][lane] = total;
+    const int n0 = nt * 16 + 4 * q;
+    float bi[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p.bias && wv == 0)
+#pragma unroll
+        for (int i = 0; i < 4; i++) bi[i] = p.bias[min(n0 + i, p.n - 1)];
+    __syncthreads();
+    if (wv != 0 || row >= p.m || half || n0 >= p.n) return;
+    f32x4 v = red[0][lane];
+#pragma unroll
+    for (int z = 1; z < NW; z++) v += red[z][lane];
+    if constexpr (!R16) {
+        f32x4 l = red[0][lane + 8];
+#pragma unroll
+        for (int z = 1; z < NW; z++) l += red[z][lane + 8];
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = fmaf(l[i], LO_DOWN, v[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        v[i] = ldexpf(v[i], -s_exp);
+        if (p.bias) v[i] = v[i] + bi[i];
+        v[i] = fnn_activation(v[i], p.act);
+    }
+    const int64_t at = (int64_t)row * p.n + n0;
+    if (p.vec4) {
+        *reinterpret_cast<f32x4 *>(p.out + at) = v;
+        if (p.residual) *reinterpret_cast<f32x4 *>(p.sum_out + at) = v + *reinterpret_cast<const f32x4 *>(p.residual + at);
+        return;
+    }
+    for (int i = 0; i < 4 && n0 + i < p.n; i++) {
+        p.out[at + i] = v[i];
+        if (p.residual) p.sum_out[at + i] = v[i] + p.residual[at + i];
+    }
+}
+
+// Microseconds expected here, and of the kernels behind: the streaming kernel (K a multiple of 128) or the tiles that decode the nibbles.
+// Fitted to 420 drawn calls of 5 to 16 rows, weights from memory (8, 14 and 6 % mean error).  What takes time here is a round of workgroups over
+// the CUs, the pieces of a wave and the activations, which every workgroup reads whole: 4096 x 4096 from 5 to 8 rows 11.0 -> 12.1 us.
+float here_us(int64_t m, int64_t n, int64_t k)
+{
+    const int64_t kblocks = (k + 127) / 128, per = (kblocks + NW - 1) / NW, tiles = (n + 15) / 16, rounds = (tiles + 255) / 256;
+    return 1.42f + (float)rounds * (2.56f + (m <= 8 ? 0.848f : 0.124f) * (float)per + 1.267e-4f * (float)(m * k)) + 2.82e-4f * (float)(tiles * kblocks);
+}
+float others_us(int64_t m, int64_t n, int64_t k)
+{
+    const float nk = (float)(n * k) / 1e6f, ks = (float)k / 1e3f;
+    return k % 128 == 0 ? 6.05f + 0.299f * nk + 0.738f * ks : 10.97f + 0.390f * nk + 1.629f * ks + 4.86e-6f * (float)(m * n);
+}
+
+}  // namespace
+
+int fnn_codebook_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, bool *handled)
+{
+    *handled = false;
+    // (up to four rows the FMA kernels add in f32 from exact products: 1.0e-7 off against 64 bits, 1.5e-7 here and in the kernels behind)
+    if (w->dtype != FNN_DT_I4CB || q.m < 5 || q.m > 16 || q.qblock != 32 || q.as_written || q.n != w->rows || q.k != w->inner) return FNN_OK;
+    if (flags & (FNN_FLAG_ACT_F16_SINGLE | FNN_FLAG_ACT_QUANT | FNN_FLAG_FORCE_GENERIC | FNN_FLAG_PREFER_FMA)) return FNN_OK;
+    if (fnn_ctx_option(ctx, FNN_OPT_FRAGMENT) != 0 || fnn_ctx_option(ctx, FNN_OPT_CODEBOOK_EXPANDED) != 0 || !fnn_frag_options_untouched(ctx)) return FNN_OK;
+    // 32-bit buffer offsets
+    if (q.n < 1 || q.k < 1 || q.m * q.k >= 1ll << 28 || q.n * q.bpr >= 1ll << 28 || q.n >= 1ll << 24) return FNN_OK;
+    // (the margin: where the two are about equal what was there stays.  Of the drawn calls 0.7 % then lose more than 5 %, the worst 1.12 times; all
+    // together take 0.79 of the time: 8 x 3072 x 3072 13.0 -> 9.5 us, 8 x 1003 x 3333 14.1 -> 6.7, 16 x 1024 x 1024 7.8 -> 6.0)
+    if (here_us(q.m, q.n, q.k) > (q.k % 128 == 0 ? 0.90f : 0.97f) * others_us(q.m, q.n, q.k)) return FNN_OK;
+    CodebookArgs p = {};
+    p.kblocks = (int)((w->kp + 15) / 16);
+    if (int rc = fnn_frag_words(ctx, s, w, p.kblocks, &p.wf, &p.kp)) return rc;
+    p.bscales = q.scales; p.codebook = q.codebook; p.a = q.a; p.bias = q.bias; p.out = q.out;
+    p.m = (int)q.m; p.n = (int)q.n; p.k = (int)q.k; p.bpr = (int)q.bpr; p.act = q.act;
+    fnn_take_residual(ctx, q.out, q.m * q.n, &p.residual, &p.sum_out);
+    p.vec4 = p.n % 4 == 0 && ((reinterpret_cast<uintptr_t>(p.out) | reinterpret_cast<uintptr_t>(p.residual) | reinterpret_cast<uintptr_t>(p.sum_out)) & 15) == 0;
+    const dim3 grid((unsigned)((p.n + 15) / 16)), block(NW * 64);
+    if (q.m > 8) hipLaunchKernelGGL(qgemm_codebook_kernel<true>, grid, block, 0, s, p);
+    else hipLaunchKernelGGL(qgemm_codebook_kernel<false>, grid, block, 0, s, p);
+    if (const hipError_t e = hipGetLastError(); e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
+    *handled = true;
+    return FNN_OK;
+}
