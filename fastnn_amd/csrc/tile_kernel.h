@@ -4,6 +4,7 @@
 // qgemm_tiled.hip for the design.
 #pragma once
 #include <climits>
+#include <type_traits>
 
 struct TileArgs {
     const uint32_t *words;
@@ -87,6 +88,49 @@ template <int N>
 __device__ __forceinline__ void wait_loads_but()
 {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// The results of a wave, o[r][tn] = row m0 + 8 (r / 4) + r % 4 + 4 h, column n0 + 32 tn + lr: bias, activation, stores, each in a pass of
+// its own with its (uniform) test in front.  With all of them inside one loop an output was some 60 instructions, 15 to 40 KB of code
+// that a wave fetches and runs once while its matrix core idles.
+template <int R, int TN>
+__device__ __forceinline__ void tile_finish(float (&o)[R][TN], float *dst, int64_t m0, int64_t n0, int64_t m, int64_t n, const float (&bi)[TN], bool has_bias,
+                                            int act, int lr, int h)
+{
+    if (has_bias) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int tn = 0; tn < TN; tn++) o[r][tn] = o[r][tn] + bi[tn];
+    }
+    auto activate = [&](auto a) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int tn = 0; tn < TN; tn++) o[r][tn] = fnn_activation(o[r][tn], decltype(a)::value);
+    };
+    if (act == FNN_ACT_SILU) activate(std::integral_constant<int, FNN_ACT_SILU>{});
+    else if (act == FNN_ACT_GELU) activate(std::integral_constant<int, FNN_ACT_GELU>{});
+    else if (act == FNN_ACT_RELU) activate(std::integral_constant<int, FNN_ACT_RELU>{});
+    float *first = dst + m0 * n + n0;
+    const uint32_t lane = (uint32_t)(4 * h) * (uint32_t)n + (uint32_t)lr;
+    if (m0 + 2 * R <= m && n0 + 32 * TN <= n) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            float *row = first + (int64_t)((r >> 2) * 8 + (r & 3)) * n;   // (uniform: scalar arithmetic)
+#pragma unroll
+            for (int tn = 0; tn < TN; tn++) row[lane + tn * 32] = o[r][tn];
+        }
+    } else {
+        const int rows = (int)(m - m0 < 2 * R ? m - m0 : 2 * R) - 4 * h, cols = (int)(n - n0 < 32 * TN ? n - n0 : 32 * TN) - lr;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            float *row = first + (int64_t)((r >> 2) * 8 + (r & 3)) * n;
+#pragma unroll
+            for (int tn = 0; tn < TN; tn++)
+                if ((r >> 2) * 8 + (r & 3) < rows && tn * 32 < cols) row[lane + tn * 32] = o[r][tn];
+        }
+    }
 }
 
 // INT8 = false: f16 operands, v_mfma_f32_32x32x16_f16, 64 k-values per stage, float epilogue.
@@ -545,118 +589,59 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
 
     // ---- epilogue.  acc[i] of a 32x32 block: row (i/4)*8 + h*4 + i%4, column lr.  With hi/lo
     // operands a block holds 16 output rows: hi in rows 0..15 (i < 8), lo in rows 16..31 (i + 8).
-    if constexpr (INT8 && DIG == 3) {
-        // slab q of the wave (operand rows 8q .. 8q + 7, q = tm*4 + i/4) = plane q % 3 of the activation rows
-        // 8 (q/3) .. + 7; a lane holds rows 4h + t of every slab in acc[q / 4][tn][(q % 4) * 4 + t]
-        constexpr int SHIFT = (DT == FNN_DT_I4) ? 4 : 0;   // 4-bit signed lanes entered as 16*q
-        constexpr int GR = TM * 4 / 3;                      // groups of 8 activation rows per wave
-        const int64_t mrow0 = ((int64_t)mt * BM + wm * TM * 32) / 3;
+    const int wvu = __builtin_amdgcn_readfirstlane(wv), wmu = wvu / WGN, wnu = wvu % WGN;
+    const int64_t ncol0 = n0 + wnu * TN * 32;   // the wave's first column
+    const int64_t ncol = ncol0 + lr;            // this lane's first
+    if constexpr (INT8 && DIG > 0) {
+        // Three planes: slab q of the wave (operand rows 8q .. 8q + 7, q = tm*4 + i/4) = plane q % 3 of the activation rows 8 (q/3) .. + 7; a
+        // lane holds rows 4h + t of every slab in acc[q / 4][tn][(q % 4) * 4 + t].  Two and four planes: row r of the lane in block tm and plane j =
+        // block row j*RPB + (r/4)*8 + h*4 + r%4 = (i/4)*8 + h*4 + i%4
+        constexpr int RPB = 32 / DIG;
+        constexpr int NR = RPB / 2;                             // activation rows of a 32-row block that a lane holds (two and four planes)
+        constexpr int R = DIG == 3 ? TM * 16 / 3 : TM * NR;     // ... and of the wave's rows
+        constexpr int SHIFT = (DT == FNN_DT_I4) ? 4 : 0;        // 4-bit signed lanes entered as 16*q
+        const int64_t mrow0 = DIG == 3 ? ((int64_t)mt * BM + wmu * TM * 32) / 3 : ((int64_t)mt * (BM / 32) + wmu * TM) * RPB;
         const bool split = p.splits > 1;
         float sc[TN], zp[TN], bi[TN];
 #pragma unroll
         for (int tn = 0; tn < TN; tn++) {
-            const int64_t n = n0 + (wn * TN + tn) * 32 + lr;
+            const int64_t n = ncol + tn * 32;
             const bool ok = n < p.n && !split;
             sc[tn] = ok ? p.scales[n] : 0.0f;
             zp[tn] = ok ? p.zeros[n] : 0.0f;
             bi[tn] = (ok && p.bias) ? p.bias[n] : 0.0f;
         }
-        int rexp[GR][4];
-        float rxs[GR][4];
+        const int last = (int)(p.m - 1 - mrow0);
+        if (last < 0) return;   // (padding rows only)
+        int rexp[R];
+        float rxs[R];
+        const int *rexp0 = p.rexp + mrow0;
+        const float *xsum0 = p.xsum + mrow0;
 #pragma unroll
-        for (int u = 0; u < GR; u++)
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                int64_t m = mrow0 + u * 8 + h * 4 + t;
-                if (m > p.m - 1) m = p.m - 1;
-                rexp[u][t] = p.rexp[m];
-                rxs[u][t] = split ? 0.0f : p.xsum[m];
-            }
-#pragma unroll
-        for (int u = 0; u < GR; u++)
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const int64_t m = mrow0 + u * 8 + h * 4 + t;
-                if (m >= p.m) continue;
-                const int e = rexp[u][t];
-                const bool bad = e == INT_MIN;      // the row holds a non-finite activation
-#pragma unroll
-                for (int tn = 0; tn < TN; tn++) {
-                    const int64_t n = n0 + (wn * TN + tn) * 32 + lr;
-                    if (n >= p.n) continue;
-                    float v = 0.0f;
-#pragma unroll
-                    for (int j = 2; j >= 0; j--) {
-                        const int q = 3 * u + j;
-                        v = fmaf(v, 256.0f, (float)__float_as_int(acc[q >> 2][tn][(q & 3) * 4 + t]));
-                    }
-                    const float d = bad ? __builtin_nanf("") : ldexpf(v, -e - SHIFT);
-                    if (split) {
-                        p.part[((int64_t)z * p.m + m) * p.n + n] = d;
-                    } else {
-                        float o = d * sc[tn] + zp[tn] * rxs[u][t];
-                        if (p.bias) o = o + bi[tn];
-                        p.out[m * p.n + n] = fnn_activation(o, p.act);
-                    }
-                }
-            }
-        return;
-    } else if constexpr (INT8 && DIG > 0) {
-        constexpr int RPB = 32 / DIG;        // activation rows per 32-row block
-        constexpr int NR = RPB / 2;          // ... of which a lane holds NR (the other half belongs to lanes h ^ 1)
-        constexpr int SHIFT = (DT == FNN_DT_I4) ? 4 : 0;   // 4-bit signed lanes entered as 16*q
-        const int64_t mrow0 = ((int64_t)mt * (BM / 32) + wm * TM) * RPB;
-        const bool split = p.splits > 1;
-        float sc[TN], zp[TN], bi[TN];
-#pragma unroll
-        for (int tn = 0; tn < TN; tn++) {
-            const int64_t n = n0 + (wn * TN + tn) * 32 + lr;
-            const bool ok = n < p.n && !split;
-            sc[tn] = ok ? p.scales[n] : 0.0f;
-            zp[tn] = ok ? p.zeros[n] : 0.0f;
-            bi[tn] = (ok && p.bias) ? p.bias[n] : 0.0f;
+        for (int r = 0; r < R; r++) {
+            const int at = min((r >> 2) * 8 + (r & 3) + 4 * h, last);
+            rexp[r] = rexp0[at];
+            rxs[r] = split ? 0.0f : xsum0[at];
         }
-        // acc index of (row r of the lane, plane j): block row j*RPB + (r/4)*8 + h*4 + r%4 = (i/4)*8 + h*4 + i%4
-        int rexp[TM][NR];
-        float rxs[TM][NR];
+        float o[R][TN];
 #pragma unroll
-        for (int tm = 0; tm < TM; tm++)
+        for (int r = 0; r < R; r++) {
+            const bool bad = rexp[r] == INT_MIN;      // the row holds a non-finite activation
 #pragma unroll
-            for (int r = 0; r < NR; r++) {
-                int64_t m = mrow0 + tm * RPB + (r / 4) * 8 + h * 4 + (r % 4);
-                if (m > p.m - 1) m = p.m - 1;
-                rexp[tm][r] = p.rexp[m];
-                rxs[tm][r] = split ? 0.0f : p.xsum[m];
-            }
+            for (int tn = 0; tn < TN; tn++) {
+                float v = 0.0f;
 #pragma unroll
-        for (int tm = 0; tm < TM; tm++)
-#pragma unroll
-            for (int r = 0; r < NR; r++) {
-                const int64_t m = mrow0 + tm * RPB + (r / 4) * 8 + h * 4 + (r % 4);
-                if (m >= p.m) continue;
-                const int e = rexp[tm][r];
-                const bool bad = e == INT_MIN;      // the row holds a non-finite activation
-#pragma unroll
-                for (int tn = 0; tn < TN; tn++) {
-                    const int64_t n = n0 + (wn * TN + tn) * 32 + lr;
-                    if (n >= p.n) continue;
-                    float v = 0.0f;
-#pragma unroll
-                    for (int j = DIG - 1; j >= 0; j--) {
-                        const int i = j * (RPB / 8) * 4 + (r / 4) * 4 + (r % 4);
-                        const float bits = acc[tm][tn][i];
-                        v = fmaf(v, 256.0f, (float)__float_as_int(bits));
-                    }
-                    float d = bad ? __builtin_nanf("") : ldexpf(v, -e - SHIFT);
-                    if (split) {
-                        p.part[((int64_t)z * p.m + m) * p.n + n] = d;
-                    } else {
-                        float o = d * sc[tn] + zp[tn] * rxs[tm][r];
-                        if (p.bias) o = o + bi[tn];
-                        p.out[m * p.n + n] = fnn_activation(o, p.act);
-                    }
+                for (int j = DIG - 1; j >= 0; j--) {
+                    const int q = 3 * (r >> 2) + j;   // three planes
+                    const float bits = DIG == 3 ? acc[q >> 2][tn][(q & 3) * 4 + (r & 3)] : acc[r / NR][tn][j * (RPB / 8) * 4 + r % NR];
+                    v = fmaf(v, 256.0f, (float)__float_as_int(bits));
                 }
+                const float d = bad ? __builtin_nanf("") : ldexpf(v, -rexp[r] - SHIFT);
+                o[r][tn] = split ? d : d * sc[tn] + zp[tn] * rxs[r];
             }
+        }
+        tile_finish<R, TN>(o, split ? p.part + (int64_t)z * p.m * p.n : p.out, mrow0, ncol0, p.m, p.n, bi, p.bias != nullptr && !split,
+                           split ? (int)FNN_ACT_NONE : p.act, lr, h);
         return;
     } else if constexpr (INT8 && CONV) {
         __syncthreads();   // the row tables
@@ -766,48 +751,41 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
         }
         return;
     } else if constexpr (INT8) {
-        const int64_t mrow = ((int64_t)mt * (BM / 32) + wm * TM) * 32;
+        const int64_t mrow = ((int64_t)mt * (BM / 32) + wmu * TM) * 32;
         if (!FP8 && !p.c_i32) {   // (uniform) one pass instead of a matrix of sums written and read again
             const float sa = p.act_q[0], za = p.act_q[1], kza = (float)p.k_values * za;
             float sw[TN], zw[TN], zws[TN], bs[TN];
 #pragma unroll
             for (int tn = 0; tn < TN; tn++) {
-                int64_t n = n0 + (wn * TN + tn) * 32 + lr;
+                int64_t n = ncol + tn * 32;
                 if (n > p.n - 1) n = p.n - 1;
                 sw[tn] = p.scales[n];
                 zw[tn] = p.zeros[n];
                 zws[tn] = za * (float)p.word_sum[n];
                 bs[tn] = p.bias ? p.bias[n] : 0.0f;
             }
-            const bool has_bias = p.bias != nullptr;
+            constexpr int R = TM * 16;
+            const int last = (int)(p.m - 1 - mrow);
+            if (last < 0) return;   // (padding rows only)
+            const int32_t *code_sum = p.code_sum + mrow;
+            float o[R][TN];
 #pragma unroll
-            for (int tm = 0; tm < TM; tm++) {
-                int qs[16];
+            for (int r = 0; r < R; r++) {
+                const float input_sum = (float)code_sum[min((r >> 2) * 8 + (r & 3) + 4 * h, last)] * sa + kza;
 #pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    int64_t m = mrow + tm * 32 + (i / 4) * 8 + h * 4 + (i % 4);
-                    qs[i] = p.code_sum[m > p.m - 1 ? p.m - 1 : m];
-                }
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int64_t m = mrow + tm * 32 + (i / 4) * 8 + h * 4 + (i % 4);
-                    if (m >= p.m) continue;
-                    const float input_sum = (float)qs[i] * sa + kza;
-#pragma unroll
-                    for (int tn = 0; tn < TN; tn++) {
-                        const int64_t n = n0 + (wn * TN + tn) * 32 + lr;
-                        if (n >= p.n) continue;
-                        const float bits = acc[tm][tn][i];
-                        int a = __float_as_int(bits);
-                        if constexpr (DT == FNN_DT_I4) a >>= 4;
-                        const float dot = za != 0.0f ? (float)a * sa + zws[tn] : (float)a * sa;
-                        float v = dot * sw[tn] + zw[tn] * input_sum;
-                        if (has_bias) v = v + bs[tn];
-                        p.out[m * p.n + n] = fnn_activation(v, p.act);
-                        if (p.acc_out) p.acc_out[m * p.n + n] = za != 0.0f ? 0 : a;
+                for (int tn = 0; tn < TN; tn++) {
+                    const float bits = acc[r >> 4][tn][r & 15];
+                    int a = __float_as_int(bits);
+                    if constexpr (DT == FNN_DT_I4) a >>= 4;
+                    const float dot = za != 0.0f ? (float)a * sa + zws[tn] : (float)a * sa;
+                    o[r][tn] = dot * sw[tn] + zw[tn] * input_sum;
+                    if (p.acc_out) {
+                        const int64_t m = mrow + (r >> 2) * 8 + (r & 3) + 4 * h, n = ncol + tn * 32;
+                        if (m < p.m && n < p.n) p.acc_out[m * p.n + n] = za != 0.0f ? 0 : a;
                     }
                 }
             }
+            tile_finish<R, TN>(o, p.out, mrow, ncol0, p.m, p.n, bs, p.bias != nullptr, p.act, lr, h);
             return;
         }
 #pragma unroll
@@ -830,12 +808,15 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
     }
     constexpr int RPB = PRECISE ? 16 : 32;           // output rows per block
     constexpr int NI = PRECISE ? 8 : 16;
-    const int64_t mrow0 = ((int64_t)mt * (BM / 32) + wm * TM) * RPB;
+    constexpr int R = TM * NI;
+    const int64_t mrow0 = ((int64_t)mt * (BM / 32) + wmu * TM) * RPB;
+    const int last = (int)(p.m - 1 - mrow0);
+    if (last < 0) return;   // (padding rows only)
     float sc[TN], zp[TN], bi[TN], um[TN];
     const bool split = p.splits > 1;
 #pragma unroll
     for (int tn = 0; tn < TN; tn++) {
-        const int64_t n = n0 + (wn * TN + tn) * 32 + lr;
+        const int64_t n = ncol + tn * 32;
         const bool ok = n < p.n && !split;
         if constexpr (CB) {   // block scales are applied in the loop; what is left is the table's power of two
             sc[tn] = ok ? ldexpf(1.0f, -cb_exp) : 0.0f;
@@ -847,48 +828,40 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
         bi[tn] = (ok && p.bias) ? p.bias[n] : 0.0f;
         um[tn] = (!PRECISE && ok && p.umean) ? p.umean[n] : 0.0f;
     }
-    // row constants of every output row this lane holds, requested together (clamped rows, masked
-    // later) so that their latencies overlap instead of chaining behind the stores
-    int rexp[TM][NI];
-    float rxs[TM][NI], rcorr[TM][NI];
+    // row constants of every output row this lane holds, requested together (clamped rows) so that their latencies
+    // overlap instead of chaining
+    int rexp[R];
+    float rxs[R], rcorr[R];
+    const int *rexp0 = p.rexp + mrow0;
+    const float *xsum0 = p.xsum + mrow0, *esum0 = PRECISE ? nullptr : p.esum + mrow0;
 #pragma unroll
-    for (int tm = 0; tm < TM; tm++)
+    for (int r = 0; r < R; r++) {
+        const int at = min((r >> 2) * 8 + (r & 3) + 4 * h, last);
+        rexp[r] = rexp0[at];
+        rxs[r] = split ? 0.0f : xsum0[at];
+        rcorr[r] = (!PRECISE && !split) ? esum0[at] : 0.0f;
+    }
+    float o[R][TN];
 #pragma unroll
-        for (int i = 0; i < NI; i++) {
-            int64_t m = mrow0 + tm * RPB + (i / 4) * 8 + h * 4 + (i % 4);
-            if (m > p.m - 1) m = p.m - 1;
-            rexp[tm][i] = p.rexp[m];
-            rxs[tm][i] = split ? 0.0f : p.xsum[m];
-            rcorr[tm][i] = (!PRECISE && !split) ? p.esum[m] : 0.0f;
-        }
+    for (int r = 0; r < R; r++) {
+        const int e = rexp[r];
+        float corr = 0.0f;
+        if constexpr (!PRECISE) corr = ldexpf(rcorr[r], -e);
 #pragma unroll
-    for (int tm = 0; tm < TM; tm++)
-#pragma unroll
-        for (int i = 0; i < NI; i++) {
-            const int64_t m = mrow0 + tm * RPB + (i / 4) * 8 + h * 4 + (i % 4);
-            if (m >= p.m) continue;
-            const int e = rexp[tm][i];
-            const float xs = rxs[tm][i];
-            float corr = 0.0f;
-            if constexpr (!PRECISE) corr = ldexpf(rcorr[tm][i], -e);
-#pragma unroll
-            for (int tn = 0; tn < TN; tn++) {
-                const int64_t n = n0 + (wn * TN + tn) * 32 + lr;
-                if (n >= p.n) continue;
-                float v;
-                if constexpr (PRECISE) v = acc[tm][tn][i] + acc[tm][tn][i + 8] * LO_DOWN;
-                else v = acc[tm][tn][i];
-                float d = ldexpf(v, -e);   // this workgroup's share of sum_k A[m,k]*u(W[n,k])
-                if (split) {
-                    p.part[((int64_t)z * p.m + m) * p.n + n] = d;
-                } else {
-                    if constexpr (!PRECISE) d = d - um[tn] * corr;
-                    float o = d * sc[tn] + zp[tn] * xs;
-                    if (p.bias) o = o + bi[tn];
-                    p.out[m * p.n + n] = fnn_activation(o, p.act);
-                }
+        for (int tn = 0; tn < TN; tn++) {
+            float v;
+            if constexpr (PRECISE) v = acc[r / NI][tn][r % NI] + acc[r / NI][tn][r % NI + 8] * LO_DOWN;
+            else v = acc[r / NI][tn][r % NI];
+            float d = ldexpf(v, -e);   // this workgroup's share of sum_k A[m,k]*u(W[n,k])
+            if (!split) {
+                if constexpr (!PRECISE) d = d - um[tn] * corr;
+                d = d * sc[tn] + zp[tn] * rxs[r];
             }
+            o[r][tn] = d;
         }
+    }
+    tile_finish<R, TN>(o, split ? p.part + (int64_t)z * p.m * p.n : p.out, mrow0, ncol0, p.m, p.n, bi, p.bias != nullptr && !split,
+                       split ? (int)FNN_ACT_NONE : p.act, lr, h);
 }
 
 // sum of the K-split partial tiles in split order + affine / bias / activation epilogue.  A thread owns one
