@@ -99,6 +99,7 @@ int fnn_mfma_rows16(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, co
                     int flags, bool *handled);
 
 // I8 activations x I8/I4 weights and the quantised Conv2d on int8 MFMA tiles with i32 accumulators.
+float fnn_i8_tiled_us(int dt, int64_t m, int64_t n, int64_t k);   // microseconds expected of the LDS tiles
 int fnn_i8_tiled_matmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const I8ActArgs &p, bool *handled);
 // p.actq must already hold the (image, group) activation scales.
 int fnn_i8_tiled_conv(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QConvArgs &p, bool *handled);

@@ -66,28 +66,36 @@ __global__ void __launch_bounds__(256) frag_codes_reduce_kernel(FragIntArgs p)
     if (p.acc_out) p.acc_out[i] = za != 0.0f ? 0 : acc;
 }
 
-// Microseconds of quantisation + MatMul in a form, least squares over 3 500 drawn shapes (7 % mean error; the terms as in
-// qgemm_frag.hip), and of the LDS-tiled form.  Reading the payload in the kernel touches 16 separate 64-byte pieces per wave
-// load (3.5 times the L1 time of a contiguous KB) and saves the launch that lays the codes out.
+// Which form: an estimate in microseconds (quantisation included), least squares over 3 500 drawn shapes in all their forms (7 % mean error; the terms as
+// in qgemm_frag.hip).  Reading the payload in the kernel touches 16 separate 64-byte pieces per wave load (3.5 times the L1
+// time of a contiguous KB) and saves the launch that lays the codes out.
 struct IntShape { int mb, nb; };
 constexpr IntShape kIntShapes[] = {{1, 1}, {1, 2}, {2, 2}, {2, 4}, {4, 4}};
 
-float codes_us(IntShape t, bool direct, int splits, int64_t m, int64_t n, int64_t k, int groups, bool four)
+struct IntLoad { float rounds, bytes, mfma, area, mn, mk, nk; };
+IntLoad codes_load(IntShape t, bool direct, int splits, int64_t m, int64_t n, int64_t k, int groups, bool four)
 {
-    const float area = (float)(t.mb * t.nb), mn = (float)m * (float)n;
+    const float area = (float)(t.mb * t.nb);
     const float x = (float)((m + 16 * t.mb - 1) / (16 * t.mb)) * (float)((n + 16 * t.nb - 1) / (16 * t.nb)) * (float)splits / 256.f, cx = (float)(int)(x + 0.99999f);
     float r = area > 8.f ? cx : (x <= 4.f ? 0.5f * (cx + x) : x + 0.25f);
     if (r < 1.f) r = 1.f;
     const float seg = (float)(((groups + splits - 1) / splits + FRAG_NW - 1) / FRAG_NW), wb = four ? 64.f : 128.f;
-    const float bytes = seg * 8.f * ((float)t.mb * 2048.f * (direct ? 3.5f : 1.f) + (float)t.nb * 16.f * wb) / 1e5f, mfma = seg * area * 64.f / 2400.f;
-    const float two = splits > 1 ? 1.f : 0.f, mk = (float)m * (float)k * 9.f / 1e6f, nk = (float)n * (float)groups * wb / 1e6f;
-    return direct ? 10.22f + r * (0.25f * bytes + 2.596f * mfma) + two * 2.91f + 0.277f * mn * 4.f / 1e6f + 0.267f * mk + 0.0116f * nk
-                  : 12.76f + r * (0.387f * bytes + 1.563f * mfma) + two * 3.12f + 0.438f * mn * 4.f / 1e6f + 0.308f * mk + 0.013f * nk;
+    return {r, seg * 8.f * ((float)t.mb * 2048.f * (direct ? 3.5f : 1.f) + (float)t.nb * 16.f * wb) / 1e5f, seg * area * 64.f / 2400.f, area,
+            (float)m * (float)n * 4.f / 1e6f, (float)m * (float)k * 9.f / 1e6f, (float)n * (float)groups * wb / 1e6f};
 }
-float codes_tiled_us(int64_t m, int64_t n, int64_t k)
+float codes_order(const IntLoad &l, bool direct, int splits)
 {
-    const float fm = (float)m, fn = (float)n, fk = (float)k;
-    return 15.1f + 1.144f * fm * fn * fk / 1e9f + 1.273f * fm * fn / 1e6f + 0.0721f * fn * fk / 1e6f + 3.114f * fm * fk / 1e6f + 0.995f * fk / 1e3f;
+    const float two = splits > 1 ? 1.f : 0.f;
+    return direct ? 10.22f + l.rounds * (0.25f * l.bytes + 2.596f * l.mfma) + two * 2.91f + 0.277f * l.mn + 0.267f * l.mk + 0.0116f * l.nk
+                  : 12.76f + l.rounds * (0.387f * l.bytes + 1.563f * l.mfma) + two * 3.12f + 0.438f * l.mn + 0.308f * l.mk + 0.013f * l.nk;
+}
+// Microseconds of the form that it picks (operand kernel + MatMul), to be compared with the LDS tiles': least squares over 590 drawn calls
+// whose products are below 8e9 MACs, 7 % mean error.
+float codes_us(const IntLoad &l, bool direct, int splits)
+{
+    const float two = splits > 1 ? 1.f : 0.f;
+    return direct ? 2.59f + l.rounds * (0.388f * l.bytes + 3.112f * l.mfma + 0.0384f + 0.0094f * l.area) + two * 2.91f + 0.501f * l.mn + 0.134f * l.mk + 0.1066f * l.nk
+                  : 5.11f + l.rounds * (0.567f * l.bytes + 1.415f * l.mfma + 0.0537f * l.area) + two * 3.12f + 0.401f * l.mn + 0.172f * l.mk + 0.1011f * l.nk;
 }
 
 }  // namespace
@@ -115,7 +123,7 @@ int fnn_frag_i8act(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, con
     } else {
         // (products beyond that run at the matrix cores' rate on the LDS tiles: 2048 x 4096 x 4096 78 us there, 112 here)
         if ((double)q.m * (double)q.n * (double)q.k > 8e9) return FNN_OK;
-        float best = 1e30f;
+        float best = 1e30f, us = 0.f;
         for (IntShape t : kIntShapes) {
             if (t.mb > 1 && (t.mb / 2) * 16 >= q.m) continue;
             const int64_t wgs = ((q.m + 16 * t.mb - 1) / (16 * t.mb)) * ((q.n + 16 * t.nb - 1) / (16 * t.nb));
@@ -123,12 +131,13 @@ int fnn_frag_i8act(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, con
                 if (sp > 1 && (wgs * sp > 600 || sp * 8 > p.ks.kblocks)) break;
                 for (int d = 0; d < 2; d++) {
                     if (d && (!direct_ok || q.m > 256)) continue;
-                    const float us = codes_us(t, d != 0, sp, q.m, q.n, q.k, p.ks.kblocks, four);
-                    if (us < best) { best = us; mb = t.mb; nb = t.nb; splits = sp; direct = d != 0; }
+                    const IntLoad l = codes_load(t, d != 0, sp, q.m, q.n, q.k, p.ks.kblocks, four);
+                    const float o = codes_order(l, d != 0, sp);
+                    if (o < best) { best = o; us = codes_us(l, d != 0, sp); mb = t.mb; nb = t.nb; splits = sp; direct = d != 0; }
                 }
             }
         }
-        if (best > 0.93f * codes_tiled_us(q.m, q.n, q.k)) return FNN_OK;
+        if (us > 0.97f * fnn_i8_tiled_us(w->dtype, q.m, q.n, q.k)) return FNN_OK;
     }
     const int shape = mb * 16 + nb;
     if (shape != 0x11 && shape != 0x12 && shape != 0x22 && shape != 0x24 && shape != 0x44) return FNN_OK;

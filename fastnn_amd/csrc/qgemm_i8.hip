@@ -420,8 +420,8 @@ hipError_t launch_i8_tile(const TileArgs &p, hipStream_t s)
     static std::atomic<uint64_t> lds_raised{0};
     hipError_t e = fnn_raise_lds_limit(lds_raised, reinterpret_cast<const void *>(kern), (int)lds);
     if (e != hipSuccess) return e;
-    // (a ring of three requests only the stages its K range has: one LDS buffer per stage, at most three)
-    const int bufs = (NS == 3 && p.ips < NS) ? p.ips : NS;
+    // (only the stages of the K range are requested: one LDS buffer per stage, at most the ring)
+    const int bufs = p.ips < NS ? p.ips : NS;
     hipLaunchKernelGGL(kern, dim3((unsigned)p.mtiles * p.ntiles * p.splits), dim3(WGM * WGN * 64), lds / NS * bufs, s, p);
     return hipGetLastError();
 }
@@ -488,8 +488,15 @@ hipError_t run_i8_gemm(const uint32_t *words, int64_t kp, int64_t rows_total, in
         return conv ? launch_i8_tile<DT, 4, 1, 1, 2, 3, true>(t, s) : launch_i8_tile<DT, 4, 1, 1, 2, 3>(t, s);
     }
     t.ntiles = (int)((n + 127) / 128);
-    if (!conv && form == 1) return launch_i8_tile<DT, 2, 4, 2, 1, 3>(t, s);      // 128 x 128 on eight waves of 64 x 32
-    if (!conv && form == 2) {                                                    // 256 x 128 on eight waves of 64 x 64
+    // 128 x 128 on eight waves of 64 x 32, four stages: with three a stage is requested one stage before it is waited for, and the wait is
+    // its latency and its transfer (32 KB, 0.4 us of a CU's 32 bytes a clock) one behind the other (384 x 4096 x 8192 48.8 -> 38.5 us,
+    // 512 x 2048 x 8192 33.4 -> 28.7, five stages 29.0).  4-bit weights beyond one round keep three: two workgroups to a CU (72 KB each)
+    // hide more (1594 x 1856 x 14843 81 against 98 us).
+    if (!conv && form == 1) {
+        if (DT == FNN_DT_I4 && (int64_t)t.mtiles * t.ntiles * t.splits > 256) return launch_i8_tile<DT, 2, 4, 2, 1, 3>(t, s);
+        return launch_i8_tile<DT, 2, 4, 2, 1, 4>(t, s);
+    }
+    if (!conv && form == 2) {   // 256 x 128 on eight waves of 64 x 64 (three stages: a fourth fits with 4-bit weights, and gains nothing)
         t.mtiles = (int)((rows_pad + 255) / 256);
         return launch_i8_tile<DT, 4, 2, 2, 2, 3>(t, s);
     }
@@ -683,6 +690,64 @@ int fnn_row_qsum(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const
     return FNN_OK;
 }
 
+namespace {
+
+// Tile form (1: 128 x 128 on eight waves of 64 x 32, 2: 256 x 128 on eight waves of 64 x 64) and K split.
+// K split over workgroups while the tiles alone leave CUs idle: the partial matrices are exact integers, so the epilogue adds them in
+// any order (4096 x 4096 at M = 256: 64 tiles, 31 -> 24 us with four K ranges); more than four partial matrices cost more than the idle
+// CUs they fill (M = 128 23.8 -> 20.5 us).
+struct I8TileForm { int form, splits; };
+I8TileForm i8_tile_form(int form, int64_t rows_pad, int64_t n, int iters)
+{
+    const int64_t tiles = (rows_pad / 128) * (n <= 64 ? 1 : (n + 127) / 128);
+    int splits = (int)(256 / (tiles > 0 ? tiles : 1));
+    if (form == 2) splits *= 2;
+    if (splits > 4) splits = 4;
+    if (splits > iters / 4) splits = iters / 4;
+    return {form, splits < 1 ? 1 : splits};
+}
+
+// Microseconds of operand kernel + tiles (+ reduction) in a form: least squares over 740 drawn calls (M 17 .. 2048, K 256 .. 8192,
+// N 256 .. 16384), 4 % mean error.  Whole rounds of workgroups decide: 405 x 7808 x 8373 is 264 tiles of 128 x 128, two rounds, and 132
+// of 256 x 128, one: 80 against 64 us.  The form with the lower figure is 0.3 % off the better one on average (taken only from 256
+// tiles of 256 x 128 on it was 0.9 % off).
+float i8_tile_us(I8TileForm f, int dt, int64_t m, int64_t rows_pad, int64_t n, int64_t k)
+{
+    static const float kFit[2][2][9] = {   // launches, round, stage of a round, M N / 1e6, K split, M N / 1e6 per split, M K / 1e6, weight MB, stages of all
+                                           // tiles / 256
+        {{6.58f, 1.549f, 0.4699f, 0.901f, 0.556f, 2.422f, 0.460f, 0.0f, 0.1759f}, {6.90f, 1.131f, 0.4796f, 0.875f, 0.390f, 2.780f, 0.574f, 0.0194f, 0.1036f}},
+        {{6.69f, 3.651f, 0.7511f, 0.650f, 1.304f, 1.617f, 0.526f, 0.0f, 0.2313f}, {4.39f, 6.079f, 0.6951f, 0.503f, 0.912f, 1.709f, 0.768f, 0.1648f, 0.0760f}}};
+    const float *c = kFit[f.form == 2][dt == FNN_DT_I4];
+    const int iters = (int)((k + KB - 1) / KB), ips = (iters + f.splits - 1) / f.splits, splits = (iters + ips - 1) / ips;
+    const int64_t tiles = (f.form == 2 ? rows_pad / 256 : rows_pad / 128) * ((n + 127) / 128) * splits;
+    const float rounds = (float)((tiles + 255) / 256), mn = (float)m * (float)n / 1e6f;
+    return c[0] + rounds * (c[1] + c[2] * (float)ips) + c[3] * mn + (splits > 1 ? c[4] + c[5] * (float)splits * mn : 0.f) + c[6] * (float)m * (float)k / 1e6f +
+           c[7] * (float)n * (float)k * (dt == FNN_DT_I4 ? 0.5f : 1.f) / 1e6f + c[8] * (float)tiles * (float)ips / 256.f;
+}
+
+I8TileForm i8_tile_choice(int dt, int64_t m, int64_t n, int64_t k, float *us)
+{
+    const int64_t rows_pad = (m + 127) / 128 * 128;
+    const int iters = (int)((k + KB - 1) / KB);
+    I8TileForm f = i8_tile_form(1, rows_pad, n, iters);
+    *us = i8_tile_us(f, dt, m, rows_pad, n, k);
+    if (rows_pad % 256 == 0 && n > 64) {
+        const I8TileForm tall = i8_tile_form(2, rows_pad, n, iters);
+        const float t = i8_tile_us(tall, dt, m, rows_pad, n, k);
+        if (t < 0.98f * *us) { f = tall; *us = t; }
+    }
+    return f;
+}
+
+}  // namespace
+
+float fnn_i8_tiled_us(int dt, int64_t m, int64_t n, int64_t k)
+{
+    float us;
+    (void)i8_tile_choice(dt, m, n, k, &us);
+    return us;
+}
+
 int fnn_i8_tiled_matmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const I8ActArgs &p, bool *handled)
 {
     *handled = false;
@@ -696,20 +761,19 @@ int fnn_i8_tiled_matmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w
     const size_t q_off = (a_bytes + 255) / 256 * 256;
     void *ws0 = nullptr, *ws1 = nullptr;
     int rc;
-    // K split over workgroups while the tiles alone leave CUs idle: the partial matrices are exact integers, so the
-    // epilogue adds them in any order (4096 x 4096 at M = 256: 64 tiles, 31 -> 24 us with four K ranges)
-    const int64_t tiles = (rows_pad / 128) * (p.n <= 64 ? (p.n + 63) / 64 : (p.n + 127) / 128);
     const int iters = (int)(kpad / KB);
-    int splits = (int)(256 / (tiles > 0 ? tiles : 1));
-    // Tile form: 128 x 128 on eight waves of 64 x 32 (every wave issues loads: 4096 x 4096 at M = 256 25.7 -> 24.3 us, M = 128
-    // 21.9 -> 20.5), 256 x 128 on eight waves of 64 x 64 once those fill the chip unsplit (M = 2048: 90.6 -> 70.1 us);
-    // FNN_OPT_TILE_SHAPE 0 / 1 / 2 picks the four-wave tiles / either of these.
+    // FNN_OPT_TILE_SHAPE 0 / 1 / 2: the four-wave tiles / either form
+    float us;
+    const I8TileForm f = i8_tile_choice(w->dtype, p.m, p.n, p.k, &us);
     int form = (int)fnn_ctx_option(ctx, FNN_OPT_TILE_SHAPE);
-    if (form < 0 || form > 2) form = (rows_pad % 256 == 0 && (rows_pad / 256) * ((p.n + 127) / 128) >= 256) ? 2 : 1;
+    if (form < 0 || form > 2) form = f.form;
     if (p.n <= 64) form = 0;
     if (form == 2 && rows_pad % 256) form = 1;
-    if (form == 2) splits *= 2;
-    if (splits > 4) splits = 4;   // (more partial matrices cost more than the idle CUs they fill: M = 128 23.8 -> 20.5 us)
+    int splits = form == f.form ? f.splits : i8_tile_form(form, rows_pad, p.n, iters).splits;
+    if (form == 2 && splits > 1 && !fnn_ctx_tmp_fits(ctx, 1, (size_t)splits * p.m * p.n * 4 + 256)) {   // (its splits need the most room)
+        form = 1;
+        splits = i8_tile_form(1, rows_pad, p.n, iters).splits;
+    }
     if (const int64_t forced = fnn_ctx_option(ctx, FNN_OPT_TILE_SPLIT); forced > 0) splits = (int)forced;
     if (splits > iters / 4) splits = iters / 4;
     if (splits > 16) splits = 16;

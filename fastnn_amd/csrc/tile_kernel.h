@@ -318,8 +318,7 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
     // dense f16 weights ([hi | lo] halves): rows are whole stages long and the activations are swept twice;
     // packed weights: one sweep, and the last stage of a row may be partly past its end
     constexpr bool DENSE = !INT8 && D::WPS == 4;
-    // running source pointers: advanced after every stage, frozen once the K range is exhausted
-    // (the extra requests of the last iterations re-read the final stage and are never consumed)
+    // running source pointers: advanced after every stage
 #pragma unroll
     for (int j = 0; j < A_LPW; j++) a_src[j] += (int64_t)(DENSE ? it0 % p.a_wrap : it0) * a_step;
 #pragma unroll
@@ -361,17 +360,15 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
             else if (n == 2) load_group_to_lds16<2>(a_src[g], a_src[g + 1 < A_LPW ? g + 1 : g], nullptr, nullptr, base);
             else load_group_to_lds16<1>(a_src[g], nullptr, nullptr, nullptr, base);
         }
-        const bool more = it + 1 < it1;           // wave-uniform
-        int64_t astep = more ? a_step : 0;
-        if (DENSE && more && ++a_pos == p.a_wrap) {   // second sweep over the activations
+        int64_t astep = a_step;
+        if (DENSE && ++a_pos == p.a_wrap) {   // second sweep over the activations
             a_pos = 0;
             astep = -(int64_t)(p.a_wrap - 1) * a_step;
         }
-        const int wstep = !more ? 0 : w_stride;
 #pragma unroll
         for (int j = 0; j < A_LPW; j++) a_src[j] += astep;
 #pragma unroll
-        for (int j = 0; j < W_LPW; j++) w_src[j] += wstep;
+        for (int j = 0; j < W_LPW; j++) w_src[j] += w_stride;
     };
 
     f32x16 acc[TM][TN];
@@ -502,23 +499,16 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
                     }
         };
 
-        // With a ring of three a hand-over waits for every outstanding load, so stages past the K range need not be
-        // requested to keep the wait counts right: a short K range (the first conv layers: one or two stages)
-        // then moves no byte twice and needs one LDS buffer per stage it has (the launcher sizes LDS to that).
-        // Deeper rings keep requesting (re-reads of the final stage that nothing consumes).
-        constexpr bool EXACT = NS == 3;
-        const bool one_stage = EXACT && it1 - it0 == 1;   // (workgroup-uniform)
-        if (one_stage) {
-            issue(it0, 0);
-        } else {
+        // Stages past the K range are not requested, so a short one moves no byte twice and needs one LDS buffer per stage it has (the
+        // launcher sizes a ring of three to that); where fewer are on their way than the wait counts, it waits for all of them.
 #pragma unroll
-            for (int st = 0; st < NS - 1; st++) issue(it0 + st, st);
-        }
+        for (int st = 0; st < NS - 1; st++)
+            if (it0 + st < it1) issue(it0 + st, st);
         uint32_t wq[TN][WQW], wqn[TN][WQW];
         f16x8 af[4][TM], bfr[2][TN], bfl[2][CB ? TN : 1];
         if constexpr (CB) load_bscales(it0, bs_cur);
         // first stage: this wave's part has landed
-        if (one_stage) wait_loads_but<0>();
+        if (it1 - it0 < NS - 1) wait_loads_but<0>();
         else if (w_on) wait_loads_but<(NS - 2) * LPS>();
         else wait_loads_but<(NS - 2) * A_LPW>();
         __syncthreads();                    // ... and everybody else's
@@ -545,12 +535,13 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
             mfmas(af[1], bfr[1], bfl[1], 1);
             // hand-over
             // this wave's part of the next stage has landed
-            if (w_on) wait_loads_but<(NS - 3) * LPS>();
+            if (NS == 3 || it + NS - 1 > it1) wait_loads_but<0>();
+            else if (w_on) wait_loads_but<(NS - 3) * LPS>();
             else wait_loads_but<(NS - 3) * A_LPW>();
             __syncthreads();                    // everybody's; the stage before the current one is free
             int fb = buf + NS - 1;
             if (fb >= NS) fb -= NS;
-            if (!EXACT || it + NS - 1 < it1) issue(it + NS - 1, fb);
+            if (it + NS - 1 < it1) issue(it + NS - 1, fb);
             // step 2, with the first reads of the next stage
             read_w(nbase, wqn);
             read_a(nbase, 0, af[0]);
