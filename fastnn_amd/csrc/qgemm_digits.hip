@@ -16,7 +16,7 @@
 // twice the f16 rate), a fraction of the vector instructions per stage, and a tighter result: the only rounding
 // before the epilogue is rint() at 2^-30 (2^-22 with three planes) of the row's largest magnitude.
 //
-// Launches: digit_prep_kernel (once per call), qgemm_tile_kernel<int8, DIG>, and with K split over workgroups
+// Launches: digit_prep_kernel or digit_groups_kernel (once per call), qgemm_tile_kernel<int8, DIG> or qgemm_wave_kernel, and with K split over workgroups
 // splitk_epilogue_kernel (partials added in split order: results do not depend on scheduling).
 // A row holding a non-finite activation comes out as NaN in every column (the reference yields inf or NaN there
 // depending on the weights' signs and zeros).
@@ -62,26 +62,17 @@ __device__ __forceinline__ void transpose4(uint32_t a, uint32_t b, uint32_t c, u
 // operand layout.  Operand row of (activation row m, plane j): (m / RPB) * 32 + j * RPB + m % RPB, RPB = 32 / DIG, for
 // two and four planes; with three planes ((m / 8) * 3 + j) * 8 + m % 8 (groups of 24 rows: 8 activation rows x 3 planes).
 // IL: the nibble decoders deliver k = 0,2,4,6,1,3,5,7 of each 8, and the activations are stored in that order.
-// FRAG (three planes): the fragment order of qgemm_wave_impl.h instead of tile-major rows.
-template <int DIG, bool IL, bool FRAG = false>
+template <int DIG, bool IL>
 __global__ void __launch_bounds__(256) digit_prep_kernel(DigitArgs p)
 {
     constexpr int RPB = DIG == 3 ? 8 : 32 / DIG;
     constexpr uint32_t BIAS = DIG == 4 ? 0x80808080u : (DIG == 3 ? 0x00808080u : 0x00008080u);
     __shared__ float red[2][4];
-    // (fragment order: eight activation rows share 128-byte lines of a plane; their workgroups go to one XCD)
-    const int64_t m = FRAG && (blockIdx.x | 63u) < gridDim.x ? (blockIdx.x & ~63u) + (blockIdx.x & 7) * 8 + ((blockIdx.x >> 3) & 7) : blockIdx.x;
+    const int64_t m = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int64_t nchunks = p.kpad / 16;
     const int64_t row0 = DIG == 3 ? (m / 8) * 24 + m % 8 : (m / RPB) * 32 + m % RPB;
     auto chunk_at = [&](int j, int64_t c) {
-        if constexpr (FRAG) {
-            // chunk of 16 k-values -> (step, half): 32 s + 16 h, or for nibbles 128 b + 64 p + 32 h + 16 t with step 4 b + 2 p + t
-            const int64_t step = IL ? (c >> 3) * 4 + ((c >> 1) & 2) + (c & 1) : c >> 1;
-            const int half = IL ? (int)(c >> 1) & 1 : (int)c & 1;
-            const int64_t r = row0 + j * RPB;
-            return p.planes + (((r >> 5) * p.nsteps + step) * 64 + half * 32 + (r & 31)) * 16;
-        }
         return p.planes + (((c >> 3) * p.rows_pad + row0 + j * RPB) * KB + (c & 7) * 16);
     };
     if (m >= p.m) {   // padding rows of the last tile
@@ -182,6 +173,121 @@ __global__ void __launch_bounds__(256) digit_prep_kernel(DigitArgs p)
     }
 }
 
+// Fragment order: byte of a chunk of 16 k-values inside a block of 32 operand rows, from (step, half): 32 s + 16 h, or for nibbles
+// 128 b + 64 p + 32 h + 16 t with step 4 b + 2 p + t
+template <bool IL>
+__device__ __forceinline__ int chunk_bytes(int c)
+{
+    const int step = IL ? (c >> 3) * 4 + ((c >> 1) & 2) + (c & 1) : c >> 1, half = IL ? (c >> 1) & 1 : c & 1;
+    return (step * 64 + half * 32) * 16;
+}
+// the power of two of three planes: |x * 2^e| < 2^22 for every |x| <= mx
+__device__ __forceinline__ int scale3(float mx)
+{
+    if (!(mx > 0.0f && mx < __builtin_huge_valf())) return 0;
+    int ex;
+    (void)frexpf(mx, &ex);   // mx = f * 2^ex, f in [0.5, 1)
+    return 22 - ex;
+}
+
+// Three planes in the fragment order of qgemm_wave_impl.h, one workgroup per activation row slot.  Bound: the chain of a launch (one trip to
+// memory, one reduction, one store), at many rows the 16-byte pieces of the stores.  A thread holds groups of four values, GROUPS_NT of them
+// apart: a wave's load is one contiguous KB (with 16 consecutive values a thread every load touched every line of it), and few values a thread
+// keep the chain short.  256 x 4096 7.4 -> 6.0 us, 512 x 4096 8.2 -> 6.6, 2048 x 4096 20.2 -> 18.3; 256 threads 7.5, 7.8 and 18.2, 1024 threads 6.2, 6.6
+// and 20.8; eight rows a workgroup, every line stored whole, 9.9, 9.5 and 13.1.  (Tile-major rows are stored in whole
+// lines either way, there the kernel above is ahead at many rows: 2048 x 4096 10.9 against 13.1.)  Eight rows share the 128-byte lines of a
+// plane: their workgroups go to one XCD.
+constexpr int GROUPS_NT = 512, GROUPS_KEEP = 4;   // groups of a thread that stay in registers between the two passes
+template <bool IL>
+__global__ void __launch_bounds__(GROUPS_NT) digit_groups_kernel(DigitArgs p)
+{
+    constexpr int NT = GROUPS_NT, NW = NT / 64;
+    __shared__ float red[2][NW];
+    const int64_t m = (blockIdx.x | 63u) < gridDim.x ? (blockIdx.x & ~63u) + (blockIdx.x & 7) * 8 + ((blockIdx.x >> 3) & 7) : blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, groups = p.nsteps * 8;
+    const float *x = p.a + m * p.k;
+    const bool vec = (p.k % 4 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0), real = m < p.m;
+    auto load4 = [&](int g, float (&v)[4]) {
+        const int64_t k0 = (int64_t)g * 4;
+        if (vec && real && k0 + 4 <= p.k) {
+            const float4 t = *reinterpret_cast<const float4 *>(x + k0);
+            v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = (real && k0 + i < p.k) ? x[k0 + i] : 0.0f;
+        }
+    };
+    float keep[GROUPS_KEEP][4];
+    float mx = 0.0f, sum = 0.0f;
+    auto stats = [&](const float (&v)[4]) {
+        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+        sum += (v[0] + v[1]) + (v[2] + v[3]);
+    };
+    const bool in_regs = groups <= NT * GROUPS_KEEP;   // (uniform)
+    if (in_regs) {
+#pragma unroll
+        for (int i = 0; i < GROUPS_KEEP; i++) {
+            keep[i][0] = keep[i][1] = keep[i][2] = keep[i][3] = 0.0f;
+            if (tid + i * NT < groups) load4(tid + i * NT, keep[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < GROUPS_KEEP; i++) stats(keep[i]);
+    } else {
+        for (int g = tid; g < groups; g += NT) { load4(g, keep[0]); stats(keep[0]); }
+    }
+    // fmaxf drops NaN operands: the sum carries them (and +-inf); either makes the row's maximum infinite
+    if (!(fabsf(sum) < __builtin_huge_valf())) mx = __builtin_huge_valf();
+    mx = wave_max(mx);
+    sum = wave_sum(sum);
+    if (lane == 0) { red[0][wv] = mx; red[1][wv] = sum; }
+    __syncthreads();
+    mx = 0.0f;
+    sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; w += 2) {
+        mx = fmaxf(mx, fmaxf(red[0][w], red[0][w + 1]));
+        sum += red[1][w] + red[1][w + 1];
+    }
+    const bool finite = mx < __builtin_huge_valf();
+    const int e = scale3(mx);
+    const int row0 = (int)(m / 8) * 24 + (int)(m & 7);
+    auto convert = [&](int g, const float (&v)[4]) {
+        uint32_t t[4], w[4];   // w[plane]
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int vi = finite ? (int)rintf(ldexpf(v[i], e)) : 0;
+            t[i] = ((uint32_t)vi + 0x00808080u) ^ 0x00808080u;    // byte j = digit j as a signed byte
+        }
+        if (IL) {   // the neighbour (lane ^ 1) holds the other half of the eight: its first and third or second and fourth values
+            transpose4(t[0], t[2], t[1], t[3], w);
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)w[j], 0xB1, 0xF, 0xF, true);
+                w[j] = __builtin_amdgcn_perm(other, w[j], (lane & 1) ? 0x03020706u : 0x05040100u);
+            }
+        } else {
+            transpose4(t[0], t[1], t[2], t[3], w);
+        }
+        const int64_t at = chunk_bytes<IL>(g >> 2) + (g & 3) * 4;
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const int row = row0 + j * 8;
+            *reinterpret_cast<uint32_t *>(p.planes + (int64_t)(row >> 5) * p.nsteps * 1024 + (row & 31) * 16 + at) = w[j];
+        }
+    };
+    if (in_regs) {
+#pragma unroll
+        for (int i = 0; i < GROUPS_KEEP; i++)
+            if (tid + i * NT < groups) convert(tid + i * NT, keep[i]);
+    } else {
+        for (int g = tid; g < groups; g += NT) { load4(g, keep[0]); convert(g, keep[0]); }
+    }
+    if (tid == 0) {
+        p.rexp[m] = finite ? e : INT_MIN;
+        p.xsum[m] = sum;
+    }
+}
+
 // Three planes on the wave tiles (qgemm_wave_impl.h); wk: waves that share a tile.
 template <int DT>
 int run_digits_wave(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int wk, bool *handled)
@@ -215,7 +321,7 @@ int run_digits_wave(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, co
     d.xsum = (float *)(d.rexp + m_pad);
     d.m = q.m; d.k = q.k; d.kpad = (int64_t)p.nsteps * 32; d.rows_pad = 0;
     d.nsteps = p.nsteps;
-    hipLaunchKernelGGL((digit_prep_kernel<3, IL, true>), dim3((unsigned)m_pad), dim3(256), 0, s, d);
+    hipLaunchKernelGGL((digit_groups_kernel<IL>), dim3((unsigned)m_pad), dim3(GROUPS_NT), 0, s, d);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
     p.af = d.planes; p.rexp = d.rexp; p.xsum = d.xsum;
