@@ -114,6 +114,11 @@ class ExecutablePlan:
         """MatMul instructions whose activation operand the MatMul before them prepared."""
         return int(self.lib.fnn_plan_operands_handed(self.handle))
 
+    @property
+    def halved(self) -> bool:
+        """Whether the last pass was a forward pass in two halves of its images."""
+        return bool(self.lib.fnn_plan_halved(self.handle))
+
     def _ok(self, rc, what):
         if rc:
             msg = self.lib.fnn_backend_last_error(None)

@@ -1335,3 +1335,32 @@ FnnResidualIo *fnn_ctx_residual_io(fnn_hip_ctx *ctx) { return &ctx->residual; }
 FnnPrepIo *fnn_ctx_prep_io(fnn_hip_ctx *ctx) { return &ctx->prep; }
 FnnPreparedOperand *fnn_ctx_prepared(fnn_hip_ctx *ctx) { return &ctx->prepared; }
 bool fnn_ctx_static_mode(fnn_hip_ctx *ctx) { return ctx->static_mode; }
+int fnn_ctx_parts_begin(fnn_hip_ctx *ctx)
+{
+    return guarded(ctx, "parts", [&]() -> int {
+        if (ctx->capturing) return fail(ctx, FNN_ERR_DISPATCH, "transfer from host memory during graph capture");
+        HIP_TRY(ctx, FNN_ERR_MEMORY, ctx->io.begin_parts(ctx->stream));
+        return FNN_OK;
+    });
+}
+int fnn_ctx_part_in(fnn_hip_ctx *ctx, int part, void *dst_dev, const void *src, size_t bytes)
+{
+    return guarded(ctx, "copy in", [&]() -> int {
+        HIP_TRY(ctx, FNN_ERR_MEMORY, ctx->io.in_part(ctx->stream, part, dst_dev, src, bytes));
+        return FNN_OK;
+    });
+}
+int fnn_ctx_part_mark(fnn_hip_ctx *ctx, int part)
+{
+    return guarded(ctx, "parts", [&]() -> int {
+        HIP_TRY(ctx, FNN_ERR_DISPATCH, ctx->io.mark_part(ctx->stream, part));
+        return FNN_OK;
+    });
+}
+int fnn_ctx_part_out(fnn_hip_ctx *ctx, int part, void *dst, const void *src_dev, size_t bytes)
+{
+    return guarded(ctx, "copy out", [&]() -> int {
+        HIP_TRY(ctx, FNN_ERR_MEMORY, ctx->io.out_part(part, dst, src_dev, bytes));
+        return FNN_OK;
+    });
+}

@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <exception>
 #include <map>
+#include <memory>
 #include <new>
 #include <string>
 #include <vector>
@@ -131,6 +132,11 @@ struct fnn_plan {
     uint64_t residuals_fused = 0;     // such Adds in the last host-side pass
     size_t prep_ready = (size_t)-1;   // index of a MatMul whose operand the call before it has prepared
     uint64_t operands_handed = 0;     // such MatMuls in the last host-side pass
+    // the plan over each half of its images, where every instruction works image by image (split_images); constants stay with this plan
+    std::unique_ptr<fnn_plan> half[2];
+    bool halves_tried = false, last_halved = false;
+    std::vector<fnn_slice> halved;    // the slices that are halved: what a forward pass may write and read
+    ~fnn_plan() { if (graph) fnn_hip_graph_destroy(nullptr, graph); }   // every dispatch ends with a sync: nothing in flight
 };
 
 struct fnn_backend {
@@ -1113,6 +1119,21 @@ int run_instr(fnn_backend *b, fnn_plan *p, size_t idx, bool consts_resident)
     return FNN_OK;
 }
 
+// are the plan's constants where an earlier dispatch of it left them?
+bool constants_in_place(fnn_backend *b, fnn_plan *p)
+{
+    if (p->resident_uid != b->uid || p->resident_generation != b->generation) return false;
+    if (p->resident_seq == b->write_seq) return true;
+    // the host wrote into the arena since: in place unless a constant was hit
+    for (const auto &hw : b->host_writes) {
+        if (hw.first <= p->resident_seq) continue;
+        for (const auto &c : p->instrs)
+            if (c.kind == K_WRITE_CONST && overlaps(c.dst, hw.second)) return false;
+    }
+    p->resident_seq = b->write_seq;
+    return true;
+}
+
 // first / stopped_at: a caller that runs unsupported kernels elsewhere dispatches in segments.  With stopped_at given,
 // an instruction that returns FNN_ERR_UNSUPPORTED_OP ends the segment (index in *stopped_at, nothing of it has run)
 // and the caller resumes at the next index; a plan that ever stopped this way is not replayed as a graph.
@@ -1124,18 +1145,8 @@ int dispatch_impl(fnn_backend *b, fnn_plan *p, uint64_t *elapsed_ns, uint64_t n_
     if (p->arena_size > b->arena_bytes) return fail(b, FNN_ERR_MEMORY, "dispatch: plan needs an arena of %llu bytes, backend holds %llu", (unsigned long long)p->arena_size, (unsigned long long)b->arena_bytes);
     if (elapsed_ns && n_elapsed < p->instrs.size()) return fail(b, FNN_ERR_DISPATCH, "dispatch_profile: room for %llu timings, plan has %llu instructions", (unsigned long long)n_elapsed, (unsigned long long)p->instrs.size());
     if (!p->analysed) analyse(p);
-    bool resident = p->resident_uid == b->uid && p->resident_generation == b->generation;
-    if (first > 0) resident = p->segment_resident;   // later segment of one pass: as the first segment found it
-    else if (resident && p->resident_seq != b->write_seq) {
-        // the host wrote into the arena since: still resident unless a constant was hit
-        for (const auto &hw : b->host_writes) {
-            if (hw.first <= p->resident_seq) continue;
-            for (const auto &c : p->instrs)
-                if (c.kind == K_WRITE_CONST && overlaps(c.dst, hw.second)) { resident = false; break; }
-            if (!resident) break;
-        }
-        if (resident) p->resident_seq = b->write_seq;
-    }
+    p->last_halved = false;
+    const bool resident = first > 0 ? p->segment_resident : constants_in_place(b, p);   // (later segment of one pass: as the first segment found it)
 
     // Replay: a plan whose constants are in place, whose weights are all cached and whose
     // workspaces have their final size launches as one HIP graph (the executor's static-shape
@@ -1243,6 +1254,207 @@ int read_slice(fnn_backend *b, uint64_t offset, void *out, uint64_t size)
     if (size == 0) return FNN_OK;
     if (!out) return fail(b, FNN_ERR_DISPATCH, "read_arena: NULL destination");
     return lift(b, fnn_ctx_copy_out(b->ctx, out, b->arena + offset, size));
+}
+
+// ---- a forward pass in two halves of its images: while the first is computed the second's input is on its way, and while
+// the second is computed the first's results are.  A plan of the whole batch and its halves leave the same bytes in the arena: the
+// instructions below work image by image, in integers or value by value, so what an image's results are does not depend on how
+// many go together.
+fnn_slice half_of(const fnn_slice &s, int g) { return {s.offset + (uint64_t)g * (s.size / 2), s.size / 2}; }
+
+uint64_t next_plan_uid()
+{
+    static std::atomic<uint64_t> next{1};
+    return next++;
+}
+
+// The call `in` on half g of `images` images; false: it does not work image by image, or its slices are not what its sizes say.
+bool halve(const Instr &in, uint64_t images, int g, Instr *out)
+{
+    if (in.kind != K_CALL || in.has_param_dims || in.has_secondary || in.inputs.empty()) return false;
+    const uint64_t elems = in.dst.size / 4, in0 = in.inputs[0].size / 4;
+    const std::vector<uint64_t> &p = in.params;
+    *out = in;
+    size_t tensors = in.inputs.size();   // the first of the inputs are tensors of images, the others constants
+    for (const fnn_slice &s : in.inputs)
+        if (overlaps(s, in.dst)) return false;
+    ConvInput ci;
+    if (ranged_conv_input(in, &ci)) {
+        if (ci.images != images || in.inputs.size() > 3 || in.meta.shape.empty() || p[0] == 0 || p[2] == 0) return false;
+        const uint64_t eh = p[2] * (p[7] - 1) + 1, ew = p[2] * (p[8] - 1) + 1, h = p[5] + 2 * p[1], w = p[6] + 2 * p[1];
+        if (p[7] < 1 || p[8] < 1 || h < eh || w < ew) return false;
+        if (elems != images * in.meta.shape[0] * ((h - eh) / p[0] + 1) * ((w - ew) / p[0] + 1)) return false;
+        tensors = 1;
+    } else if (in.kernel == "add_f32") {
+        if (in.inputs.size() != 2 || in0 != elems || in.inputs[1].size / 4 != elems) return false;
+    } else if (in.kernel == "relu_f32" || in.kernel == "gelu_f32" || in.kernel == "silu_f32") {
+        if (in.inputs.size() != 1 || in0 != elems) return false;
+    } else if (in.kernel == "concat") {
+        uint64_t sum = 0;
+        for (const fnn_slice &s : in.inputs) {
+            sum += s.size / 4;
+            if (p.size() < 3 || p[2] == 0 || s.size / 4 % p[2]) return false;
+        }
+        if (p[2] % images || sum != elems) return false;
+        out->params[2] = p[2] / 2;
+    } else if (in.kernel == "slice_f32") {
+        if (in.inputs.size() != 1 || p.size() != 4 || p[2] <= p[1] || p[3] == 0 || elems == 0) return false;
+        const uint64_t range = p[2] - p[1], dim = in0 * range / elems;
+        if (dim == 0 || dim * elems != in0 * range || p[2] > dim || in0 % (dim * p[3]) || in0 / (dim * p[3]) % images) return false;
+    } else if (in.kernel == "pool_f32") {
+        if (in.inputs.size() != 1 || p.size() != 8 || p[4] != images || p[1] == 0 || in0 != images * p[5] * p[6] * p[7]) return false;
+        if (p[6] + 2 * p[2] < p[0] || p[7] + 2 * p[2] < p[0]) return false;
+        if (elems != images * p[5] * ((p[6] + 2 * p[2] - p[0]) / p[1] + 1) * ((p[7] + 2 * p[2] - p[0]) / p[1] + 1)) return false;
+        out->params[4] = images / 2;
+    } else if (in.kernel == "upsample_nearest2d") {
+        if (in.inputs.size() != 1 || p.size() != 4 || p[0] * p[1] * p[2] * p[3] == 0 || in0 % (p[2] * p[3] * images) || elems != in0 * p[0] * p[1]) return false;
+    } else {
+        return false;
+    }
+    auto cut = [&](fnn_slice *s) {
+        if (s->size % (images * 4) || s->size / 2 % 64) return false;   // whole images, and a start as aligned as the slots are
+        *s = half_of(*s, g);
+        return true;
+    };
+    for (size_t i = 0; i < tensors; i++)
+        if (!cut(&out->inputs[i])) return false;
+    return cut(&out->dst);
+}
+
+// Builds p->half once.  Left empty where an instruction is none of those above or the halves could meet in the arena.
+void split_images(fnn_plan *p)
+{
+    if (p->halves_tried) return;
+    p->halves_tried = true;
+    if (p->uploads_every_run || p->has_unsupported) return;
+    uint64_t images = 0;
+    ConvInput ci;
+    for (const Instr &in : p->instrs)
+        if (!images && ranged_conv_input(in, &ci)) images = ci.images;
+    if (images < 2 || images % 2) return;
+    struct Use { fnn_slice s; bool written; };
+    std::vector<Use> uses;                 // tensors of images
+    std::vector<fnn_slice> constants;
+    std::unique_ptr<fnn_plan> h[2];
+    for (int g = 0; g < 2; g++) {
+        h[g].reset(new fnn_plan());
+        h[g]->arena_size = p->arena_size;
+        h[g]->uid = next_plan_uid();
+    }
+    auto use = [&](const fnn_slice &s, bool written) {
+        for (Use &u : uses)
+            if (u.s.offset == s.offset && u.s.size == s.size) { u.written |= written; return; }
+        uses.push_back(Use{s, written});
+    };
+    for (const Instr &in : p->instrs) {
+        if (in.kind == K_WRITE_CONST) {
+            constants.push_back(fnn_slice{in.dst.offset, in.data.size()});
+            continue;
+        }
+        for (int g = 0; g < 2; g++) {
+            Instr part;
+            if (!halve(in, images, g, &part)) return;
+            h[g]->instrs.push_back(std::move(part));
+        }
+        for (size_t i = 0; i < in.inputs.size(); i++) {
+            const bool halved = h[0]->instrs.back().inputs[i].size != in.inputs[i].size;
+            if (halved) use(in.inputs[i], false);
+            else constants.push_back(in.inputs[i]);
+        }
+        use(in.dst, true);
+    }
+    // one half's bytes are never the other's, and constants are nobody's
+    for (const Use &a : uses) {
+        for (const Use &c : uses)
+            if ((a.written || c.written) && overlaps(half_of(a.s, 0), half_of(c.s, 1))) return;
+        for (const fnn_slice &c : constants)
+            if (a.written && overlaps(a.s, c)) return;
+    }
+    for (const Use &a : uses) {
+        bool constant = false;
+        for (const fnn_slice &c : constants) constant |= overlaps(a.s, c);
+        if (!constant) p->halved.push_back(a.s);
+    }
+    for (int g = 0; g < 2; g++) p->half[g] = std::move(h[g]);
+}
+
+// Whether this forward pass goes in halves.  A half costs all of the plan's launches again, about 7 us each where the images are
+// few; what it hides is half of the bytes, 57 GB/s either way.  A YOLOv8n-shaped backbone and neck at 640 x 640 (69 calls): 16 images, 124
+// MB, 3.78 -> 3.29 ms, 12 images 2.97 -> 2.80; 8 images, 62 MB, would gain what the runs differ by.  Four parts gain no more (the launches again).
+bool forward_in_halves(fnn_backend *b, fnn_plan *p, const fnn_host_slice *inputs, uint64_t n_inputs, const fnn_host_slice *outputs, uint64_t n_outputs)
+{
+    constexpr uint64_t kBytesPerCall = 900u << 10, kLeast = 4u << 20;
+    // (the first pass goes whole and leaves the constants and the weights in place, the second as the plan's graph)
+    if (!b->graph_replay || !p->last_replayed || !b->arena || p->arena_size > b->arena_bytes || !p->analysed || p->has_unsupported || !n_inputs || !n_outputs) return false;
+    uint64_t bytes = 0;
+    for (uint64_t i = 0; i < n_inputs; i++) {
+        if (inputs[i].size < kLeast || !inputs[i].data) return false;
+        bytes += inputs[i].size;
+    }
+    for (uint64_t i = 0; i < n_outputs; i++) {
+        if (!outputs[i].data) return false;
+        bytes += outputs[i].size;
+    }
+    uint64_t calls = 0;
+    for (const Instr &in : p->instrs) calls += in.kind == K_CALL;
+    if (bytes < calls * kBytesPerCall) return false;
+    split_images(p);
+    if (!p->half[0]) return false;
+    auto halved = [&](uint64_t offset, uint64_t size) {
+        for (const fnn_slice &s : p->halved)
+            if (s.offset == offset && s.size == size) return true;
+        return false;
+    };
+    for (uint64_t i = 0; i < n_inputs; i++)
+        if (!halved(inputs[i].offset, inputs[i].size)) return false;
+    for (uint64_t i = 0; i < n_outputs; i++) {
+        if (!halved(outputs[i].offset, outputs[i].size)) return false;
+        for (uint64_t k = 0; k < n_inputs; k++) {   // the first half's results come while the second's input is read
+            const uintptr_t o = reinterpret_cast<uintptr_t>(outputs[i].data), x = reinterpret_cast<uintptr_t>(inputs[k].data);
+            if (o < x + inputs[k].size && x < o + outputs[i].size) return false;
+        }
+    }
+    return constants_in_place(b, p);
+}
+
+int run_halves(fnn_backend *b, fnn_plan *p, const fnn_host_slice *inputs, uint64_t n_inputs, const fnn_host_slice *outputs, uint64_t n_outputs)
+{
+    for (auto &h : p->half) {
+        if (h->resident_uid == b->uid && h->resident_generation == b->generation) continue;
+        // Its first pass here: no constants of its own, the weights are there, and with its range tables it can be recorded at once.
+        if (!h->analysed) analyse(h.get());
+        for (size_t i = 0; i < h->instrs.size(); i++) {
+            fnn_slice covered{0, 0};
+            int pending = -1;
+            if (leaves_ranges(h->instrs[i])) request_ranges(b, h.get(), i, &covered, &pending);
+        }
+        *fnn_ctx_range_io(b->ctx) = FnnRangeIo{};
+        clear_ranges(b);
+        h->resident_uid = b->uid; h->resident_generation = b->generation; h->resident_seq = b->write_seq;
+    }
+    int st = lift(b, fnn_ctx_parts_begin(b->ctx));
+    b->write_seq++;
+    for (uint64_t i = 0; i < n_inputs; i++) log_write(b, fnn_slice{inputs[i].offset, inputs[i].size});
+    for (int g = 0; g < 2 && !st; g++) {
+        for (uint64_t i = 0; i < n_inputs && !st; i++) {
+            const fnn_slice s = half_of(fnn_slice{inputs[i].offset, inputs[i].size}, g);
+            st = lift(b, fnn_ctx_part_in(b->ctx, g, b->arena + s.offset, (const uint8_t *)inputs[i].data + (uint64_t)g * s.size, s.size));
+        }
+        if (!st) st = dispatch_impl(b, p->half[g].get(), nullptr, 0, 0, nullptr, false);
+        if (!st) st = lift(b, fnn_ctx_part_mark(b->ctx, g));
+    }
+    for (int g = 0; g < 2 && !st; g++)
+        for (uint64_t i = 0; i < n_outputs && !st; i++) {
+            const fnn_slice s = half_of(fnn_slice{outputs[i].offset, outputs[i].size}, g);
+            st = lift(b, fnn_ctx_part_out(b->ctx, g, (uint8_t *)outputs[i].data + (uint64_t)g * s.size, b->arena + s.offset, s.size));
+        }
+    if (st) return st;
+    p->last_halved = true;
+    p->last_replayed = p->half[0]->last_replayed && p->half[1]->last_replayed;
+    p->ranges_used = p->half[0]->ranges_used;
+    p->residuals_fused = p->half[0]->residuals_fused;
+    p->operands_handed = p->half[0]->operands_handed;
+    return FNN_OK;
 }
 
 }  // namespace
@@ -1360,18 +1572,15 @@ int fnn_plan_create(uint64_t arena_size, fnn_plan **out)
 {
     return guarded(nullptr, "fnn_plan_create", [&]() -> int {
         if (!out) return fail(nullptr, FNN_ERR_DISPATCH, "fnn_plan_create: out is NULL");
-        static std::atomic<uint64_t> next_uid{1};
         *out = new fnn_plan();
         (*out)->arena_size = arena_size;
-        (*out)->uid = next_uid++;
+        (*out)->uid = next_plan_uid();
         return FNN_OK;
     });
 }
 
 void fnn_plan_destroy(fnn_plan *p)
 {
-    if (!p) return;
-    if (p->graph) fnn_hip_graph_destroy(nullptr, p->graph);   // every dispatch ends with a sync: nothing in flight
     delete p;
 }
 
@@ -1382,6 +1591,7 @@ int fnn_plan_replayed(const fnn_plan *p) { return p && p->last_replayed ? 1 : 0;
 uint64_t fnn_plan_ranges_used(const fnn_plan *p) { return p ? p->ranges_used : 0; }
 uint64_t fnn_plan_residuals_fused(const fnn_plan *p) { return p ? p->residuals_fused : 0; }
 uint64_t fnn_plan_operands_handed(const fnn_plan *p) { return p ? p->operands_handed : 0; }
+int fnn_plan_halved(const fnn_plan *p) { return p && p->last_halved ? 1 : 0; }
 
 static void touched(fnn_plan *p)
 {
@@ -1390,6 +1600,9 @@ static void touched(fnn_plan *p)
     p->uploads_every_run = false;
     p->resident_uid = 0;
     p->revision++;
+    p->half[0].reset();
+    p->half[1].reset();
+    p->halves_tried = false;
     if (p->graph) {
         fnn_hip_graph_destroy(nullptr, p->graph);
         p->graph = nullptr;
@@ -1535,9 +1748,13 @@ int fnn_backend_forward(fnn_backend *b, fnn_plan *p, const fnn_host_slice *input
         b->shape_env.clear();
         b->shape_env_sig.clear();
         int st = FNN_OK;
-        for (uint64_t i = 0; i < n_inputs && !st; i++) st = write_slice(b, inputs[i].offset, inputs[i].data, inputs[i].size, true);
-        if (!st) st = dispatch_impl(b, p, nullptr, 0, 0, nullptr, false);
-        for (uint64_t i = 0; i < n_outputs && !st; i++) st = read_slice(b, outputs[i].offset, outputs[i].data, outputs[i].size);
+        if (forward_in_halves(b, p, inputs, n_inputs, outputs, n_outputs)) {
+            st = run_halves(b, p, inputs, n_inputs, outputs, n_outputs);
+        } else {
+            for (uint64_t i = 0; i < n_inputs && !st; i++) st = write_slice(b, inputs[i].offset, inputs[i].data, inputs[i].size, true);
+            if (!st) st = dispatch_impl(b, p, nullptr, 0, 0, nullptr, false);
+            for (uint64_t i = 0; i < n_outputs && !st; i++) st = read_slice(b, outputs[i].offset, outputs[i].data, outputs[i].size);
+        }
         if (!st) return lift(b, fnn_ctx_wait(b->ctx));
         fnn_hip_sync(b->ctx);
         fnn_ctx_drop(b->ctx);

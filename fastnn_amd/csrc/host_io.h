@@ -26,6 +26,17 @@ struct FnnHostIo {
 
     bool touched = false;               // transfers from or to the caller's own (pinned) memory may be under way
 
+    // A call that works in parts: the transfers of one part pass beside the kernels of another, inputs on `ahead`, outputs on `behind`
+    // (made on first use, at the default priority).  The stream `s` waits for a part's input, `behind` for its mark.
+    static constexpr int kParts = 2;
+    hipStream_t ahead = nullptr, behind = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_in[kParts] = {}, ev_part[kParts] = {}, ev_out = nullptr;
+    bool out_behind = false;            // `behind` has transfers that no wait has joined yet
+    hipError_t begin_parts(hipStream_t s);                                                   // behind everything enqueued on s so far
+    hipError_t in_part(hipStream_t s, int part, void *dst, const void *src, size_t bytes);   // more than kSmallTransfer; src held
+    hipError_t mark_part(hipStream_t s, int part);                                           // the part's kernels are enqueued
+    hipError_t out_part(int part, void *dst, const void *src, size_t bytes);
+
     void destroy();
     // enqueues host -> device; the transfer is done when the stream gets there.  held: the caller leaves `src` alone until the
     // wait that ends its call (also one that fails: abandon); else it may be reused on return

@@ -125,6 +125,45 @@ void FnnHostIo::destroy()
     if (flag) (void)hipHostFree(flag);
     small = nullptr;
     flag = nullptr;
+    for (hipStream_t *t : {&ahead, &behind})
+        if (*t) {
+            (void)hipStreamSynchronize(*t);
+            (void)hipStreamDestroy(*t);
+            *t = nullptr;
+        }
+    for (hipEvent_t *e : {&ev_fork, &ev_in[0], &ev_in[1], &ev_part[0], &ev_part[1], &ev_out})
+        if (*e) {
+            (void)hipEventDestroy(*e);
+            *e = nullptr;
+        }
+}
+
+hipError_t FnnHostIo::begin_parts(hipStream_t s)
+{
+    hipError_t e;
+    for (hipStream_t *t : {&ahead, &behind})
+        if (!*t && (e = hipStreamCreateWithFlags(t, hipStreamNonBlocking)) != hipSuccess) return e;
+    for (hipEvent_t *v : {&ev_fork, &ev_in[0], &ev_in[1], &ev_part[0], &ev_part[1], &ev_out})
+        if (!*v && (e = hipEventCreateWithFlags(v, hipEventDisableTiming)) != hipSuccess) return e;
+    if ((e = hipEventRecord(ev_fork, s)) != hipSuccess) return e;
+    return hipStreamWaitEvent(ahead, ev_fork, 0);
+}
+
+hipError_t FnnHostIo::in_part(hipStream_t s, int part, void *dst, const void *src, size_t bytes)
+{
+    hipError_t e;
+    if (bytes <= kSmallTransfer) return hipErrorInvalidValue;   // (those share staging memory that a wait on s hands out anew)
+    if ((e = in(ahead, dst, src, bytes, true)) != hipSuccess || (e = hipEventRecord(ev_in[part], ahead)) != hipSuccess) return e;
+    return hipStreamWaitEvent(s, ev_in[part], 0);
+}
+
+hipError_t FnnHostIo::mark_part(hipStream_t s, int part) { return hipEventRecord(ev_part[part], s); }
+
+hipError_t FnnHostIo::out_part(int part, void *dst, const void *src, size_t bytes)
+{
+    const hipError_t e = hipStreamWaitEvent(behind, ev_part[part], 0);
+    touched = out_behind = true;
+    return e != hipSuccess ? e : hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, behind);
 }
 
 hipError_t FnnHostIo::take_small(hipStream_t s, size_t bytes, size_t align_like, unsigned char **p)
@@ -253,10 +292,16 @@ hipError_t FnnHostIo::wait(hipStream_t s)
         if ((e = hipHostMalloc((void **)&flag, 64, hipHostMallocCoherent)) != hipSuccess) return e;
         *flag = 0;
     }
+    if (out_behind) {   // (`ahead` is joined already: s waits for every input)
+        if ((e = hipEventRecord(ev_out, behind)) == hipSuccess) e = hipStreamWaitEvent(s, ev_out, 0);
+        if (e != hipSuccess) (void)hipStreamSynchronize(behind);
+        out_behind = false;
+    }
     // A word that the stream's last kernel writes reaches the host 3.7 us before hipStreamSynchronize returns; after
     // kSpin of polling the runtime's wait takes over (it is also the one that reports a failed kernel).
     signal_kernel<<<1, 1, 0, s>>>(flag, ++epoch);
-    if ((e = hipGetLastError()) == hipSuccess) {
+    if (hipError_t launched = hipGetLastError(); e == hipSuccess) e = launched;
+    if (e == hipSuccess) {
         const auto until = std::chrono::steady_clock::now() + kSpin;
         for (int i = 1; !(seen = __atomic_load_n(flag, __ATOMIC_ACQUIRE) == epoch); i++) {
             _mm_pause();
@@ -279,6 +324,12 @@ hipError_t FnnHostIo::wait(hipStream_t s)
 
 void FnnHostIo::abandon(hipStream_t s)
 {
+    if (ahead) {
+        (void)hipStreamSynchronize(ahead);
+        (void)hipStreamSynchronize(s);   // (`behind` waits for marks on it)
+        if (behind) (void)hipStreamSynchronize(behind);
+        out_behind = false;
+    }
     if (touched) (void)hipStreamSynchronize(s);
     touched = false;
     pending.clear();   // (what it staged stays taken until the next wait)

@@ -93,3 +93,9 @@ int fnn_ctx_copy_in(fnn_hip_ctx *ctx, void *dst_dev, const void *src, size_t byt
 int fnn_ctx_copy_out(fnn_hip_ctx *ctx, void *dst, const void *src_dev, size_t bytes);
 int fnn_ctx_wait(fnn_hip_ctx *ctx);
 void fnn_ctx_drop(fnn_hip_ctx *ctx);
+// The same for a call that works in two parts (host_io.h): between begin and fnn_ctx_wait (fnn_ctx_drop) a part's input, its kernels on
+// the context's stream, its mark, and its outputs, which may be asked for once both parts are marked.
+int fnn_ctx_parts_begin(fnn_hip_ctx *ctx);
+int fnn_ctx_part_in(fnn_hip_ctx *ctx, int part, void *dst_dev, const void *src, size_t bytes);
+int fnn_ctx_part_mark(fnn_hip_ctx *ctx, int part);
+int fnn_ctx_part_out(fnn_hip_ctx *ctx, int part, void *dst, const void *src_dev, size_t bytes);

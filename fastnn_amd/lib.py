@@ -69,7 +69,7 @@ BACKEND_SYMBOLS = [
     "fnn_backend_set_kernel_flags", "fnn_backend_set_graph_replay", "fnn_backend_set_option",
     "fnn_backend_allocate_arena", "fnn_backend_write_arena", "fnn_backend_read_arena",
     "fnn_plan_create", "fnn_plan_destroy", "fnn_plan_add_write_const", "fnn_plan_add_fill",
-    "fnn_plan_add_memcopy", "fnn_plan_add_call_kernel", "fnn_plan_len", "fnn_plan_replayed", "fnn_plan_ranges_used", "fnn_plan_residuals_fused", "fnn_plan_operands_handed", "fnn_plan_arena_size",
+    "fnn_plan_add_memcopy", "fnn_plan_add_call_kernel", "fnn_plan_len", "fnn_plan_replayed", "fnn_plan_ranges_used", "fnn_plan_residuals_fused", "fnn_plan_operands_handed", "fnn_plan_halved", "fnn_plan_arena_size",
     "fnn_plan_set_param_dims", "fnn_plan_from_bincode", "fnn_plan_to_bincode", "fnn_plan_describe",
     "fnn_backend_dispatch", "fnn_backend_forward", "fnn_backend_dispatch_env", "fnn_backend_dispatch_from", "fnn_backend_dispatch_profile",
     "fnn_backend_dispatch_profile_env",
@@ -217,6 +217,7 @@ def _prototype(l):
     l.fnn_plan_residuals_fused.restype = C.c_uint64
     l.fnn_plan_operands_handed.argtypes = [_vp]
     l.fnn_plan_operands_handed.restype = C.c_uint64
+    l.fnn_plan_halved.argtypes = [_vp]
     l.fnn_backend_dispatch.argtypes = [_vp, _vp]
     l.fnn_backend_forward.argtypes = [_vp, _vp, C.POINTER(HostSlice), _u64, C.POINTER(HostSlice), _u64]
     l.fnn_backend_dispatch_env.argtypes = [_vp, _vp, C.POINTER(C.c_char_p), C.POINTER(_u64), _u64]

@@ -152,6 +152,9 @@ uint64_t fnn_plan_residuals_fused(const fnn_plan *p);
 /* MatMul instructions of the plan that, on its last pass (or in its recorded graph), found their activation operand
  * prepared by the split-K reduction of the MatMul before them (FNN_OPT_FUSE_PREP; no counterpart in fastnn). */
 uint64_t fnn_plan_operands_handed(const fnn_plan *p);
+/* 1: the plan's last pass was a forward pass in two halves of its images (transfers of one half beside the kernels of the
+ * other; the results and the arena are those of the whole pass) */
+int fnn_plan_halved(const fnn_plan *p);
 /* Backend::dispatch_profile, src/backend/mod.rs:178-211: elapsed_ns[i] per instruction */
 int fnn_backend_dispatch_profile(fnn_backend *b, fnn_plan *p, uint64_t *elapsed_ns, uint64_t n);
 /* The same under the ShapeEnv the trait method is handed (symbolic param_dims are resolved against it, as

@@ -1,0 +1,90 @@
+"""A forward pass in two halves of its images (transfers of one half beside the kernels of the other) leaves the bytes that the whole
+pass leaves: in the outputs, in every other value, call after call; plans that do not work image by image go whole."""
+import numpy as np
+import pytest
+
+from fastnn_amd.aot import AotExecutor
+
+pytestmark = pytest.mark.gpu
+
+
+def node(op, inputs, outputs, **attributes):
+    return {"name": outputs[0], "op_type": op, "inputs": "[" + ", ".join(inputs) + "]", "outputs": "[" + ", ".join(outputs) + "]",
+            **{k: str(v) for k, v in attributes.items()}}
+
+
+def graph(rng, size):
+    """Every kind of instruction that is halved: Conv (with an Add, with a Concat behind it), Split, MaxPool, Concat, Resize, Silu, Add."""
+    params = {"w1": rng.standard_normal((16, 3, 3, 3)).astype(np.float32), "b1": rng.standard_normal(16).astype(np.float32),
+              "w2": rng.standard_normal((8, 8, 3, 3)).astype(np.float32) * 0.2, "w3": rng.standard_normal((8, 24, 1, 1)).astype(np.float32) * 0.2}
+    nodes = [node("Conv", ["x", "w1", "b1"], ["c1"], strides=2, pads=1, group=1), node("Silu", ["c1"], ["s1"]), node("Split", ["s1"], ["l", "r"], axis=1),
+             node("Conv", ["r", "w2"], ["c2"], strides=1, pads=1, group=1), node("Add", ["c2", "r"], ["a"]),
+             node("MaxPool", ["a"], ["p"], kernel_shape=5, strides=1, pads=2), node("Concat", ["r", "l", "p"], ["k"], axis=1),
+             node("Conv", ["k", "w3"], ["c3"], strides=1, pads=0, group=1), node("Relu", ["c3"], ["out"]),
+             node("Resize", ["out"], ["up"], mode="nearest", scale_h=2, scale_w=2)]
+    return nodes, params
+
+
+def executor(rng, batch, size, quantize=8, outputs=("up", "out")):
+    nodes, params = graph(rng, size)
+    return AotExecutor(nodes, params, ["x"], list(outputs), {"x": [batch, 3, size, size]}, quantize=quantize)
+
+
+@pytest.mark.parametrize("quantize", [8, 4])
+@pytest.mark.parametrize("batch,size", [(2, 640), (6, 352), (16, 224)])
+def test_the_same_bytes(batch, size, quantize):
+    rng = np.random.default_rng(batch)
+    ex = executor(np.random.default_rng(7), batch, size, quantize)
+    whole = executor(np.random.default_rng(7), batch, size, quantize)
+    whole.set_graph_replay(False)
+    try:
+        for call in range(6):     # the first two go whole, the second as a graph, the others as the graphs of their halves
+            x = rng.standard_normal((batch, 3, size, size)).astype(np.float32) * (call + 1)
+            got, want = ex.forward({"x": x}), whole.forward({"x": x})
+            assert not whole._plan.halved and ex._plan.halved == (call > 1)
+            assert ex.replayed == (call > 0)
+            for name in want:
+                assert got[name].tobytes() == want[name].tobytes(), (call, name)
+            for name in ("l", "a", "p", "k"):
+                assert ex.read_output(name).tobytes() == whole.read_output(name).tobytes(), (call, name)
+            # between the passes: the whole plan on other inputs, and on these again
+            if call == 3:
+                y = x[::-1].copy()
+                ex.write_inputs({"x": y})
+                ex.dispatch()
+                whole.write_inputs({"x": y})
+                whole.dispatch()
+                assert ex.read_output("up").tobytes() == whole.read_output("up").tobytes()
+    finally:
+        ex.close()
+        whole.close()
+
+
+def test_what_goes_whole():
+    """An odd number of images, one image, floating-point weights (their kernels add in an order that depends on the batch), few bytes."""
+    for batch, size, quantize in ((3, 640, 8), (1, 1024, 8), (2, 640, "f8"), (2, 64, 8)):
+        ex = executor(np.random.default_rng(7), batch, size, quantize)
+        x = np.random.default_rng(1).standard_normal((batch, 3, size, size)).astype(np.float32)
+        first = ex.forward({"x": x})
+        for _ in range(3):
+            again = ex.forward({"x": x})
+            assert not ex._plan.halved
+            assert all(again[n].tobytes() == first[n].tobytes() for n in first)
+        ex.close()
+
+
+def test_results_in_memory_of_the_input():
+    """The caller may have the results written over its input: that pass goes whole."""
+    batch, size = 2, 640
+    rng = np.random.default_rng(3)
+    ex = executor(np.random.default_rng(7), batch, size, outputs=("up",))
+    x = rng.standard_normal((batch, 3, size, size)).astype(np.float32)
+    want = ex.forward({"x": x})["up"].copy()
+    slots = [ex._values[n].slot[0] for n in ("x", "up")]
+    buffer = np.empty(max(x.size, want.size), np.float32)
+    for _ in range(4):
+        buffer[:x.size] = x.reshape(-1)
+        ex._backend.forward(ex._plan, [(slots[0], buffer[:x.size])], [(slots[1], buffer[:want.size])])
+        assert not ex._plan.halved
+        assert buffer[:want.size].tobytes() == want.tobytes()
+    ex.close()
