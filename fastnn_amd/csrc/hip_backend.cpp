@@ -1434,7 +1434,10 @@ int run_halves(fnn_backend *b, fnn_plan *p, const fnn_host_slice *inputs, uint64
     }
     int st = lift(b, fnn_ctx_parts_begin(b->ctx));
     b->write_seq++;
-    for (uint64_t i = 0; i < n_inputs; i++) log_write(b, fnn_slice{inputs[i].offset, inputs[i].size});
+    for (uint64_t i = 0; i < n_inputs; i++) {   // (as write_slice: another plan's weights may have been there)
+        drop_weights_overlapping(b, fnn_slice{inputs[i].offset, inputs[i].size});
+        log_write(b, fnn_slice{inputs[i].offset, inputs[i].size});
+    }
     for (int g = 0; g < 2 && !st; g++) {
         for (uint64_t i = 0; i < n_inputs && !st; i++) {
             const fnn_slice s = half_of(fnn_slice{inputs[i].offset, inputs[i].size}, g);
