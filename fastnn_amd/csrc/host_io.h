@@ -4,7 +4,7 @@
 // either way.  Up to kSmallTransfer bytes a copy kernel in the stream reads (writes) the pinned staging memory: it costs
 // one dependent launch, 3.5 us, where a transfer by the copy engine between kernels of the stream costs two hand-overs
 // between queues (64 KB in, a kernel, 64 KB out: 18 against 30 us).  From there on the copy engine's rate is the better
-// one (5 MB: 99 against 132 us); the blocks of a large input are copied into staging memory by several threads while the
+// one (5 MB in: 99 against 132 us; results that go to pinned memory stay with the kernel up to 8 MB); the blocks of a large input are copied into staging memory by several threads while the
 // engine moves those before them.
 #pragma once
 #include <hip/hip_runtime.h>
