@@ -4,7 +4,7 @@
 // rows) asks for 224 bytes per k-value with 8-bit and 160 with 4-bit weights against 12 clocks of its SIMD's matrix core, so
 // the four waves of a CU need 14 and 10 clocks of L1 time in the same 12.  No LDS, no barrier: the operands lie in memory in
 // fragment order, a wave's load is contiguous, and RING steps of 32 k-values are in flight per wave.  What is left at large M
-// is the epilogue, which nothing overlaps at one wave per SIMD (10 to 15 us per round of tiles), and a matrix core that is
+// is the epilogue, which nothing overlaps at one wave per SIMD (7 to 12 us per round of tiles), and a matrix core that is
 // busy half the time: I8 4096 x 4096 M = 2048 1.88 POP/s, matrix cores busy 47 % of the launch's clocks, waves waiting 24 % of
 // theirs; M = 256 (one tile per CU, a chain of latencies) 21 % and 31 %.
 // Measured against the LDS tiles of qgemm_digits.hip: I8 4096 x 4096 M = 256 29.6 -> 27.4 us, M = 1024 72.5 -> 65.5,
@@ -22,6 +22,7 @@ namespace {
 using namespace dech;
 typedef int wi32x4 __attribute__((ext_vector_type(4)));
 typedef int wi32x16 __attribute__((ext_vector_type(16)));
+typedef float wf32x4 __attribute__((ext_vector_type(4)));
 
 // Operand rows in groups of 24 = 8 activation rows x 3 planes (plane j in rows [8j, 8j + 8) of the group).  WK: waves of the
 // four that share an output tile and split K (they meet in LDS at the end); the others lie side by side (WK = 1: 2 x 2,
@@ -35,8 +36,8 @@ __global__ void __launch_bounds__(256, 1) qgemm_wave_kernel(WaveArgs p)
     constexpr int RING = WAVE_RING(W8);                // steps in flight, and the unit in which K is dealt out
     constexpr int SHIFT = DT == FNN_DT_I4 ? 4 : 0;     // 4-bit signed lanes enter as 16 q
     constexpr int WL = W8 ? RING : RING / 2;           // weight loads per ring: a 16-byte piece is one step or two
-    extern __shared__ __attribute__((aligned(16))) float wred[];   // [wave][value][lane]
-    __shared__ int2 row_const[4][WAVE_ROWS];
+    extern __shared__ __attribute__((aligned(16))) wf32x4 wred[];   // [wave][group of rows][column block][lane]
+    __shared__ __attribute__((aligned(16))) int2 row_const[4][WAVE_ROWS];
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, h = lane >> 5;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wk = WK == 1 ? 0 : (WK == 2 ? wv >> 1 : wv);
@@ -67,7 +68,6 @@ __global__ void __launch_bounds__(256, 1) qgemm_wave_kernel(WaveArgs p)
 
     // Row and column constants of the outputs: requested before the last unit, so that the epilogue, which nothing overlaps
     // on this SIMD, does not begin with a trip to memory.
-    auto slot_row = [&](int r) { return (r >> 2) * 8 + h * 4 + (r & 3); };   // of a lane's 16 row slots
     float sc[TN], zp[TN], bi[TN];
     int rexp = 0;
     float xsum = 0.0f;
@@ -154,71 +154,102 @@ __global__ void __launch_bounds__(256, 1) qgemm_wave_kernel(WaveArgs p)
     }
 
     // D: acc[i][j][e] is operand row 32 i + (e / 4) * 8 + h * 4 + e % 4, column 32 j + lr.
-    // A value of this lane, (row slot r, column block j): the three planes of one activation row combined
-    auto value = [&](int r, int j) {
+    // A value of this lane, (row 8 g + 4 h + t, column block j): the three planes of one activation row combined
+    auto value = [&](int g, int t, int j) {
         float v = 0.0f;
 #pragma unroll
         for (int d = 2; d >= 0; d--) {
-            const int slab = 3 * (r >> 2) + d;
-            v = fmaf(v, 256.0f, (float)acc[slab >> 2][j][(slab & 3) * 4 + (r & 3)]);
+            const int slab = 3 * g + d;
+            v = fmaf(v, 256.0f, (float)acc[slab >> 2][j][(slab & 3) * 4 + t]);
         }
         return v;
     };
     if (h == 0) row_const[wv][lr] = make_int2(rexp, __float_as_int(xsum));
-    const bool has_bias = p.bias != nullptr;
-    // row slot r, its TN values
-    auto finish = [&](int r, const float (&v)[TN]) {
-        const int64_t m = m0 + slot_row(r);
-        if (m >= p.m) return;
-        float o[TN];
-        const int2 rc = row_const[wv][slot_row(r)];
-        const bool bad = rc.x == INT_MIN;   // a non-finite row
+    // The waves that split K hand each other their sums through LDS, four rows of a column as one piece, and share the groups of rows.
+    // Then scale, bias, activation and stores, each in a pass of its own with its uniform test in front: nothing overlaps this part at one
+    // wave per SIMD, and a wave fetches its code to run it once (0.25 us a KB).  Against single values
+    // through LDS and the formula in a loop over rows, the kernel alone: I8 4096 x 4096 M = 256 19.6 -> 18.6 us, M = 2048 108 -> 102, 2048 x 8192
+    // M = 1024 66 -> 59, I4 4096 x 4096 M = 1536 83 -> 78.
+    constexpr int OWN = 4 / WK;   // groups of rows that this wave finishes
+    float o[OWN][4][TN];
+    if constexpr (WK == 1) {
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const float d = bad ? __builtin_nanf("") : ldexpf(v[j], -rc.x - SHIFT);
-            o[j] = d * sc[j] + zp[j] * __int_as_float(rc.y);
-        }
-        if (has_bias)
+        for (int x = 0; x < OWN; x++)
 #pragma unroll
-            for (int j = 0; j < TN; j++) o[j] = o[j] + bi[j];
-        if (p.act != FNN_ACT_NONE)
+            for (int t = 0; t < 4; t++)
 #pragma unroll
-            for (int j = 0; j < TN; j++) o[j] = fnn_activation(o[j], p.act);
-        const int64_t at = m * p.n + n0 + lr;
+                for (int j = 0; j < TN; j++) o[x][t][j] = value(x, t, j);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            if (n0 + j * 32 + lr >= p.n) continue;
-            p.out[at + j * 32] = o[j];
-            if (p.residual) p.sum_out[at + j * 32] = o[j] + p.residual[at + j * 32];
-        }
+        for (int g = 0; g < 4; g++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) wred[((wv * 4 + g) * TN + j) * 64 + lane] = wf32x4{value(g, 0, j), value(g, 1, j), value(g, 2, j), value(g, 3, j)};
+        __syncthreads();
+        const wf32x4 *q = wred + ((wn * 4 + wk * OWN) * TN) * 64 + lane;   // (the partners lie WN waves apart)
+#pragma unroll
+        for (int x = 0; x < OWN; x++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                wf32x4 v = q[(x * TN + j) * 64];
+#pragma unroll
+                for (int y = 1; y < WK; y++) v += q[((y * WN * 4 + x) * TN + j) * 64];
+#pragma unroll
+                for (int t = 0; t < 4; t++) o[x][t][j] = v[t];
+            }
+    }
+#pragma unroll
+    for (int x = 0; x < OWN; x++) {
+        const wi32x4 *rc = reinterpret_cast<const wi32x4 *>(&row_const[wv][(wk * OWN + x) * 8 + h * 4]);
+        const wi32x4 r01 = rc[0], r23 = rc[1];
+        const int re[4] = {r01[0], r01[2], r23[0], r23[2]}, rs[4] = {r01[1], r01[3], r23[1], r23[3]};
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                const float d = re[t] == INT_MIN ? __builtin_nanf("") : ldexpf(o[x][t][j], -re[t] - SHIFT);   // (a non-finite row)
+                o[x][t][j] = d * sc[j] + zp[j] * __int_as_float(rs[t]);
+            }
+    }
+    auto every = [&](auto f) {
+#pragma unroll
+        for (int x = 0; x < OWN; x++)
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) f(x, t, j);
     };
-    // The sums go through LDS and the formula runs in a loop over them: unrolled over the registers it is some 40 KB of code
-    // that every wave runs once, and fetching that took 10 us.
-    constexpr int VALUES = 16 * TN, OWN = 16 / WK;
-#pragma unroll
-    for (int r = 0; r < 16; r++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) wred[(wv * VALUES + r * TN + j) * 64 + lane] = value(r, j);
-    __syncthreads();
-    // wave wk finishes its share of the slots; its partners' values lie WN waves apart
-    const float *q = wred + ((WK == 1 ? wv : wn) * VALUES + wk * OWN * TN) * 64 + lane;
-#pragma unroll 2
-    for (int x = 0; x < OWN; x++, q += TN * 64) {
-        float v[TN];
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            v[j] = q[j * 64];
-#pragma unroll
-            for (int y = 1; y < WK; y++) v[j] += q[(y * WN * VALUES + j) * 64];
-        }
-        finish(wk * OWN + x, v);
+    if (p.bias) every([&](int x, int t, int j) { o[x][t][j] = o[x][t][j] + bi[j]; });
+    auto activate = [&](auto a) { every([&](int x, int t, int j) { o[x][t][j] = fnn_activation(o[x][t][j], decltype(a)::value); }); };
+    if (p.act == FNN_ACT_SILU) activate(std::integral_constant<int, FNN_ACT_SILU>{});
+    else if (p.act == FNN_ACT_GELU) activate(std::integral_constant<int, FNN_ACT_GELU>{});
+    else if (p.act == FNN_ACT_RELU) activate(std::integral_constant<int, FNN_ACT_RELU>{});
+    const int64_t base = (m0 + wk * OWN * 8) * p.n + n0;                   // (uniform)
+    const uint32_t lane_at = (uint32_t)(4 * h) * (uint32_t)p.n + (uint32_t)lr;
+    const bool whole = m0 + WAVE_ROWS <= p.m && n0 + WAVE_COLS <= p.n;
+    const int rows = (int)(p.m - m0 < WAVE_ROWS ? p.m - m0 : WAVE_ROWS) - wk * OWN * 8 - 4 * h, cols = (int)(p.n - n0 < WAVE_COLS ? p.n - n0 : WAVE_COLS) - lr;
+    auto store = [&](float *dst) {
+        if (whole) every([&](int x, int t, int j) { (dst + base + (int64_t)(x * 8 + t) * p.n)[lane_at + j * 32] = o[x][t][j]; });
+        else
+            every([&](int x, int t, int j) {
+                if (x * 8 + t < rows && j * 32 < cols) (dst + base + (int64_t)(x * 8 + t) * p.n)[lane_at + j * 32] = o[x][t][j];
+            });
+    };
+    store(p.out);
+    if (p.residual) {
+        every([&](int x, int t, int j) {
+            if (x * 8 + t < rows && j * 32 < cols) o[x][t][j] = o[x][t][j] + (p.residual + base + (int64_t)(x * 8 + t) * p.n)[lane_at + j * 32];
+        });
+        store(p.sum_out);
     }
 }
 
 template <int DT, int WK>
 hipError_t wave_launch_one(const WaveArgs &p, hipStream_t s)
 {
-    constexpr int lds = 4 * 16 * WAVE_COLS / 32 * 256;
+    constexpr int lds = WK == 1 ? 0 : 4 * 16 * WAVE_COLS / 32 * 256;
     auto kern = qgemm_wave_kernel<DT, WK>;
     static std::atomic<uint64_t> raised{0};
     const hipError_t e = fnn_raise_lds_limit(raised, reinterpret_cast<const void *>(kern), lds);
