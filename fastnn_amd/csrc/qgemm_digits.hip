@@ -580,38 +580,36 @@ int run_digits3(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const 
 
 }  // namespace
 
-// Microseconds of preparation + three planes on the LDS tiles: least squares over 1480 drawn calls (M 17 .. 2048, K 256 .. 16384,
-// N 16 .. 16384, weights from memory and from cache; 4 to 7 % mean error)
+// Microseconds of preparation + three planes on the LDS tiles: least squares over 1450 drawn calls (M 17 .. 2048, 8-bit weights from 96
+// on, K 512 .. 8192, N 512 .. 16384, more than 2048 x 2048 elements; 3 to 5 % mean error)
 float fnn_digits3_us(int dt, int64_t m, int64_t n, int64_t k)
 {
-    static const float kFit[3][11] = {   // launch, stage of a round, round, M N / 1e6 per split, second launch, M N, M K, M K of ragged rows, N K / 1e6,
-                                         // workgroups / 256, K / 1e3
-        {7.48f, 0.457f, 0.f, 1.157f, 3.00f, 1.151f, 1.160f, 3.593f, 0.0564f, 2.443f, 0.495f},      // 4-bit, 192 x 128
-        {6.41f, 1.075f, 1.72f, 0.f, 0.f, 0.097f, 0.597f, 3.272f, 0.f, 6.814f, 0.f},                // 4-bit, 192 x 256
-        {3.68f, 0.714f, 2.17f, 0.425f, 4.77f, 0.417f, 1.060f, 1.826f, 0.0286f, 6.016f, 0.265f}};   // 8-bit, 192 x 128
+    static const float kFit[3][12] = {   // launch, stage of a round, round, M N / 1e6 per split, second launch, M N, M K, M K of rows that are no whole
+                                         // float4s, N K / 1e6, workgroups / 256, their stages / 256, stage of a workgroup
+        {0.f, 0.478f, 8.68f, 2.951f, 2.18f, 0.f, 1.201f, 3.19f, 0.0169f, 1.18f, 0.192f, 0.f},      // 4-bit, 192 x 128
+        {5.41f, 0.819f, 3.94f, 0.f, 0.f, 0.664f, 0.801f, 2.21f, 0.f, 0.f, 0.370f, 0.102f},         // 4-bit, 192 x 256
+        {5.42f, 0.446f, 3.56f, 2.313f, 2.92f, 0.f, 1.303f, 2.74f, 0.f, 1.20f, 0.369f, 0.f}};       // 8-bit, 192 x 128
     const bool w8 = dt == FNN_DT_I8;
     const Digits3Form f = digits3_form(!w8, m, n, k);
-    const float *c = kFit[w8 ? 2 : f.wide], rounds = (float)((f.tiles * f.splits + 255) / 256), mn = (float)m * (float)n / 1e6f, mk = (float)m * (float)k / 1e6f;
-    const bool ragged = (w8 ? (k + 3) / 4 : (k + 7) / 8) % 4 != 0;
-    return c[0] + rounds * (c[1] * (float)f.ips + c[2]) + (f.splits > 1 ? c[3] * (float)f.splits * mn + c[4] : 0.f) + c[5] * mn +
-           (c[6] + (ragged ? c[7] : 0.f)) * mk + c[8] * (float)n * (float)k / 1e6f + c[9] * (float)(f.tiles * f.splits) / 256.f + c[10] * (float)k / 1e3f;
+    const float *c = kFit[w8 ? 2 : f.wide], wgs = (float)(f.tiles * f.splits) / 256.f, rounds = (float)((f.tiles * f.splits + 255) / 256);
+    const float mn = (float)m * (float)n / 1e6f, mk = (float)m * (float)k / 1e6f, ips = (float)f.ips;
+    return c[0] + rounds * (c[1] * ips + c[2]) + (f.splits > 1 ? c[3] * (float)f.splits * mn + c[4] : 0.f) + c[5] * mn + (c[6] + (k % 4 ? c[7] : 0.f)) * mk +
+           c[8] * (float)n * (float)k / 1e6f + wgs * (c[9] + c[10] * ips) + c[11] * ips;
 }
 
-// Microseconds of preparation + MatMul on the wave tiles, against the LDS tiles of run_digits3: least squares over 950 drawn calls
-// (M 96 .. 2048, K 256 .. 16384, N 257 .. 16384, weights from memory and from cache; 8 % mean error for 8-bit, 4 to 6 % for 4-bit
-// weights).  Both count whole rounds of workgroups over the 256 CUs: which one ends with the emptier round decides more than
-// their rates do; with few rows the weight's bytes and the steps that a wave walks alone count beside them (without those two
-// 15 % of the I8 calls of 96 .. 160 rows lost more than 3 %, 119 x 6016 x 8704 51.8 us against 42.8; now none, at 0.87 of the LDS tiles'
-// time on average, the best choice 0.86).  Taken from 96 rows on (8-bit weights below have four planes), up to the rows that
-// were measured, where it is ahead by more than 5 %.
+// Microseconds expected of preparation + MatMul on the wave tiles, against the LDS tiles of run_digits3: least squares over the 1200 of those calls
+// from 96 rows on, each form and kernel timed on all of them (2 to 3 % mean error).  Both count whole rounds of workgroups over the 256 CUs: which one ends
+// with the emptier round decides more than their rates do.  On 400 other calls the form and kernel with the lower figure is 0.3 % off the
+// best one on average, five are more than 5 % off; with fits of the kernels as they were before it was 3.2 % (955 x 7610 x 1344 I4
+// 74.5 us on the LDS tiles, 52.0 here).  Taken from 96 rows on (8-bit weights below have four planes), up to the rows that were measured.
 int fnn_wave_choice(int dtype, int64_t m, int64_t n, int64_t k, float *us)
 {
-    static const float kWave[2][3][8] = {   // [8-bit][wk 1, 2, 4]: launch, 100 steps of a round, round, M N / 1e6, M K / 1e6, weight MB, 100 steps of all
-                                            // tiles / 256, 100 steps of a wave
-        {{6.26f, 22.15f, 5.061f, 1.073f, 1.556f, 0.1649f, 1.445f, 0.f}, {4.91f, 21.54f, 5.071f, 0.766f, 1.519f, 0.1213f, 3.563f, 2.75f},
-         {4.99f, 24.77f, 4.294f, 0.165f, 1.970f, 0.1820f, 2.357f, 2.19f}},
-        {{1.21f, 15.25f, 8.626f, 0.664f, 0.519f, 0.2031f, 8.724f, 12.22f}, {3.00f, 18.95f, 6.416f, 0.212f, 0.532f, 0.0494f, 14.53f, 14.06f},
-         {2.92f, 22.45f, 4.955f, 0.034f, 1.345f, 0.1360f, 11.79f, 15.26f}}};
+    static const float kWave[2][3][9] = {   // [8-bit][wk 1, 2, 4]: launch, 100 steps of a round, round, M N / 1e6, M K / 1e6, weight MB, 100 steps of all
+                                            // tiles / 256, 100 steps of a wave, M K of rows that are no whole float4s
+        {{8.16f, 19.12f, 3.40f, 0.924f, 1.089f, 0.f, 6.07f, 1.43f, 0.308f}, {7.16f, 21.68f, 4.14f, 0.817f, 1.218f, 0.0334f, 4.72f, 0.f, 0.346f},
+         {6.73f, 23.65f, 3.81f, 0.505f, 1.512f, 0.0936f, 3.91f, 0.f, 0.373f}},
+        {{7.46f, 21.00f, 3.36f, 1.035f, 1.059f, 0.f, 8.02f, 0.f, 0.295f}, {6.78f, 25.69f, 3.54f, 1.309f, 1.131f, 0.006f, 6.46f, 0.f, 0.281f},
+         {6.35f, 29.38f, 3.42f, 1.094f, 1.584f, 0.0429f, 4.38f, 0.f, 0.492f}}};
     if (dtype != FNN_DT_I8 && dtype != FNN_DT_I4 && dtype != FNN_DT_U4) return 0;
     if (m < 96 || m > 2048 || n * k <= (int64_t)2048 * 2048) return 0;
     const bool w8 = dtype == FNN_DT_I8;
@@ -624,12 +622,12 @@ int fnn_wave_choice(int dtype, int64_t m, int64_t n, int64_t k, float *us)
         const int64_t rows = i == 0 ? 2 * WAVE_ROWS : WAVE_ROWS, cols = i == 2 ? WAVE_COLS : 2 * WAVE_COLS;
         const int64_t tiles = ceil_div(m, rows) * ceil_div(n, cols);
         const float *c = kWave[w8][i], rounds = (float)ceil_div(tiles, 256), steps = (float)(ceil_div(units, 1 << i) * ring) / 100.f;
-        const float t = c[0] + c[1] * rounds * steps + c[2] * rounds + c[3] * mn + c[4] * mk + c[5] * (float)n * (float)k * (w8 ? 1.f : 0.5f) / 1e6f +
-                        c[6] * (float)tiles / 256.f * steps + c[7] * steps;
+        const float t = c[0] + c[1] * rounds * steps + c[2] * rounds + c[3] * mn + (c[4] + (k % 4 ? c[8] : 0.f)) * mk +
+                        c[5] * (float)n * (float)k * (w8 ? 1.f : 0.5f) / 1e6f + c[6] * (float)tiles / 256.f * steps + c[7] * steps;
         if (t < best) { best = t; wk = 1 << i; }
     }
     *us = best;
-    return best < 0.95f * fnn_digits3_us(dtype, m, n, k) ? wk : 0;
+    return best < 0.98f * fnn_digits3_us(dtype, m, n, k) ? wk : 0;
 }
 
 // what the kernels of this file can multiply at all
