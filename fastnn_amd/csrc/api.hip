@@ -896,9 +896,33 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
             // fused-dequant MatMul per group (bias and activation in its epilogue), [pixel, channel] -> NCHW
             const int64_t cg = c / groups, ocg = oc / groups, kk = cg * kh * kw, np = ho * wo, rows = b * np;
             if (rows > (1ll << 31) || b > 65535) return fail(ctx, FNN_ERR_UNSUPPORTED_OP, "conv2d: %lld output pixels exceed the f32 path's limit", (long long)rows);
-            if ((rc = ensure(ctx, ctx->st_col, (size_t)rows * kk * 4 + 256))) return rc;
             if ((rc = ensure(ctx, ctx->st_rows, (size_t)rows * ocg * 4 + 256))) return rc;
-            float *col = (float *)ctx->st_col.ptr, *rows_out = (float *)ctx->st_rows.ptr;
+            float *rows_out = (float *)ctx->st_rows.ptr;
+            // More pixels than the fragment kernels take as rows: the f16 tiles, whose operand comes straight from the image.  (U4 weights
+            // go to digit planes; 31-bit byte offsets and positions.)
+            const int64_t small = 1 << 24;
+            if (groups == 1 && rows > 2048 && w->dtype != FNN_DT_U4 && !(flags & FNN_FLAG_FORCE_GENERIC) && fnn_ctx_option(ctx, FNN_OPT_FRAGMENT) <= 0 &&
+                xin < (1ull << 31) && kk < small && h < small && wd < small && np < (1ll << 31) && pad < small && (ho - 1) * stride < small &&
+                (wo - 1) * stride < small && (int64_t)kh * dil < small && (int64_t)kw * dil < small) {
+                QMatmulArgs q;
+                q.words = w->words; q.scales = w->scales; q.zeros = w->zeros; q.codebook = w->codebook;
+                q.a = nullptr; q.bias = dbias; q.out = rows_out;
+                q.m = rows; q.n = oc; q.k = kk; q.kp = w->kp; q.bpr = w->bpr; q.qblock = w->qblock; q.act = act;
+                q.as_written = 0;
+                const ConvSource src = {dx, (int)c, (int)h, (int)wd, kh, kw, stride, pad, dil, (int)wo, (int)np, (unsigned)xin};
+                bool handled = false;
+                if ((rc = fnn_tiled_qmatmul(ctx, ctx->stream, w, q, flags & FNN_FLAG_ACT_F16_SINGLE, &handled, &src))) return rc;
+                if (handled) {
+                    HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_rows_to_nchw(rows_out, dy, b, np, oc, 0, oc, ctx->stream));
+                    if (!dev) {
+                        if (int rc_ = stage_out(ctx, y, dy, yout)) return rc_;
+                        if (int rc_ = finish(ctx)) return rc_;
+                    }
+                    return FNN_OK;
+                }
+            }
+            if ((rc = ensure(ctx, ctx->st_col, (size_t)rows * kk * 4 + 256))) return rc;
+            float *col = (float *)ctx->st_col.ptr;
             for (int g = 0; g < groups; g++) {
                 HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_im2col_f32(dx, col, b, c, groups, g, h, wd, ho, wo, kh, kw, stride, pad, dil, ctx->stream));
                 if (groups == 1) {

@@ -3,7 +3,8 @@
 // (src/backend/cpu/mod.rs:4204-4257, src/backend/cpu/microkernels/conv.rs:509-660).  Here the
 // im2col matrix [B*Ho*Wo, C/g*KH*KW] is written as f32 rows, the fused-dequant MatMul kernels
 // multiply it with the packed weight rows (bias and activation in their epilogue), and the
-// [pixel, channel] result is turned into NCHW.
+// [pixel, channel] result is turned into NCHW.  (More than 2048 pixels, one group: the matrix is not written, the
+// tiles' operand comes straight from the image, conv_prep_kernel.h.)
 #include "common.h"
 
 namespace {

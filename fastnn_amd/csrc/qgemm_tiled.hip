@@ -275,6 +275,7 @@ __global__ void __launch_bounds__(64) row_umean_kernel(const uint32_t *words, in
 }
 
 #include "tile_kernel.h"
+#include "conv_prep_kernel.h"
 
 // Split-K reduction that also prepares the operand of the MatMul reading this one's result (a plan's next layer):
 // workgroup m owns output row m whole.  Thread (r, tid) of its RW * 256 threads owns the columns 8 * (tid + 256 r),
@@ -568,7 +569,7 @@ int tile_splits(double t_bits, int cfg, int base, int iters, int64_t M, int64_t 
 
 template <int DT>
 int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags,
-              const DenseOperand *dense = nullptr)
+              const ConvSource *conv, const DenseOperand *dense = nullptr)
 {
     const int64_t M = q.m, N = q.n, K = q.k;
     const TileLayout L = tile_layout<DT>(ctx, M, N, K, flags, dense != nullptr);
@@ -603,7 +604,7 @@ int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QM
     FnnPrepIo *pio = fnn_ctx_prep_io(ctx);
     FnnPreparedOperand *have = fnn_ctx_prepared(ctx);
     constexpr int kInterleaved = DecH<DT>::INTERLEAVED ? 1 : 0;
-    const bool handed = pio->offered && !dense && have->buffer && !have->fragments && have->a == q.a && have->m == M && have->k == K && have->kpad == kpad &&
+    const bool handed = pio->offered && !dense && !conv && have->buffer && !have->fragments && have->a == q.a && have->m == M && have->k == K && have->kpad == kpad &&
                         have->rows_pad == rows_pad && have->precise == (precise ? 1 : 0) && have->interleaved == kInterleaved;
     const int own_slot = handed ? have->slot : 0;
     void *ws0 = handed ? have->buffer : nullptr, *ws1 = nullptr;
@@ -634,8 +635,11 @@ int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QM
     pa.interleaved = DecH<DT>::INTERLEAVED ? 1 : 0;
     hipError_t e = hipSuccess;
     if (!handed) {
-        hipLaunchKernelGGL(act_prep_kernel, dim3((unsigned)m_pad), dim3(256), 0, s, pa);
-        e = hipGetLastError();
+        if (conv) e = launch_conv_prep(pa, *conv, m_pad, s);
+        else {
+            hipLaunchKernelGGL(act_prep_kernel, dim3((unsigned)m_pad), dim3(256), 0, s, pa);
+            e = hipGetLastError();
+        }
         if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
     }
 
@@ -781,7 +785,7 @@ __global__ void __launch_bounds__(256) expand_codebook_kernel(const uint32_t *wo
     }
 }
 
-int run_tiled_codebook(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags)
+int run_tiled_codebook(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, const ConvSource *conv)
 {
     const int64_t kpad = (q.k + BK - 1) / BK * BK;
     const size_t op_bytes = (size_t)q.n * 2 * kpad * 2;
@@ -812,7 +816,7 @@ int run_tiled_codebook(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w,
         if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
     }
     DenseOperand d{(const uint32_t *)op, row_scale, row_zero};
-    return run_tiled<DT_F16_DENSE>(ctx, s, w, q, flags, &d);
+    return run_tiled<DT_F16_DENSE>(ctx, s, w, q, flags, conv, &d);
 }
 
 }  // namespace
@@ -861,7 +865,8 @@ float fnn_tiled_us(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, in
            (sp > 1 ? c[3] + c[4] * mn * (float)sp : 0.f) + c[5] * mn + (c[6] + (ragged ? c[9] : 0.f)) * mk + c[7] * (float)n * (float)k / 1e6f + c[8] * (float)k / 1e3f;
 }
 
-int fnn_tiled_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, bool *handled)
+int fnn_tiled_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, int flags, bool *handled,
+                      const ConvSource *conv)
 {
     *handled = false;
     const int64_t min_m = fnn_ctx_option(ctx, FNN_OPT_TILE_MIN_M);
@@ -884,13 +889,13 @@ int fnn_tiled_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, 
             int rc;
             if (q.words == w->words && (rc = fnn_aligned_rows(ctx, s, w, &qa.words, &qa.kp))) return rc;
             if (qa.kp % 4 == 0 && !(reinterpret_cast<uintptr_t>(qa.words) & 15)) {
-                rc = run_tiled<FNN_DT_I4CB>(ctx, s, w, qa, flags);
+                rc = run_tiled<FNN_DT_I4CB>(ctx, s, w, qa, flags, conv);
                 if (rc) return rc;
                 *handled = true;
                 return FNN_OK;
             }
         }
-        int rc = run_tiled_codebook(ctx, s, w, q, flags);
+        int rc = run_tiled_codebook(ctx, s, w, q, flags, conv);
         if (rc) return rc;
         *handled = true;
         return FNN_OK;
@@ -904,13 +909,13 @@ int fnn_tiled_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, 
     if (q.words == w->words && (rc = fnn_aligned_rows(ctx, s, w, &qa.words, &qa.kp))) return rc;
     if (qa.kp % 4 != 0 || (reinterpret_cast<uintptr_t>(qa.words) & 15)) return FNN_OK;
     switch (w->dtype) {
-    case FNN_DT_I8: rc = run_tiled<FNN_DT_I8>(ctx, s, w, qa, flags); break;
-    case FNN_DT_I4: rc = run_tiled<FNN_DT_I4>(ctx, s, w, qa, flags); break;
-    case FNN_DT_U8: rc = run_tiled<FNN_DT_U8>(ctx, s, w, qa, flags); break;
-    case FNN_DT_U4: rc = run_tiled<FNN_DT_U4>(ctx, s, w, qa, flags); break;
-    case FNN_DT_F8: rc = run_tiled<FNN_DT_F8>(ctx, s, w, qa, flags); break;
-    case FNN_DT_F8R: rc = run_tiled<FNN_DT_F8R>(ctx, s, w, qa, flags); break;
-    case FNN_DT_F4: rc = run_tiled<FNN_DT_F4>(ctx, s, w, qa, flags); break;
+    case FNN_DT_I8: rc = run_tiled<FNN_DT_I8>(ctx, s, w, qa, flags, conv); break;
+    case FNN_DT_I4: rc = run_tiled<FNN_DT_I4>(ctx, s, w, qa, flags, conv); break;
+    case FNN_DT_U8: rc = run_tiled<FNN_DT_U8>(ctx, s, w, qa, flags, conv); break;
+    case FNN_DT_U4: rc = run_tiled<FNN_DT_U4>(ctx, s, w, qa, flags, conv); break;
+    case FNN_DT_F8: rc = run_tiled<FNN_DT_F8>(ctx, s, w, qa, flags, conv); break;
+    case FNN_DT_F8R: rc = run_tiled<FNN_DT_F8R>(ctx, s, w, qa, flags, conv); break;
+    case FNN_DT_F4: rc = run_tiled<FNN_DT_F4>(ctx, s, w, qa, flags, conv); break;
     default: return FNN_OK;
     }
     if (rc) return rc;

@@ -1,0 +1,71 @@
+"""The f32 Conv2d of more than 2048 output pixels, whose f16 operand comes straight from the image, against im2col rows and their preparation."""
+import numpy as np
+import pytest
+
+import fastnn_amd
+from fastnn_amd import lib as flib
+from gpu_common import assert_close, to_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    with fastnn_amd.HipContext(0) as c:
+        yield c
+
+
+# batch, channels, height, width, output channels, kernel (h, w), stride, padding, dilation
+GEOMETRIES = [
+    (1, 3, 64, 33, 16, 3, 3, 1, 1, 1),      # one k block, part of it padding; 2112 pixels end on no tile
+    (2, 17, 66, 71, 20, 3, 3, 2, 1, 1),     # 153 values; blocks of pixels that span two images
+    (3, 32, 29, 31, 130, 1, 1, 1, 0, 1),    # 1x1
+    (1, 6, 61, 57, 33, 5, 2, 1, 3, 2),      # dilated, a kernel that is not square, more padding than it reaches
+    (1, 64, 50, 47, 48, 3, 3, 1, 1, 1),     # nine k blocks: the most that stay in registers
+    (2, 80, 40, 41, 24, 3, 3, 1, 1, 1),     # 720 values: three blocks read twice
+    (3, 8, 97, 95, 40, 2, 3, 3, 0, 1),      # rows and columns that no tap reaches
+]
+
+
+def both(ctx, handle, x, oc, args, **kw):
+    got = ctx.qconv2d(handle, x, oc, *args, 1, **kw)
+    ctx.set_option(flib.OPT_FRAGMENT, 1)    # (no tile of the fragment kernels: the call runs on im2col rows)
+    try:
+        return got, ctx.qconv2d(handle, x, oc, *args, 1, **kw)
+    finally:
+        ctx.set_option(flib.OPT_FRAGMENT, 0)
+
+
+@pytest.mark.parametrize("wdt", [flib.DT_U8, flib.DT_F8, flib.DT_F8R, flib.DT_F4, flib.DT_I4CB])
+@pytest.mark.parametrize("geo", GEOMETRIES)
+def test_operand_from_the_image_equals_prepared_rows(ctx, orc, geo, wdt):
+    """The operand's halves are the same bits, so is every product; a row sum, which zero points (U8, FP4) multiply, may differ in its
+    last place (f32 of a double against f32 sums: 1e-6 of the sum of magnitudes, as the stated 2e-5 against the oracle)."""
+    b, c, h, w, oc, kh, kw, stride, pad, dil = geo
+    rng = np.random.default_rng(5 + c + oc)
+    kk = c * kh * kw
+    x = rng.uniform(-0.3, 1, (b, c, h, w)).astype(np.float32)
+    bias = (rng.standard_normal(oc) * 0.05).astype(np.float32)
+    pw = fastnn_amd.quantize_weights(wdt, (rng.standard_normal((oc, kk)) * np.sqrt(2.0 / kk)).astype(np.float32))
+    args = (kh, kw, stride, pad, dil)
+    want = orc.qconv2d_float(x, to_oracle(orc, pw), *args, 1, bias=bias, act=flib.ACT_SILU)
+    assert b * want.shape[2] * want.shape[3] > 2048
+    handle = ctx.register(pw)
+    got, rows = both(ctx, handle, x, oc, args, bias=bias, act=flib.ACT_SILU)
+    assert_close(got, want, 2e-5)
+    if wdt in (flib.DT_U8, flib.DT_F4):
+        assert_close(got, rows, 2e-6)
+    else:
+        assert np.array_equal(got, rows)
+    single, rows = both(ctx, handle, x, oc, args, bias=bias, act=flib.ACT_SILU, flags=flib.FLAG_ACT_F16_SINGLE)
+    assert_close(single, rows, 2e-6)
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_not_a_number_and_infinities_as_in_the_rows(ctx, value):
+    rng = np.random.default_rng(9)
+    x = rng.standard_normal((1, 16, 50, 48)).astype(np.float32)
+    x[0, 3, 20, 21] = value
+    handle = ctx.register(fastnn_amd.quantize_weights(flib.DT_F8, rng.standard_normal((24, 144)).astype(np.float32)))
+    got, rows = both(ctx, handle, x, 24, (3, 3, 1, 1, 1))
+    assert np.array_equal(got, rows, equal_nan=True)
