@@ -22,7 +22,6 @@
 
 hipError_t launch_im2col_f32(const float *x, float *col, int64_t b, int64_t c, int groups, int g, int64_t h, int64_t w,
                              int64_t ho, int64_t wo, int kh, int kw, int stride, int pad, int dil, hipStream_t s);
-hipError_t launch_rows_to_nchw(const float *src, float *y, int64_t b, int64_t np, int64_t oc, int64_t ch0, int64_t ocg, hipStream_t s);
 hipError_t launch_fill(float *dst, uint64_t n, float value, hipStream_t s);
 hipError_t launch_eltwise(int op, const float *a, const float *b, uint64_t nb, float *out, uint64_t n, hipStream_t s, FnnRangeIo *rio);
 hipError_t launch_copy2d(float *dst, uint64_t dst_pitch, uint64_t dst_len, const float *src, uint64_t src_pitch, uint64_t src_len,
@@ -909,11 +908,10 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
                 q.a = nullptr; q.bias = dbias; q.out = rows_out;
                 q.m = rows; q.n = oc; q.k = kk; q.kp = w->kp; q.bpr = w->bpr; q.qblock = w->qblock; q.act = act;
                 q.as_written = 0;
-                const ConvSource src = {dx, (int)c, (int)h, (int)wd, kh, kw, stride, pad, dil, (int)wo, (int)np, (unsigned)xin};
+                const ConvSource src = {dx, (int)c, (int)h, (int)wd, kh, kw, stride, pad, dil, (int)wo, (int)np, (unsigned)xin, dy};
                 bool handled = false;
                 if ((rc = fnn_tiled_qmatmul(ctx, ctx->stream, w, q, flags & FNN_FLAG_ACT_F16_SINGLE, &handled, &src))) return rc;
                 if (handled) {
-                    HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_rows_to_nchw(rows_out, dy, b, np, oc, 0, oc, ctx->stream));
                     if (!dev) {
                         if (int rc_ = stage_out(ctx, y, dy, yout)) return rc_;
                         if (int rc_ = finish(ctx)) return rc_;

@@ -64,11 +64,13 @@ int fnn_frag_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, int
 int fnn_row_qsum(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const int32_t **qsum);
 // microseconds expected of the f16 tiles (per-channel types)
 float fnn_tiled_us(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags);
+hipError_t launch_rows_to_nchw(const float *src, float *y, int64_t b, int64_t np, int64_t oc, int64_t ch0, int64_t ocg, hipStream_t s);
 // (conv: the activations are a convolution's windows of its NCHW input, p.m output pixels of p.k values; p.a is not read)
 struct ConvSource {
     const float *x;
     int c, h, w, kh, kw, stride, pad, dil, wo, np;   // np: output pixels of an image
     unsigned bytes;                                  // of x
+    float *y;                                        // the result, [image][channel][np] (p.out: rows, where K is split)
 };
 int fnn_tiled_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p,
                       int flags, bool *handled, const ConvSource *conv = nullptr);

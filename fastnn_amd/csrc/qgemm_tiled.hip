@@ -657,6 +657,11 @@ int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QM
     if (splits > 1) fnn_take_residual(ctx, q.out, M * N, &t.residual, &t.sum_out);
     t.m = M; t.n = N; t.kp = q.kp; t.kpad = kpad; t.rows_pad = rows_pad;
     t.a_wrap = 0;
+    if (conv && splits == 1) {
+        t.cv.y = conv->y;
+        t.cv.np = (uint32_t)conv->np;
+        t.cv.vec4 = conv->np % 4 == 0 && !(reinterpret_cast<uintptr_t>(conv->y) & 15);
+    }
     t.bscales = nullptr; t.codebook = nullptr; t.bpr = 0;
     if constexpr (DT == FNN_DT_I4CB) {
         t.bscales = q.scales; t.codebook = q.codebook; t.bpr = q.bpr;
@@ -692,7 +697,7 @@ int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QM
         // whole rows per workgroup, in the other operand buffer than the one this call's own row tables live in.
         TileLayout NL;
         int n_il = 0;
-        const bool may_prepare = pio->next_w && !dense && !t.codebook && !fnn_ctx_static_mode(ctx) && M >= 17 && N % 64 == 0 && N <= 2048 * PREP_RG &&
+        const bool may_prepare = pio->next_w && !dense && !conv && !t.codebook && !fnn_ctx_static_mode(ctx) && M >= 17 && N % 64 == 0 && N <= 2048 * PREP_RG &&
                                  (pio->next_a == q.out || (t.residual && pio->next_a == t.sum_out)) &&
                                  pio->next_w->inner == N && tile_layout_of(ctx, pio->next_w->dtype, M, pio->next_w->rows, N, pio->next_flags, &NL, &n_il) &&
                                  NL.kpad == N && !((reinterpret_cast<uintptr_t>(t.scales) | reinterpret_cast<uintptr_t>(t.zeros) | reinterpret_cast<uintptr_t>(t.out) |
@@ -727,6 +732,7 @@ int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QM
         if (rowb > 65535) rowb = 65535;
         hipLaunchKernelGGL(splitk_epilogue_kernel, dim3((unsigned)colb, (unsigned)rowb), dim3(256), 0, s, t, precise ? 0 : 1);
         e = hipGetLastError();
+        if (e == hipSuccess && conv) e = launch_rows_to_nchw(q.out, conv->y, M / conv->np, conv->np, N, 0, N, s);
         if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
     }
     return FNN_OK;

@@ -37,7 +37,8 @@ struct TileArgs {
     const float *codebook;
     int64_t bpr;
     // quantised Conv2d epilogue inside the int8 kernel (CONV): scales / zeros / bias above are those of the group's
-    // channels; y and acc_out start at the group's first channel of image 0
+    // channels; y and acc_out start at the group's first channel of image 0.  The f16 kernels read y, np and vec4 only: non-null y
+    // takes the results there instead of to `out` (one group, K in one split)
     struct Conv {
         float *y;                  // [B, OC, np]
         int32_t *acc_out;          // same shape, or null
@@ -94,8 +95,7 @@ __device__ __forceinline__ void wait_loads_but()
 // its own with its (uniform) test in front.  With all of them inside one loop an output was some 60 instructions, 15 to 40 KB of code
 // that a wave fetches and runs once while its matrix core idles.
 template <int R, int TN>
-__device__ __forceinline__ void tile_finish(float (&o)[R][TN], float *dst, int64_t m0, int64_t n0, int64_t m, int64_t n, const float (&bi)[TN], bool has_bias,
-                                            int act, int lr, int h)
+__device__ __forceinline__ void tile_activate(float (&o)[R][TN], const float (&bi)[TN], bool has_bias, int act)
 {
     if (has_bias) {
 #pragma unroll
@@ -112,6 +112,11 @@ __device__ __forceinline__ void tile_finish(float (&o)[R][TN], float *dst, int64
     if (act == FNN_ACT_SILU) activate(std::integral_constant<int, FNN_ACT_SILU>{});
     else if (act == FNN_ACT_GELU) activate(std::integral_constant<int, FNN_ACT_GELU>{});
     else if (act == FNN_ACT_RELU) activate(std::integral_constant<int, FNN_ACT_RELU>{});
+}
+
+template <int R, int TN>
+__device__ __forceinline__ void tile_store(const float (&o)[R][TN], float *dst, int64_t m0, int64_t n0, int64_t m, int64_t n, int lr, int h)
+{
     float *first = dst + m0 * n + n0;
     const uint32_t lane = (uint32_t)(4 * h) * (uint32_t)n + (uint32_t)lr;
     if (m0 + 2 * R <= m && n0 + 32 * TN <= n) {
@@ -129,6 +134,46 @@ __device__ __forceinline__ void tile_finish(float (&o)[R][TN], float *dst, int64
 #pragma unroll
             for (int tn = 0; tn < TN; tn++)
                 if ((r >> 2) * 8 + (r & 3) < rows && tn * 32 < cols) row[lane + tn * 32] = o[r][tn];
+        }
+    }
+}
+
+template <int R, int TN>
+__device__ __forceinline__ void tile_finish(float (&o)[R][TN], float *dst, int64_t m0, int64_t n0, int64_t m, int64_t n, const float (&bi)[TN], bool has_bias,
+                                            int act, int lr, int h)
+{
+    tile_activate<R, TN>(o, bi, has_bias, act);
+    tile_store<R, TN>(o, dst, m0, n0, m, n, lr, h);
+}
+
+// The same outputs, o after bias and activation, as a convolution's [image, channel, pixel]: rows are output pixels.  A lane's four consecutive
+// rows are one 16-byte store where an image has a multiple of four pixels (32 bytes of a channel by the two halves of a wave, whole lines in L2
+// by the wave's passes); instead of rows that another kernel turns: 45 launches of 4 .. 6.5 us in a 640 x 640 detector, F8 weights.
+template <int R, int TN>
+__device__ __forceinline__ void tile_store_nchw(const float (&o)[R][TN], float *y, uint32_t np, int vec4, int64_t m0, int64_t n0, int64_t m, int64_t n, int lr, int h)
+{
+#pragma unroll
+    for (int q = 0; q < R / 4; q++) {
+        const int64_t row = m0 + q * 8 + 4 * h;
+        if (row >= m) continue;
+        uint32_t img = (uint32_t)row / np, px = (uint32_t)row - img * np;
+        if (vec4) {
+            float *first = y + ((int64_t)img * n + n0 + lr) * np + px;
+#pragma unroll
+            for (int tn = 0; tn < TN; tn++)
+                if (n0 + tn * 32 + lr < n)
+                    *reinterpret_cast<float4 *>(first + (int64_t)(tn * 32) * np) = make_float4(o[q * 4][tn], o[q * 4 + 1][tn], o[q * 4 + 2][tn], o[q * 4 + 3][tn]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (row + j < m) {
+                    float *first = y + ((int64_t)img * n + n0 + lr) * np + px;
+#pragma unroll
+                    for (int tn = 0; tn < TN; tn++)
+                        if (n0 + tn * 32 + lr < n) first[(int64_t)(tn * 32) * np] = o[q * 4 + j][tn];
+                }
+                if (++px == np) { px = 0; img++; }
+            }
         }
     }
 }
@@ -851,8 +896,9 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
             o[r][tn] = d;
         }
     }
-    tile_finish<R, TN>(o, split ? p.part + (int64_t)z * p.m * p.n : p.out, mrow0, ncol0, p.m, p.n, bi, p.bias != nullptr && !split,
-                       split ? (int)FNN_ACT_NONE : p.act, lr, h);
+    tile_activate<R, TN>(o, bi, p.bias != nullptr && !split, split ? (int)FNN_ACT_NONE : p.act);
+    if (p.cv.y) tile_store_nchw<R, TN>(o, p.cv.y, p.cv.np, p.cv.vec4, mrow0, ncol0, p.m, p.n, lr, h);   // (a convolution's pixels; K in one split)
+    else tile_store<R, TN>(o, split ? p.part + (int64_t)z * p.m * p.n : p.out, mrow0, ncol0, p.m, p.n, lr, h);
 }
 
 // sum of the K-split partial tiles in split order + affine / bias / activation epilogue.  A thread owns one
