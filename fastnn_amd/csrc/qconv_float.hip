@@ -10,24 +10,22 @@
 namespace {
 
 // col[r, e] = x[b, g*cg + ic, oh*s + i*d - pad, ow*s + j*d - pad] (0 outside), r = b*np + oh*wo + ow,
-// e = (ic*KH + i)*KW + j (src/backend/cpu/im2col.rs:32-52).  Consecutive lanes take consecutive e.
-__global__ void __launch_bounds__(256) im2col_f32_kernel(const float *x, float *col, int64_t rows, int64_t np, int64_t wo,
-                                                         int64_t c, int64_t cg, int g, int64_t h, int64_t w, int kh, int kw,
-                                                         int stride, int pad, int dil, int64_t kk)
+// e = (ic*KH + i)*KW + j (src/backend/cpu/im2col.rs:32-52).  Consecutive lanes take consecutive e.  I: the type that positions are counted
+// in, 32 bits wherever they fit (the divisions of 64 bits were most of the time).
+template <typename I>
+__global__ void __launch_bounds__(256) im2col_f32_kernel(const float *x, float *col, I total, I np, I wo, I c, I cg, int g, I h, I w, int kh, int kw,
+                                                         int stride, int pad, int dil, I kk)
 {
-    const int64_t total = rows * kk;
-    const int khw = kh * kw;
-    for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * 256) {
-        const int64_t r = idx / kk;
-        const int e = (int)(idx - r * kk);
-        const int64_t nn = r / np, p = r - nn * np;
-        const int64_t oh = p / wo, ow = p - oh * wo;
-        const int ic = e / khw, rem = e - ic * khw;
-        const int i = rem / kw, j = rem - i * kw;
-        const int64_t ih = oh * stride + (int64_t)i * dil - pad, iw = ow * stride + (int64_t)j * dil - pad;
-        float v = 0.0f;
-        if (ih >= 0 && ih < h && iw >= 0 && iw < w) v = x[((nn * c + (int64_t)g * cg + ic) * h + ih) * w + iw];
-        col[idx] = v;
+    const unsigned khw = (unsigned)(kh * kw);
+    for (I idx = (I)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (I)gridDim.x * 256) {
+        const I r = idx / kk;
+        const unsigned e = (unsigned)(idx - r * kk);
+        const I nn = r / np, p = r - nn * np;
+        const I oh = p / wo, ow = p - oh * wo;
+        const unsigned ic = e / khw, rem = e - ic * khw;
+        const unsigned i = rem / (unsigned)kw, j = rem - i * (unsigned)kw;
+        const I ih = oh * (I)stride + (I)i * (I)dil - (I)pad, iw = ow * (I)stride + (I)j * (I)dil - (I)pad;   // (unsigned: above the image wraps round to past it)
+        col[idx] = ih < h && iw < w ? x[((nn * c + (I)g * cg + ic) * h + ih) * w + iw] : 0.0f;
     }
 }
 
@@ -60,8 +58,15 @@ hipError_t launch_im2col_f32(const float *x, float *col, int64_t b, int64_t c, i
     int64_t blocks = (rows * kk + 255) / 256;
     if (blocks > 65535 * 16) blocks = 65535 * 16;
     if (blocks < 1) return hipSuccess;
-    hipLaunchKernelGGL(im2col_f32_kernel, dim3((unsigned)blocks), dim3(256), 0, s, x, col, rows, np, wo, c, cg, g, h, w, kh, kw,
-                       stride, pad, dil, kk);
+    const dim3 grid((unsigned)blocks);
+    // (the last step of the loop may pass `total` by the grid; positions above and left of the image wrap to 2^32 - pad ..)
+    const int64_t lim = 1ll << 31;
+    if (rows * kk < lim && b * c * h * w < lim && pad < (1 << 30) && (ho - 1) * stride + (int64_t)(kh - 1) * dil < lim && (wo - 1) * stride + (int64_t)(kw - 1) * dil < lim)
+        hipLaunchKernelGGL(im2col_f32_kernel<uint32_t>, grid, dim3(256), 0, s, x, col, (uint32_t)(rows * kk), (uint32_t)np, (uint32_t)wo, (uint32_t)c, (uint32_t)cg,
+                           g, (uint32_t)h, (uint32_t)w, kh, kw, stride, pad, dil, (uint32_t)kk);
+    else
+        hipLaunchKernelGGL(im2col_f32_kernel<uint64_t>, grid, dim3(256), 0, s, x, col, (uint64_t)(rows * kk), (uint64_t)np, (uint64_t)wo, (uint64_t)c, (uint64_t)cg,
+                           g, (uint64_t)h, (uint64_t)w, kh, kw, stride, pad, dil, (uint64_t)kk);
     return hipGetLastError();
 }
 
