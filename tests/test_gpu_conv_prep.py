@@ -17,13 +17,18 @@ def ctx():
 
 # batch, channels, height, width, output channels, kernel (h, w), stride, padding, dilation
 GEOMETRIES = [
+    # 64 pixels a workgroup
     (1, 3, 64, 33, 16, 3, 3, 1, 1, 1),      # one k block, part of it padding; 2112 pixels end on no tile
     (2, 17, 66, 71, 20, 3, 3, 2, 1, 1),     # 153 values; blocks of pixels that span two images
     (3, 32, 29, 31, 130, 1, 1, 1, 0, 1),    # 1x1
     (1, 6, 61, 57, 33, 5, 2, 1, 3, 2),      # dilated, a kernel that is not square, more padding than it reaches
-    (1, 64, 50, 47, 48, 3, 3, 1, 1, 1),     # nine k blocks: the most that stay in registers
-    (2, 80, 40, 41, 24, 3, 3, 1, 1, 1),     # 720 values: three blocks read twice
     (3, 8, 97, 95, 40, 2, 3, 3, 0, 1),      # rows and columns that no tap reaches
+    (1, 72, 259, 257, 8, 3, 3, 1, 1, 1),    # more than 65536 pixels, 11 k blocks: two of them read twice
+    # 16 pixels
+    (1, 64, 50, 47, 48, 3, 3, 1, 1, 1),     # nine k blocks in three steps
+    (2, 90, 40, 41, 24, 3, 3, 1, 1, 1),     # 810 values in four
+    (1, 40, 46, 47, 20, 8, 8, 1, 3, 1),     # 2560 values: a step of four k blocks read twice
+    (3, 230, 33, 31, 16, 1, 1, 1, 0, 1),    # 1x1, one step
 ]
 
 
