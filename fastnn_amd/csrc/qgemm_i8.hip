@@ -490,10 +490,21 @@ hipError_t run_i8_gemm(const uint32_t *words, int64_t kp, int64_t rows_total, in
     t.ntiles = (int)((n + 127) / 128);
     // 128 x 128 on eight waves of 64 x 32, four stages: with three a stage is requested one stage before it is waited for, and the wait is
     // its latency and its transfer (32 KB, 0.4 us of a CU's 32 bytes a clock) one behind the other (384 x 4096 x 8192 48.8 -> 38.5 us,
-    // 512 x 2048 x 8192 33.4 -> 28.7, five stages 29.0).  4-bit weights beyond one round keep three: two workgroups to a CU (72 KB each)
+    // 640 x 2048 x 5120 33.7 -> 29.2; five stages gain no more).  4-bit weights beyond one round keep three: two workgroups to a CU (72 KB each)
     // hide more (1594 x 1856 x 14843 81 against 98 us).
+    // Where 8-bit tiles fill (nearly) every CU of every round, eight waves on four stages are as much as the chip sustains: back to back for
+    // milliseconds they take 26.0 us on one device and 31.8 on another (512 x 2048 x 8192, quantisation included; weights from memory 28.7 and
+    // 34.3), where three stages take 28.3 on both (33.5; three stages before the rings ended with their range 29.6, 34.9).  Four waves of
+    // 64 x 64 on four stages are as steady, 29.4 (31.6), and ahead on a longer K: 512 x 4096 x 8192 three stages 41.0 (50.2), four waves
+    // 41.1 (43.3), eight on four 41.6 to 42.3 (45.1); 256 x 8192 x 8192, K in two splits, 55.8 (58.0), 54.3 (54.3).  At 224 workgroups eight on four
+    // are ahead on both devices (512 x 2048 x 7168 27.4 against 26.7, from memory 33.0 against 28.9), at 240 they are not (27.7 against 29.9).
     if (!conv && form == 1) {
-        if (DT == FNN_DT_I4 && (int64_t)t.mtiles * t.ntiles * t.splits > 256) return launch_i8_tile<DT, 2, 4, 2, 1, 3>(t, s);
+        const int64_t wgs = (int64_t)t.mtiles * t.ntiles * t.splits, last = wgs % 256;
+        if constexpr (DT == FNN_DT_I8) {
+            if (last == 0 || last > 224) return t.ips <= 16 ? launch_i8_tile<DT, 2, 4, 2, 1, 3>(t, s) : launch_i8_tile<DT, 2, 2, 2, 2, 4>(t, s);
+        } else {
+            if (wgs > 256) return launch_i8_tile<DT, 2, 4, 2, 1, 3>(t, s);
+        }
         return launch_i8_tile<DT, 2, 4, 2, 1, 4>(t, s);
     }
     if (!conv && form == 2) {   // 256 x 128 on eight waves of 64 x 64 (three stages: a fourth fits with 4-bit weights, and gains nothing)

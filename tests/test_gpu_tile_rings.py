@@ -46,6 +46,33 @@ def test_i8_activations(ctx, orc, dt, m, n, k):
         ctx.release(h)
 
 
+# 256 tiles of 128 x 128, and 240: every CU has one, and the 8-bit tiles run on three stages up to 16 of them, on four waves and four stages beyond
+@pytest.mark.parametrize("m,n,k", [(2000, 2040, 100), (2000, 2040, 380), (2000, 2040, 2048), (2000, 2040, 2050), (2000, 1920, 2300)])
+def test_i8_activations_on_every_cu(ctx, orc, m, n, k):
+    """The sums of the first and the last rows equal the oracle's, all of them those of the four-wave tiles."""
+    rng = np.random.default_rng(k + n)
+    pw = weight(rng, flib.DT_I8, n, k)
+    payload = np.frombuffer(orc.quantize_activations(rng.standard_normal((m, k)).astype(np.float32)), np.uint8)
+    h = ctx.register(pw)
+    try:
+        ctx.set_option(flib.OPT_FRAGMENT, -1)
+        outs = []
+        for shape in (0, 1):
+            ctx.set_option(flib.OPT_TILE_SHAPE, shape)
+            outs.append(ctx.qmatmul_i8act(h, payload, m, n, want_acc=True))
+        assert np.array_equal(outs[0][1], outs[1][1])
+        assert_close(outs[0][0], outs[1][0], 1e-6, "all rows")
+        for first in (0, m - 20):
+            part = np.concatenate([payload[:8], payload[8 + first * k:8 + (first + 20) * k]])
+            want, want_acc = orc.qmatmul_i8act(to_oracle(orc, pw), part, 20, want_acc=True)
+            assert np.array_equal(outs[1][1][first:first + 20], want_acc)
+            assert_close(outs[1][0][first:first + 20], want, 1e-6, f"rows {first} ..")
+    finally:
+        ctx.set_option(flib.OPT_FRAGMENT, 0)
+        ctx.set_option(flib.OPT_TILE_SHAPE, -1)
+        ctx.release(h)
+
+
 # f16 tiles (stages of 64 values, rings of three to six) and digit planes (128 values, three to six)
 @pytest.mark.parametrize("dt", [flib.DT_I8, flib.DT_I4, flib.DT_U4, flib.DT_F8])
 @pytest.mark.parametrize("k", [60, 128, 190, 256, 384, 500, 640, 770])
