@@ -498,6 +498,7 @@ hipError_t run_i8_gemm(const uint32_t *words, int64_t kp, int64_t rows_total, in
     // 64 x 64 on four stages are as steady, 29.4 (31.6), and ahead on a longer K: 512 x 4096 x 8192 three stages 41.0 (50.2), four waves
     // 41.1 (43.3), eight on four 41.6 to 42.3 (45.1); 256 x 8192 x 8192, K in two splits, 55.8 (58.0), 54.3 (54.3).  At 224 workgroups eight on four
     // are ahead on both devices (512 x 2048 x 7168 27.4 against 26.7, from memory 33.0 against 28.9), at 240 they are not (27.7 against 29.9).
+    // 4-bit weights, with fewer bytes a stage, stay ahead there: 512 x 2048 x 8192 28.1 with three stages, 25.0 to 26.0 with four.
     if (!conv && form == 1) {
         const int64_t wgs = (int64_t)t.mtiles * t.ntiles * t.splits, last = wgs % 256;
         if constexpr (DT == FNN_DT_I8) {
