@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(NW * 64) qgemm_codebook_kernel(CodebookArgs p)
     for (int b = b0; b < b1; b += PB) {
         if (b > b0) request(b);
         // ---- the activations of the piece: one power of two per row, f16 hi + lo
-        if (p.k % 4 != 0 && b + PB >= p.kblocks) {   // (uniform) the last values of a row run into the next row: they do not count
+        if (p.k % VALS != 0 && b + PB >= p.kblocks) {   // (uniform) the last values of a lane run into the next row: they do not count
 #pragma unroll
             for (int s = 0; s < STEPS; s++)
 #pragma unroll

@@ -80,3 +80,22 @@ def test_values_that_are_no_numbers(ctx, m):
     got = ctx.qmatmul(handle, a, n)
     assert np.isnan(got[:, 7]).all() and np.isfinite(np.delete(got, 7, axis=1)).all()
     ctx.release(handle)
+
+
+# K that ends anywhere in a lane's group of eight values (or four): what lies behind a row's last value is the next row's first
+@pytest.mark.parametrize("k", [204, 205, 206, 207, 208, 300, 1004])
+@pytest.mark.parametrize("m", [6, 13])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf, -3.4e38, 1e30])
+def test_the_first_values_of_a_row_do_not_reach_the_row_before(ctx, m, k, value):
+    rng = np.random.default_rng(k)
+    n = 40
+    pw = codebook_weight(rng, n, k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    handle = ctx.register(pw)
+    clean = ctx.qmatmul(handle, a, n)
+    for row in (1, m - 1):
+        bad = a.copy()
+        bad[row, :4] = value
+        got = ctx.qmatmul(handle, bad, n)
+        assert np.delete(got, row, axis=0).tobytes() == np.delete(clean, row, axis=0).tobytes(), row
+    ctx.release(handle)
