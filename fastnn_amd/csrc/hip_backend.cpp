@@ -1606,6 +1606,7 @@ static void touched(fnn_plan *p)
     p->half[0].reset();
     p->half[1].reset();
     p->halves_tried = false;
+    p->halved.clear();
     if (p->graph) {
         fnn_hip_graph_destroy(nullptr, p->graph);
         p->graph = nullptr;

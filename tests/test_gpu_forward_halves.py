@@ -3,7 +3,10 @@ pass leaves: in the outputs, in every other value, call after call; plans that d
 import numpy as np
 import pytest
 
+import fastnn_amd
+from fastnn_amd import lib as flib
 from fastnn_amd.aot import AotExecutor
+from fastnn_amd.backend import ExecutablePlan, HipBackend, meta_of
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +91,68 @@ def test_results_in_memory_of_the_input():
         assert not ex._plan.halved
         assert buffer[:want.size].tobytes() == want.tobytes()
     ex.close()
+
+
+class TwoImages:
+    """x -> Conv 1x1 -> c -> Relu -> r on two images of three channels, as a plan that goes in halves; `take` lays further slots out."""
+
+    C, SIZE = 4, 640
+
+    def __init__(self):
+        rng = np.random.default_rng(11)
+        self.top = 0
+        self.pw = fastnn_amd.quantize_weights(flib.DT_I8, (rng.standard_normal((self.C, 3)) * 0.4).astype(np.float32))
+        self.pw2 = fastnn_amd.quantize_weights(flib.DT_I8, (rng.standard_normal((self.C, self.C)) * 0.4).astype(np.float32))
+        plane = 2 * self.SIZE * self.SIZE * 4
+        self.x, self.c, self.r, self.z = (self.take(n * plane) for n in (3, self.C, self.C, self.C))
+        self.w, self.w2 = self.take(self.pw.words.nbytes), self.take(self.pw2.words.nbytes)
+        self.rng = rng
+
+    def take(self, nbytes):
+        off = self.top
+        self.top += (nbytes + 63) // 64 * 64
+        return (off, nbytes)
+
+    def conv(self, src, channels, w, pw, dst, bias=()):
+        return ("conv2d_i8", [src, w, *bias], dst, [1, 0, 1, 1, channels, self.SIZE, self.SIZE, 1, 1], meta_of(pw, [self.C, channels, 1, 1]))
+
+    def plan(self):
+        p = ExecutablePlan(self.top).write_const(self.w[0], self.pw.words).write_const(self.w2[0], self.pw2.words)
+        p.call_kernel(*self.conv(self.x, 3, self.w, self.pw, self.c))
+        return p.call_kernel("relu_f32", [self.c], self.r, [self.c[1] // 4])
+
+    def input(self):
+        return self.rng.standard_normal(self.x[1] // 4).astype(np.float32)
+
+    def pass_(self, be, plan, x, outputs):
+        out = [np.empty(s[1] // 4, np.float32) for s in outputs]
+        be.forward(plan, [(self.x[0], x)], [(s[0], o) for s, o in zip(outputs, out)])
+        return out
+
+    def same_as_whole(self, be, plan, outputs, halved, extend=None, passes=4):
+        """`passes` passes on new inputs equal those of a plan that never goes in halves; the later ones go in halves or not, as said."""
+        with HipBackend(0) as other:
+            other.allocate_arena(self.top)
+            other.set_graph_replay(False)
+            whole = self.plan()
+            if extend:
+                whole.call_kernel(*extend)
+            for i in range(passes):
+                x = self.input()
+                got, want = self.pass_(be, plan, x, outputs), self.pass_(other, whole, x, outputs)
+                assert all(g.tobytes() == w.tobytes() for g, w in zip(got, want)), i
+            assert plan.halved == halved
+            whole.close()
+
+
+def test_an_instruction_added_after_halved_passes():
+    """The new instruction reads the last bytes of the input as a constant (a bias): what could be halved before it no longer can."""
+    t = TwoImages()
+    with HipBackend(0) as be:
+        be.allocate_arena(t.top)
+        plan = t.plan()
+        t.same_as_whole(be, plan, [t.r], halved=True)
+        extend = t.conv(t.r, t.C, t.w2, t.pw2, t.z, [(t.x[0] + t.x[1] - 4 * t.C, 4 * t.C)])
+        plan.call_kernel(*extend)
+        t.same_as_whole(be, plan, [t.z], halved=False, extend=extend)
+        plan.close()
