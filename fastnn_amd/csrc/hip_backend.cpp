@@ -1363,10 +1363,11 @@ void split_images(fnn_plan *p)
         }
         use(in.dst, true);
     }
-    // one half's bytes are never the other's, and constants are nobody's
+    // one half's bytes are never the other's (also where neither is written by a call: a transfer writes the inputs), and constants
+    // are nobody's
     for (const Use &a : uses) {
         for (const Use &c : uses)
-            if ((a.written || c.written) && overlaps(half_of(a.s, 0), half_of(c.s, 1))) return;
+            if (overlaps(half_of(a.s, 0), half_of(c.s, 1))) return;
         for (const fnn_slice &c : constants)
             if (a.written && overlaps(a.s, c)) return;
     }

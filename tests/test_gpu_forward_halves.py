@@ -156,3 +156,16 @@ def test_an_instruction_added_after_halved_passes():
         plan.call_kernel(*extend)
         t.same_as_whole(be, plan, [t.z], halved=False, extend=extend)
         plan.close()
+
+
+def test_a_tensor_inside_the_input():
+    """The second image is read as a tensor of its own: its first half would be read while the input's second half arrives."""
+    t = TwoImages()
+    second = (t.x[0] + t.x[1] // 2, t.x[1] // 2)
+    s_y = t.take(second[1])
+    with HipBackend(0) as be:
+        be.allocate_arena(t.top)
+        extend = ("relu_f32", [second], s_y, [second[1] // 4])
+        plan = t.plan().call_kernel(*extend)
+        t.same_as_whole(be, plan, [t.r, s_y], halved=False, extend=extend)
+        plan.close()
