@@ -1410,10 +1410,15 @@ bool forward_in_halves(fnn_backend *b, fnn_plan *p, const fnn_host_slice *inputs
         if (!halved(inputs[i].offset, inputs[i].size)) return false;
     for (uint64_t i = 0; i < n_outputs; i++) {
         if (!halved(outputs[i].offset, outputs[i].size)) return false;
-        for (uint64_t k = 0; k < n_inputs; k++) {   // the first half's results come while the second's input is read
-            const uintptr_t o = reinterpret_cast<uintptr_t>(outputs[i].data), x = reinterpret_cast<uintptr_t>(inputs[k].data);
-            if (o < x + inputs[k].size && x < o + outputs[i].size) return false;
-        }
+        // the first half's results come while the second's input is read, and before the second half's of results named earlier
+        auto meets = [&](const fnn_host_slice &other) {
+            const uintptr_t o = reinterpret_cast<uintptr_t>(outputs[i].data), x = reinterpret_cast<uintptr_t>(other.data);
+            return o < x + other.size && x < o + outputs[i].size;
+        };
+        for (uint64_t k = 0; k < n_inputs; k++)
+            if (meets(inputs[k])) return false;
+        for (uint64_t k = 0; k < i; k++)
+            if (meets(outputs[k])) return false;
     }
     return constants_in_place(b, p);
 }

@@ -169,3 +169,20 @@ def test_a_tensor_inside_the_input():
         plan = t.plan().call_kernel(*extend)
         t.same_as_whole(be, plan, [t.r, s_y], halved=False, extend=extend)
         plan.close()
+
+
+def test_results_that_overlap():
+    """Two results in overlapping memory of the caller: the later one wins, in every byte, as when the pass goes whole."""
+    t = TwoImages()
+    n = t.c[1] // 4
+    with HipBackend(0) as be:
+        be.allocate_arena(t.top)
+        plan = t.plan()
+        for _ in range(4):
+            x = t.input()
+            buffer = np.empty(n + n // 2, np.float32)
+            be.forward(plan, [(t.x[0], x)], [(t.c[0], buffer[:n]), (t.r[0], buffer[n // 2:])])
+            c, r = (be.read_arena(*s, np.float32) for s in (t.c, t.r))
+            assert np.array_equal(buffer[:n // 2], c[:n // 2]) and np.array_equal(buffer[n // 2:], r)
+        assert not plan.halved
+        plan.close()
