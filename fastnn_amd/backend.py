@@ -115,6 +115,11 @@ class ExecutablePlan:
         return int(self.lib.fnn_plan_operands_handed(self.handle))
 
     @property
+    def one_launch_convs(self) -> int:
+        """Quantised Conv2d instructions that ran as one launch (of one half where the pass went in halves)."""
+        return int(self.lib.fnn_plan_one_launch_convs(self.handle))
+
+    @property
     def halved(self) -> bool:
         """Whether the last pass was a forward pass in two halves of its images."""
         return bool(self.lib.fnn_plan_halved(self.handle))

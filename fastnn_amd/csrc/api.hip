@@ -67,6 +67,7 @@ struct fnn_hip_ctx {
     FnnPrepIo prep;                       // a prepared operand handed from one MatMul call to the next (range_io.h)
     FnnPreparedOperand prepared;
     FnnHostIo io;                         // transfers of the calls that take host pointers
+    uint64_t one_launch_convs = 0;        // quantised Conv2d calls that took the one-launch kernel
 };
 
 // Workspace of fnn_hip_qmatmul_static, part of the library's device image: every GPU the library runs on holds one
@@ -1010,7 +1011,10 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
             else HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_qconv2d_i8(p, ctx->stream, 4, &nparts));
             bool handled = patch;
             int rc2 = FNN_OK;
-            if (patch) rc2 = fnn_patch_conv(ctx, ctx->stream, w, p, shape);
+            if (patch) {
+                rc2 = fnn_patch_conv(ctx, ctx->stream, w, p, shape);
+                ctx->one_launch_convs++;
+            }
             else if (!many_groups) rc2 = fnn_i8_tiled_conv(ctx, ctx->stream, w, p, &handled);
             if (rc2) return rc2;
             if (!handled) {
@@ -1277,6 +1281,8 @@ int fnn_hip_graph_launch(fnn_hip_ctx *ctx, fnn_hip_graph *g)
         return FNN_OK;
     });
 }
+
+uint64_t fnn_hip_one_launch_convs(const fnn_hip_ctx *ctx) { return ctx ? ctx->one_launch_convs : 0; }
 
 uint64_t fnn_hip_workspace_epoch(const fnn_hip_ctx *ctx) { return ctx ? ctx->ws_epoch : 0; }
 

@@ -132,6 +132,7 @@ struct fnn_plan {
     uint64_t residuals_fused = 0;     // such Adds in the last host-side pass
     size_t prep_ready = (size_t)-1;   // index of a MatMul whose operand the call before it has prepared
     uint64_t operands_handed = 0;     // such MatMuls in the last host-side pass
+    uint64_t one_launch_convs = 0;    // quantised convolutions of the last host-side pass that took the one-launch kernel
     // the plan over each half of its images, where every instruction works image by image (split_images); constants stay with this plan
     std::unique_ptr<fnn_plan> half[2];
     bool halves_tried = false, last_halved = false;
@@ -1104,7 +1105,9 @@ int run_instr(fnn_backend *b, fnn_plan *p, size_t idx, bool consts_resident)
                 }
             }
         }
+        const uint64_t convs = fnn_hip_one_launch_convs(b->ctx);
         const int st = run_call_with_ranges(b, p, idx);
+        p->one_launch_convs += fnn_hip_one_launch_convs(b->ctx) - convs;
         if (st == FNN_OK && res->used) {
             p->add_done = idx + 1;
             p->residuals_fused++;
@@ -1168,6 +1171,7 @@ int dispatch_impl(fnn_backend *b, fnn_plan *p, uint64_t *elapsed_ns, uint64_t n_
             p->ranges_used = 0;
             p->residuals_fused = 0;
             p->operands_handed = 0;
+            p->one_launch_convs = 0;
             p->add_done = (size_t)-1;
             p->prep_ready = (size_t)-1;
             for (size_t i = 0; i < p->instrs.size() && st == FNN_OK; i++) st = run_instr(b, p, i, true);
@@ -1198,7 +1202,7 @@ int dispatch_impl(fnn_backend *b, fnn_plan *p, uint64_t *elapsed_ns, uint64_t n_
     }
 
     clear_ranges(b);   // ranges never outlive a pass: between passes anyone may write into the arena
-    if (first == 0) { p->ranges_used = 0; p->residuals_fused = 0; p->operands_handed = 0; }
+    if (first == 0) { p->ranges_used = 0; p->residuals_fused = 0; p->operands_handed = 0; p->one_launch_convs = 0; }
     p->add_done = (size_t)-1;
     p->prep_ready = (size_t)-1;
     for (size_t i = (size_t)first; i < p->instrs.size(); i++) {
@@ -1463,6 +1467,7 @@ int run_halves(fnn_backend *b, fnn_plan *p, const fnn_host_slice *inputs, uint64
     p->ranges_used = p->half[0]->ranges_used;
     p->residuals_fused = p->half[0]->residuals_fused;
     p->operands_handed = p->half[0]->operands_handed;
+    p->one_launch_convs = p->half[0]->one_launch_convs;
     return FNN_OK;
 }
 
@@ -1600,6 +1605,7 @@ int fnn_plan_replayed(const fnn_plan *p) { return p && p->last_replayed ? 1 : 0;
 uint64_t fnn_plan_ranges_used(const fnn_plan *p) { return p ? p->ranges_used : 0; }
 uint64_t fnn_plan_residuals_fused(const fnn_plan *p) { return p ? p->residuals_fused : 0; }
 uint64_t fnn_plan_operands_handed(const fnn_plan *p) { return p ? p->operands_handed : 0; }
+uint64_t fnn_plan_one_launch_convs(const fnn_plan *p) { return p ? p->one_launch_convs : 0; }
 int fnn_plan_halved(const fnn_plan *p) { return p && p->last_halved ? 1 : 0; }
 
 static void touched(fnn_plan *p)

@@ -60,7 +60,7 @@ EXPORTED_SYMBOLS = [
     "fnn_hip_qmatmul", "fnn_hip_qmatmul_static", "fnn_hip_quantize_activations", "fnn_hip_dequantize_activations", "fnn_hip_quantize_activations_per_channel", "fnn_hip_dequantize_activations_per_channel", "fnn_hip_qmatmul_i8act", "fnn_hip_qconv2d", "fnn_hip_qconv2d_i8act",
     "fnn_hip_timer_start", "fnn_hip_timer_stop",
     "fnn_hip_graph_begin", "fnn_hip_graph_end", "fnn_hip_graph_launch", "fnn_hip_graph_destroy",
-    "fnn_hip_workspace_epoch",
+    "fnn_hip_workspace_epoch", "fnn_hip_one_launch_convs",
     "fnn_packed_words", "fnn_quantize_weights", "fnn_quantize_weights_kn", "fnn_transpose_kn_to_nk", "fnn_hip_version",
 ]
 # every symbol include/fastnn_hip_backend.h declares
@@ -69,7 +69,7 @@ BACKEND_SYMBOLS = [
     "fnn_backend_set_kernel_flags", "fnn_backend_set_graph_replay", "fnn_backend_set_option",
     "fnn_backend_allocate_arena", "fnn_backend_write_arena", "fnn_backend_read_arena",
     "fnn_plan_create", "fnn_plan_destroy", "fnn_plan_add_write_const", "fnn_plan_add_fill",
-    "fnn_plan_add_memcopy", "fnn_plan_add_call_kernel", "fnn_plan_len", "fnn_plan_replayed", "fnn_plan_ranges_used", "fnn_plan_residuals_fused", "fnn_plan_operands_handed", "fnn_plan_halved", "fnn_plan_arena_size",
+    "fnn_plan_add_memcopy", "fnn_plan_add_call_kernel", "fnn_plan_len", "fnn_plan_replayed", "fnn_plan_ranges_used", "fnn_plan_residuals_fused", "fnn_plan_operands_handed", "fnn_plan_one_launch_convs", "fnn_plan_halved", "fnn_plan_arena_size",
     "fnn_plan_set_param_dims", "fnn_plan_from_bincode", "fnn_plan_to_bincode", "fnn_plan_describe",
     "fnn_backend_dispatch", "fnn_backend_forward", "fnn_backend_dispatch_env", "fnn_backend_dispatch_from", "fnn_backend_dispatch_profile",
     "fnn_backend_dispatch_profile_env",
@@ -177,6 +177,8 @@ def _prototype(l):
     l.fnn_hip_graph_end.argtypes = [_vp, C.POINTER(_vp)]
     l.fnn_hip_graph_launch.argtypes = [_vp, _vp]
     l.fnn_hip_graph_destroy.argtypes = [_vp, _vp]
+    l.fnn_hip_one_launch_convs.argtypes = [_vp]
+    l.fnn_hip_one_launch_convs.restype = _u64
     l.fnn_hip_workspace_epoch.argtypes = [_vp]
     l.fnn_hip_workspace_epoch.restype = _u64
     l.fnn_packed_words.argtypes = [C.c_int, _i64, _i64]
@@ -217,6 +219,8 @@ def _prototype(l):
     l.fnn_plan_residuals_fused.restype = C.c_uint64
     l.fnn_plan_operands_handed.argtypes = [_vp]
     l.fnn_plan_operands_handed.restype = C.c_uint64
+    l.fnn_plan_one_launch_convs.argtypes = [_vp]
+    l.fnn_plan_one_launch_convs.restype = C.c_uint64
     l.fnn_plan_halved.argtypes = [_vp]
     l.fnn_backend_dispatch.argtypes = [_vp, _vp]
     l.fnn_backend_forward.argtypes = [_vp, _vp, C.POINTER(HostSlice), _u64, C.POINTER(HostSlice), _u64]
@@ -414,6 +418,11 @@ class HipContext:
         v = _i64()
         self._check(self.lib.fnn_hip_get_option(self.handle, option, C.byref(v)))
         return v.value
+
+    @property
+    def one_launch_convs(self) -> int:
+        """Quantised Conv2d calls so far that ran as one launch from a patch of the input."""
+        return int(self.lib.fnn_hip_one_launch_convs(self.handle))
 
     def alloc(self, nbytes: int) -> DeviceBuffer:
         return DeviceBuffer(self, nbytes)

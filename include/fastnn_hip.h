@@ -325,6 +325,9 @@ int fnn_hip_graph_destroy(fnn_hip_ctx *ctx, fnn_hip_graph *g);
  * fastnn).  A captured graph holds the workspace addresses of its capture: when the count has
  * changed since, the graph is stale and must be captured again instead of launched. */
 uint64_t fnn_hip_workspace_epoch(const fnn_hip_ctx *ctx);
+/* Counts the context's fnn_hip_qconv2d calls that ran, or were captured, as one launch from a patch of the input
+ * (FNN_OPT_CONV_IMPLICIT; no counterpart in fastnn: lets tests see which path ran). */
+uint64_t fnn_hip_one_launch_convs(const fnn_hip_ctx *ctx);
 
 /* ---- host-side weight quantisers (no GPU needed): the packers the
  * quantisation pass calls (src/compiler/passes/quantization.rs:170-260,

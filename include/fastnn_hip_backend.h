@@ -152,6 +152,9 @@ uint64_t fnn_plan_residuals_fused(const fnn_plan *p);
 /* MatMul instructions of the plan that, on its last pass (or in its recorded graph), found their activation operand
  * prepared by the split-K reduction of the MatMul before them (FNN_OPT_FUSE_PREP; no counterpart in fastnn). */
 uint64_t fnn_plan_operands_handed(const fnn_plan *p);
+/* Quantised Conv2d instructions of the plan that, on its last pass (or in its recorded graph; of one half where it went in
+ * halves), ran as one launch from a patch of the input (FNN_OPT_CONV_IMPLICIT; no counterpart in fastnn). */
+uint64_t fnn_plan_one_launch_convs(const fnn_plan *p);
 /* 1: the plan's last pass was a forward pass in two halves of its images (transfers of one half beside the kernels of the
  * other; the results and the arena are those of the whole pass) */
 int fnn_plan_halved(const fnn_plan *p);

@@ -48,14 +48,25 @@ def test_every_shape_gives_the_same_integers_and_floats(ctx, orc, geo, wdt):
     handle = ctx.register(pw)
     try:
         ctx.set_option(flib.OPT_CONV_IMPLICIT, 2)
+        before = ctx.one_launch_convs
         pair, pair_acc = ctx.qconv2d(handle, x, oc, *args, bias=bias, act=flib.ACT_SILU, want_acc=True)
         assert np.array_equal(pair_acc, want_acc)
+        assert ctx.one_launch_convs == before
         ctx.set_option(flib.OPT_CONV_IMPLICIT, 1)
+        ran = set()
         for form in FORMS:
             ctx.set_option(flib.OPT_CONV_PATCH, form)
+            before = ctx.one_launch_convs
             got, acc = ctx.qconv2d(handle, x, oc, *args, bias=bias, act=flib.ACT_SILU, want_acc=True)
             assert np.array_equal(acc, want_acc), form
             assert np.array_equal(got, pair), form
+            if ctx.one_launch_convs > before:
+                ran.add(form)
+        # the launch ran: by rule, with K shared by waves and not (all of them over pixels and channels), four waves and eight
+        if kk < 4000:
+            shared = {f for f in ran if f and (f & 3) + (f >> 2 & 3) < 2 + (f >> 4 & 1)}
+            assert 0 in ran and shared and ran - shared - {0}
+            assert {f >> 4 & 1 for f in ran if f} == {0, 1}
         assert_close(pair, want, 1e-5)
     finally:
         ctx.set_option(flib.OPT_CONV_IMPLICIT, 0)
@@ -68,14 +79,18 @@ def test_a_weight_used_with_another_kernel_geometry(ctx, orc):
     rng = np.random.default_rng(5)
     pw = fastnn_amd.quantize_weights(flib.DT_I8, (rng.standard_normal((24, 36)) * 0.2).astype(np.float32))
     handle = ctx.register(pw)
+    ctx.set_option(flib.OPT_CONV_IMPLICIT, 1)
     for _ in range(2):
         for c, k in ((4, 3), (36, 1)):
+            before = ctx.one_launch_convs
             x = rng.uniform(-1, 1, (1, c, 10, 12)).astype(np.float32)
             args = (k, k, 1, k // 2, 1, 1)
             want, want_acc, _, _ = orc.qconv2d_i8(x, to_oracle(orc, pw), *args, want_acc=True)
             got, acc = ctx.qconv2d(handle, x, 24, *args, want_acc=True)
             assert np.array_equal(acc, want_acc)
             assert_close(got, want, 1e-5)
+            assert ctx.one_launch_convs - before == (1 if k == 3 else 0)
+    ctx.set_option(flib.OPT_CONV_IMPLICIT, 0)
     ctx.release(handle)
 
 
@@ -90,7 +105,9 @@ def test_not_a_number_and_infinities_as_in_the_pair(ctx, value):
     try:
         for option in (1, 2):
             ctx.set_option(flib.OPT_CONV_IMPLICIT, option)
+            before = ctx.one_launch_convs
             res.append(ctx.qconv2d(handle, x, 40, 3, 3, 1, 1, 1, 1, act=flib.ACT_RELU, want_acc=True))
+            assert ctx.one_launch_convs - before == 2 - option
     finally:
         ctx.set_option(flib.OPT_CONV_IMPLICIT, 0)
         ctx.release(handle)
