@@ -67,6 +67,7 @@ struct fnn_hip_ctx {
     FnnPrepIo prep;                       // a prepared operand handed from one MatMul call to the next (range_io.h)
     FnnPreparedOperand prepared;
     FnnHostIo io;                         // transfers of the calls that take host pointers
+    bool prepare_only = false;            // a quantised Conv2d call builds what it keeps with its weight and goes no further
     uint64_t one_launch_convs = 0;        // quantised Conv2d calls that took the one-launch kernel
 };
 
@@ -968,6 +969,7 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
             HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_row_qsum(w, wm->row_qsum, ctx->stream));
         }
         p.row_qsum = wm->row_qsum;
+        if (ctx->prepare_only) return FNN_OK;
         FnnRangeIo &rio = ctx->range;
         rio.in_used = 0;
         if (flags & FNN_FLAG_FORCE_GENERIC) {
@@ -1363,6 +1365,7 @@ FnnResidualIo *fnn_ctx_residual_io(fnn_hip_ctx *ctx) { return &ctx->residual; }
 FnnPrepIo *fnn_ctx_prep_io(fnn_hip_ctx *ctx) { return &ctx->prep; }
 FnnPreparedOperand *fnn_ctx_prepared(fnn_hip_ctx *ctx) { return &ctx->prepared; }
 bool fnn_ctx_static_mode(fnn_hip_ctx *ctx) { return ctx->static_mode; }
+void fnn_ctx_prepare_only(fnn_hip_ctx *ctx, bool on) { ctx->prepare_only = on; }
 int fnn_ctx_parts_begin(fnn_hip_ctx *ctx)
 {
     return guarded(ctx, "parts", [&]() -> int {

@@ -1122,6 +1122,22 @@ int run_instr(fnn_backend *b, fnn_plan *p, size_t idx, bool consts_resident)
     return FNN_OK;
 }
 
+// What a recorded pass of the plan may not allocate: the copies of weights that its convolutions read in the kernels they choose.  The
+// passes before it may have chosen others (under other options, or as the whole of a pass that now goes in halves).  A call that
+// fails here fails in the pass as well, which says so.
+void prepare_convs(fnn_backend *b, fnn_plan *p)
+{
+    *fnn_ctx_range_io(b->ctx) = FnnRangeIo{};
+    fnn_ctx_prepare_only(b->ctx, true);
+    for (Instr &in : p->instrs) {
+        if (in.kind != K_CALL) continue;
+        const KernelName kn = split_activation(in.kernel);
+        if ((kn.base == "conv2d_i8" || kn.base == "conv2d_i4") && in.meta.present && in.meta.codebook.empty()) (void)run_call(b, in);
+    }
+    fnn_ctx_prepare_only(b->ctx, false);
+    b->err[0] = 0;
+}
+
 // are the plan's constants where an earlier dispatch of it left them?
 bool constants_in_place(fnn_backend *b, fnn_plan *p)
 {
@@ -1164,6 +1180,7 @@ int dispatch_impl(fnn_backend *b, fnn_plan *p, uint64_t *elapsed_ns, uint64_t n_
         p->graph = nullptr;
     }
     if (may_replay && !p->graph) {
+        prepare_convs(b, p);
         const uint64_t w0 = b->weights_epoch, s0 = fnn_hip_workspace_epoch(b->ctx), c0 = b->scratch_epoch;
         if (fnn_hip_graph_begin(b->ctx) == FNN_OK) {
             int st = FNN_OK;

@@ -99,3 +99,5 @@ int fnn_ctx_parts_begin(fnn_hip_ctx *ctx);
 int fnn_ctx_part_in(fnn_hip_ctx *ctx, int part, void *dst_dev, const void *src, size_t bytes);
 int fnn_ctx_part_mark(fnn_hip_ctx *ctx, int part);
 int fnn_ctx_part_out(fnn_hip_ctx *ctx, int part, void *dst, const void *src_dev, size_t bytes);
+// On: the integer convolutions called through fnn_hip_qconv2d build the copies of their weights (which a capture may not allocate) and return
+void fnn_ctx_prepare_only(fnn_hip_ctx *ctx, bool on);

@@ -186,3 +186,23 @@ def test_results_that_overlap():
             assert np.array_equal(buffer[:n // 2], c[:n // 2]) and np.array_equal(buffer[n // 2:], r)
         assert not plan.halved
         plan.close()
+
+
+@pytest.mark.parametrize("forward", [True, False])
+def test_recorded_passes_run_the_kernels_that_their_calls_choose(forward):
+    """Passes on the operand kernel + GEMM pair, then one launch a convolution asked for: a pass that is recorded at once (as the halves of a
+    pass are, and a plan after a change of options) has the copies of its weights all the same."""
+    t = TwoImages()
+    with HipBackend(0) as be:
+        be.allocate_arena(t.top)
+        plan = t.plan()
+        run = (lambda: t.pass_(be, plan, x, [t.r])[0]) if forward else (lambda: (be.write_arena(t.x[0], x), be.dispatch(plan), be.read_arena(*t.r, np.float32))[2])
+        x = t.input()
+        be.set_option(flib.OPT_CONV_IMPLICIT, 2)
+        want = [run() for _ in range(2)]
+        assert plan.replayed and plan.one_launch_convs == 0
+        be.set_option(flib.OPT_CONV_IMPLICIT, 1)
+        got = [run() for _ in range(2)]
+        assert plan.replayed and plan.halved == forward and plan.one_launch_convs == 1
+        assert all(np.array_equal(g, want[0]) for g in want + got)
+        plan.close()
