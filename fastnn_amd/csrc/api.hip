@@ -897,8 +897,6 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
             // fused-dequant MatMul per group (bias and activation in its epilogue), [pixel, channel] -> NCHW
             const int64_t cg = c / groups, ocg = oc / groups, kk = cg * kh * kw, np = ho * wo, rows = b * np;
             if (rows > (1ll << 31) || b > 65535) return fail(ctx, FNN_ERR_UNSUPPORTED_OP, "conv2d: %lld output pixels exceed the f32 path's limit", (long long)rows);
-            if ((rc = ensure(ctx, ctx->st_rows, (size_t)rows * ocg * 4 + 256))) return rc;
-            float *rows_out = (float *)ctx->st_rows.ptr;
             // More pixels than the fragment kernels take as rows: the f16 tiles, whose operand comes straight from the image.  (U4 weights
             // go to digit planes; 31-bit byte offsets and positions.)
             const int64_t small = 1 << 24;
@@ -907,7 +905,7 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
                 (wo - 1) * stride < small && (int64_t)kh * dil < small && (int64_t)kw * dil < small) {
                 QMatmulArgs q;
                 q.words = w->words; q.scales = w->scales; q.zeros = w->zeros; q.codebook = w->codebook;
-                q.a = nullptr; q.bias = dbias; q.out = rows_out;
+                q.a = nullptr; q.bias = dbias; q.out = nullptr;
                 q.m = rows; q.n = oc; q.k = kk; q.kp = w->kp; q.bpr = w->bpr; q.qblock = w->qblock; q.act = act;
                 q.as_written = 0;
                 const ConvSource src = {dx, (int)c, (int)h, (int)wd, kh, kw, stride, pad, dil, (int)wo, (int)np, (unsigned)xin, dy};
@@ -922,7 +920,8 @@ int fnn_hip_qconv2d(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const float *x, i
                 }
             }
             if ((rc = ensure(ctx, ctx->st_col, (size_t)rows * kk * 4 + 256))) return rc;
-            float *col = (float *)ctx->st_col.ptr;
+            if ((rc = ensure(ctx, ctx->st_rows, (size_t)rows * ocg * 4 + 256))) return rc;
+            float *col = (float *)ctx->st_col.ptr, *rows_out = (float *)ctx->st_rows.ptr;
             for (int g = 0; g < groups; g++) {
                 HIP_TRY(ctx, FNN_ERR_DISPATCH, launch_im2col_f32(dx, col, b, c, groups, g, h, wd, ho, wo, kh, kw, stride, pad, dil, ctx->stream));
                 if (groups == 1) {
@@ -1304,10 +1303,10 @@ int fnn_hip_graph_destroy(fnn_hip_ctx *ctx, fnn_hip_graph *g)
 
 // staging access for the matrix-core translation units
 // 0: prepared operands, 1: partial tiles / accumulators, 2 and 3: conv operand, transient weight expansion,
-// 4: the prepared operand one MatMul call leaves for the next
+// 4: the prepared operand one MatMul call leaves for the next, 5: rows of results that become [image, channel, pixel]
 static Staging &tmp_slot(fnn_hip_ctx *ctx, int which)
 {
-    return which == 0 ? ctx->st_tmp : (which == 1 ? ctx->st_tmp2 : (which == 4 ? ctx->st_tmp4 : ctx->st_tmp3));
+    return which == 0 ? ctx->st_tmp : (which == 1 ? ctx->st_tmp2 : (which == 4 ? ctx->st_tmp4 : (which == 5 ? ctx->st_rows : ctx->st_tmp3)));
 }
 // fnn_hip_qmatmul_static: fixed regions of the static workspace, nothing grows
 static size_t static_room(const fnn_hip_ctx *ctx, int which) { return which == 0 ? ctx->static_operand_room : (which == 1 ? kStaticPartialBytes : 0); }

@@ -53,7 +53,7 @@ float fnn_digits3_us(int dt, int64_t m, int64_t n, int64_t k);   // microseconds
 // a middle number of activation rows (and any number with ragged weight rows), per-channel types: both operands in the order the
 // matrix cores take them; asked first, takes what it is expected to finish before the kernels it would replace (qgemm_frag.hip)
 int fnn_frag_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
-// 3 to 16 rows, codebook weights with blocks of 32 (qgemm_codebook.hip)
+// 5 to 16 rows, codebook weights with blocks of 32 (qgemm_codebook.hip)
 int fnn_codebook_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, int flags, bool *handled);
 int fnn_frag_i8act(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const I8ActArgs &p, bool *handled);
 // fragment-major copy of a weight's packed words, built on first use; null when it does not exist and this call may not build it
@@ -70,7 +70,7 @@ struct ConvSource {
     const float *x;
     int c, h, w, kh, kw, stride, pad, dil, wo, np;   // np: output pixels of an image
     unsigned bytes;                                  // of x
-    float *y;                                        // the result, [image][channel][np] (p.out: rows, where K is split)
+    float *y;                                        // the result, [image][channel][np] (p.out is not used)
 };
 int fnn_tiled_qmatmul(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p,
                       int flags, bool *handled, const ConvSource *conv = nullptr);

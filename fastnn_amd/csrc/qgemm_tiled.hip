@@ -611,6 +611,8 @@ int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QM
     int rc;
     if (!handed && (rc = fnn_ctx_ensure_tmp(ctx, 0, L.ws_bytes, &ws0))) return rc;
     if (splits > 1 && (rc = fnn_ctx_ensure_tmp(ctx, 1, (size_t)splits * M * N * 4, &ws1))) return rc;
+    void *rows = q.out;   // a convolution's results go straight to its y; their rows are wanted only where K is split
+    if (conv && splits > 1 && (rc = fnn_ctx_ensure_tmp(ctx, 5, (size_t)M * N * 4 + 256, &rows))) return rc;
     *have = FnnPreparedOperand{};   // (whatever was there is used by this call or stale)
     pio->consumed = handed ? 1 : 0;
 
@@ -652,9 +654,9 @@ int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QM
     t.zero_chunk = q.words + w->rows * q.kp;    // the zeroed margin behind the last row
     t.scales = q.scales; t.zeros = q.zeros; t.umean = want_umean ? wm->umean : nullptr; t.bias = q.bias;
     t.ap = pa.ap; t.rexp = pa.rexp; t.xsum = pa.xsum; t.esum = pa.esum;
-    t.out = q.out; t.part = (float *)ws1;
+    t.out = (float *)rows; t.part = (float *)ws1;
     t.residual = nullptr; t.sum_out = nullptr;
-    if (splits > 1) fnn_take_residual(ctx, q.out, M * N, &t.residual, &t.sum_out);
+    if (splits > 1) fnn_take_residual(ctx, t.out, M * N, &t.residual, &t.sum_out);
     t.m = M; t.n = N; t.kp = q.kp; t.kpad = kpad; t.rows_pad = rows_pad;
     t.a_wrap = 0;
     if (conv && splits == 1) {
@@ -732,7 +734,7 @@ int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QM
         if (rowb > 65535) rowb = 65535;
         hipLaunchKernelGGL(splitk_epilogue_kernel, dim3((unsigned)colb, (unsigned)rowb), dim3(256), 0, s, t, precise ? 0 : 1);
         e = hipGetLastError();
-        if (e == hipSuccess && conv) e = launch_rows_to_nchw(q.out, conv->y, M / conv->np, conv->np, N, 0, N, s);
+        if (e == hipSuccess && conv) e = launch_rows_to_nchw(t.out, conv->y, M / conv->np, conv->np, N, 0, N, s);
         if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
     }
     return FNN_OK;

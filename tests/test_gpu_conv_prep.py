@@ -1,4 +1,6 @@
 """The f32 Conv2d of more than 2048 output pixels, whose f16 operand comes straight from the image, against im2col rows and their preparation."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -74,3 +76,23 @@ def test_not_a_number_and_infinities_as_in_the_rows(ctx, value):
     handle = ctx.register(fastnn_amd.quantize_weights(flib.DT_F8, rng.standard_normal((24, 144)).astype(np.float32)))
     got, rows = both(ctx, handle, x, 24, (3, 3, 1, 1, 1))
     assert np.array_equal(got, rows, equal_nan=True)
+
+
+def test_no_room_for_rows_of_results_that_go_straight_to_the_image():
+    """1 -> 128 channels over 512 x 512 pixels: the operand is 64 values of two halves a pixel (64 MiB), the result 128 MiB in the caller's memory."""
+    def free():
+        bytes_free, total = C.c_size_t(), C.c_size_t()
+        assert c.lib.hipMemGetInfo(C.byref(bytes_free), C.byref(total)) == 0
+        return bytes_free.value
+
+    with fastnn_amd.HipContext(0) as c:
+        handle = c.register(fastnn_amd.quantize_weights(flib.DT_F8, np.ones((128, 9), np.float32)))
+        x, y = c.to_device(np.ones((512, 512), np.float32)), c.alloc(128 * 512 * 512 * 4)
+        c.sync()
+        before = free()
+        rc = c.lib.fnn_hip_qconv2d(c.handle, handle, x.ptr, 1, 1, 512, 512, 3, 3, 1, 1, 1, 1, None, flib.ACT_NONE, y.ptr, None, flib.FLAG_DEVICE_PTRS)
+        c.sync()
+        assert rc == 0 and before - free() < 100 << 20
+        got = y.download(np.float32, 128 * 512 * 512).reshape(128, 512, 512)
+        assert (got[:, 1:-1, 1:-1] == 9).all() and (got[:, 0, 0] == 4).all()
+        c.release(handle)
