@@ -5,9 +5,15 @@
 // rectangle (all channels, halo included), quantises every value once with the image's scale and leaves it in LDS, channels
 // innermost: [chunk of 16 channels][patch pixel][16 bytes].  Phase 2: a tap of the kernel is then a fixed LDS offset, and the
 // 16 bytes that a lane (pixel lane & 31, k half lane >> 5) reads there are the A operand of v_mfma_i32_32x32x32_i8 as they
-// are, for k in the order (kernel row, kernel column, channel).  The weights are kept in that order, one KB per block of 32
-// channels and step (conv_words_kernel, built with the row sums on a weight's first call).  The waves share pixel blocks,
+// are, for k in the order (chunk of 16 channels, kernel row, kernel column, channel).  The weights are kept in that order, one KB per
+// block of 32 channels and step (conv_words_kernel, built with the row sums on a weight's first call).  The waves share pixel blocks,
 // channel blocks and, where there is little work, the K range; K parts meet in LDS and then share the epilogue.
+//
+// Where patch and weights of all channels do not fit LDS, or leave room for one small rectangle only, the channels come in segments: both
+// phases for one segment after the other, the sums stay in registers, and the next segment's weights arrive in a second
+// buffer during phase 2.  Against the operand kernel + GEMM pair, which has to run such layers else (and a kernel that fetched im2col taps at
+// any K): 8 x 320 x 160 x 160 -> 24 channels 5x5 1427 (721) -> 214 us with the range scan, 512 x 80 x 80 -> 32 3x3 47.6 (45.5) -> 27.2, 16 x
+// 512 x 40 x 40 -> 64 3x3 101 (101) -> 61.
 //
 // What bounded the kernels that fetched im2col taps was vector instructions and their chain: a 3 x 3 layer fetched and quantised every
 // input value nine times, about 11 instructions a tap; here it is about 1.4 times (18 x 10 pixels under 16 x 8) and the tap arithmetic
@@ -44,10 +50,13 @@ struct PatchArgs {
     int pw, pp, pgroups;      // patch width, pixels, groups of 64 pixels
     int split;                // patches of up to 32 pixels: the two halves of a wave take a chunk each
     int nch;                  // chunks of 16 channels (up to 4 channels: one chunk = 4 pixels of 4 channels)
-    int nsteps, nkc;          // K steps of two chunks, chunks
+    int nsteps, nkc;          // K steps of two chunks of K, chunks of K
     int lnw, lwch, lwks;      // log2 of the waves, of those over channels, over K
     int w_at, tab_at, red_at; // LDS offsets behind the patch
-    FastDiv dpw, dpg, dparts, dtx, dper, dkw;   // (dper: chunks per tap, or per kernel row of up to 4 channels)
+    FastDiv dpw, dpg, dparts, dtx, dper, dkw;   // (dper: taps, or chunks per kernel row of up to 4 channels)
+    // segments of the channels that follow each other in LDS, chunks and steps of a whole one (last: the other forms do not load them)
+    int segs, cs, nss;
+    FastDiv dnss;
 };
 
 // 64 lanes' 16 bytes each from memory into LDS, without registers: lane i's land at lds + 16 i.  The compiler does not see these loads.
@@ -75,8 +84,8 @@ constexpr uint32_t NOWHERE = 0x80000000u;   // a buffer offset past every slab (
 constexpr int MAX_WAVES = 8;
 constexpr int MAX_LDS = 152 * 1024;   // beside the static part
 
-// C4: up to four channels in a group.  KS: the K range is shared by 1 << lwks waves.
-template <bool KS, bool C4>
+// C4: up to four channels in a group.  KS: the K range is shared by 1 << lwks waves.  SEG: the channels come in segments.
+template <bool KS, bool C4, bool SEG>
 __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs p)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -94,8 +103,10 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
 
     // ---- loads of phase 1: a unit is 64 patch pixels of one chunk (or 32 of two); a channel's plane is a scalar offset, so
     // that only the pixel costs address arithmetic, once for 16 loads
-    const int units = C4 ? p.pgroups : (p.split ? (p.nch + 1) >> 1 : p.pgroups * p.nch);
-    auto unit_at = [&](int u, int &chunk, int &pix) {   // (chunk: uniform but for split patches)
+    const int segs = SEG ? p.segs : 1, nss = SEG ? p.nss : p.nsteps;
+    auto chunks_of = [&](int sg) { return SEG ? min(p.cs, p.nch - sg * p.cs) : p.nch; };
+    auto units_of = [&](int sg) { return C4 ? p.pgroups : (p.split ? (chunks_of(sg) + 1) >> 1 : p.pgroups * chunks_of(sg)); };
+    auto unit_at = [&](int u, int &chunk, int &pix) {   // (chunk: of the segment; uniform but for split patches)
         if (!C4 && p.split) {
             chunk = 2 * u + hf;
             pix = lr;
@@ -104,7 +115,7 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
             pix = (u - chunk * p.pgroups) * 64 + lane;
         }
     };
-    auto fetch = [&](int u, int t, float(&v)[16]) {
+    auto fetch = [&](int u, int t, int sg, float(&v)[16]) {
         const int ty = __builtin_amdgcn_readfirstlane((int)p.dtx.div((uint32_t)t)), tx = t - ty * (int)p.dtx.d;
         const int iy0 = ty * p.th * p.stride - p.pad, ix0 = (tx << p.twl) * p.stride - p.pad;
         int chunk, pix;
@@ -116,10 +127,14 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
         if (!C4) {
             chunk0 = p.split ? 2 * u : __builtin_amdgcn_readfirstlane(chunk);
             if (p.split) {
-                ok = ok && chunk < p.nch;
+                ok = ok && chunk < chunks_of(sg);
                 vo += hf ? (uint32_t)(16 * chstep) : 0u;
                 wide = 32;
             }
+        }
+        if constexpr (SEG) {
+            chunk0 += sg * p.cs;
+            chunk += sg * p.cs;
         }
         vo = ok ? vo : NOWHERE;   // outside the image: zero by the range check
         int so = chunk0 * 16 * chstep;
@@ -134,7 +149,7 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
         }
     };
     float v0[16], v1[16];
-    if (wv < units) fetch(wv, t0, v0);
+    if (wv < units_of(0)) fetch(wv, t0, 0, v0);
 
     // ---- this lane's channel: a wave works on one block of 32
     const bool share = !KS && p.ocg <= 16;   // (uniform) up to 16 channels: the lanes of channels 16 .. 31 take half of
@@ -143,33 +158,44 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
     const float sw = p.scales[ch], zw = p.zeros[ch], bi = p.bias ? p.bias[ch] : 0.0f;
     const int qw = p.qsum[ch];
 
-    // ---- LDS offset of every chunk of K, relative to a pixel's first tap; bits 24 up: how many of its four words count
-    uint32_t *tab = reinterpret_cast<uint32_t *>(lds + p.tab_at);   // [2 halves][nsteps]
-    for (int kc = tid; kc < 2 * p.nsteps; kc += nw * 64) {
+    // ---- LDS offset of every chunk of K of a segment, relative to a pixel's first tap; bits 24 up: how many of its four words
+    // count (of the segments', the last step of the last one may hold half a step)
+    uint32_t *tab = reinterpret_cast<uint32_t *>(lds + p.tab_at);   // [2 halves][nss]
+    for (int kc = tid; kc < 2 * nss; kc += nw * 64) {
         uint32_t e = 0;
-        if (kc < p.nkc) {
-            const int tap = (int)p.dper.div((uint32_t)kc), r = kc - tap * (int)p.dper.d;
+        if (SEG || kc < p.nkc) {   // (a segment is whole steps)
+            const int q = (int)p.dper.div((uint32_t)kc), r = kc - q * (int)p.dper.d;
             if (C4) {
-                e = (uint32_t)((tap * p.pw + r * 4) * p.dil * 4) | ((uint32_t)min(4, p.kw - r * 4) << 24);
+                e = (uint32_t)((q * p.pw + r * 4) * p.dil * 4) | ((uint32_t)min(4, p.kw - r * 4) << 24);
             } else {
-                const int i = (int)p.dkw.div((uint32_t)tap), j = tap - i * p.kw;
-                e = (uint32_t)((r * p.pp + (i * p.pw + j) * p.dil) * 16) | (4u << 24);
+                const int i = (int)p.dkw.div((uint32_t)r), j = r - i * p.kw;
+                e = (uint32_t)((q * p.pp + (i * p.pw + j) * p.dil) * 16) | (4u << 24);
             }
         }
-        tab[(kc & 1) * p.nsteps + (kc >> 1)] = e;
+        tab[(kc & 1) * nss + (kc >> 1)] = e;
     }
 
-    // ---- the workgroup's weights on their way into LDS, where every rectangle and every wave finds them
-    auto weights = [&]() {
-        const int kbs = p.nsteps << p.lwch;
-        const unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)lds + p.w_at);
-        const char *src = reinterpret_cast<const char *>(p.cw) + (int64_t)blockIdx.y * kbs * 1024 + lane * 16;
-        for (int i = wv; i < kbs; i += nw) load_kb(src + (int64_t)i * 1024, base + i * 1024);
+    // ---- the workgroup's weights on their way into LDS, where every rectangle and every wave finds them: all of them once, or a segment's
+    // into one of two buffers while the segment before it is multiplied
+    const int wbytes = (nss << p.lwch) * 1024;
+    auto weights = [&](int sg, int buf) {
+        const unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)lds + p.w_at + buf * wbytes);
+        const char *src = reinterpret_cast<const char *>(p.cw) + ((int64_t)blockIdx.y * (p.nsteps << p.lwch) + sg * nss) * 1024 + lane * 16;
+        const int kbs = min(wch, ((p.ocg + 31) >> 5) - (int)blockIdx.y * wch) * nss;   // (of blocks that exist: what the others multiply is not stored)
+        for (int i = wv; i < kbs; i += nw) {
+            int from = i;
+            if constexpr (SEG) {   // (a block's segments follow each other)
+                const int blk = __builtin_amdgcn_readfirstlane((int)p.dnss.div((uint32_t)i)), s = i - blk * nss;
+                if (sg * nss + s >= p.nsteps) continue;
+                from = blk * p.nsteps + s;
+            }
+            load_kb(src + (int64_t)from * 1024, base + i * 1024);
+        }
     };
 
     // ---- activation scale of the image: from partial ranges, or ready-made
     float sa, za, inv;
-    weights();
+    weights(0, 0);
     if (p.npairs > 0) {
         float mn = p.range_zero ? 0.0f : INFINITY, mx = p.range_zero ? 0.0f : -INFINITY;
         conv_fold_partial_ranges(p.pairs + (int64_t)nn * p.pair_stride * 2, p.npairs, tid, nw * 64, mn, mx);
@@ -197,7 +223,7 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
     const int bq = p.bias ? conv_bias_q(bi, sa, sw) : 0;
 
     const int qlo = p.wbits == 4 ? -8 : -128, qhi = p.wbits == 4 ? 7 : 127;
-    auto quantise = [&](int u, const float(&v)[16]) {
+    auto quantise = [&](int u, int sg, const float(&v)[16]) {
         int chunk, pix;
         unit_at(u, chunk, pix);
         uint32_t w[4];
@@ -214,12 +240,12 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
             w[i] = __builtin_amdgcn_perm((uint32_t)q[1], (uint32_t)q[0], 0x0c0c0400u) | __builtin_amdgcn_perm((uint32_t)q[3], (uint32_t)q[2], 0x04000c0cu);
         }
         if (C4 || (p.cg & 15)) {   // bytes of channels that do not exist are zero
-            const int left = p.cg - chunk * 16;
+            const int left = p.cg - ((SEG ? sg * p.cs : 0) + chunk) * 16;
 #pragma unroll
             for (int i = 0; i < (C4 ? 1 : 4); i++)
                 if (left < i * 4 + 4) w[i] = left <= i * 4 ? 0u : w[i] & (0xffffffffu >> (8 * (i * 4 + 4 - left)));
         }
-        if (pix >= p.pp || (!C4 && p.split && chunk >= p.nch)) return;
+        if (pix >= p.pp || (!C4 && p.split && chunk >= chunks_of(sg))) return;
         if (C4) reinterpret_cast<uint32_t *>(lds)[pix] = w[0];
         else reinterpret_cast<u32x4 *>(lds)[chunk * p.pp + pix] = u32x4{w[0], w[1], w[2], w[3]};
     };
@@ -227,35 +253,47 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
     const int np = p.ho * p.wo, tw1 = (1 << p.twl) - 1;
     const int pl = px_ * 32 + lr;
     const unsigned char *a_lds = lds + ((pl >> p.twl) * p.pw + (pl & tw1)) * p.stride * (C4 ? 4 : 16);
-    const unsigned char *w_lds = lds + p.w_at + cw_ * p.nsteps * 1024 + lane * 16;
-    const int s0 = (p.nsteps * kw_) >> lwks, s1 = (p.nsteps * (kw_ + 1)) >> lwks;
+    const unsigned char *w_lds = lds + p.w_at + cw_ * nss * 1024 + lane * 16;
+    const int tail = (p.nkc & 1) && hf ? 0 : 0x01010101;   // (an odd number of chunks of K: the last step's second half is no chunk)
     int *red = reinterpret_cast<int *>(lds + p.red_at);
     float mn = INFINITY, mx = -INFINITY;
 
-    for (int t = t0; t < t1; t++) {
+    int wbuf = 0;   // (segments) the buffer of this segment's weights
+    i32x16 acc;
+    int qs = 0, sg = 0;
+    for (int t = t0; t < t1;) {
         // ---- phase 1
+        const int units = units_of(sg);
         for (int u = wv; u < units; u += 2 * nw) {
-            if (u + nw < units) fetch(u + nw, t, v1);
-            quantise(u, v0);
+            if (u + nw < units) fetch(u + nw, t, sg, v1);
+            quantise(u, sg, v0);
             if (u + nw < units) {
-                if (u + 2 * nw < units) fetch(u + 2 * nw, t, v0);
-                quantise(u + nw, v1);
+                if (u + 2 * nw < units) fetch(u + 2 * nw, t, sg, v0);
+                quantise(u + nw, sg, v1);
             }
         }
-        if (t == t0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the weights are there
+        if (SEG || t == t0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the weights are there
         __syncthreads();
-        if (t + 1 < t1 && wv < units) fetch(wv, t + 1, v0);   // the next patch's first loads pass under phase 2
+        const int sn = SEG && sg + 1 < segs ? sg + 1 : 0, tn = sn ? t : t + 1;   // the next patch
+        if (tn < t1) {
+            if (wv < units_of(sn)) fetch(wv, tn, sn, v0);   // its first loads pass under phase 2
+            if constexpr (SEG) weights(sn, wbuf ^ 1);
+        }
 
         // ---- phase 2
-        i32x16 acc;
+        if (!SEG || sg == 0) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) acc[i] = 0;
-        int qs = 0;
+            for (int i = 0; i < 16; i++) acc[i] = 0;
+            qs = 0;
+        }
+        const int first = SEG ? sg * nss : 0, steps = SEG ? min(nss, p.nsteps - first) : nss;
+        const int s0 = (steps * kw_) >> lwks, s1 = blk * 32 < p.ocg ? (steps * (kw_ + 1)) >> lwks : s0;   // (uniform; no block: nothing to multiply)
+        const unsigned char *w_at = w_lds + (SEG ? wbuf * wbytes : 0);
         for (int s = s0; s < s1; s += 4) {
             uint32_t e[4];
             i32x4 af[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) e[i] = tab[hf * p.nsteps + min(s + i, s1 - 1)];
+            for (int i = 0; i < 4; i++) e[i] = tab[hf * nss + min(s + i, s1 - 1)];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const unsigned char *at = a_lds + (e[i] & 0xffffffu);
@@ -269,16 +307,25 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 if (s + i >= s1) break;   // (wave-uniform)
-                acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], *reinterpret_cast<const i32x4 *>(w_lds + (s + i) * 1024), acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], *reinterpret_cast<const i32x4 *>(w_at + (s + i) * 1024), acc, 0, 0, 0);
                 if constexpr (C4) {
 #pragma unroll
                     for (int q = 0; q < 4; q++) qs = __builtin_amdgcn_sdot4(af[i][q], q < (int)(e[i] >> 24) ? 0x01010101 : 0, qs, false);
                 } else {
-                    const int ones = (e[i] >> 24) ? 0x01010101 : 0;
+                    const int ones = SEG ? (first + s + i == p.nsteps - 1 ? tail : 0x01010101) : ((e[i] >> 24) ? 0x01010101 : 0);
 #pragma unroll
                     for (int q = 0; q < 4; q++) qs = __builtin_amdgcn_sdot4(af[i][q], ones, qs, false);
                 }
             }
+        }
+        if constexpr (SEG) {
+            wbuf ^= 1;
+            if (sn) {   // (uniform) more of this rectangle's channels
+                sg = sn;
+                __syncthreads();   // this segment is read before the next one is written
+                continue;
+            }
+            sg = 0;
         }
         // ---- the K parts meet (exact integers: any order), and every wave that held one finishes its share of the pixels
         qs += __shfl_xor(qs, 32, 64);   // the two k halves of a pixel
@@ -371,7 +418,7 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
                     finish(i32x4{acc[t4 * 4], acc[t4 * 4 + 1], acc[t4 * 4 + 2], acc[t4 * 4 + 3]}, rs, at, ow);
             }
         }
-        if (t + 1 < t1) __syncthreads();   // this patch is read before the next one is written
+        if (++t < t1) __syncthreads();   // this patch is read before the next one is written
     }
 
     if (p.range_out) {
@@ -405,11 +452,11 @@ __global__ void __launch_bounds__(64) conv_words_kernel(const uint32_t *words, i
     int sum = 0;
     for (int kc = lane; kc < 2 * nsteps; kc += 64) {
         u32x4 o = {0, 0, 0, 0};
-        const int per = c4 ? kwc : nch, tap = kc / per, r = kc - tap * per;
-        if (n < ocg && tap < (c4 ? kh : kh * kw)) {
+        const int per = c4 ? kwc : kh * kw, q = kc / per, r = kc - q * per;   // (kernel row, four columns) or (sixteen channels, tap)
+        if (n < ocg && q < (c4 ? kh : nch)) {
 #pragma unroll
             for (int b = 0; b < 16; b++) {
-                const int c = c4 ? b & 3 : r * 16 + b, j = c4 ? r * 4 + (b >> 2) : tap % kw, i = c4 ? tap : tap / kw;
+                const int c = c4 ? b & 3 : q * 16 + b, j = c4 ? r * 4 + (b >> 2) : r % kw, i = c4 ? q : r / kw;
                 if (c >= cg || j >= kw) continue;
                 const int k = (c * kh + i) * kw + j;
                 const int q = bits == 4 ? ((int)(row[k >> 3] << (28 - 4 * (k & 7)))) >> 28 : (int)(int8_t)(row[k >> 2] >> (8 * (k & 3)));
@@ -453,8 +500,8 @@ bool place(const QConvArgs &p, const Geometry &q, Shape &s)
         const int64_t pw = (int64_t)(tw - 1) * p.stride + (int64_t)(p.kw - 1) * p.dil + 1, ph = (int64_t)(th - 1) * p.stride + (int64_t)(p.kh - 1) * p.dil + 1;
         if (pw * ph > 1 << 16) continue;
         const int64_t pp = pw * ph, tx = (wo + tw - 1) / tw, tiles = tx * ((ho + th - 1) / th);
-        const int64_t patch = cg <= 4 ? (pp * 4 + 4 * 4 * p.dil + 15) / 16 * 16 : pp * q.nch * 16;
-        const int64_t bytes = patch + (int64_t)s.wch * q.nsteps * 1024 + (q.nsteps * 8 + 15) / 16 * 16 + (s.wks > 1 ? 4096 * s.nw : 0);
+        const int64_t patch = cg <= 4 ? (pp * 4 + 4 * 4 * p.dil + 15) / 16 * 16 : pp * s.cs * 16;
+        const int64_t bytes = patch + (int64_t)s.wch * s.nss * 1024 * (s.segs > 1 ? 2 : 1) + (s.nss * 8 + 15) / 16 * 16 + (s.wks > 1 ? 4096 * s.nw : 0);
         if (bytes > MAX_LDS) continue;
         // vector instructions: 8 a patch value, 18 an output; narrow rectangles use less of a cache line
         const double cost = (double)tiles * ((double)((pp + 63) / 64 * 64) * (cg <= 4 ? cg : q.nch * 16) * 8 + 32.0 * s.wpx * ((ocg + 31) / 32 * 32) * 18) * (1 + 0.4 / tw);
@@ -465,43 +512,60 @@ bool place(const QConvArgs &p, const Geometry &q, Shape &s)
     return found;
 }
 
-// Microseconds expected of a shape, and of the operand kernel + GEMM pair (qgemm_i8.hip).  Fitted by least squares to kernel times of 239
-// layers (YOLOv8n's at 224 to 640 pixels a side and batches of 1 to 16, ResNet's at 1, 8 and 32) in some 35 shapes each; the shape with the
-// lowest figure is 3 % off the best on average, and 22 % below the kernels that were there before (4052 -> 3141 us over all layers).
+// Microseconds expected of a shape, and of the operand kernel + GEMM pair (qgemm_i8.hip); both with a range scan's launch, without its bytes.  Fitted
+// by least squares to 678 layers (YOLOv8n's at 224 to 640 pixels a side and batches of 1 to 16, ResNet's at 1, 8 and 32, VGG's, U-Net's, heads, and
+// 400 drawn ones: 3 to 2048 channels in and out, kernels of 1 to 7, dilated, grouped, odd widths) in every shape that fits, 32 700 timings.  A
+// rectangle is a chain of latencies or what its waves issue, whichever is longer.  On 150 layers that the fit had not seen the choice is
+// 2 % off the best one on average (5 % of them more than 12 %), with the fit to 239 layers of two networks, which held no long K, 3.4 %.
 float patch_us(const QConvArgs &p, const Geometry &q, const Shape &s)
 {
     const int64_t cg = p.c / p.groups, ocg = p.oc / p.groups;
-    const bool c4 = cg <= 4, split = !c4 && s.pp <= 32 && q.nch > 1;
-    const int groups = (s.pp + 63) / 64, units = c4 ? groups : (split ? (q.nch + 1) / 2 : groups * q.nch);
-    const float units_wave = (float)((units + s.nw - 1) / s.nw) * (c4 ? 0.25f : 1.0f);
-    const int steps = (q.nsteps + s.wks - 1) / s.wks, items = s.wks == 1 ? (ocg <= 16 ? 2 : 4) : (s.wks < 4 ? 4 / s.wks : 1);
+    const bool c4 = cg <= 4, split = !c4 && s.pp <= 32 && s.cs > 1, flat = p.kh == 1 && p.kw == 1 && p.pad == 0 && p.stride == 1;
+    const int groups = (s.pp + 63) / 64, rest = s.segs - 1;
+    auto units_of = [&](int chunks) { return (float)(((split ? (chunks + 1) / 2 : groups * chunks) + s.nw - 1) / s.nw); };
+    auto fours_of = [&](int steps) { return (float)(((steps + s.wks - 1) / s.wks + 3) / 4); };
+    const float units = c4 ? 0.61f * units_of(1) : rest * units_of(s.cs) + units_of(q.nch - rest * s.cs), fours = rest * fours_of(s.nss) + fours_of(q.nsteps - rest * s.nss);
+    const float steps = (float)((q.nsteps + s.wks - 1) / s.wks) * (float)(s.wch < q.ncb ? s.wch : q.ncb) / (float)s.wch;
+    const float items = s.wks == 1 ? (ocg <= 16 ? 2.f : 4.f) : (s.wks < 4 ? 4.f / s.wks : 1.f);
     const int64_t wgs = p.b * ((s.tiles + s.per - 1) / s.per) * s.gy, per_cu = (wgs + 255) / 256;
-    const int64_t resident = 160 * 1024 / (int64_t)(s.lds + 1300) < 16 / s.nw ? 160 * 1024 / (int64_t)(s.lds + 1300) : 16 / s.nw;
-    const float seq = (float)((per_cu + resident - 1) / resident) * s.per, all = (float)(per_cu * s.per);
-    const float issue = units_wave * 170 + steps * 12 + items * 75 + 40 + 15 * (s.wks - 1);   // vector instructions of a wave and rectangle
-    return 3.58f + seq * (0.271f + 0.285f * units_wave + 0.432f * ((steps + 3) / 4) + 0.397f * items + (s.wks > 1 ? 0.516f : 0.0f)) +
-           0.0307f * per_cu * s.wch * q.nsteps + 0.0000072f * all * s.pp * cg + 0.000149f * all * s.nw * issue + 0.102f * per_cu * s.nw;
+    int64_t resident = 160 * 1024 / (int64_t)(s.lds + 1300) < 16 / s.nw ? 160 * 1024 / (int64_t)(s.lds + 1300) : 16 / s.nw;
+    if (resident < 1) resident = 1;
+    const float seq = (float)((per_cu + resident - 1) / resident) * s.per, waves = (float)(per_cu * s.per * s.nw);
+    const float chain = seq * (0.559f * units + 0.429f * fours + 0.319f * items + (s.wks > 1 ? 0.649f : 0.f) + 0.371f * rest);
+    const float issue = waves * (0.0591f + 0.0242f * units + 0.01352f * steps + 0.0189f * items);
+    const float c2 = chain * chain, i2 = issue * issue;
+    const float out_mb = (float)(p.b * p.oc) * (float)(p.ho * p.wo) * 4e-6f, patch_mb = (float)(p.b * s.tiles * s.gy) * (float)s.pp * (float)cg * 4e-6f;
+    const bool vec4 = (flat ? p.ho * p.wo : p.wo) % 4 == 0;
+    const float each = sqrtf(sqrtf(c2 * c2 + i2 * i2)) + 0.0177f * (float)(per_cu * s.wch * q.nsteps) * (float)(rest ? s.per : 1) + 0.1087f * (float)(per_cu * s.nw) +
+                       0.05f * patch_mb;
+    return 3.14f + 3.75f * p.groups + p.groups * each + (vec4 ? 0.058f : 0.527f) * out_mb;
 }
 float pair_us(const QConvArgs &p)
 {
-    const float rows = (float)(p.b * p.ho * p.wo), ocg = (float)(p.oc / p.groups);
-    const float stages = (float)(((p.c / p.groups) * p.kh * p.kw + 127) / 128);
-    const float wgs = ceilf(rows / 64) * ceilf(ocg / 64);
-    return 8.87f + 0.443f * stages + 41.8e-6f * rows * stages + 1.24e-6f * rows * ocg + 0.0741f * ceilf(wgs / 256) * stages + 0.0015625f * wgs * stages;
+    const int64_t np = p.ho * p.wo;
+    const float rows = (float)(p.b * np), ocg = (float)(p.oc / p.groups), kk = (float)((p.c / p.groups) * p.kh * p.kw);
+    const float stages = ceilf(kk / 128), wgs = ceilf(rows / 64) * ceilf(ocg / 64), rounds = ceilf(wgs / 256);
+    const float in_mb = (float)(p.b * p.c) * (float)(p.h * p.w) * 4e-6f, out_mb = rows * (float)p.oc * 4e-6f;
+    const float each = (0.298f + 0.203f * rounds + 0.000446f * wgs) * stages + 0.352f * rounds +
+                       rows * (1.28e-6f * ocg + (0.141e-6f + (p.kh * p.kw > 1 ? 0.341e-6f : 0.f) + (p.stride > 1 ? 0.117e-6f : 0.f)) * kk);
+    return 2.71f + 8.25f * p.groups + p.groups * each + (np < 64 ? 1.3f : 0.f) + (np % 4 ? 0.55f : 0.f) * out_mb + 0.09f * in_mb;
 }
 
 // false: the pair runs this convolution.  form: FNN_OPT_CONV_PATCH
 bool choose(const QConvArgs &p, const Geometry &q, int option, int form, Shape &best)
 {
     // waves over pixels and over channels, all of them (the rest share K)
-    static const int8_t shapes[][3] = {{1, 1, 4}, {1, 1, 8}, {1, 2, 4}, {1, 2, 8}, {1, 4, 4}, {1, 4, 8}, {2, 1, 4}, {2, 1, 8}, {2, 2, 4}, {2, 4, 8}, {4, 1, 4}, {4, 1, 8}, {4, 2, 8}, {8, 1, 8}};
+    static const int8_t shapes[][3] = {{1, 1, 4}, {1, 1, 8}, {1, 2, 4}, {1, 2, 8}, {1, 4, 4}, {1, 4, 8}, {2, 1, 4}, {2, 1, 8}, {2, 2, 4}, {2, 4, 8}, {1, 8, 8}, {4, 1, 4}, {4, 1, 8}, {4, 2, 8}, {8, 1, 8}};
     float us = 0;
     bool found = false;
-    auto consider = [&](int wpx, int wch, int nw, int per) {
+    auto consider = [&](int wpx, int wch, int nw, int per, int cs) {   // cs: chunks of a segment, 0: all of them in one
         Shape s;
         s.wpx = wpx; s.wch = wch; s.nw = nw; s.wks = nw / (wpx * wch); s.per = per;
-        if (q.ncb % wch) return;
-        s.gy = q.ncb / wch;
+        if (wch >= 2 * q.ncb || (cs && (cs >= q.nch || p.c / p.groups <= 4))) return;
+        s.cs = cs ? cs : q.nch;
+        s.segs = (q.nch + s.cs - 1) / s.cs;
+        s.nss = cs ? cs * p.kh * p.kw / 2 : q.nsteps;
+        s.gy = (q.ncb + wch - 1) / wch;
         if (!place(p, q, s)) return;
         // several rectangles a workgroup only where that leaves work for most CUs
         for (int k = 1; k <= (per ? 1 : 4); k *= 2) {
@@ -513,13 +577,16 @@ bool choose(const QConvArgs &p, const Geometry &q, int option, int form, Shape &
     };
     if (form) {
         const int wpx = 1 << (form & 3), wch = 1 << ((form >> 2) & 3), nw = 4 << ((form >> 4) & 1);
-        if (wpx * wch <= nw) consider(wpx, wch, nw, 1 << ((form >> 5) & 3));
+        if (wpx * wch <= nw) consider(wpx, wch, nw, 1 << ((form >> 5) & 3), (form >> 8) & 7 ? 1 << ((form >> 8) & 7) : 0);
         return found;
     }
-    for (const auto &c : shapes) consider(c[0], c[1], c[2], 0);
-    // many channels and a long K under many pixels: every workgroup loads its channels' weights and quantises the pixels again, the pair does
-    // that once (16 x 128 x 40 x 40 -> 256 3x3 stride 2: 28.8 against 24.6 us; 32 x 256 x 40 x 40: 164 against 64)
-    return found && (option != 0 || us < pair_us(p) * 0.95f);
+    for (const auto &c : shapes) consider(c[0], c[1], c[2], 0, 0);
+    // (segments: an even number of chunks, so that a segment is whole steps of two; up to 24 KB of weights a block they gain nothing)
+    for (int cs = 2; cs < q.nch && q.nsteps > 24; cs *= 2)
+        for (const auto &c : shapes) consider(c[0], c[1], c[2], 0, cs);
+    // many channels under many pixels: every workgroup loads its channels' weights and quantises the pixels again, the pair does that once
+    // (16 x 128 x 40 x 40 -> 256 3x3 stride 2: 28.8 against 24.6 us)
+    return found && (option != 0 || us < pair_us(p));
 }
 
 bool plan(const fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QConvArgs &p, Geometry &q, Shape &s)
@@ -534,15 +601,15 @@ bool plan(const fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QConvArgs &p, G
     return choose(p, q, option, (int)fnn_ctx_option(ctx, FNN_OPT_CONV_PATCH), s) && p.b * s.tiles < 1ll << 30;
 }
 
-template <bool KS, bool C4>
+template <bool KS, bool C4, bool SEG>
 hipError_t launch(const PatchArgs &p, dim3 grid, size_t lds, hipStream_t s)
 {
     static std::atomic<uint64_t> raised{0};
     if (lds > 48 * 1024) {
-        const hipError_t e = fnn_raise_lds_limit(raised, (const void *)conv_patch_kernel<KS, C4>, MAX_LDS);
+        const hipError_t e = fnn_raise_lds_limit(raised, (const void *)conv_patch_kernel<KS, C4, SEG>, MAX_LDS);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((conv_patch_kernel<KS, C4>), grid, dim3(64u << p.lnw), lds, s, p);
+    hipLaunchKernelGGL((conv_patch_kernel<KS, C4, SEG>), grid, dim3(64u << p.lnw), lds, s, p);
     return hipGetLastError();
 }
 
@@ -598,15 +665,17 @@ int fnn_patch_conv(fnn_hip_ctx *ctx, hipStream_t stream, const fnn_hip_weight *w
     a.ho = flat ? 1 : (int)p.ho; a.wo = flat ? (int)np : (int)p.wo;
     a.kw = p.kw; a.stride = p.stride; a.pad = p.pad; a.dil = p.dil;
     a.twl = s.twl; a.th = s.th; a.tiles = s.tiles; a.per = s.per; a.parts = (s.tiles + s.per - 1) / s.per;
-    a.pw = s.pw; a.pp = s.pp; a.pgroups = (s.pp + 63) / 64; a.split = !c4 && s.pp <= 32 && q.nch > 1;
+    a.pw = s.pw; a.pp = s.pp; a.pgroups = (s.pp + 63) / 64; a.split = !c4 && s.pp <= 32 && s.cs > 1;
     a.nch = q.nch; a.nsteps = q.nsteps; a.nkc = q.nkc;
+    a.segs = s.segs; a.cs = s.cs; a.nss = s.nss;
     auto log2of = [](int v) { int l = 0; while (1 << l < v) l++; return l; };
     a.lnw = log2of(s.nw); a.lwch = log2of(s.wch); a.lwks = log2of(s.wks);
-    a.w_at = c4 ? (s.pp * 4 + 4 * 4 * p.dil + 15) / 16 * 16 : s.pp * q.nch * 16;
-    a.tab_at = a.w_at + s.wch * q.nsteps * 1024;
-    a.red_at = a.tab_at + (q.nsteps * 8 + 15) / 16 * 16;
+    a.w_at = c4 ? (s.pp * 4 + 4 * 4 * p.dil + 15) / 16 * 16 : s.pp * s.cs * 16;
+    a.tab_at = a.w_at + s.wch * s.nss * 1024 * (s.segs > 1 ? 2 : 1);
+    a.red_at = a.tab_at + (s.nss * 8 + 15) / 16 * 16;
     a.dpw = fast_div((uint32_t)s.pw); a.dpg = fast_div((uint32_t)a.pgroups); a.dparts = fast_div((uint32_t)a.parts);
-    a.dtx = fast_div((uint32_t)s.tiles_x); a.dper = fast_div((uint32_t)(c4 ? q.kwc : q.nch)); a.dkw = fast_div((uint32_t)p.kw);
+    a.dtx = fast_div((uint32_t)s.tiles_x); a.dper = fast_div((uint32_t)(c4 ? q.kwc : p.kh * p.kw)); a.dkw = fast_div((uint32_t)p.kw);
+    a.dnss = fast_div((uint32_t)s.nss);
     const bool with_sum = p.residual && p.sum_out;
     a.vec4 = (a.wo % 4 == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 && (!p.acc_out || (reinterpret_cast<uintptr_t>(p.acc_out) & 15) == 0) &&
               (!with_sum || ((reinterpret_cast<uintptr_t>(p.residual) | reinterpret_cast<uintptr_t>(p.sum_out)) & 15) == 0)) ? 1 : 0;
@@ -632,8 +701,9 @@ int fnn_patch_conv(fnn_hip_ctx *ctx, hipStream_t stream, const fnn_hip_weight *w
         a.residual = with_sum ? p.residual + oc0 * np : nullptr;
         a.sum_out = with_sum ? p.sum_out + oc0 * np : nullptr;
         hipError_t e;
-        if (s.wks > 1) e = c4 ? launch<true, true>(a, grid, s.lds, stream) : launch<true, false>(a, grid, s.lds, stream);
-        else e = c4 ? launch<false, true>(a, grid, s.lds, stream) : launch<false, false>(a, grid, s.lds, stream);
+        if (s.segs > 1) e = s.wks > 1 ? launch<true, false, true>(a, grid, s.lds, stream) : launch<false, false, true>(a, grid, s.lds, stream);
+        else if (s.wks > 1) e = c4 ? launch<true, true, false>(a, grid, s.lds, stream) : launch<true, false, false>(a, grid, s.lds, stream);
+        else e = c4 ? launch<false, true, false>(a, grid, s.lds, stream) : launch<false, false, false>(a, grid, s.lds, stream);
         if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
     }
     if (with_sum) fnn_ctx_residual_io(ctx)->used = 1;   // the epilogue stored y + residual as well

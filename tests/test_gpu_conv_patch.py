@@ -26,9 +26,14 @@ GEOMETRIES = [
     (3, 64, 5, 5, 128, 1, 1, 1, 0, 1, 1),     # fewer pixels than a block
     (1, 36, 17, 23, 40, 3, 3, 2, 0, 1, 2),    # groups, rows and columns of the input that no tap reaches
     (2, 40, 12, 14, 96, 1, 1, 2, 0, 1, 1),    # 1x1 with a stride
-    (1, 512, 9, 9, 32, 3, 3, 1, 1, 1, 1),     # K = 4608: most shapes do not fit the LDS
+    (1, 512, 9, 9, 32, 3, 3, 1, 1, 1, 1),     # K = 4608: does not fit the LDS whole
+    (2, 150, 11, 13, 72, 3, 3, 1, 1, 1, 1),   # ten chunks, the last of six channels: segments of two, four and two, eight and two; an even K
+    (1, 230, 9, 10, 40, 1, 5, 2, 2, 2, 1),    # fifteen chunks of five taps: the last segment is one chunk, the last step half a one
+    (2, 72, 30, 31, 24, 5, 5, 1, 2, 1, 1),    # five chunks of 25 taps
 ]
-FORMS = [0] + [128 + a + 4 * b + 16 * w + 32 * t for w in (0, 1) for a in range(4) for b in range(3) if a + b <= 2 + w for t in (0, 1, 3)]
+FORMS = [0] + [128 + a + 4 * b + 16 * w + 32 * t for w in (0, 1) for a in range(4) for b in range(4) if a + b <= 2 + w for t in (0, 1, 3)]
+# ... with the channels in segments of two, four and eight chunks of 16
+FORMS += [f + 256 * s for f in FORMS[1:] if f >> 5 & 3 != 3 for s in (1, 2, 3)]
 
 
 @pytest.mark.parametrize("wdt", [flib.DT_I8, flib.DT_I4])
@@ -63,6 +68,8 @@ def test_every_shape_gives_the_same_integers_and_floats(ctx, orc, geo, wdt):
             if ctx.one_launch_convs > before:
                 ran.add(form)
         # the launch ran: by rule, with K shared by waves and not (all of them over pixels and channels), four waves and eight
+        segments = {f >> 8 for f in ran if f} - {0}
+        assert segments == {s for s in (1, 2, 3) if -(-c // groups // 16) > 1 << s and c // groups > 4}
         if kk < 4000:
             shared = {f for f in ran if f and (f & 3) + (f >> 2 & 3) < 2 + (f >> 4 & 1)}
             assert 0 in ran and shared and ran - shared - {0}
@@ -72,6 +79,26 @@ def test_every_shape_gives_the_same_integers_and_floats(ctx, orc, geo, wdt):
         ctx.set_option(flib.OPT_CONV_IMPLICIT, 0)
         ctx.set_option(flib.OPT_CONV_PATCH, 0)
         ctx.release(handle)
+
+
+@pytest.mark.parametrize("geo", [(1, 512, 40, 40, 16, 3), (2, 320, 33, 30, 24, 5), (1, 1024, 60, 50, 40, 3), (4, 96, 100, 100, 8, 7)])
+def test_few_output_channels_and_a_long_k_run_as_one_launch(ctx, orc, geo):
+    """Layers whose weights do not fit LDS: by rule one launch, the channels in segments, with the pair's bits."""
+    b, c, h, w, oc, k = geo
+    rng = np.random.default_rng(3 + c)
+    x = rng.uniform(-0.3, 1, (b, c, h, w)).astype(np.float32)
+    pw = fastnn_amd.quantize_weights(flib.DT_I8, (rng.standard_normal((oc, c * k * k)) * 0.02).astype(np.float32))
+    handle = ctx.register(pw)
+    before = ctx.one_launch_convs
+    got, acc = ctx.qconv2d(handle, x, oc, k, k, 1, k // 2, 1, 1, act=flib.ACT_SILU, want_acc=True)
+    assert ctx.one_launch_convs == before + 1
+    try:
+        ctx.set_option(flib.OPT_CONV_IMPLICIT, 2)
+        pair, pair_acc = ctx.qconv2d(handle, x, oc, k, k, 1, k // 2, 1, 1, act=flib.ACT_SILU, want_acc=True)
+    finally:
+        ctx.set_option(flib.OPT_CONV_IMPLICIT, 0)
+        ctx.release(handle)
+    assert np.array_equal(acc, pair_acc) and np.array_equal(got, pair)
 
 
 def test_a_weight_used_with_another_kernel_geometry(ctx, orc):
