@@ -167,7 +167,7 @@ const OptionSpec kOptions[FNN_OPT_COUNT] = {
     {0, 0, 4},        // FNN_OPT_DIGIT_PLANES
     {1, 0, 2},        // FNN_OPT_GEMV_TILE_MAJOR
     {0, -1, 0xffff},  // FNN_OPT_FRAGMENT
-    {0, 0, 0x7ff},    // FNN_OPT_CONV_PATCH
+    {0, 0, 0x3fff},   // FNN_OPT_CONV_PATCH
 };
 
 #define HIP_TRY(ctx, code, expr)                                                              \

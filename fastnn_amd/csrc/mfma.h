@@ -81,7 +81,7 @@ int64_t fnn_conv_operand_workgroups(const QConvArgs &p);
 // the convolution from an int8 patch in LDS (qconv_patch.hip), asked first: rectangles of 32 * wpx pixels, nw waves over pixels (wpx), blocks of 32
 // channels (wch) and K (wks), `per` rectangles a workgroup, gy workgroups over the channels
 struct FnnPatchShape {
-    int nw, wpx, wch, wks, gy, per, segs, cs, nss, twl, th, pw, pp, tiles_x, tiles;
+    int nw, wpx, wch, wks, gy, per, segs, cs, nss, sets, twl, th, pw, pp, tiles_x, tiles;
     size_t lds;
     int64_t workgroups(int64_t images) const { return images * ((tiles + per - 1) / per) * gy; }
 };

@@ -15,6 +15,11 @@
 // any K): 8 x 320 x 160 x 160 -> 24 channels 5x5 1427 (721) -> 214 us with the range scan, 512 x 80 x 80 -> 32 3x3 47.6 (45.5) -> 27.2, 16 x
 // 512 x 40 x 40 -> 64 3x3 101 (101) -> 61.
 //
+// Under many output channels every workgroup of a few blocks quantises the same pixels again.  There a wave works on several blocks, one after
+// the other on the one patch, and fetches their weights itself, four steps ahead (from L2; no wave shares them, so LDS would only cost
+// room): no barrier behind the patch's.  Against the pair (and a kernel with pixels in LDS and im2col taps): 16 x 512 x 28 x 28 -> 1024 1x1
+// 71 (55) -> 39 us, 512 x 320 x 320 -> 192 1x1 176 (124) -> 98, 256 x 208 x 208 -> 384 3x3 179 (166) -> 144.
+//
 // What bounded the kernels that fetched im2col taps was vector instructions and their chain: a 3 x 3 layer fetched and quantised every
 // input value nine times, about 11 instructions a tap; here it is about 1.4 times (18 x 10 pixels under 16 x 8) and the tap arithmetic
 // is gone.  One image: 64 -> 64 channels 3x3 at 40 x 40 10.5 -> 6.6 us (before: operand kernel + GEMM), 128 -> 128 3x3 at 20 x 20 12.0 -> 7.2,
@@ -57,6 +62,7 @@ struct PatchArgs {
     // segments of the channels that follow each other in LDS, chunks and steps of a whole one (last: the other forms do not load them)
     int segs, cs, nss;
     FastDiv dnss;
+    int sets;   // blocks of output channels of a wave
 };
 
 // 64 lanes' 16 bytes each from memory into LDS, without registers: lane i's land at lds + 16 i.  The compiler does not see these loads.
@@ -84,8 +90,10 @@ constexpr uint32_t NOWHERE = 0x80000000u;   // a buffer offset past every slab (
 constexpr int MAX_WAVES = 8;
 constexpr int MAX_LDS = 152 * 1024;   // beside the static part
 
-// C4: up to four channels in a group.  KS: the K range is shared by 1 << lwks waves.  SEG: the channels come in segments.
-template <bool KS, bool C4, bool SEG>
+// C4: up to four channels in a group.  KS: the K range is shared by 1 << lwks waves.  SEGMENTS: the channels come in segments.  SETS: a wave
+// works on several blocks of output channels, one after the other, and fetches their weights itself.
+enum Form { WHOLE, SEGMENTS, SETS };
+template <bool KS, bool C4, Form FORM>
 __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs p)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -103,6 +111,7 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
 
     // ---- loads of phase 1: a unit is 64 patch pixels of one chunk (or 32 of two); a channel's plane is a scalar offset, so
     // that only the pixel costs address arithmetic, once for 16 loads
+    constexpr bool SEG = FORM == SEGMENTS, MANY = FORM == SETS;
     const int segs = SEG ? p.segs : 1, nss = SEG ? p.nss : p.nsteps;
     auto chunks_of = [&](int sg) { return SEG ? min(p.cs, p.nch - sg * p.cs) : p.nch; };
     auto units_of = [&](int sg) { return C4 ? p.pgroups : (p.split ? (chunks_of(sg) + 1) >> 1 : p.pgroups * chunks_of(sg)); };
@@ -152,11 +161,16 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
     if (wv < units_of(0)) fetch(wv, t0, 0, v0);
 
     // ---- this lane's channel: a wave works on one block of 32
-    const bool share = !KS && p.ocg <= 16;   // (uniform) up to 16 channels: the lanes of channels 16 .. 31 take half of
-    const int blk = (int)blockIdx.y * wch + cw_, n = blk * 32 + (share ? (lr & 15) : lr);   // the pixels of the lane 16 below in the epilogue
-    const int ch = n < p.ocg ? n : 0;
-    const float sw = p.scales[ch], zw = p.zeros[ch], bi = p.bias ? p.bias[ch] : 0.0f;
-    const int qw = p.qsum[ch];
+    const bool share = !KS && !MANY && p.ocg <= 16;   // (uniform) up to 16 channels: the lanes of channels 16 .. 31 take half of
+    int blk = (int)blockIdx.y * wch * (MANY ? p.sets : 1) + cw_, n, qw;   // the pixels of the lane 16 below in the epilogue
+    float sw, zw, bi;
+    auto channel = [&]() {
+        n = blk * 32 + (share ? (lr & 15) : lr);
+        const int ch = n < p.ocg ? n : 0;
+        sw = p.scales[ch]; zw = p.zeros[ch]; bi = p.bias ? p.bias[ch] : 0.0f;
+        qw = p.qsum[ch];
+    };
+    channel();
 
     // ---- LDS offset of every chunk of K of a segment, relative to a pixel's first tap; bits 24 up: how many of its four words
     // count (of the segments', the last step of the last one may hold half a step)
@@ -195,7 +209,7 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
 
     // ---- activation scale of the image: from partial ranges, or ready-made
     float sa, za, inv;
-    weights(0, 0);
+    if constexpr (!MANY) weights(0, 0);
     if (p.npairs > 0) {
         float mn = p.range_zero ? 0.0f : INFINITY, mx = p.range_zero ? 0.0f : -INFINITY;
         conv_fold_partial_ranges(p.pairs + (int64_t)nn * p.pair_stride * 2, p.npairs, tid, nw * 64, mn, mx);
@@ -219,8 +233,13 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
         const float *q = p.actq + (int64_t)nn * p.actq_stride;
         sa = q[0]; za = q[1]; inv = q[2];
     }
-    const float wt = sw * (float)qw;
-    const int bq = p.bias ? conv_bias_q(bi, sa, sw) : 0;
+    float wt;
+    int bq;
+    auto channel_terms = [&]() {
+        wt = sw * (float)qw;
+        bq = p.bias ? conv_bias_q(bi, sa, sw) : 0;
+    };
+    channel_terms();
 
     const int qlo = p.wbits == 4 ? -8 : -128, qhi = p.wbits == 4 ? 7 : 127;
     auto quantise = [&](int u, int sg, const float(&v)[16]) {
@@ -257,6 +276,153 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
     const int tail = (p.nkc & 1) && hf ? 0 : 0x01010101;   // (an odd number of chunks of K: the last step's second half is no chunk)
     int *red = reinterpret_cast<int *>(lds + p.red_at);
     float mn = INFINITY, mx = -INFINITY;
+
+    int oy0, ox0;   // the rectangle's first pixel
+    auto rectangle = [&](int t) {
+        const int ty = __builtin_amdgcn_readfirstlane((int)p.dtx.div((uint32_t)t));
+        oy0 = ty * p.th;
+        ox0 = (t - ty * (int)p.dtx.d) << p.twl;
+    };
+    // pixels 8 ig + 4 hf + (0 .. 3) of the block: scale times the sum of their codes, place in a plane (false: outside)
+    auto pixels = [&](int ig, float(&rs)[4], int &at, int &ow) {
+        const int pq = ig * 8 + hf * 4, pt = px_ * 32 + pq, oh = oy0 + (pt >> p.twl);
+        ow = ox0 + (pt & tw1);
+        at = oh * p.wo + ow;
+        i32x4 q4 = *reinterpret_cast<const i32x4 *>(&s_qs[wv - kw_][pq]);
+        if constexpr (KS)
+            for (int k2 = 1; k2 < wks; k2++) {
+                const i32x4 o4 = *reinterpret_cast<const i32x4 *>(&s_qs[wv - kw_ + k2][pq]);
+#pragma unroll
+                for (int j = 0; j < 4; j++) q4[j] += o4[j];
+            }
+#pragma unroll
+        for (int j = 0; j < 4; j++) rs[j] = sa * (float)q4[j];
+        return oh < p.ho && ow < p.wo;
+    };
+    auto finish = [&](const i32x4 &a4, const float(&rs)[4], int at, int ow) {
+        if (n >= p.ocg) return;
+        float v[4];
+        int av[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = conv_affine(a4[j], sa, za, rs[j], sw, zw, wt, bq, p.kk, &av[j]);
+        conv_act4(v, p.act);
+        const int64_t o = nn * p.y_image + (uint32_t)(n * np + at);
+        // a residual: the Add behind this convolution; v becomes the sums, whose ranges travel on instead of y's
+        if (p.vec4) {
+            *reinterpret_cast<float4 *>(p.y + o) = make_float4(v[0], v[1], v[2], v[3]);
+            if (p.acc_out) *reinterpret_cast<int4 *>(p.acc_out + o) = make_int4(av[0], av[1], av[2], av[3]);
+            if (p.residual) {
+                const float4 r4 = *reinterpret_cast<const float4 *>(p.residual + o);
+                v[0] = v[0] + r4.x; v[1] = v[1] + r4.y; v[2] = v[2] + r4.z; v[3] = v[3] + r4.w;
+                *reinterpret_cast<float4 *>(p.sum_out + o) = make_float4(v[0], v[1], v[2], v[3]);
+            }
+            mn = fminf(fminf(mn, fminf(v[0], v[1])), fminf(v[2], v[3]));
+            mx = fmaxf(fmaxf(mx, fmaxf(v[0], v[1])), fmaxf(v[2], v[3]));
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (ow + j >= p.wo) continue;
+                p.y[o + j] = v[j];
+                if (p.acc_out) p.acc_out[o + j] = av[j];
+                if (p.residual) {
+                    v[j] = v[j] + p.residual[o + j];
+                    p.sum_out[o + j] = v[j];
+                }
+                mn = fminf(mn, v[j]);
+                mx = fmaxf(mx, v[j]);
+            }
+        }
+    };
+
+    if constexpr (MANY) {
+        const int all = (p.ocg + 31) >> 5, units = units_of(0);
+        const char *w0 = reinterpret_cast<const char *>(p.cw) + lane * 16;
+        auto weights_of = [&](int b, int s, i32x4(&w)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[i] = *reinterpret_cast<const i32x4 *>(w0 + ((int64_t)b * p.nsteps + min(s + i, p.nsteps - 1)) * 1024);
+        };
+        i32x4 w[4], wn[4];
+        if (blk < all) weights_of(blk, 0, w);
+        for (int u = wv; u < units; u += 2 * nw) {
+            if (u + nw < units) fetch(u + nw, t0, 0, v1);
+            quantise(u, 0, v0);
+            if (u + nw < units) {
+                if (u + 2 * nw < units) fetch(u + 2 * nw, t0, 0, v0);
+                quantise(u + nw, 0, v1);
+            }
+        }
+        rectangle(t0);
+        __syncthreads();
+        // from here on a wave is on its own
+        int qs = 0;
+        for (int set = 0; set < p.sets && blk < all; set++, blk += wch) {
+            i32x16 acc;
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[i] = 0;
+            if (set > 0) channel();
+            for (int s = 0; s < p.nsteps; s += 4) {
+                const bool more = s + 4 < p.nsteps;   // (uniform)
+                weights_of(more || blk + wch >= all ? blk : blk + wch, more ? s + 4 : 0, wn);
+                uint32_t e[4];
+                i32x4 af[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) e[i] = tab[hf * nss + min(s + i, p.nsteps - 1)];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const unsigned char *at = a_lds + (e[i] & 0xffffffu);
+                    if constexpr (C4) {
+#pragma unroll
+                        for (int q = 0; q < 4; q++) af[i][q] = *reinterpret_cast<const int *>(at + q * p.dil * 4);
+                    } else {
+                        af[i] = *reinterpret_cast<const i32x4 *>(at);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (s + i >= p.nsteps) break;   // (uniform)
+                    acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], w[i], acc, 0, 0, 0);
+                }
+                if (set == 0) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+                            const bool counts = s + i < p.nsteps && (C4 ? q < (int)(e[i] >> 24) : (e[i] >> 24) != 0);
+                            qs = __builtin_amdgcn_sdot4(af[i][q], counts ? 0x01010101 : 0, qs, false);
+                        }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) w[i] = wn[i];
+            }
+            if (set == 0) {
+                qs += __shfl_xor(qs, 32, 64);
+                if (hf == 0) s_qs[wv][lr] = qs;
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            } else {
+                channel_terms();
+            }
+            float rs[4];
+            int at, ow;
+#pragma unroll
+            for (int t4 = 0; t4 < 4; t4++)
+                if (pixels(t4, rs, at, ow)) finish(i32x4{acc[t4 * 4], acc[t4 * 4 + 1], acc[t4 * 4 + 2], acc[t4 * 4 + 3]}, rs, at, ow);
+            if (p.range_out) {   // one pair per wave and block
+                mn = wave_min(mn);
+                mx = wave_max(mx);
+                if (lane == 0) {
+                    const int wpx = nw >> p.lwch;
+                    float *dst = p.range_out + ((int64_t)nn * p.range_stride + (int64_t)blk * p.parts * wpx + part * wpx + px_) * 2;
+                    dst[0] = mn;
+                    dst[1] = mx;
+                }
+                mn = INFINITY;
+                mx = -INFINITY;
+            }
+        }
+        return;
+    }
 
     int wbuf = 0;   // (segments) the buffer of this segment's weights
     i32x16 acc;
@@ -346,57 +512,7 @@ __global__ void __launch_bounds__(64 * MAX_WAVES, 4) conv_patch_kernel(PatchArgs
                 for (int i = 0; i < 8; i++) acc[i] = (int)__builtin_amdgcn_permlane16_swap((uint32_t)acc[i], (uint32_t)acc[i + 8], false, false)[0];
             }
         }
-        const int ty = __builtin_amdgcn_readfirstlane((int)p.dtx.div((uint32_t)t)), oy0 = ty * p.th, ox0 = (t - ty * (int)p.dtx.d) << p.twl;
-        // pixels 8 ig + 4 hf + (0 .. 3) of the block: scale times the sum of their codes, place in a plane (false: outside)
-        auto pixels = [&](int ig, float(&rs)[4], int &at, int &ow) {
-            const int pq = ig * 8 + hf * 4, pt = px_ * 32 + pq, oh = oy0 + (pt >> p.twl);
-            ow = ox0 + (pt & tw1);
-            at = oh * p.wo + ow;
-            i32x4 q4 = *reinterpret_cast<const i32x4 *>(&s_qs[wv - kw_][pq]);
-            if constexpr (KS)
-                for (int k2 = 1; k2 < wks; k2++) {
-                    const i32x4 o4 = *reinterpret_cast<const i32x4 *>(&s_qs[wv - kw_ + k2][pq]);
-#pragma unroll
-                    for (int j = 0; j < 4; j++) q4[j] += o4[j];
-                }
-#pragma unroll
-            for (int j = 0; j < 4; j++) rs[j] = sa * (float)q4[j];
-            return oh < p.ho && ow < p.wo;
-        };
-        auto finish = [&](const i32x4 &a4, const float(&rs)[4], int at, int ow) {
-            if (n >= p.ocg) return;
-            float v[4];
-            int av[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = conv_affine(a4[j], sa, za, rs[j], sw, zw, wt, bq, p.kk, &av[j]);
-            conv_act4(v, p.act);
-            const int64_t o = nn * p.y_image + (uint32_t)(n * np + at);
-            // a residual: the Add behind this convolution; v becomes the sums, whose ranges travel on instead of y's
-            if (p.vec4) {
-                *reinterpret_cast<float4 *>(p.y + o) = make_float4(v[0], v[1], v[2], v[3]);
-                if (p.acc_out) *reinterpret_cast<int4 *>(p.acc_out + o) = make_int4(av[0], av[1], av[2], av[3]);
-                if (p.residual) {
-                    const float4 r4 = *reinterpret_cast<const float4 *>(p.residual + o);
-                    v[0] = v[0] + r4.x; v[1] = v[1] + r4.y; v[2] = v[2] + r4.z; v[3] = v[3] + r4.w;
-                    *reinterpret_cast<float4 *>(p.sum_out + o) = make_float4(v[0], v[1], v[2], v[3]);
-                }
-                mn = fminf(fminf(mn, fminf(v[0], v[1])), fminf(v[2], v[3]));
-                mx = fmaxf(fmaxf(mx, fmaxf(v[0], v[1])), fmaxf(v[2], v[3]));
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    if (ow + j >= p.wo) continue;
-                    p.y[o + j] = v[j];
-                    if (p.acc_out) p.acc_out[o + j] = av[j];
-                    if (p.residual) {
-                        v[j] = v[j] + p.residual[o + j];
-                        p.sum_out[o + j] = v[j];
-                    }
-                    mn = fminf(mn, v[j]);
-                    mx = fmaxf(mx, v[j]);
-                }
-            }
-        };
+        rectangle(t);
         float rs[4];
         int at, ow;
         if constexpr (KS) {
@@ -501,7 +617,7 @@ bool place(const QConvArgs &p, const Geometry &q, Shape &s)
         if (pw * ph > 1 << 16) continue;
         const int64_t pp = pw * ph, tx = (wo + tw - 1) / tw, tiles = tx * ((ho + th - 1) / th);
         const int64_t patch = cg <= 4 ? (pp * 4 + 4 * 4 * p.dil + 15) / 16 * 16 : pp * s.cs * 16;
-        const int64_t bytes = patch + (int64_t)s.wch * s.nss * 1024 * (s.segs > 1 ? 2 : 1) + (s.nss * 8 + 15) / 16 * 16 + (s.wks > 1 ? 4096 * s.nw : 0);
+        const int64_t bytes = patch + (s.sets ? 0 : (int64_t)s.wch * s.nss * 1024 * (s.segs > 1 ? 2 : 1)) + (s.nss * 8 + 15) / 16 * 16 + (s.wks > 1 ? 4096 * s.nw : 0);
         if (bytes > MAX_LDS) continue;
         // vector instructions: 8 a patch value, 18 an output; narrow rectangles use less of a cache line
         const double cost = (double)tiles * ((double)((pp + 63) / 64 * 64) * (cg <= 4 ? cg : q.nch * 16) * 8 + 32.0 * s.wpx * ((ocg + 31) / 32 * 32) * 18) * (1 + 0.4 / tw);
@@ -514,9 +630,9 @@ bool place(const QConvArgs &p, const Geometry &q, Shape &s)
 
 // Microseconds expected of a shape, and of the operand kernel + GEMM pair (qgemm_i8.hip); both with a range scan's launch, without its bytes.  Fitted
 // by least squares to 678 layers (YOLOv8n's at 224 to 640 pixels a side and batches of 1 to 16, ResNet's at 1, 8 and 32, VGG's, U-Net's, heads, and
-// 400 drawn ones: 3 to 2048 channels in and out, kernels of 1 to 7, dilated, grouped, odd widths) in every shape that fits, 32 700 timings.  A
+// 400 drawn ones: 3 to 2048 channels in and out, kernels of 1 to 7, dilated, grouped, odd widths) in every shape that fits, 38 700 timings.  A
 // rectangle is a chain of latencies or what its waves issue, whichever is longer.  On 150 layers that the fit had not seen the choice is
-// 2 % off the best one on average (5 % of them more than 12 %), with the fit to 239 layers of two networks, which held no long K, 3.4 %.
+// 1.8 % off the best one on average (5 % of them more than 11 %).
 float patch_us(const QConvArgs &p, const Geometry &q, const Shape &s)
 {
     const int64_t cg = p.c / p.groups, ocg = p.oc / p.groups;
@@ -524,21 +640,23 @@ float patch_us(const QConvArgs &p, const Geometry &q, const Shape &s)
     const int groups = (s.pp + 63) / 64, rest = s.segs - 1;
     auto units_of = [&](int chunks) { return (float)(((split ? (chunks + 1) / 2 : groups * chunks) + s.nw - 1) / s.nw); };
     auto fours_of = [&](int steps) { return (float)(((steps + s.wks - 1) / s.wks + 3) / 4); };
-    const float units = c4 ? 0.61f * units_of(1) : rest * units_of(s.cs) + units_of(q.nch - rest * s.cs), fours = rest * fours_of(s.nss) + fours_of(q.nsteps - rest * s.nss);
-    const float steps = (float)((q.nsteps + s.wks - 1) / s.wks) * (float)(s.wch < q.ncb ? s.wch : q.ncb) / (float)s.wch;
-    const float items = s.wks == 1 ? (ocg <= 16 ? 2.f : 4.f) : (s.wks < 4 ? 4.f / s.wks : 1.f);
+    const int sets = s.sets ? s.sets : 1, blocks = s.wch * sets * s.gy;
+    const float units = c4 ? 0.5f * units_of(1) : rest * units_of(s.cs) + units_of(q.nch - rest * s.cs);
+    const float fours = (float)sets * (rest * fours_of(s.nss) + fours_of(q.nsteps - rest * s.nss)), busy = (float)(blocks < q.ncb ? blocks : q.ncb) / (float)blocks;
+    const float steps = (float)((q.nsteps + s.wks - 1) / s.wks * sets) * busy;
+    const float items = s.wks == 1 ? (ocg <= 16 && !s.sets ? 2.f : 4.f * sets) : (s.wks < 4 ? 4.f / s.wks : 1.f);
     const int64_t wgs = p.b * ((s.tiles + s.per - 1) / s.per) * s.gy, per_cu = (wgs + 255) / 256;
     int64_t resident = 160 * 1024 / (int64_t)(s.lds + 1300) < 16 / s.nw ? 160 * 1024 / (int64_t)(s.lds + 1300) : 16 / s.nw;
     if (resident < 1) resident = 1;
     const float seq = (float)((per_cu + resident - 1) / resident) * s.per, waves = (float)(per_cu * s.per * s.nw);
-    const float chain = seq * (0.559f * units + 0.429f * fours + 0.319f * items + (s.wks > 1 ? 0.649f : 0.f) + 0.371f * rest);
-    const float issue = waves * (0.0591f + 0.0242f * units + 0.01352f * steps + 0.0189f * items);
+    const float chain = seq * (0.576f * units + (s.sets ? 0.346f : 0.422f) * fours + 0.296f * items + (s.wks > 1 ? 0.61f : 0.f) + 0.397f * rest + (s.sets ? 0.674f : 0.f));
+    const float issue = waves * (0.055f + 0.0368f * units + (s.sets ? 0.01505f : 0.01222f) * steps + 0.01463f * items);
     const float c2 = chain * chain, i2 = issue * issue;
     const float out_mb = (float)(p.b * p.oc) * (float)(p.ho * p.wo) * 4e-6f, patch_mb = (float)(p.b * s.tiles * s.gy) * (float)s.pp * (float)cg * 4e-6f;
     const bool vec4 = (flat ? p.ho * p.wo : p.wo) % 4 == 0;
-    const float each = sqrtf(sqrtf(c2 * c2 + i2 * i2)) + 0.0177f * (float)(per_cu * s.wch * q.nsteps) * (float)(rest ? s.per : 1) + 0.1087f * (float)(per_cu * s.nw) +
-                       0.05f * patch_mb;
-    return 3.14f + 3.75f * p.groups + p.groups * each + (vec4 ? 0.058f : 0.527f) * out_mb;
+    const float weights = s.sets ? 0.00455e-3f * (float)(wgs * s.wch * s.sets) * (float)q.nsteps * busy : 0.0185f * (float)(per_cu * s.wch * q.nsteps) * (float)(rest ? s.per : 1);
+    const float each = sqrtf(sqrtf(c2 * c2 + i2 * i2)) + weights + 0.11f * (float)(per_cu * s.nw) + 0.0448f * patch_mb;
+    return 3.11f + 3.77f * p.groups + p.groups * each + (vec4 ? 0.076f : 0.579f) * out_mb;
 }
 float pair_us(const QConvArgs &p)
 {
@@ -558,35 +676,39 @@ bool choose(const QConvArgs &p, const Geometry &q, int option, int form, Shape &
     static const int8_t shapes[][3] = {{1, 1, 4}, {1, 1, 8}, {1, 2, 4}, {1, 2, 8}, {1, 4, 4}, {1, 4, 8}, {2, 1, 4}, {2, 1, 8}, {2, 2, 4}, {2, 4, 8}, {1, 8, 8}, {4, 1, 4}, {4, 1, 8}, {4, 2, 8}, {8, 1, 8}};
     float us = 0;
     bool found = false;
-    auto consider = [&](int wpx, int wch, int nw, int per, int cs) {   // cs: chunks of a segment, 0: all of them in one
+    // cs: chunks of a segment, 0: all of them in one; sets: blocks of a wave that fetches its weights itself
+    auto consider = [&](int wpx, int wch, int nw, int per, int cs, int sets = 0) {
         Shape s;
         s.wpx = wpx; s.wch = wch; s.nw = nw; s.wks = nw / (wpx * wch); s.per = per;
-        if (wch >= 2 * q.ncb || (cs && (cs >= q.nch || p.c / p.groups <= 4))) return;
+        if (wch * (sets ? sets : 1) >= 2 * q.ncb || (sets && s.wks > 1) || (cs && (cs >= q.nch || p.c / p.groups <= 4))) return;
         s.cs = cs ? cs : q.nch;
         s.segs = (q.nch + s.cs - 1) / s.cs;
         s.nss = cs ? cs * p.kh * p.kw / 2 : q.nsteps;
-        s.gy = (q.ncb + wch - 1) / wch;
+        s.sets = sets;
+        s.gy = (q.ncb + wch * (sets ? sets : 1) - 1) / (wch * (sets ? sets : 1));
         if (!place(p, q, s)) return;
         // several rectangles a workgroup only where that leaves work for most CUs
-        for (int k = 1; k <= (per ? 1 : 4); k *= 2) {
+        for (int k = 1; k <= (per || sets ? 1 : 4); k *= 2) {
             if (!per) s.per = k;
             if (!per && k > 1 && p.b * ((s.tiles + k - 1) / k) * s.gy < 200) break;
-            const float t = patch_us(p, q, s);
+            const float t = patch_us(p, q, s) * (sets ? 1.04f : 1.0f);   // (the margin: a shape in sets has to be ahead beyond the fit's noise)
             if (!found || t < us) { us = t; best = s; found = true; }
         }
     };
     if (form) {
         const int wpx = 1 << (form & 3), wch = 1 << ((form >> 2) & 3), nw = 4 << ((form >> 4) & 1);
-        if (wpx * wch <= nw) consider(wpx, wch, nw, 1 << ((form >> 5) & 3), (form >> 8) & 7 ? 1 << ((form >> 8) & 7) : 0);
+        const int per = 1 << ((form >> 5) & 3), cs = (form >> 8) & 7 ? 1 << ((form >> 8) & 7) : 0, sets = (form >> 11) & 7 ? 1 << (((form >> 11) & 7) - 1) : 0;
+        if (wpx * wch <= nw && !(sets && (cs || per > 1))) consider(wpx, wch, nw, per, cs, sets);
         return found;
     }
     for (const auto &c : shapes) consider(c[0], c[1], c[2], 0, 0);
     // (segments: an even number of chunks, so that a segment is whole steps of two; up to 24 KB of weights a block they gain nothing)
     for (int cs = 2; cs < q.nch && q.nsteps > 24; cs *= 2)
         for (const auto &c : shapes) consider(c[0], c[1], c[2], 0, cs);
-    // many channels under many pixels: every workgroup loads its channels' weights and quantises the pixels again, the pair does that once
-    // (16 x 128 x 40 x 40 -> 256 3x3 stride 2: 28.8 against 24.6 us)
-    return found && (option != 0 || us < pair_us(p));
+    // (sets: the best shape of 3 % of the layers with one block of output channels, of 21 % with two, of 39 % from three on)
+    for (const auto &c : shapes)
+        for (int sets = 1; sets <= 8; sets *= 2) consider(c[0], c[1], c[2], 0, 0, sets);
+    return found && (option != 0 || us < 1.05f * pair_us(p));   // (large layers take the pair up to 30 % longer than expected)
 }
 
 bool plan(const fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QConvArgs &p, Geometry &q, Shape &s)
@@ -601,15 +723,15 @@ bool plan(const fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QConvArgs &p, G
     return choose(p, q, option, (int)fnn_ctx_option(ctx, FNN_OPT_CONV_PATCH), s) && p.b * s.tiles < 1ll << 30;
 }
 
-template <bool KS, bool C4, bool SEG>
+template <bool KS, bool C4, Form FORM>
 hipError_t launch(const PatchArgs &p, dim3 grid, size_t lds, hipStream_t s)
 {
     static std::atomic<uint64_t> raised{0};
     if (lds > 48 * 1024) {
-        const hipError_t e = fnn_raise_lds_limit(raised, (const void *)conv_patch_kernel<KS, C4, SEG>, MAX_LDS);
+        const hipError_t e = fnn_raise_lds_limit(raised, (const void *)conv_patch_kernel<KS, C4, FORM>, MAX_LDS);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((conv_patch_kernel<KS, C4, SEG>), grid, dim3(64u << p.lnw), lds, s, p);
+    hipLaunchKernelGGL((conv_patch_kernel<KS, C4, FORM>), grid, dim3(64u << p.lnw), lds, s, p);
     return hipGetLastError();
 }
 
@@ -667,25 +789,26 @@ int fnn_patch_conv(fnn_hip_ctx *ctx, hipStream_t stream, const fnn_hip_weight *w
     a.twl = s.twl; a.th = s.th; a.tiles = s.tiles; a.per = s.per; a.parts = (s.tiles + s.per - 1) / s.per;
     a.pw = s.pw; a.pp = s.pp; a.pgroups = (s.pp + 63) / 64; a.split = !c4 && s.pp <= 32 && s.cs > 1;
     a.nch = q.nch; a.nsteps = q.nsteps; a.nkc = q.nkc;
-    a.segs = s.segs; a.cs = s.cs; a.nss = s.nss;
+    a.segs = s.segs; a.cs = s.cs; a.nss = s.nss; a.sets = s.sets;
     auto log2of = [](int v) { int l = 0; while (1 << l < v) l++; return l; };
     a.lnw = log2of(s.nw); a.lwch = log2of(s.wch); a.lwks = log2of(s.wks);
     a.w_at = c4 ? (s.pp * 4 + 4 * 4 * p.dil + 15) / 16 * 16 : s.pp * s.cs * 16;
-    a.tab_at = a.w_at + s.wch * s.nss * 1024 * (s.segs > 1 ? 2 : 1);
+    a.tab_at = a.w_at + (s.sets ? 0 : s.wch * s.nss * 1024 * (s.segs > 1 ? 2 : 1));
     a.red_at = a.tab_at + (s.nss * 8 + 15) / 16 * 16;
     a.dpw = fast_div((uint32_t)s.pw); a.dpg = fast_div((uint32_t)a.pgroups); a.dparts = fast_div((uint32_t)a.parts);
     a.dtx = fast_div((uint32_t)s.tiles_x); a.dper = fast_div((uint32_t)(c4 ? q.kwc : p.kh * p.kw)); a.dkw = fast_div((uint32_t)p.kw);
     a.dnss = fast_div((uint32_t)s.nss);
     const bool with_sum = p.residual && p.sum_out;
-    a.vec4 = (a.wo % 4 == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 && (!p.acc_out || (reinterpret_cast<uintptr_t>(p.acc_out) & 15) == 0) &&
-              (!with_sum || ((reinterpret_cast<uintptr_t>(p.residual) | reinterpret_cast<uintptr_t>(p.sum_out)) & 15) == 0)) ? 1 : 0;
-    const int64_t parts = (int64_t)q.ncb * a.parts;
+    const uintptr_t places = reinterpret_cast<uintptr_t>(p.y) | reinterpret_cast<uintptr_t>(p.acc_out) |
+                             (with_sum ? reinterpret_cast<uintptr_t>(p.residual) | reinterpret_cast<uintptr_t>(p.sum_out) : 0);
+    a.vec4 = a.wo % 4 == 0 && (places & 15) == 0;
+    const int64_t pairs = (int64_t)a.parts * (s.sets ? s.wpx : 1), parts = q.ncb * pairs;   // of a block, of an image
     a.range_out = nullptr;
     if (p.range_out && p.groups == 1 && parts <= p.range_out_stride) {
         FnnRangeIo *rio = fnn_ctx_range_io(ctx);
         rio->out_parts = (int)parts;
         rio->out_tile_elems = 32 * (uint64_t)np;
-        rio->out_tile_pairs = a.parts;
+        rio->out_tile_pairs = (int)pairs;
         a.range_out = p.range_out;
     }
     const dim3 grid((unsigned)(p.b * a.parts), (unsigned)s.gy);
@@ -701,9 +824,10 @@ int fnn_patch_conv(fnn_hip_ctx *ctx, hipStream_t stream, const fnn_hip_weight *w
         a.residual = with_sum ? p.residual + oc0 * np : nullptr;
         a.sum_out = with_sum ? p.sum_out + oc0 * np : nullptr;
         hipError_t e;
-        if (s.segs > 1) e = s.wks > 1 ? launch<true, false, true>(a, grid, s.lds, stream) : launch<false, false, true>(a, grid, s.lds, stream);
-        else if (s.wks > 1) e = c4 ? launch<true, true, false>(a, grid, s.lds, stream) : launch<true, false, false>(a, grid, s.lds, stream);
-        else e = c4 ? launch<false, true, false>(a, grid, s.lds, stream) : launch<false, false, false>(a, grid, s.lds, stream);
+        if (s.sets) e = c4 ? launch<false, true, SETS>(a, grid, s.lds, stream) : launch<false, false, SETS>(a, grid, s.lds, stream);
+        else if (s.segs > 1) e = s.wks > 1 ? launch<true, false, SEGMENTS>(a, grid, s.lds, stream) : launch<false, false, SEGMENTS>(a, grid, s.lds, stream);
+        else if (s.wks > 1) e = c4 ? launch<true, true, WHOLE>(a, grid, s.lds, stream) : launch<true, false, WHOLE>(a, grid, s.lds, stream);
+        else e = c4 ? launch<false, true, WHOLE>(a, grid, s.lds, stream) : launch<false, false, WHOLE>(a, grid, s.lds, stream);
         if (e != hipSuccess) return fnn_ctx_fail(ctx, FNN_ERR_DISPATCH, hipGetErrorString(e));
     }
     if (with_sum) fnn_ctx_residual_io(ctx)->used = 1;   // the epilogue stored y + residual as well

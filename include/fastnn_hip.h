@@ -179,8 +179,9 @@ enum {
                                   /* digit planes, w waves of a workgroup sharing a tile                                            */
     FNN_OPT_CONV_PATCH = 25,      /* shape of that launch: 0 (default) = by rule, else 128 + log2 of the waves over pixels + 4 * log2  */
                                   /* over channels + 16 (eight waves instead of four) + 32 * log2 of the rectangles of a workgroup + */
-                                  /* 256 * log2 of the chunks of 16 channels that are in LDS at a time (0: all of them); a shape    */
-                                  /* that does not fit leaves the call to the pair                                                  */
+                                  /* 256 * log2 of the chunks of 16 channels that are in LDS at a time (0: all of them) + 2048 *    */
+                                  /* (1 + log2 of the blocks of 32 output channels of a wave, which then fetches their weights      */
+                                  /* itself); a shape that does not fit leaves the call to the pair                                 */
     FNN_OPT_COUNT = 26
 };
 int fnn_hip_set_option(fnn_hip_ctx *ctx, int option, int64_t value);

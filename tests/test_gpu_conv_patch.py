@@ -34,6 +34,8 @@ GEOMETRIES = [
 FORMS = [0] + [128 + a + 4 * b + 16 * w + 32 * t for w in (0, 1) for a in range(4) for b in range(4) if a + b <= 2 + w for t in (0, 1, 3)]
 # ... with the channels in segments of two, four and eight chunks of 16
 FORMS += [f + 256 * s for f in FORMS[1:] if f >> 5 & 3 != 3 for s in (1, 2, 3)]
+# ... with one, two and four blocks of output channels a wave, which fetches their weights itself
+FORMS += [f + 2048 * s for f in FORMS[1:] if f < 256 and f >> 5 & 3 == 0 and (f & 3) + (f >> 2 & 3) == 2 + (f >> 4 & 1) for s in (1, 2, 3)]
 
 
 @pytest.mark.parametrize("wdt", [flib.DT_I8, flib.DT_I4])
@@ -68,8 +70,9 @@ def test_every_shape_gives_the_same_integers_and_floats(ctx, orc, geo, wdt):
             if ctx.one_launch_convs > before:
                 ran.add(form)
         # the launch ran: by rule, with K shared by waves and not (all of them over pixels and channels), four waves and eight
-        segments = {f >> 8 for f in ran if f} - {0}
+        segments = {f >> 8 & 7 for f in ran if f} - {0}
         assert segments == {s for s in (1, 2, 3) if -(-c // groups // 16) > 1 << s and c // groups > 4}
+        assert any(f >> 11 for f in ran)
         if kk < 4000:
             shared = {f for f in ran if f and (f & 3) + (f >> 2 & 3) < 2 + (f >> 4 & 1)}
             assert 0 in ran and shared and ran - shared - {0}
@@ -81,9 +84,9 @@ def test_every_shape_gives_the_same_integers_and_floats(ctx, orc, geo, wdt):
         ctx.release(handle)
 
 
-@pytest.mark.parametrize("geo", [(1, 512, 40, 40, 16, 3), (2, 320, 33, 30, 24, 5), (1, 1024, 60, 50, 40, 3), (4, 96, 100, 100, 8, 7)])
-def test_few_output_channels_and_a_long_k_run_as_one_launch(ctx, orc, geo):
-    """Layers whose weights do not fit LDS: by rule one launch, the channels in segments, with the pair's bits."""
+@pytest.mark.parametrize("geo", [(1, 512, 40, 40, 16, 3), (2, 320, 33, 30, 24, 5), (1, 1024, 60, 50, 40, 3), (4, 96, 100, 100, 8, 7), (8, 512, 38, 38, 512, 1)])
+def test_layers_with_more_weights_than_lds_holds_run_as_one_launch(ctx, orc, geo):
+    """A long K under few output channels, many channels under many pixels: by rule one launch, with the pair's bits."""
     b, c, h, w, oc, k = geo
     rng = np.random.default_rng(3 + c)
     x = rng.uniform(-0.3, 1, (b, c, h, w)).astype(np.float32)
