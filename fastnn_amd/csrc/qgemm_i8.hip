@@ -498,6 +498,8 @@ hipError_t run_i8_gemm(const uint32_t *words, int64_t kp, int64_t rows_total, in
     // 64 x 64 on four stages are as steady, 29.4 (31.6), and ahead on a longer K: 512 x 4096 x 8192 three stages 41.0 (50.2), four waves
     // 41.1 (43.3), eight on four 41.6 to 42.3 (45.1); 256 x 8192 x 8192, K in two splits, 55.8 (58.0), 54.3 (54.3).  At 224 workgroups eight on four
     // are ahead on both devices (512 x 2048 x 7168 27.4 against 26.7, from memory 33.0 against 28.9), at 240 they are not (27.7 against 29.9).
+    // The line between three stages and four waves: from cache four waves are ahead from 19 to 28 stages on, from memory from 9 or 10 (512 x K x 8192
+    // and 1024 x K x 8192; at 16 28.2 against 28.6 us, from memory 32.0 against 29.8).
     // 4-bit weights, with fewer bytes a stage, stay ahead there: 512 x 2048 x 8192 28.1 with three stages, 25.0 to 26.0 with four.
     if (!conv && form == 1) {
         const int64_t wgs = (int64_t)t.mtiles * t.ntiles * t.splits, last = wgs % 256;
@@ -720,7 +722,8 @@ I8TileForm i8_tile_form(int form, int64_t rows_pad, int64_t n, int iters)
 }
 
 // Microseconds of operand kernel + tiles (+ reduction) in a form: least squares over 740 drawn calls (M 17 .. 2048, K 256 .. 8192,
-// N 256 .. 16384), 4 % mean error.  Whole rounds of workgroups decide: 405 x 7808 x 8373 is 264 tiles of 128 x 128, two rounds, and 132
+// N 256 .. 16384) with eight waves on four stages everywhere, 4 % mean error; 5 % (7 % where three stages or four waves take the full rounds) on 260
+// others with the kernels as they are, of which the form and the fragment kernels' route together are 0.6 % off the best.  Whole rounds of workgroups decide: 405 x 7808 x 8373 is 264 tiles of 128 x 128, two rounds, and 132
 // of 256 x 128, one: 80 against 64 us.  The form with the lower figure is 0.3 % off the better one on average (taken only from 256
 // tiles of 256 x 128 on it was 0.9 % off).
 float i8_tile_us(I8TileForm f, int dt, int64_t m, int64_t rows_pad, int64_t n, int64_t k)

@@ -545,7 +545,7 @@ __global__ void __launch_bounds__(WGM * WGN * 64) qgemm_tile_kernel(TileArgs p)
         };
 
         // Stages past the K range are not requested, so a short one moves no byte twice and needs one LDS buffer per stage it has (the
-        // launcher sizes a ring of three to that); where fewer are on their way than the wait counts, it waits for all of them.
+        // launcher of the int8 tiles allots no more); where fewer are on their way than the wait counts, it waits for all of them.
 #pragma unroll
         for (int st = 0; st < NS - 1; st++)
             if (it0 + st < it1) issue(it0 + st, st);
