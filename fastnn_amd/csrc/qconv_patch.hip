@@ -632,7 +632,7 @@ bool place(const QConvArgs &p, const Geometry &q, Shape &s)
 // by least squares to 678 layers (YOLOv8n's at 224 to 640 pixels a side and batches of 1 to 16, ResNet's at 1, 8 and 32, VGG's, U-Net's, heads, and
 // 400 drawn ones: 3 to 2048 channels in and out, kernels of 1 to 7, dilated, grouped, odd widths) in every shape that fits, 38 700 timings.  A
 // rectangle is a chain of latencies or what its waves issue, whichever is longer.  On 150 layers that the fit had not seen the choice is
-// 1.8 % off the best one on average (5 % of them more than 11 %).
+// 1.5 % off the best one on average (5 % of them more than 9 %).
 float patch_us(const QConvArgs &p, const Geometry &q, const Shape &s)
 {
     const int64_t cg = p.c / p.groups, ocg = p.oc / p.groups;
@@ -641,7 +641,7 @@ float patch_us(const QConvArgs &p, const Geometry &q, const Shape &s)
     auto units_of = [&](int chunks) { return (float)(((split ? (chunks + 1) / 2 : groups * chunks) + s.nw - 1) / s.nw); };
     auto fours_of = [&](int steps) { return (float)(((steps + s.wks - 1) / s.wks + 3) / 4); };
     const int sets = s.sets ? s.sets : 1, blocks = s.wch * sets * s.gy;
-    const float units = c4 ? 0.5f * units_of(1) : rest * units_of(s.cs) + units_of(q.nch - rest * s.cs);
+    const float units = c4 ? 0.25f * units_of(1) : rest * units_of(s.cs) + units_of(q.nch - rest * s.cs);
     const float fours = (float)sets * (rest * fours_of(s.nss) + fours_of(q.nsteps - rest * s.nss)), busy = (float)(blocks < q.ncb ? blocks : q.ncb) / (float)blocks;
     const float steps = (float)((q.nsteps + s.wks - 1) / s.wks * sets) * busy;
     const float items = s.wks == 1 ? (ocg <= 16 && !s.sets ? 2.f : 4.f * sets) : (s.wks < 4 ? 4.f / s.wks : 1.f);
@@ -649,14 +649,17 @@ float patch_us(const QConvArgs &p, const Geometry &q, const Shape &s)
     int64_t resident = 160 * 1024 / (int64_t)(s.lds + 1300) < 16 / s.nw ? 160 * 1024 / (int64_t)(s.lds + 1300) : 16 / s.nw;
     if (resident < 1) resident = 1;
     const float seq = (float)((per_cu + resident - 1) / resident) * s.per, waves = (float)(per_cu * s.per * s.nw);
-    const float chain = seq * (0.576f * units + (s.sets ? 0.346f : 0.422f) * fours + 0.296f * items + (s.wks > 1 ? 0.61f : 0.f) + 0.397f * rest + (s.sets ? 0.674f : 0.f));
-    const float issue = waves * (0.055f + 0.0368f * units + (s.sets ? 0.01505f : 0.01222f) * steps + 0.01463f * items);
+    // (a row of the patch begins and ends inside a line; pieces: rows that 64 of its pixels lie in)
+    const float pieces = 64.f / (float)s.pw, row_mb = (float)(p.b * s.tiles * s.gy) * (float)(s.pp / s.pw) * (float)cg * 64e-6f;
+    const float chain = seq * (((c4 ? 0.825f : 0.573f) + 0.0177f * (pieces < 16.f ? pieces : 16.f)) * units + (s.sets ? 0.319f : (c4 ? 0.485f : 0.39f)) * fours +
+                               0.317f * items + (s.wks > 1 ? 0.5f : 0.f) + 0.412f * rest + (s.sets ? 0.458f : 0.f));
+    const float issue = waves * (0.019f + ((c4 ? 0.0222f : 0.0541f) + 0.00169f * pieces) * units + (s.sets ? 0.01304f : (c4 ? 0.0118f : 0.00967f)) * steps + 0.0195f * items);
     const float c2 = chain * chain, i2 = issue * issue;
     const float out_mb = (float)(p.b * p.oc) * (float)(p.ho * p.wo) * 4e-6f, patch_mb = (float)(p.b * s.tiles * s.gy) * (float)s.pp * (float)cg * 4e-6f;
     const bool vec4 = (flat ? p.ho * p.wo : p.wo) % 4 == 0;
-    const float weights = s.sets ? 0.00455e-3f * (float)(wgs * s.wch * s.sets) * (float)q.nsteps * busy : 0.0185f * (float)(per_cu * s.wch * q.nsteps) * (float)(rest ? s.per : 1);
-    const float each = sqrtf(sqrtf(c2 * c2 + i2 * i2)) + weights + 0.11f * (float)(per_cu * s.nw) + 0.0448f * patch_mb;
-    return 3.11f + 3.77f * p.groups + p.groups * each + (vec4 ? 0.076f : 0.579f) * out_mb;
+    const float weights = s.sets ? 0.f : 0.0108f * (float)(per_cu * s.wch * q.nsteps) * (float)(rest ? s.per : 1);
+    const float each = sqrtf(sqrtf(c2 * c2 + i2 * i2)) + weights + 0.116f * (float)(per_cu * s.nw) + 0.0036f * patch_mb + 0.0946f * row_mb;
+    return 3.06f + 3.88f * p.groups + p.groups * each + (vec4 ? 0.08f : 0.57f) * out_mb;
 }
 float pair_us(const QConvArgs &p)
 {
@@ -666,7 +669,7 @@ float pair_us(const QConvArgs &p)
     const float in_mb = (float)(p.b * p.c) * (float)(p.h * p.w) * 4e-6f, out_mb = rows * (float)p.oc * 4e-6f;
     const float each = (0.298f + 0.203f * rounds + 0.000446f * wgs) * stages + 0.352f * rounds +
                        rows * (1.28e-6f * ocg + (0.141e-6f + (p.kh * p.kw > 1 ? 0.341e-6f : 0.f) + (p.stride > 1 ? 0.117e-6f : 0.f)) * kk);
-    return 2.71f + 8.25f * p.groups + p.groups * each + (np < 64 ? 1.3f : 0.f) + (np % 4 ? 0.55f : 0.f) * out_mb + 0.09f * in_mb;
+    return 2.71f + 8.25f * p.groups + p.groups * each + (np < 64 ? 1.3f : 0.f) + (np % 4 ? 0.55f : 0.f) * out_mb + 0.075f * in_mb;
 }
 
 // false: the pair runs this convolution.  form: FNN_OPT_CONV_PATCH
