@@ -1285,13 +1285,18 @@ int write_slice(fnn_backend *b, uint64_t offset, const void *data, uint64_t size
     return lift(b, fnn_ctx_copy_in(b->ctx, b->arena + offset, data, size, held));
 }
 
-int read_slice(fnn_backend *b, uint64_t offset, void *out, uint64_t size)
+int check_read(fnn_backend *b, uint64_t offset, const void *out, uint64_t size)
 {
     fnn_slice s{offset, size};
     if (!b->arena || !in_arena(b, s)) return fail(b, FNN_ERR_MEMORY, "read_arena: %llu bytes at %llu outside the arena of %llu bytes", (unsigned long long)size, (unsigned long long)offset, (unsigned long long)b->arena_bytes);
-    if (size == 0) return FNN_OK;
-    if (!out) return fail(b, FNN_ERR_DISPATCH, "read_arena: NULL destination");
-    return lift(b, fnn_ctx_copy_out(b->ctx, out, b->arena + offset, size));
+    if (size && !out) return fail(b, FNN_ERR_DISPATCH, "read_arena: NULL destination");
+    return FNN_OK;
+}
+
+int read_slice(fnn_backend *b, uint64_t offset, void *out, uint64_t size)
+{
+    const int st = check_read(b, offset, out, size);
+    return st || size == 0 ? st : lift(b, fnn_ctx_copy_out(b->ctx, out, b->arena + offset, size));
 }
 
 // ---- results that leave while the rest of the pass runs.  A result is final behind the last instruction that writes into it; where enough of the
@@ -1351,10 +1356,12 @@ struct EarlyResults {
     int mark(size_t c) const { return plan->first_mark + (int)(c < plan->cuts.size() ? c : kMostCuts); }
     int mark_end(fnn_backend *b) { return lift(b, fnn_ctx_mark(b->ctx, mark(plan->cuts.size()))); }
     bool leaves_early(size_t i) const { return results[i].last != kNever; }
-    // everything is enqueued: the results follow their marks
+    // everything is enqueued: the results follow their marks.  (Refused as read_slice refuses them, and then none leaves.)
     int send(fnn_backend *b, bool marked_end)
     {
         int st = FNN_OK;
+        for (const Result &r : results)
+            if (!st) st = check_read(b, r.to.offset, r.to.data, r.to.size);
         for (size_t c = 0; c < plan->cuts.size() + (marked_end ? 1 : 0) && !st; c++)
             for (Result &r : results) {
                 if (st || r.sent || r.last == kNever || (c < plan->cuts.size() && r.last > plan->cuts[c])) continue;

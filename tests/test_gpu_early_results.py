@@ -105,3 +105,30 @@ def test_a_plan_that_another_backend_has_cut():
             b.dispatch(plan)
             assert b.read_arena(*chain.v[9], np.float32).tobytes() == want[9].tobytes()
         plan.close()
+
+
+@pytest.mark.parametrize("past", [4, 64, 4096])
+def test_a_pinned_result_that_ends_outside_the_arena(past):
+    """It begins in a tensor that leaves early and ends past the arena: refused as every such read is, nothing leaves, and the next pass is whole."""
+    n = 1 << 18
+    chain = Chain(n)
+    end = (chain.arena, n * 4)          # the arena's last tensor, written first
+    plan = ExecutablePlan(chain.arena + chain.step)
+    plan.call_kernel("relu_f32", [chain.x], end, [n])
+    plan.call_kernel("relu_f32", [chain.x], chain.v[0], [n])
+    for a, b in zip(chain.v, chain.v[1:]):
+        plan.call_kernel("add_f32", [a, chain.x], b, [n])
+    x = np.random.default_rng(4).standard_normal(n).astype(np.float32)
+    want = np.maximum(x, 0)
+    with HipBackend(0) as be:
+        be.allocate_arena(chain.arena + chain.step)
+        for _ in range(4):
+            whole, longer = flib.result_array((n,)), flib.result_array((n + past // 4,))
+            whole[...] = longer[...] = 7.0
+            with pytest.raises(flib.FnnError) as e:
+                be.forward(plan, [(chain.x[0], x)], [(end[0], whole), (end[0], longer)])
+            assert "outside the arena" in str(e.value)
+            assert (longer == 7.0).all() and (whole == 7.0).all()
+            be.forward(plan, [(chain.x[0], x)], [(end[0], whole)])
+            assert whole.tobytes() == want.tobytes()
+        plan.close()
