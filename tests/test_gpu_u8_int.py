@@ -70,3 +70,21 @@ def test_register_tiles(form, m, k, n):
         broken = ctx.qmatmul(h, bad, n, bias=bias)
         assert not np.isfinite(broken[7]).any() and np.array_equal(broken[keep], got[keep])
         ctx.release(h)
+
+
+@pytest.mark.parametrize("form", [1, 2, 4, 1 | 2 << 3])
+def test_long_rows_with_the_tiles_asked_for(form):
+    """A lane and the zero point's shift are up to 384 together: 384 * 128 * K passes 2^31 from K = 43691 on, so that longer rows are another kernel's whatever the
+    option asks for (in 32-bit sums -128849 for 134324).  The sums are f32 then, of products of one sign, added 16 and more at a time: 45000 / 16
+    additions, each half of 2^-24 of the sum off at most, 8.4e-5 where all err to one side."""
+    m, k, n = 40, 45000, 64
+    q = np.full((n, k), 255, np.uint8)       # 1.5, and one weight of 0.5
+    q[:, 7] = 0
+    words = np.concatenate([q.reshape(-1).view(np.uint32), np.zeros(16, np.uint32)])
+    pw = fastnn_amd.PackedWeight(flib.DT_U8, n, k, words, np.full(n, 1 / 255, np.float32), np.full(n, 0.5, np.float32))
+    a = np.full((m, k), 1.99, np.float32)
+    with fastnn_amd.HipContext(0) as ctx:
+        h = ctx.register(pw)
+        ctx.set_option(flib.OPT_FRAGMENT, 1 << 14 | form)
+        assert off(ctx.qmatmul(h, a, n), exact(pw, a, n, k, 0.0)) < 8.4e-5
+        ctx.release(h)
