@@ -21,7 +21,7 @@ HIP_SOURCES = ["api.hip", "host_io.hip", "qgemv.hip", "qgemm_generic.hip", "qgem
                "qgemm_stream.hip", "qgemm_stream_i8.hip", "qgemm_stream_i4.hip", "qgemm_stream_u4.hip", "qgemm_stream_u8.hip",
                "qgemm_stream_f8.hip", "qgemm_stream_f8r.hip", "qgemm_stream_f4.hip", "qgemm_stream_i4cb.hip",
                "qgemm_codebook.hip", "qgemm_frag.hip", "qgemm_frag_i8.hip", "qgemm_frag_i4.hip", "qgemm_frag_u8.hip", "qgemm_frag_u4.hip", "qgemm_frag_f8.hip",
-               "qgemm_frag_f8r.hip", "qgemm_frag_f4.hip", "qgemm_frag_int.hip", "qgemm_frag_int_i8.hip", "qgemm_frag_int_i4.hip",                "qgemm_wave_i8.hip", "qgemm_wave_u8.hip", "qgemm_wave_i4.hip", "qgemm_wave_u4.hip"]
+               "qgemm_frag_f8r.hip", "qgemm_frag_f4.hip", "qgemm_frag_int.hip", "qgemm_frag_int_i8.hip", "qgemm_frag_int_i4.hip",                "qgemm_wave_i8.hip", "qgemm_wave_i4.hip", "qgemm_wave_u4.hip"]
 HOST_SOURCES = ["quantize_host.cpp", "quantize_simd_avx512.cpp", "quantize_simd_avx2.cpp", "quantize_simd_base.cpp", "host_pool.cpp", "hip_backend.cpp"]
 # the weight packers are compiled once per instruction set and chosen at run time
 SOURCE_FLAGS = {"quantize_simd_avx512.cpp": ["-O3", "-mavx512f", "-mavx512bw", "-mavx512dq", "-mavx512vl", "-mprefer-vector-width=512"],

@@ -169,16 +169,6 @@ struct DecI<FNN_DT_I4> {
         return pack8((w[0] << 4) & 0xF0F0F0F0u, w[0] & 0xF0F0F0F0u, (w[1] << 4) & 0xF0F0F0F0u, w[1] & 0xF0F0F0F0u);
     }
 };
-// unsigned bytes as signed ones, q - 128: the caller adds 128 to the zero point (in units of the scale)
-template <>
-struct DecI<FNN_DT_U8> {
-    static constexpr int WPS = 4;
-    static constexpr bool INTERLEAVED = false;
-    __device__ static __forceinline__ f16x8 step(const uint32_t *w)
-    {
-        return pack8(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u, w[2] ^ 0x80808080u, w[3] ^ 0x80808080u);
-    }
-};
 // unsigned 4-bit lanes fit a signed byte as they are (0..15): low nibbles in place, high nibbles shifted down
 template <>
 struct DecI<FNN_DT_U4> {

@@ -62,8 +62,8 @@ int fnn_fragment_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w,
 int fnn_frag_words(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, int64_t kblocks, const uint32_t **words, int *kp);
 // sum of the integer lanes per weight row (I8, I4), built on first use
 int fnn_row_qsum(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const int32_t **qsum);
-// microseconds expected of the f16 tiles (per-channel types), and their split of K
-float fnn_tiled_us(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags, int *splits = nullptr);
+// microseconds expected of the f16 tiles (per-channel types)
+float fnn_tiled_us(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags);
 hipError_t launch_rows_to_nchw(const float *src, float *y, int64_t b, int64_t np, int64_t oc, int64_t ch0, int64_t ocg, hipStream_t s);
 // (conv: the activations are a convolution's windows of its NCHW input, p.m output pixels of p.k values; p.a is not read)
 struct ConvSource {

@@ -421,8 +421,7 @@ bool frag_plan(fnn_hip_ctx *ctx, const fnn_hip_weight *w, int64_t m, int flags, 
         // (9 .. 16 rows: at 0.90 0.2 % of the drawn calls lose more than 3 %, 8 % at the worst; at 0.97 a sixth do.)
         const float margin = m <= 16 || m >= 500 || 4.f * (float)m * (float)f.ks.kblocks * (f.four_bit ? 128.f : 64.f) > 4e6f ? 0.90f : 0.97f;
         if (best > 1e29f || best > margin * others) return false;
-        // (U8: the register tiles' error is above the one here, 1.9e-7 against 1.5e-7)
-        if (float us; w->dtype != FNN_DT_U8 && fnn_wave_choice(w->dtype, m, n, k, &us) && best > margin * us) return false;
+        if (float us; fnn_wave_choice(w->dtype, m, n, k, &us) && best > margin * us) return false;
     }
     f.op_mb = f.mb; f.op_nb = f.nb;
     if (f.direct) {

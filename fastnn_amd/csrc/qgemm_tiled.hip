@@ -28,7 +28,6 @@
 // FNN_FLAG_ACT_F16_SINGLE keeps hi only and removes the first-order effect of the rounding
 // on rows with a non-zero mean lane value: dot -= mean_k(u[n,k]) * sum_k (hi - x').
 #include "mfma.h"
-#include "qgemm_wave.h"
 #include "dech.h"
 #include "range_io.h"
 
@@ -700,11 +699,9 @@ int run_tiled(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QM
         // whole rows per workgroup, in the other operand buffer than the one this call's own row tables live in.
         TileLayout NL;
         int n_il = 0;
-        float next_us;
         const bool may_prepare = pio->next_w && !dense && !conv && !t.codebook && !fnn_ctx_static_mode(ctx) && M >= 17 && N % 64 == 0 && N <= 2048 * PREP_RG &&
                                  (pio->next_a == q.out || (t.residual && pio->next_a == t.sum_out)) &&
                                  pio->next_w->inner == N && tile_layout_of(ctx, pio->next_w->dtype, M, pio->next_w->rows, N, pio->next_flags, &NL, &n_il) &&
-                                 !(pio->next_w->dtype == FNN_DT_U8 && fnn_wave_form(ctx, FNN_DT_U8, M, pio->next_w->rows, N, pio->next_flags, &next_us)) &&
                                  NL.kpad == N && !((reinterpret_cast<uintptr_t>(t.scales) | reinterpret_cast<uintptr_t>(t.zeros) | reinterpret_cast<uintptr_t>(t.out) |
                                                     reinterpret_cast<uintptr_t>(t.sum_out) | reinterpret_cast<uintptr_t>(t.part)) & 15);
         void *nb = nullptr;
@@ -861,7 +858,7 @@ int fnn_row_means(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, cons
 // Least squares over 5080 drawn calls (M 17 .. 2048, K 256 .. 16384, N 16 .. 16384, weights from memory and from cache; 8 % mean
 // error): a CU's stages, rounds of resident workgroups, the K split's second launch and partials, output, operand and weight
 // bytes, the longest row, ragged rows.
-float fnn_tiled_us(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags, int *splits)
+float fnn_tiled_us(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, int flags)
 {
     static const float kFit[2][11] = {{5.03f, 0.2922f, 2.760f, 2.696f, 1.447f, 2.021f, 1.363f, 0.194f, 0.841f, 5.68f, 0.0748f},    // 8-bit
                                       {7.12f, 0.3122f, 0.972f, 2.467f, 1.069f, 1.962f, 2.417f, 0.146f, 0.717f, 3.81f, 0.0050f}};   // 4-bit
@@ -869,7 +866,6 @@ float fnn_tiled_us(fnn_hip_ctx *ctx, int dt, int64_t m, int64_t n, int64_t k, in
     const TileLayout L = four ? tile_layout<FNN_DT_F4>(ctx, m, n, k, flags, false) : tile_layout<FNN_DT_U8>(ctx, m, n, k, flags, false);
     const int iters = (int)(L.kpad / BK), base = L.mtiles * L.ntiles;
     const int sp0 = tile_splits(four ? 0.4 : 0.7, L.cfg, base, iters, m, n, false), ips = (iters + sp0 - 1) / sp0, sp = (iters + ips - 1) / ips;
-    if (splits) *splits = sp;
     const int load = (base * sp + 255) / 256, per_cu = L.bm == 32 ? 4 : (L.bm == 64 ? 3 : 2);
     const float *c = kFit[four], mn = (float)m * (float)n / 1e6f, mk = (float)m * (float)k / 1e6f;
     const bool ragged = (four ? (k + 7) / 8 : (k + 3) / 4) % 4 != 0;

@@ -12,7 +12,6 @@ struct WaveArgs {
     const int8_t *af;            // [block of 32 operand rows][step][h 0..1][row][16 bytes]
     const int *rexp;             // [m_pad] power of two applied to the row, INT_MIN: a non-finite row
     const float *xsum;           // [m_pad] sum_k A[m,k]
-    const int4 *share_sums;      // U8: [m_pad][quarter of the units] sums of the row's digits in planes 0, 1, 2
     const float *scales, *zeros, *bias;
     float *out;
     const float *residual;       // sum_out = out + residual as well
@@ -29,10 +28,7 @@ struct WaveArgs {
 // wk: waves of a workgroup that share an output tile (1, 2, 4); tail: of the tiles behind main_tiles, 0 for none (wk 1: 2, 4, wk 2: 4)
 hipError_t fnn_wave_launch_i8(int wk, int tail, const WaveArgs &p, hipStream_t s);
 hipError_t fnn_wave_launch_i4(int wk, int tail, const WaveArgs &p, hipStream_t s);
-hipError_t fnn_wave_launch_u8(int wk, int tail, const WaveArgs &p, hipStream_t s);
 hipError_t fnn_wave_launch_u4(int wk, int tail, const WaveArgs &p, hipStream_t s);
 
-// The form that the call runs in by rule (0: it is another kernel's), and of all calls that these kernels can take the form with the lowest figure:
-int fnn_wave_form(fnn_hip_ctx *ctx, int dtype, int64_t m, int64_t n, int64_t k, int flags, float *us);
 // The form for these sizes by rule, wk + 8 tail, 0 for none; *us: the time expected of it (microseconds).
 int fnn_wave_choice(int dtype, int64_t m, int64_t n, int64_t k, float *us);

@@ -33,13 +33,12 @@ __device__ __forceinline__ void wave_tile(const WaveArgs &p, unsigned rg0, unsig
 {
     using D = DecI<DT>;
     constexpr int TM = WAVE_ROWS * 3 / 32, TN = WAVE_COLS / 32;   // blocks of 32 x 32
-    constexpr bool W8 = D::WPS == 4, U8 = DT == FNN_DT_U8;
+    constexpr bool W8 = D::WPS == 4;
     constexpr int RING = WAVE_RING(W8);                // steps in flight, and the unit in which K is dealt out
     constexpr int SHIFT = DT == FNN_DT_I4 ? 4 : 0;     // 4-bit signed lanes enter as 16 q
     constexpr int WL = W8 ? RING : RING / 2;           // weight loads per ring: a 16-byte piece is one step or two
     extern __shared__ __attribute__((aligned(16))) wf32x4 wred[];   // [wave][group of rows][column block][lane]
     __shared__ __attribute__((aligned(16))) int2 row_const[4][WAVE_ROWS];
-    __shared__ __attribute__((aligned(16))) int row_sums[U8 ? 4 : 1][3][WAVE_ROWS];   // [plane][row], this wave's share of K
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, h = lane >> 5;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wk = WK == 1 ? 0 : (WK == 2 ? wv >> 1 : wv);
@@ -73,25 +72,6 @@ __device__ __forceinline__ void wave_tile(const WaveArgs &p, unsigned rg0, unsig
             sc[j] = p.scales[n];
             zp[j] = p.zeros[n];
             bi[j] = p.bias ? p.bias[n] : 0.0f;
-        }
-    };
-
-    // U8: the sums of the rows' digits over this wave's share of K wait in LDS
-    int4 sums = {0, 0, 0, 0};
-    if constexpr (U8) {
-#pragma unroll
-        for (int s = 0; s < 4 / WK; s++) {
-            const int4 t = p.share_sums[(m0 + lr) * 4 + wk * (4 / WK) + s];
-            sums.x += t.x; sums.y += t.y; sums.z += t.z;
-        }
-    }
-    auto keep_sums = [&] {
-        if constexpr (U8) {
-            if (h == 0) {
-                row_sums[wv][0][lr] = sums.x;
-                row_sums[wv][1][lr] = sums.y;
-                row_sums[wv][2][lr] = sums.z;
-            }
         }
     };
 
@@ -154,7 +134,6 @@ __device__ __forceinline__ void wave_tile(const WaveArgs &p, unsigned rg0, unsig
                 for (int j = 0; j < TN; j++)
                     if (W8 || st / 2 < WL - 1) w[W8 ? st : st / 2][j] = load_w(W8 ? u0 * RING + st : u0 * WL + st / 2, j);
         }
-        keep_sums();
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < TN; j++) wd[0][j] = decode(0, j);
@@ -162,38 +141,10 @@ __device__ __forceinline__ void wave_tile(const WaveArgs &p, unsigned rg0, unsig
         load_constants();
         unit(u1 - 1, std::true_type{});
     } else {
-        keep_sums();
         load_constants();
     }
 
     // D: acc[i][j][e] is operand row 32 i + (e / 4) * 8 + h * 4 + e % 4, column 32 j + lr.
-    if (h == 0) row_const[wv][lr] = make_int2(rexp, __float_as_int(xsum));
-    // U8 (lanes enter as q - 128): the results are small beside sums of those and beside the zero point's term, which lies off the middle of the
-    // range.  shift * (a row's digits over this wave's share of K) joins the planes while they are integers, and what is left of the zero point
-    // is half a step: the rounding to 32 bits is that of numbers of the results' own size.
-    if constexpr (U8) {
-        int shift[TN];
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const float r = rintf(fmaf(128.0f, sc[j], zp[j]) / sc[j]);
-            shift[j] = fabsf(r) <= 256.0f ? (int)r : 0;   // (not for a zero point far outside the range, or scales of 0)
-            zp[j] = fmaf((float)(128 - shift[j]), sc[j], zp[j]);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-        for (int g = 0; g < 4; g++)
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                const wi32x4 s = *reinterpret_cast<const wi32x4 *>(&row_sums[wv][d][8 * g + 4 * h]);
-                const int slab = 3 * g + d;
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-#pragma unroll
-                    for (int j = 0; j < TN; j++) acc[slab >> 2][j][(slab & 3) * 4 + t] += shift[j] * s[t];
-            }
-    }
     // A value of this lane, (row 8 g + 4 h + t, column block j): the three planes of one activation row combined
     auto value = [&](int g, int t, int j) {
         float v = 0.0f;
@@ -204,6 +155,7 @@ __device__ __forceinline__ void wave_tile(const WaveArgs &p, unsigned rg0, unsig
         }
         return v;
     };
+    if (h == 0) row_const[wv][lr] = make_int2(rexp, __float_as_int(xsum));
     // The waves that split K hand each other their sums through LDS, four rows of a column as one piece, and share the groups of rows.
     // Then scale, bias, activation and stores, each in a pass of its own with its uniform test in front: nothing overlaps this part at one
     // wave per SIMD, and a wave fetches its code to run it once (0.25 us a KB).  Against single values

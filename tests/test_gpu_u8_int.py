@@ -1,4 +1,4 @@
-"""U8 weights on the int8 matrix cores (bytes as q - 128, the zero point's whole steps added to the integer sums): the vector kernel and the register tiles."""
+"""U8 weights: few rows on the int8 matrix cores (bytes as q - 128), many rows on the f16 ones, whose activations keep 22 bits of every value whatever its row holds."""
 import numpy as np
 import pytest
 
@@ -52,7 +52,7 @@ def test_few_rows(m, k, n):
 @pytest.mark.parametrize("form", [1, 2, 4, 1 | 2 << 3, 1 | 4 << 3, 2 | 4 << 3])
 @pytest.mark.parametrize("m,k,n", [(33, 200, 129), (130, 2600, 260), (1090, 130, 3900)])
 def test_register_tiles(form, m, k, n):
-    """Activations of 24 bits: 2^-23 of a row's largest value each, 4e-7 of the result's norm at most with the values drawn here."""
+    """U8 has none of those: asked for them, a call is what it is without.  4e-7 of the result's norm at most with the values drawn here."""
     rng = np.random.default_rng(m + form)
     pw = fastnn_amd.quantize_weights(flib.DT_U8, weights(rng, n, k))
     a = rng.standard_normal((m, k)).astype(np.float32)
@@ -63,19 +63,37 @@ def test_register_tiles(form, m, k, n):
     keep = np.setdiff1d(np.arange(m), [7])
     with fastnn_amd.HipContext(0) as ctx:
         h = ctx.register(pw)
+        ctx.set_option(flib.OPT_FRAGMENT, -1)
+        plain = ctx.qmatmul(h, a, n, bias=bias)
         ctx.set_option(flib.OPT_FRAGMENT, 1 << 14 | form)
         want = exact(pw, a, n, k, bias)
         got = ctx.qmatmul(h, a, n, bias=bias)
-        assert off(got, want) < 4e-7
+        assert off(got, want) < 4e-7 and got.tobytes() == plain.tobytes()
         broken = ctx.qmatmul(h, bad, n, bias=bias)
         assert not np.isfinite(broken[7]).any() and np.array_equal(broken[keep], got[keep])
         ctx.release(h)
 
 
+@pytest.mark.parametrize("value", [0.0, 50.0, 200.0, 1e4])
+def test_rows_with_one_large_value(value):
+    """Digit planes below the row's largest value would leave the others 23 - log2(value) bits: 2.5e-6 of the result's norm off at 200.  Hi and lo halves keep 22
+    bits of each; what is left is their f32 sums, 2.8e-7 to 5.7e-7 measured."""
+    m, k, n = 512, 4096, 4096
+    rng = np.random.default_rng(1)
+    pw = fastnn_amd.quantize_weights(flib.DT_U8, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    if value:
+        a[:, 77] = value
+    sel = np.arange(0, m, 16)
+    with fastnn_amd.HipContext(0) as ctx:
+        h = ctx.register(pw)
+        assert off(ctx.qmatmul(h, a, n)[sel], exact(pw, a[sel], n, k, 0.0)) < 9e-7
+        ctx.release(h)
+
+
 @pytest.mark.parametrize("form", [1, 2, 4, 1 | 2 << 3])
 def test_long_rows_with_the_tiles_asked_for(form):
-    """A lane and the zero point's shift are up to 384 together: 384 * 128 * K passes 2^31 from K = 43691 on, so that longer rows are another kernel's whatever the
-    option asks for (in 32-bit sums -128849 for 134324).  The sums are f32 then, of products of one sign, added 16 and more at a time: 45000 / 16
+    """A lane and the zero point's steps are up to 384 together: 384 * 128 * K passes 2^31 from K = 43691 on (in 32-bit sums -128849 for 134324).  The sums are f32, of products of one sign, added 16 and more at a time: 45000 / 16
     additions, each half of 2^-24 of the sum off at most, 8.4e-5 where all err to one side."""
     m, k, n = 40, 45000, 64
     q = np.full((n, k), 255, np.uint8)       # 1.5, and one weight of 0.5
