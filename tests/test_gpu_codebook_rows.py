@@ -101,6 +101,30 @@ def test_the_first_values_of_a_row_do_not_reach_the_row_before(ctx, m, k, value)
     ctx.release(handle)
 
 
+# beside values of a normal row one of every 128 is larger, on weights that are zero: what the others are held in shows
+@pytest.mark.parametrize("m,k,n", [(5, 1003, 333), (8, 1024, 1024), (9, 1024, 1024), (16, 1003, 333)])
+def test_small_values_beside_large_ones(ctx, m, k, n):
+    """Two f16 halves hold 22 bits of every value down to 2^-29 of a piece's largest: 2^-23 of each value and of each table entry, and f32 sums, 1.1e-7 of the result's
+    norm measured at any size of the large ones, 3e-7 allowed."""
+    rng = np.random.default_rng(m + k)
+    pw = codebook_weight(rng, n, k)
+    kp, table, zero = -(-k // 8), pw.codebook.copy(), 7
+    table[zero] = 0.0
+    words = pw.words[:n * kp].reshape(n, kp).copy()
+    large = np.arange(5, k, 128)
+    for c in large:
+        words[:, c // 8] = words[:, c // 8] & ~np.uint32(15 << 4 * (c % 8)) | np.uint32(zero << 4 * (c % 8))
+    values = table[words[:, :, None] >> 4 * np.arange(8, dtype=np.uint32) & 15].reshape(n, -1)[:, :k].astype(np.float64)
+    values *= np.repeat(pw.scales.reshape(n, -1), 32, axis=1)[:, :k]
+    handle = ctx.register(fastnn_amd.PackedWeight(flib.DT_I4CB, n, k, np.concatenate([words.reshape(-1), np.zeros(16, np.uint32)]), pw.scales, pw.zeros, 32, table))
+    for value in (1.0, 2.0 ** 10, 2.0 ** 17, 2.0 ** 24, 2.0 ** 28):
+        a = rng.standard_normal((m, k)).astype(np.float32)
+        a[:, large] = value
+        want = a.astype(np.float64) @ values.T
+        assert np.linalg.norm(ctx.qmatmul(handle, a, n) - want) < 3e-7 * np.linalg.norm(want), value
+    ctx.release(handle)
+
+
 # up to four rows whose K or addresses fit no 16 bytes (the last two: columns beyond 8192): one chunk of 512 and less, several, blocks of 32 that end early, eight waves' slices
 @pytest.mark.parametrize("k,n", [(1, 1), (7, 3), (31, 15), (300, 700), (513, 9), (1003, 333), (2050, 130), (4100, 257), (9001, 48), (1024, 40), (512, 8200), (2080, 8200)])
 @pytest.mark.parametrize("m", [1, 2, 3, 4])
