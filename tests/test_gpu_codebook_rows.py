@@ -125,6 +125,19 @@ def test_small_values_beside_large_ones(ctx, m, k, n):
     ctx.release(handle)
 
 
+@pytest.mark.parametrize("m,k,n", [(6, 1024, 512), (16, 1024, 512), (8, 1003, 333), (13, 1003, 333)])
+def test_activations_at_the_end_of_the_range(ctx, m, k, n):
+    """Results of 3e38 times weights below 0.2 are numbers, and so are those of activations of 1e-37 (2e-5 of the largest, as above)."""
+    rng = np.random.default_rng(m + k)
+    pw = codebook_weight(rng, n, k)
+    weights = ctx.dequant(handle := ctx.register(pw), n, k).astype(np.float64)
+    for value in (3e38, 1e-37):
+        a = (rng.standard_normal((m, k)) * 1e-3).astype(np.float32) * np.float32(value)
+        a[m - 1, 5] = value
+        assert_close(ctx.qmatmul(handle, a, n), a.astype(np.float64) @ weights.T, 2e-5)
+    ctx.release(handle)
+
+
 # up to four rows whose K or addresses fit no 16 bytes (the last two: columns beyond 8192): one chunk of 512 and less, several, blocks of 32 that end early, eight waves' slices
 @pytest.mark.parametrize("k,n", [(1, 1), (7, 3), (31, 15), (300, 700), (513, 9), (1003, 333), (2050, 130), (4100, 257), (9001, 48), (1024, 40), (512, 8200), (2080, 8200)])
 @pytest.mark.parametrize("m", [1, 2, 3, 4])
