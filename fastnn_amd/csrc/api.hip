@@ -1406,6 +1406,7 @@ int fnn_ctx_replay(fnn_hip_ctx *ctx, fnn_hip_graph *g, bool host_busy)
 }
 int fnn_ctx_wait(fnn_hip_ctx *ctx) { return guarded(ctx, "wait", [&] { return finish(ctx); }); }
 bool fnn_ctx_may_send(fnn_hip_ctx *ctx, const void *dst, size_t bytes) { return !ctx->capturing && ctx->io.marks_ready() && fnn_is_pinned(dst, bytes); }
+bool fnn_ctx_has_marks(const fnn_hip_ctx *ctx) { return ctx->io.marks != nullptr; }
 void fnn_ctx_clear_mark(fnn_hip_ctx *ctx, int mark) { ctx->io.clear_mark(mark); }
 int fnn_ctx_mark(fnn_hip_ctx *ctx, int mark)
 {

@@ -137,8 +137,9 @@ struct fnn_plan {
     std::unique_ptr<fnn_plan> half[2];
     bool halves_tried = false, last_halved = false;
     std::vector<fnn_slice> halved;    // the slices that are halved: what a forward pass may write and read
-    // instructions behind which a forward pass marks that results may leave while the rest runs (EarlyResults); the graph holds the marks
+    // instructions behind which a forward pass marks that results may leave while the rest runs (EarlyResults)
     std::vector<size_t> cuts;
+    bool graph_marks = false;         // the graph holds their marks: not where it was recorded on a backend that had none yet
     int first_mark = 0;               // mark of cuts[0]
     bool is_half = false;             // the plan is one of another plan's `half`
     int recuts = 0;                   // times that other results moved them
@@ -1217,6 +1218,7 @@ int dispatch_impl(fnn_backend *b, fnn_plan *p, uint64_t *elapsed_ns, uint64_t n_
                 p->graph_uid = b->uid; p->graph_generation = b->generation;
                 p->graph_weights_epoch = w0; p->graph_ws_epoch = s0; p->graph_scratch_epoch = c0;
                 p->graph_env = b->shape_env_sig;
+                p->graph_marks = fnn_ctx_has_marks(b->ctx);
             } else {
                 if (g) fnn_hip_graph_destroy(b->ctx, g);
                 p->graph_failures++;
@@ -1346,6 +1348,8 @@ struct EarlyResults {
             if (p->graph) p->recuts++;
             p->drop_graph(ctx);
             p->cuts = cuts;
+        } else if (p->graph && !p->cuts.empty() && !p->graph_marks) {
+            p->drop_graph(ctx);
         }
         const size_t marks = p->cuts.size() + (marked_end ? 1 : 0);
         if (!marked_end)

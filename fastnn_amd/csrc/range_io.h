@@ -99,6 +99,7 @@ int fnn_ctx_replay(fnn_hip_ctx *ctx, fnn_hip_graph *g, bool host_busy);
 // whole pass is (it waits for the mark); done as copy_out's.  For pinned memory.
 constexpr int FNN_MARKS = 16;
 bool fnn_ctx_may_send(fnn_hip_ctx *ctx, const void *dst, size_t bytes);
+bool fnn_ctx_has_marks(const fnn_hip_ctx *ctx);   // (from the first may_send that says yes on; before that mark does nothing)
 void fnn_ctx_clear_mark(fnn_hip_ctx *ctx, int mark);
 int fnn_ctx_mark(fnn_hip_ctx *ctx, int mark);
 int fnn_ctx_send(fnn_hip_ctx *ctx, int mark, void *dst, const void *src_dev, size_t bytes);
