@@ -1897,9 +1897,9 @@ int fnn_backend_forward(fnn_backend *b, fnn_plan *p, const fnn_host_slice *input
             for (uint64_t i = 0; i < n_inputs && !st; i++) st = write_slice(b, inputs[i].offset, inputs[i].data, inputs[i].size, true);
             EarlyResults early(p, b->ctx, std::vector<fnn_host_slice>(outputs, outputs + n_outputs), false);
             if (!st) st = dispatch_impl(b, p, nullptr, 0, 0, nullptr, false);
+            if (!st) st = early.send(b, false);   // (first: a large result for ordinary memory holds the host until the stream's end)
             for (uint64_t i = 0; i < n_outputs && !st; i++)
                 if (!early.leaves_early(i)) st = read_slice(b, outputs[i].offset, outputs[i].data, outputs[i].size);
-            if (!st) st = early.send(b, false);
         }
         if (!st) return lift(b, fnn_ctx_wait(b->ctx));
         fnn_hip_sync(b->ctx);

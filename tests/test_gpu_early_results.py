@@ -146,3 +146,25 @@ def test_a_pinned_result_that_ends_outside_the_arena(past):
             be.forward(plan, [(chain.x[0], x)], [(end[0], whole)])
             assert whole.tobytes() == want.tobytes()
         plan.close()
+
+
+@pytest.mark.parametrize("first", [1, 4, 9])
+def test_results_for_ordinary_memory_beside_early_ones(first):
+    """Pinned results that leave early, large ones for ordinary memory and small ones in one call, in any order."""
+    n = 1 << 19
+    chain = Chain(n)
+    rng = np.random.default_rng(first)
+    asked = [first] + [i for i in (0, 1, 2, 4, 9) if i != first]
+    with HipBackend(0) as be:
+        be.allocate_arena(chain.arena)
+        plan = chain.plan()
+        for call in range(4):
+            x = rng.standard_normal(n).astype(np.float32)
+            out = [result("pinned" if (i + call) % 2 else "ordinary", n) for i in asked]
+            small = np.empty(100, np.float32)
+            be.forward(plan, [(chain.x[0], x)], [(chain.v[i][0], o) for i, o in zip(asked, out)] + [(chain.v[3][0], small)])
+            want = chain.expect(x)
+            for i, o in zip(asked, out):
+                assert o.tobytes() == want[i].tobytes(), (call, i)
+            assert small.tobytes() == want[3][:100].tobytes()
+        plan.close()
