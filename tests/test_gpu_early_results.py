@@ -168,3 +168,30 @@ def test_results_for_ordinary_memory_beside_early_ones(first):
                 assert o.tobytes() == want[i].tobytes(), (call, i)
             assert small.tobytes() == want[3][:100].tobytes()
         plan.close()
+
+
+def test_a_mark_that_is_long_in_coming():
+    """A pass whose first result is final after some 9 ms: the wait for it pauses (without, the processor time is the pass's; 0.65 of it measured), and the result is whole."""
+    n, calls = 1 << 24, 240
+    size = n * 4
+    plan = ExecutablePlan(4 * size)
+    plan.call_kernel("relu_f32", [(0, size)], (size, size), [n])
+    for i in range(calls):
+        a, b = ((1, 2) if i % 2 == 0 else (2, 1))
+        plan.call_kernel("add_f32", [(a * size, size), (0, size)], (b * size, size), [n])
+    plan.call_kernel("relu_f32", [(size, size)], (3 * size, size), [n])
+    for _ in range(8):
+        plan.call_kernel("add_f32", [(size, size), (0, size)], (2 * size, size), [n])
+    x = np.random.default_rng(5).integers(0, 3, n).astype(np.float32)      # (whole numbers: the sums are exact)
+    with HipBackend(0) as be:
+        be.allocate_arena(4 * size)
+        be.write_arena(0, x)
+        share = []
+        for _ in range(6):
+            out = flib.result_array((n,))
+            took, cpu = time.perf_counter(), time.process_time()
+            be.forward(plan, [(0, x[:64])], [(3 * size, out)])
+            share.append((time.process_time() - cpu) / (time.perf_counter() - took))
+            assert np.array_equal(out, x * (calls + 1))
+        assert min(share[2:]) < 0.9, share       # (the first ones allocate)
+        plan.close()
