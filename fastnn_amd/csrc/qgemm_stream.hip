@@ -34,36 +34,44 @@ bool plan_stream(bool cb, int max_tiles, int max_mb, int64_t m, int64_t n, int64
     // launches: no more workgroups than the chip holds at once (a second wave of
     // workgroups repeats every phase).  4096 x 4096 at M = 32: 14.4 against 17.9 us; 2048 -> 8192 FP8: 13.3 against 17.4;
     // 4096 x 11008 (688 workgroups): 25.0 against 23.5; M = 64 on 4096 x 4096: 21.3 against 20.0.
-    if (forced == 0 && ntiles * splits > 320 && cb && !(mb == 3 && n * k > 48000000)) {   // (those: 39 x 7680 x 15105 64.2 us with two row tiles per wave, 69.3 so)
-        // Wide outputs, codebook weights: one row tile per wave, two workgroups per CU (their LDS: rounds of 512 up to 32 rows, of 256 beyond) and
-        // the fewest rounds that leaves.  The tiles decode every nibble again for each 32 rows; two row tiles per wave cannot hide the look-ups.
-        // 4096 x 11008 M = 64 62.3 us on the tiles, 43.1 so, 2048 x 11008 39.7 and 26.6, 2048 x 16384 37.4 and 29.2; M = 32, two row tiles per wave
-        // against this, 28.0 and 27.3, 19.4 and 17.6, 21.0 and 19.3.
-        const int64_t wide_kr = mb <= 2 ? 512 : 256, total = (k + wide_kr - 1) / wide_kr;
-        for (int64_t r = 1; r <= 16; r++) {
-            const int64_t s = (total + r - 1) / r;
-            if (s > 64 || (s - 1) * r >= total || ntiles * s > 512) continue;   // (no empty split)
-            if (ntiles * s < 256) break;   // (too few workgroups)
-            *out = StreamPlan{mb, 1, (int)wide_kr, (int)s, (int)r, (int)ntiles};
-            return true;
-        }
-    }
     if (forced == 0 && ntiles * splits > 320) {
         // Wide outputs: two row tiles per wave (256 weight rows per workgroup) and as few rounds per workgroup as keep the
         // launch within one round of workgroups (one workgroup of this form per CU: at most 256).  4096 x 11008 (43 column tiles): 4 splits x 2 rounds of 512, 172 workgroups,
         // M = 17 19.2 us against 23.0 on the tiled path, M = 32 21.3 against 23.9 (8 splits x 1 round, 344 workgroups: 25.5).
-        if (mb * 2 > max_tiles) return false;
-        const int64_t ntiles2 = (n + FNN_STREAM_NW * 2 * 16 - 1) / (FNN_STREAM_NW * 2 * 16);
-        const int64_t total512 = (k + 511) / 512;
-        for (int64_t r2 = 1; r2 <= 4; r2++) {
-            const int64_t s2 = (total512 + r2 - 1) / r2;
-            if (s2 > 64 || (s2 - 1) * r2 >= total512) continue;   // (no empty split)
-            if (ntiles2 * s2 > 256) continue;   // (one workgroup of this form per CU: 270 workgroups on 5120 x 13824 ran 33.7 us against 28.0 on the tiled path)
-            if (ntiles2 * s2 < 128) break;                        // (too few workgroups: the tiled path is ahead)
-            *out = StreamPlan{mb, 2, 512, (int)s2, (int)r2, (int)ntiles2};
-            return true;
+        int64_t r2 = 0;
+        if (mb * 2 <= max_tiles) {
+            const int64_t ntiles2 = (n + FNN_STREAM_NW * 2 * 16 - 1) / (FNN_STREAM_NW * 2 * 16), total512 = (k + 511) / 512;
+            for (int64_t r = 1; r <= 4 && !r2; r++) {
+                const int64_t s = (total512 + r - 1) / r;
+                if (s > 64 || (s - 1) * r >= total512) continue;   // (no empty split)
+                if (ntiles2 * s > 256) continue;   // (one workgroup of this form per CU: 270 workgroups on 5120 x 13824 ran 33.7 us against 28.0 on the tiled path)
+                if (ntiles2 * s < 128) break;                      // (too few workgroups: the tiled path is ahead)
+                *out = StreamPlan{mb, 2, 512, (int)s, (int)r, (int)ntiles2};
+                r2 = r;
+            }
         }
-        return false;
+        // Codebook weights: one row tile per wave, two workgroups per CU (their LDS: rounds of 512 up to 32 rows, of 256 beyond) and the
+        // fewest rounds that leaves.  The tiles decode every nibble again for each 32 rows; two row tiles per wave cannot hide the look-ups.
+        // 4096 x 11008 M = 64 62.3 us on the tiles, 43.1 so, 2048 x 11008 39.7 and 26.6, 2048 x 16384 37.4 and 29.2; M = 32, two row tiles per wave
+        // against this, 28.0 and 27.3, 19.4 and 17.6, 21.0 and 19.3.
+        if (cb) {
+            const int64_t wide_kr = mb <= 2 ? 512 : 256, total = (k + wide_kr - 1) / wide_kr;
+            for (int64_t r = 1; r <= 16; r++) {
+                const int64_t s = (total + r - 1) / r;
+                if (s > 64 || (s - 1) * r >= total || ntiles * s > 512) continue;   // (no empty split)
+                if (ntiles * s < 256) break;   // (too few workgroups)
+                // A long K over few columns, from 33 rows on: workgroups of one round leave the last one of a column tile more parts to add up than they save.  90
+                // drawn calls of 17 to 60 splits take 1.18 times the tiles' time so, 1.57 at most (54 x 15104 x 976 34.6 us there, 54.5 so; 60 x 7296 x 1664 29.4
+                // and 34.6; 56 x 4992 x 2496 25.7 and 29.3), five less (38 x 5120 x 2432 29.9 and 26.1).  17 and more of two rounds are 4 to 10 % ahead.
+                if (mb > 2 && r == 1 && s > 16) continue;
+                // Two row tiles per wave in half as many rounds, each of twice the values, are ahead where those are three and more: 43 x 8448 x 10368 6 rounds against 3,
+                // 53.5 us and 50.8, 39 x 7680 x 15105 8 against 4, 65.0 and 61.0; with 4 against 2 it is 1 % behind, 5 against 3 or 7 against 4 3 to 10 %.
+                if (mb > 2 && r >= 6 && r2 && r >= 2 * r2) break;
+                *out = StreamPlan{mb, 1, (int)wide_kr, (int)s, (int)r, (int)ntiles};
+                return true;
+            }
+        }
+        return r2 != 0;
     }
     *out = StreamPlan{mb, rt, kr, (int)splits, (int)rounds, (int)ntiles};
     return true;

@@ -194,3 +194,29 @@ def test_wide_outputs(ctx, orc, m, k, n):
     handle = ctx.register(pw)
     assert_close(ctx.qmatmul(handle, a, n, bias=bias), orc.qmatmul(to_oracle(orc, pw), a, order=2, bias=bias), 2e-5)
     ctx.release(handle)
+
+
+# (splits << 8 | row tiles a wave << 4 | k-values of a round / 256; 0: none, the tiles take it)
+@pytest.mark.parametrize("m,k,n,shape", [(16, 4224, 11008, 5 << 8 | 1 << 4 | 2), (32, 2432, 11001, 5 << 8 | 1 << 4 | 2), (48, 2432, 11001, 5 << 8 | 1 << 4 | 1),
+                                         (64, 4224, 5121, 9 << 8 | 1 << 4 | 1), (33, 8448, 10368, 6 << 8 | 2 << 4 | 2), (37, 9856, 1248, 0), (60, 7296, 1664, 0)])
+def test_the_form_that_wide_outputs_run_in(ctx, m, k, n, shape):
+    """By rule the bits are those of the form named, and the other kernels', whose sums have another order, are 4e-5 of the largest result off at most (2e-5 each)."""
+    rng = np.random.default_rng(m + k)
+    pw = codebook_weight(rng, n, k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    handle = ctx.register(pw)
+    got = ctx.qmatmul(handle, a, n)
+    try:
+        ctx.set_option(flib.OPT_FRAGMENT, -1)      # (not the kernel for 5 to 16 rows)
+        ctx.set_option(flib.OPT_STREAM_SHAPE, shape)
+        named = ctx.qmatmul(handle, a, n)
+        ctx.set_option(flib.OPT_STREAM_MAX_M, 0)
+        tiles = ctx.qmatmul(handle, a, n)
+    finally:
+        ctx.set_option(flib.OPT_FRAGMENT, 0)
+        ctx.set_option(flib.OPT_STREAM_SHAPE, 0)
+        ctx.set_option(flib.OPT_STREAM_MAX_M, 32)
+    assert got.tobytes() == named.tobytes()
+    assert (got.tobytes() == tiles.tobytes()) == (shape == 0)
+    assert_close(got, tiles, 4e-5)
+    ctx.release(handle)
