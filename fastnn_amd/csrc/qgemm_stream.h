@@ -21,8 +21,12 @@ struct StreamArgs {
 constexpr int FNN_STREAM_NW = 8;   // waves per workgroup
 
 // Shape of a launch: blocks of 16 activation rows, row tiles of 16 weight rows per wave, k-values per round, K splits,
-// rounds per workgroup, column tiles
-struct StreamPlan { int mb, rt, kr, splits, rounds, ntiles; };
+// rounds per workgroup, column tiles; low_up: codebook weights, the low halves of the activations scaled (one row tile, rounds of StreamPlan::wide_kr)
+struct StreamPlan {
+    int mb, rt, kr, splits, rounds, ntiles;
+    bool low_up = false;
+    static constexpr int wide_kr(int mb) { return mb <= 2 ? 512 : 256; }
+};
 
 // one translation unit per weight type (qgemm_stream_<type>.hip)
 hipError_t fnn_stream_launch_i8(const StreamPlan &pl, const StreamArgs &p, hipStream_t s);

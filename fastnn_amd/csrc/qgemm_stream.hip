@@ -17,11 +17,13 @@ bool plan_stream(bool cb, int max_tiles, int max_mb, int64_t m, int64_t n, int64
     const int64_t nt1 = (n + FNN_STREAM_NW * 16 - 1) / (FNN_STREAM_NW * 16);
     if (nt1 * ((k + 511) / 512) < 224) kr = 256;
     int64_t splits = 0;
+    const bool low_up = forced & 128;
     if (forced > 0) {
-        rt = (int)((forced >> 4) & 15);
+        rt = (int)((forced >> 4) & 7);
         kr = (int)(forced & 15) * 256;
         splits = forced >> 8;
         if (rt < 1 || rt > 2 || (kr != 256 && kr != 512)) return false;
+        if (low_up && (!cb || rt != 1 || kr != StreamPlan::wide_kr(mb))) return false;
     }
     if (mb * rt > max_tiles) return false;   // accumulator tiles that fit the registers
     const int64_t kr_total = (k + kr - 1) / kr;   // rounds over all of K
@@ -55,7 +57,7 @@ bool plan_stream(bool cb, int max_tiles, int max_mb, int64_t m, int64_t n, int64
         // 4096 x 11008 M = 64 62.3 us on the tiles, 43.1 so, 2048 x 11008 39.7 and 26.6, 2048 x 16384 37.4 and 29.2; M = 32, two row tiles per wave
         // against this, 28.0 and 27.3, 19.4 and 17.6, 21.0 and 19.3.
         if (cb) {
-            const int64_t wide_kr = mb <= 2 ? 512 : 256, total = (k + wide_kr - 1) / wide_kr;
+            const int64_t wide_kr = StreamPlan::wide_kr(mb), total = (k + wide_kr - 1) / wide_kr;
             for (int64_t r = 1; r <= 16; r++) {
                 const int64_t s = (total + r - 1) / r;
                 if (s > 64 || (s - 1) * r >= total || ntiles * s > 512) continue;   // (no empty split)
@@ -67,13 +69,16 @@ bool plan_stream(bool cb, int max_tiles, int max_mb, int64_t m, int64_t n, int64
                 // Two row tiles per wave in half as many rounds, each of twice the values, are ahead where those are three and more: 43 x 8448 x 10368 6 rounds against 3,
                 // 53.5 us and 50.8, 39 x 7680 x 15105 8 against 4, 65.0 and 61.0; with 4 against 2 it is 1 % behind, 5 against 3 or 7 against 4 3 to 10 %.
                 if (mb > 2 && r >= 6 && r2 && r >= 2 * r2) break;
-                *out = StreamPlan{mb, 1, (int)wide_kr, (int)s, (int)r, (int)ntiles};
+                // Without two row tiles as a plan these calls are the tiles' otherwise, which hold the activations' low halves scaled by 2^11.  So does this form then: unscaled
+                // they are denormals from 2^-18 of a round's largest value on, and beside values of 2^24 on weights of zero a normal row comes out 1.7e-5 of its norm
+                // off, not 1.6e-7 (64 x 3072 x 12288).  Four fused multiply-adds a product of 32 x 16 x 16: 64 x 4096 x 11008 40.8 -> 44.5 us, 64 x 2048 x 11008 25.6 -> 27.4.
+                *out = StreamPlan{mb, 1, (int)wide_kr, (int)s, (int)r, (int)ntiles, r2 == 0};
                 return true;
             }
         }
         return r2 != 0;
     }
-    *out = StreamPlan{mb, rt, kr, (int)splits, (int)rounds, (int)ntiles};
+    *out = StreamPlan{mb, rt, kr, (int)splits, (int)rounds, (int)ntiles, low_up};
     return true;
 }
 

@@ -104,9 +104,11 @@ __device__ __forceinline__ void transpose4(uint32_t a, uint32_t b, uint32_t c, u
 
 // MB: blocks of 16 activation rows (M <= 16*MB); RT: row tiles of 16 weight rows per wave; KR: k-values per round
 // FRAG: the packed words come from the fragment-major copy (p.words_fr)
-template <int DT, int MB, int RT, int KR, bool FRAG = false>
+// LOW_UP: the low halves of the activations are scaled by 2^11 (no denormals while a value is above 2^-29 of its round's largest)
+template <int DT, int MB, int RT, int KR, bool FRAG = false, bool LOW_UP = false>
 __global__ void __launch_bounds__(NW * 64) qgemm_stream_kernel(StreamArgs p)
 {
+    constexpr float LO_UP = 2048.0f, LO_DOWN = 1.0f / 2048.0f;
     using T = StreamType<DT>;
     constexpr bool INT8 = T::INT8;
     constexpr bool CB = DT == FNN_DT_I4CB;           // nibbles look up a 16-entry table; one f32 scale per 32 values
@@ -335,7 +337,7 @@ __global__ void __launch_bounds__(NW * 64) qgemm_stream_kernel(StreamArgs p)
                         const float v = __uint_as_float(xr[u][j][e]) * inv;
                         const _Float16 h = (_Float16)v;
                         hi[e] = h;
-                        lo[e] = (_Float16)(v - (float)h);
+                        lo[e] = (_Float16)(LOW_UP ? fmaf(v, LO_UP, (float)h * -LO_UP) : v - (float)h);   // (exact but for the rounding to f16)
                     }
                     // MFMA step li / 8 of the owner's lane load, halves (li % 8) .. + 3 of its hi and of its lo fragment
                     // (codebook weights: a step is one block of 32 values, the owner holds its values 8 * owner ..)
@@ -455,9 +457,12 @@ __global__ void __launch_bounds__(NW * 64) qgemm_stream_kernel(StreamArgs p)
 #pragma unroll
                 for (int r = 0; r < RT; r++) {
                     // the block's sum (the lo x lo product is below 2^-22 of the terms), then the block scale
-                    f32x4 blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bwh[r], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bwl[r], blk, 0, 0, 0);
+                    const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, low = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bwh[r], zero, 0, 0, 0);
+                    f32x4 blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bwl[r], LOW_UP ? zero : low, 0, 0, 0);
                     blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bwh[r], blk, 0, 0, 0);
+                    if constexpr (LOW_UP)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) blk[e] = fmaf(low[e], LO_DOWN, blk[e]);
 #pragma unroll
                     for (int e = 0; e < 4; e++) acc[b][r][e] = fmaf(bsc[r], blk[e], acc[b][r][e]);
                 }
@@ -639,19 +644,19 @@ size_t stream_lds_bytes()
     return (size_t)LOADS * SUB * MB * 64 * 16;
 }
 
-template <int DT, int MB, int RT, int KR, bool FRAG = false>
+template <int DT, int MB, int RT, int KR, bool LOW_UP = false, bool FRAG = false>
 hipError_t launch_stream(const StreamArgs &p, hipStream_t s)
 {
     if constexpr (!FRAG) {
-        if (p.words_fr) return launch_stream<DT, MB, RT, KR, true>(p, s);
+        if (p.words_fr) return launch_stream<DT, MB, RT, KR, LOW_UP, true>(p, s);
     }
     static std::atomic<uint64_t> raised{0};
     const size_t lds = stream_lds_bytes<DT, MB, RT, KR>();
     if (lds > 48 * 1024) {
-        hipError_t e = fnn_raise_lds_limit(raised, (const void *)qgemm_stream_kernel<DT, MB, RT, KR, FRAG>, (int)lds);
+        hipError_t e = fnn_raise_lds_limit(raised, (const void *)qgemm_stream_kernel<DT, MB, RT, KR, FRAG, LOW_UP>, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((qgemm_stream_kernel<DT, MB, RT, KR, FRAG>), dim3((unsigned)(p.ntiles * p.splits)), dim3(NW * 64), lds, s, p);
+    hipLaunchKernelGGL((qgemm_stream_kernel<DT, MB, RT, KR, FRAG, LOW_UP>), dim3((unsigned)(p.ntiles * p.splits)), dim3(NW * 64), lds, s, p);
     return hipGetLastError();
 }
 
@@ -660,6 +665,8 @@ hipError_t launch_mb(const StreamPlan &pl, const StreamArgs &p, hipStream_t s)
 {
     using T = StreamType<DT>;
     constexpr int kTiles = T::INT8 ? 4 : (DT == FNN_DT_I4CB ? 6 : 8);   // MB * RT accumulator tiles (x 3 planes on the int8 path) that fit the registers
+    if constexpr (DT == FNN_DT_I4CB)
+        if (pl.low_up) return launch_stream<DT, MB, 1, StreamPlan::wide_kr(MB), true>(p, s);
     if (pl.rt == 2) {
         if constexpr (MB * 2 <= kTiles) {
             if (pl.kr == 512) return launch_stream<DT, MB, 2, 512>(p, s);

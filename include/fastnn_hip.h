@@ -152,7 +152,9 @@ enum {
                                   /* K = 8192 on), from M = 5 where N <= 2048, K >= 4 N and K >= 8192 (16384 for I8 / I4 / U4);  */
                                   /* from M = 9 also where K / 512 fills the last of two or more rounds of eight at most half    */
     FNN_OPT_STREAM_SHAPE = 21,    /* its launch shape: 0 (default) = by rule, else (splits << 8) | (row tiles per wave << 4) |   */
-                                  /* (k-values per round / 256), splits = 0 meaning one round per workgroup                      */
+                                  /* (k-values per round / 256), splits = 0 meaning one round per workgroup; + 128: codebook       */
+                                  /* weights, one row tile, 512 k-values a round up to M = 32 and 256 beyond: the low halves of the */
+                                  /* activations scaled (22 bits of values down to 2^-29 of a round's largest, else 2^-18)         */
     FNN_OPT_DIGIT_PLANES = 22,    /* int8 matrix-core GEMM (M >= 17, I8 / I4 / U4 weights): activation digit planes, 3 (22 bits     */
                                   /* below the row maximum, 2e-5 of max|ref| stated) or 4 (30 bits, 4e-6, a third more matrix-core */
                                   /* work and operand traffic); 0 (default) = three wherever they measured faster (4-bit weights;   */

@@ -101,11 +101,13 @@ def test_the_first_values_of_a_row_do_not_reach_the_row_before(ctx, m, k, value)
     ctx.release(handle)
 
 
-# beside values of a normal row one of every 128 is larger, on weights that are zero: what the others are held in shows
-@pytest.mark.parametrize("m,k,n", [(5, 1003, 333), (8, 1024, 1024), (9, 1024, 1024), (16, 1003, 333)])
-def test_small_values_beside_large_ones(ctx, m, k, n):
-    """Two f16 halves hold 22 bits of every value down to 2^-29 of a piece's largest: 2^-23 of each value and of each table entry, and f32 sums, 1.1e-7 of the result's
-    norm measured at any size of the large ones, 3e-7 allowed."""
+# beside values of a normal row one of every 128 is larger, on weights that are zero: what the others are held in shows.  (shape: as FNN_OPT_STREAM_SHAPE names it; by rule
+# the first four are the kernel's of 5 to 16 rows, the last one is the form for wide outputs)
+@pytest.mark.parametrize("m,k,n,shape", [(5, 1003, 333, 0), (8, 1024, 1024, 0), (9, 1024, 1024, 0), (16, 1003, 333, 0), (16, 1152, 300, 0x92), (32, 1152, 300, 0x192),
+                                         (48, 1152, 300, 0x91), (64, 1152, 300, 0x291), (57, 4224, 5121, 0)])
+def test_small_values_beside_large_ones(ctx, m, k, n, shape):
+    """Two f16 halves hold 22 bits of every value down to 2^-29 of a piece's largest: 2^-23 of each value and of each table entry, and f32 sums, 1.1e-7 to 1.6e-7 of the
+    result's norm measured at any size of the large ones, 3e-7 allowed."""
     rng = np.random.default_rng(m + k)
     pw = codebook_weight(rng, n, k)
     kp, table, zero = -(-k // 8), pw.codebook.copy(), 7
@@ -117,11 +119,24 @@ def test_small_values_beside_large_ones(ctx, m, k, n):
     values = table[words[:, :, None] >> 4 * np.arange(8, dtype=np.uint32) & 15].reshape(n, -1)[:, :k].astype(np.float64)
     values *= np.repeat(pw.scales.reshape(n, -1), 32, axis=1)[:, :k]
     handle = ctx.register(fastnn_amd.PackedWeight(flib.DT_I4CB, n, k, np.concatenate([words.reshape(-1), np.zeros(16, np.uint32)]), pw.scales, pw.zeros, 32, table))
-    for value in (1.0, 2.0 ** 10, 2.0 ** 17, 2.0 ** 24, 2.0 ** 28):
-        a = rng.standard_normal((m, k)).astype(np.float32)
-        a[:, large] = value
-        want = a.astype(np.float64) @ values.T
-        assert np.linalg.norm(ctx.qmatmul(handle, a, n) - want) < 3e-7 * np.linalg.norm(want), value
+    try:
+        if shape:
+            ctx.set_option(flib.OPT_FRAGMENT, -1)
+            ctx.set_option(flib.OPT_STREAM_SHAPE, shape)
+        for value in (1.0, 2.0 ** 10, 2.0 ** 17, 2.0 ** 24, 2.0 ** 28):
+            a = rng.standard_normal((m, k)).astype(np.float32)
+            a[:, large] = value
+            want = a.astype(np.float64) @ values.T
+            got = ctx.qmatmul(handle, a, n)
+            assert np.linalg.norm(got - want) < 3e-7 * np.linalg.norm(want), value
+            if shape:       # (the named form has run)
+                ctx.set_option(flib.OPT_STREAM_MAX_M, 0)
+                assert ctx.qmatmul(handle, a, n).tobytes() != got.tobytes()
+                ctx.set_option(flib.OPT_STREAM_MAX_M, 32)
+    finally:
+        ctx.set_option(flib.OPT_FRAGMENT, 0)
+        ctx.set_option(flib.OPT_STREAM_SHAPE, 0)
+        ctx.set_option(flib.OPT_STREAM_MAX_M, 32)
     ctx.release(handle)
 
 
@@ -196,9 +211,9 @@ def test_wide_outputs(ctx, orc, m, k, n):
     ctx.release(handle)
 
 
-# (splits << 8 | row tiles a wave << 4 | k-values of a round / 256; 0: none, the tiles take it)
+# (splits << 8 | 128, low halves scaled | row tiles a wave << 4 | k-values of a round / 256; 0: none, the tiles take it)
 @pytest.mark.parametrize("m,k,n,shape", [(16, 4224, 11008, 5 << 8 | 1 << 4 | 2), (32, 2432, 11001, 5 << 8 | 1 << 4 | 2), (48, 2432, 11001, 5 << 8 | 1 << 4 | 1),
-                                         (64, 4224, 5121, 9 << 8 | 1 << 4 | 1), (33, 8448, 10368, 6 << 8 | 2 << 4 | 2), (37, 9856, 1248, 0), (60, 7296, 1664, 0)])
+                                         (64, 4224, 5121, 9 << 8 | 128 | 1 << 4 | 1), (33, 8448, 10368, 6 << 8 | 2 << 4 | 2), (37, 9856, 1248, 0), (60, 7296, 1664, 0)])
 def test_the_form_that_wide_outputs_run_in(ctx, m, k, n, shape):
     """By rule the bits are those of the form named, and the other kernels', whose sums have another order, are 4e-5 of the largest result off at most (2e-5 each)."""
     rng = np.random.default_rng(m + k)
