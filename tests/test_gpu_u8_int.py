@@ -29,23 +29,34 @@ def off(got, want):
     return float(np.linalg.norm(got - want) / np.linalg.norm(want))
 
 
-@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8])
+# (9 to 16 rows: where the option asks for them)
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8, 9, 12, 13, 16])
+@pytest.mark.parametrize("tiles", [0, 3])
 @pytest.mark.parametrize("k,n", [(64, 16), (528, 100), (2048, 40), (2576, 264)])
-def test_few_rows(m, k, n):
-    """30-bit activations and 64-bit sums: nothing but the rounding of the result to 32 bits is left, 2^-24 a value."""
+def test_few_rows(m, tiles, k, n):
+    """30-bit activations and 64-bit sums: what is left is the rounding of the sum and of the bias added to it, 2^-24 each at most; the f16 kernels are 1.3e-7 to 3e-7 off."""
     rng = np.random.default_rng(m * 1000 + k)
     pw = fastnn_amd.quantize_weights(flib.DT_U8, weights(rng, n, k))
     a = rng.standard_normal((m, k)).astype(np.float32)
     bias = rng.standard_normal(n).astype(np.float32)
     bad = a.copy()
     bad[m - 1, k // 2] = np.nan
+    large = a.copy()
+    large[:, k // 3] = 200.0
     with fastnn_amd.HipContext(0) as ctx:
         h = ctx.register(pw)
         ctx.set_option(flib.OPT_FRAGMENT, -1)
+        ctx.set_option(flib.OPT_STREAM_MAX_M, 0)
+        ctx.set_option(flib.OPT_GEMV_INT8_MAX_M, 16)
+        ctx.set_option(flib.OPT_GEMV_ROW_TILES, tiles)
         want = exact(pw, a, n, k, bias)
-        assert off(ctx.qmatmul(h, a, n, bias=bias), want) < 3e-7
-        got = ctx.qmatmul(h, bad, n, bias=bias)
-        assert np.isnan(got[m - 1]).all() and (m == 1 or off(got[:-1], want[:-1]) < 3e-7)
+        got = ctx.qmatmul(h, a, n, bias=bias)
+        assert off(got, want) < 1.2e-7
+        assert off(ctx.qmatmul(h, large, n, bias=bias), exact(pw, large, n, k, bias)) < 1.2e-7
+        other = ctx.qmatmul(h, bad, n, bias=bias)
+        assert np.isnan(other[m - 1]).all() and np.array_equal(other[:-1], got[:-1])
+        ctx.set_option(flib.OPT_GEMV_INT8, 0)
+        assert not np.array_equal(ctx.qmatmul(h, a, n, bias=bias), got)
         ctx.release(h)
 
 

@@ -30,4 +30,6 @@ def test_the_last_round(dt, waves, tail, m, k, n):
         assert not np.isfinite(got[-1]).any()
         same = (got[:-1] == plain[:-1]).mean()
         assert same > 0.75, same
+        if k >= 300:                     # (K in several parts there: other roundings, so that the cut tiles have run)
+            assert same < 1
         ctx.release(h)
