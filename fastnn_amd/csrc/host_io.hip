@@ -42,6 +42,10 @@ __global__ __launch_bounds__(256) void copy_kernel(const T *__restrict__ src, T 
 }
 
 // Everything before this kernel in the stream is done when it starts; writes to pinned memory are not cached on the device.
+// As a mark it lets another stream's copy begin, with no wait between the two but the host's look at the word.  That holds because a
+// kernel sees what those before it in its stream wrote on any XCD: where each XCD has an L2 of its own, the end of a kernel puts its lines
+// into memory.  The release at system scope hands all that this kernel could see to whoever has seen the word, and the copy is enqueued after that.  A
+// runtime that ended kernels without their release would break this, and the kernel behind as well.
 __global__ void signal_kernel(uint32_t *flag, uint32_t value)
 {
     __hip_atomic_store(flag, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);

@@ -66,9 +66,10 @@ bool plan_stream(bool cb, int max_tiles, int max_mb, int64_t m, int64_t n, int64
                 // drawn calls of 17 to 60 splits take 1.18 times the tiles' time so, 1.57 at most (54 x 15104 x 976 34.6 us there, 54.5 so; 60 x 7296 x 1664 29.4
                 // and 34.6; 56 x 4992 x 2496 25.7 and 29.3), five less (38 x 5120 x 2432 29.9 and 26.1).  17 and more of two rounds are 4 to 10 % ahead.
                 if (mb > 2 && r == 1 && s > 16) continue;
-                // Two row tiles per wave in half as many rounds, each of twice the values, are ahead where those are three and more: 43 x 8448 x 10368 6 rounds against 3,
-                // 53.5 us and 50.8, 39 x 7680 x 15105 8 against 4, 65.0 and 61.0; with 4 against 2 it is 1 % behind, 5 against 3 or 7 against 4 3 to 10 %.
-                if (mb > 2 && r >= 6 && r2 && r >= 2 * r2) break;
+                // Two row tiles per wave in half as many rounds, each of twice the values, are ahead where those are two and more: 43 x 8448 x 10368 6 rounds against 3,
+                // 53.5 us and 50.8, 39 x 7680 x 15105 8 against 4, 65.0 and 61.0; 4 against 2 1 % behind with weights from cache, 4 to 7 % ahead from memory
+                // (43 x 4352 x 12869 44.4 and 41.6).  They are 3 to 10 % behind with 5 against 3 or 7 against 4, 13 % with 2 against 1.
+                if (mb > 2 && r >= 4 && r2 && r >= 2 * r2) break;
                 // Without two row tiles as a plan these calls are the tiles' otherwise, which hold the activations' low halves scaled by 2^11.  So does this form then: unscaled
                 // they are denormals from 2^-18 of a round's largest value on, and beside values of 2^24 on weights of zero a normal row comes out 1.7e-5 of its norm
                 // off, not 1.6e-7 (64 x 3072 x 12288).  Four fused multiply-adds a product of 32 x 16 x 16: 64 x 4096 x 11008 40.8 -> 44.5 us, 64 x 2048 x 11008 25.6 -> 27.4.
@@ -97,7 +98,9 @@ bool stream_plan_for(fnn_hip_ctx *ctx, const fnn_hip_weight *w, const QMatmulArg
     // 16.7-17.2 against 22.1-23.6 us; 4096 -> 1024 I8: 8.7 against 9.5; but 4096 -> 2048: 10.6 against 9.7, left out);
     // from M = 5 only where N <= 2048 and K >= 4 N with K >= 8192 (f16 types: 8192 -> 2048 FP8 12.0-12.2 against
     // 13.0-13.3 us) or K >= 16384 (types of the int8 GEMV, which is the better kernel below that: 16384 -> 1024 I4 13.7
-    // against 20.2-20.8 us, 8192 -> 1024 I4 13.2 against 11.4).  Not when the option was raised above its default.
+    // against 20.2-20.8 us, 8192 -> 1024 I4 13.2 against 11.4).  U8, which has that GEMV too, keeps the f16 types' line: 5 to 8 rows of 8192 to 16384 values over 256
+    // to 2048 columns 9.6 to 19.0 us here and 10.8 to 20.3 there, 8192 and 10240 -> 1024 and 10240 -> 2048 (12.5, 14.3, 14.9 and 11.0, 12.6, 13.0) apart.  Not
+    // when the option was raised above its default.
     const bool int_type = dt == FNN_DT_I8 || dt == FNN_DT_I4 || dt == FNN_DT_U4;
     if (!cb && lo <= 17) {
         // ... and from M = 9 where K leaves the eight waves of the kernel for 9 <= M <= 16 a ragged last round (its waves
