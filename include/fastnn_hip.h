@@ -109,7 +109,7 @@ enum {
     FNN_OPT_TILE_SPLIT = 6,       /* tiled GEMM: K split over this many workgroups; 0 (default) = cost model        */
     FNN_OPT_TILE_STAGES = 7,      /* tiled GEMMs: LDS ring depth where the shape has variants (3..6); 0 (default) = by shape */
     FNN_OPT_TILE_MIN_M = 8,       /* smallest M the tiled GEMM takes (default 5)                                    */
-    FNN_OPT_GEMV_INT8 = 9,        /* 1 (default): M <= 8 with I8 / I4 / U4 weights runs on the int8 matrix cores        */
+    FNN_OPT_GEMV_INT8 = 9,        /* 1 (default): M <= 8 with I8 / U8 / I4 / U4 weights runs on the int8 matrix cores   */
                                   /* (activations as four exact base-256 digit rows, integer sums, no weight decode);  */
                                   /* 0: the f16 GEMV kernel takes them too                                             */
     FNN_OPT_GEMM_INT8 = 10,       /* 1 (default): M >= FNN_OPT_GEMM_INT8_MIN_M with I8 / I4 / U4 weights runs as an int8  */
