@@ -95,8 +95,8 @@ int fnn_row_means(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, cons
 int fnn_mfma_qgemv(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p,
                    int flags, bool *handled);
 
-// M <= 4, integer weights (I8, I4, U4): int8 matrix cores, activations as three exact base-256 digit rows, one
-// workgroup per CU walking the row tiles (no decode arithmetic, activations converted once per workgroup).
+// M <= 8 (16 by option), integer weights (I8, U8, I4, U4): int8 matrix cores, activations as four exact base-256 digit rows per slice of K (no
+// decode arithmetic, activations converted once per workgroup).
 int fnn_i8dot_qgemv(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &p, bool *handled);
 // that copy for the kernels that take rows of whole 64-byte blocks only, null where it does not apply
 int fnn_fragment_blocks(fnn_hip_ctx *ctx, hipStream_t s, const fnn_hip_weight *w, const QMatmulArgs &q, const uint32_t **words_fr, int64_t *kb64);

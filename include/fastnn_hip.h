@@ -177,7 +177,7 @@ enum {
                                   /* M = 5 to 9 for short rows, from M = 9 with aligned ones, as far up as it is the faster form), -1 =  */
                                   /* off, else the shape, (direct << 15) | (K splits << 8) | (16-column blocks << 4) | (16-row       */
                                   /* blocks); a shape that does not exist for the call is ignored;                                  */
-                                  /* (1 << 14) | w, w = 1, 2 or 4: I8, I4, U4 and U8 weights on the large register tiles of three */
+                                  /* (1 << 14) | w, w = 1, 2 or 4: I8, I4 and U4 weights on the large register tiles of three     */
                                   /* digit planes, w waves of a workgroup sharing a tile                                            */
                                   /* (+ 8 t, t = 2 or 4 > w: where the tiles are more than 256, those behind the last whole round  */
                                   /* of 256 as tiles of t waves)                                                                   */
